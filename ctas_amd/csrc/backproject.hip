@@ -2,7 +2,8 @@
 // the fbp kernel of ct.cl:5-44).
 //
 // A 256-thread workgroup owns a tile of output pixels of one slice (64x64,
-// 128x64 or 128x128; each thread a 4x4, 8x4 or 8x8 lattice with stride 16).
+// 128x64 or 128x128; each thread a 4x4, 8x4 or 8x8 lattice with stride 16),
+// or the same tile of two or four slices of one centre.
 // The angles are taken in passes of AC. For each angle of a pass the
 // workgroup stages into LDS the window of the filtered row that the tile can
 // touch (a fixed length L >= the tile's diagonal + margin, placed around the
@@ -447,6 +448,151 @@ __device__ __forceinline__ void bp_tile(const Item &it, int tile, unsigned char 
   store_tile<TR, TC>(it, acc, rowf, colf);
 }
 
+// ---- slices of one geometry: CTAS sampling, float32 storage ------------------
+// Slices of one handle with the same centre share every ray coordinate, so
+// a workgroup reconstructs the same tile of NS of them: the window of an
+// angle holds the NS slices' samples at position k side by side (8 or 16
+// bytes), and one coordinate, one conversion, one address and one LDS read
+// serve NS updates. Each slice sums the same floats in the same order as on
+// its own, so the result is bit for bit that of bp_tile. The items of a
+// group lie back to back.
+template <int NS> struct GroupWord { using type = float4; };
+template <> struct GroupWord<2> { using type = float2; };
+
+template <int KIND, int AC, int NS>
+struct StageGroup {
+  using G = KindGeo<KIND>;
+  using WT = typename GroupWord<NS>::type;
+  static constexpr int L = G::L, TPA = 256 / AC, EPT = (L + TPA - 1) / TPA;
+  static constexpr size_t WIN = sizeof(WT) * AC * L;
+  static constexpr size_t HALFBUF = WIN + sizeof(float4) * AC;
+  static constexpr size_t ANGS = 2 * HALFBUF;
+  static constexpr size_t BYTES = ANGS + 2 * sizeof(float2) * AC;
+  float v[EPT][NS];
+  unsigned ok;  // bit j: element j lies inside the sinograms
+  float4 prm;
+  float2 ang, ang_next;  // table entries of the pass being fetched and of the one after
+
+  __device__ __forceinline__ void load_angle(const Item &it, int a0, int na) {
+    ang_next = ldg(it.sincos, a0 + min(static_cast<int>(threadIdx.x) / TPA, na - 1));
+  }
+  __device__ __forceinline__ void put_angle(unsigned char *lds, int slot, int na) const {
+    const int tid = threadIdx.x, a = tid / TPA;
+    if (a < na && tid - a * TPA == 0) reinterpret_cast<float2 *>(lds + ANGS)[slot * AC + a] = ang_next;
+  }
+  __device__ __forceinline__ void get_angle(const unsigned char *lds, int slot, int na) {
+    ang = reinterpret_cast<const float2 *>(lds + ANGS)[slot * AC + min(static_cast<int>(threadIdx.x) / TPA, na - 1)];
+  }
+  __device__ __forceinline__ void take_loaded() { ang = ang_next; }
+
+  __device__ __forceinline__ void fetch(const Item &it, int a0, int na, float ycm, float xcm) {
+    const int tid = threadIdx.x, a = min(tid / TPA, na - 1), sub = tid - (tid / TPA) * TPA;
+    const int w = it.w, hp = w / 2;
+    const float c = it.center;
+    const float s = ang.x, co = ang.y;
+    const float base = c + ((1.0f - s) - co) * static_cast<float>(hp);
+    const float tc = base + s * ycm + co * xcm;
+    const int lo = static_cast<int>(floorf(tc)) - G::HALF - 2;
+    prm = make_float4(base, s, co, __int_as_float((a * L - lo) * static_cast<int>(sizeof(WT))));
+    // one unsigned comparison: a group's sinograms hold fewer than 2^30 samples
+    const unsigned total = static_cast<unsigned>(it.N) * static_cast<unsigned>(w);
+    const unsigned rb = static_cast<unsigned>((a0 + a) * w + lo);
+    ok = 0;
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) {
+      const unsigned flat = rb + static_cast<unsigned>(sub + j * TPA);
+      const bool in = flat < total;
+      const unsigned at = in ? flat : 0u;
+#pragma unroll
+      for (int n = 0; n < NS; ++n) v[j][n] = ldg32(static_cast<const float *>((&it)[n].filt), at);
+      ok |= static_cast<unsigned>(in) << j;
+    }
+  }
+
+  __device__ __forceinline__ void store(unsigned char *buf, int na) const {
+    const int tid = threadIdx.x, a = tid / TPA, sub = tid - a * TPA;
+    if (a >= na) return;
+    WT *win = reinterpret_cast<WT *>(buf);
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) {
+      const int o = sub + j * TPA;
+      if (o >= L) continue;
+      const bool in = (ok >> j) & 1u;
+      WT q;
+      float *f = reinterpret_cast<float *>(&q);
+#pragma unroll
+      for (int n = 0; n < NS; ++n) f[n] = in ? v[j][n] : 0.0f;
+      win[a * L + o] = q;
+    }
+    if (sub == 0) reinterpret_cast<float4 *>(buf + WIN)[a] = prm;
+  }
+};
+
+// The same output tile of the NS items at it, (&it)[1], ...
+template <int KIND, int AC, int NS>
+__device__ __forceinline__ void bp_tile_group(const Item &it, int tile, unsigned char *lds) {
+  using G = KindGeo<KIND>;
+  using S = StageGroup<KIND, AC, NS>;
+  using WT = typename S::WT;
+  constexpr int TR = G::TR, TC = G::TC, RT = G::RT, CT = G::CT;
+  const float c = it.center;
+  const int ty0 = (tile / it.tiles_x) * RT;
+  const int tx0 = (tile % it.tiles_x) * CT;
+  const int tid = threadIdx.x;
+  const int tx = tid & 15, ty = (tid >> 6) * (4 * TR) + ((tid >> 4) & 3);
+  auto rowf = [&](int r) { return ty0 + ty + 4 * r; };
+  auto colf = [&](int q) { return tx0 + tx + 16 * q; };
+  if (tile_outside<KIND>(it, ty0, tx0)) {
+#pragma unroll
+    for (int n = 0; n < NS; ++n) zero_tile<TR, TC>((&it)[n], rowf, colf);
+    return;
+  }
+  float jc[TR], fi[TC];
+#pragma unroll
+  for (int r = 0; r < TR; ++r) jc[r] = static_cast<float>(rowf(r)) - c;
+#pragma unroll
+  for (int q = 0; q < TC; ++q) fi[q] = static_cast<float>(colf(q));
+  float acc[NS][TR][TC];
+#pragma unroll
+  for (int n = 0; n < NS; ++n)
+#pragma unroll
+    for (int r = 0; r < TR; ++r)
+#pragma unroll
+      for (int q = 0; q < TC; ++q) acc[n][r][q] = 0.0f;
+  const float ycm = static_cast<float>(ty0) + 0.5f * (RT - 1) - c;
+  const float xcm = static_cast<float>(tx0) + 0.5f * (CT - 1);
+  const bool wskip = wave_outside(it, c, ty0 + (tid >> 6) * (4 * TR), 4 * TR, tx0, CT);
+
+  run_passes<S>(it, lds, AC, ycm, xcm, wskip, [&](const unsigned char *buf, int na) {
+    const float4 *prm = reinterpret_cast<const float4 *>(buf + S::WIN);
+#pragma unroll 2
+    for (int a = 0; a < na; ++a) {
+      const float4 p = prm[a];
+      const unsigned char *wb = buf + __float_as_int(p.w);
+      float aj[TR], ci[TC];
+#pragma unroll
+      for (int r = 0; r < TR; ++r) aj[r] = p.x + p.y * jc[r];
+#pragma unroll
+      for (int q = 0; q < TC; ++q) ci[q] = p.z * fi[q];
+#pragma unroll
+      for (int r = 0; r < TR; ++r) {
+        WT vv[TC];
+#pragma unroll
+        for (int q = 0; q < TC; ++q) {
+          const int k = static_cast<int>(aj[r] + ci[q]);
+          vv[q] = *reinterpret_cast<const WT *>(wb + k * static_cast<int>(sizeof(WT)));
+        }
+#pragma unroll
+        for (int q = 0; q < TC; ++q)
+#pragma unroll
+          for (int n = 0; n < NS; ++n) acc[n][r][q] += reinterpret_cast<const float *>(&vv[q])[n];
+      }
+    }
+  });
+#pragma unroll
+  for (int n = 0; n < NS; ++n) store_tile<TR, TC>((&it)[n], acc[n], rowf, colf);
+}
+
 // ---- FP16/BF16 storage, CTAS sampling, row pairs -----------------------------
 // LDS holds, for every window position o, the pair (v[o], v[o+1]) as two
 // floats (converted from the stored 16-bit samples when staged). A lane owns
@@ -725,7 +871,14 @@ struct SlotConsts {
   int loA, loB, ba, bb, ra, rb, exact, unused;
 };
 
-template <int KIND, int AC, int ST>
+// NS slices of one centre (back to back at it, (&it)[1], ...) share their
+// coordinates: a CTAS word holds their samples side by side.
+template <int NS> struct MirrorWord;
+template <> struct MirrorWord<1> { using type = uint32_t; };
+template <> struct MirrorWord<2> { using type = uint2; };
+template <> struct MirrorWord<4> { using type = uint4; };
+
+template <int KIND, int AC, int ST, int NS>
 struct StageMirror {
   using G = KindGeo<KIND>;
   // window of D + 6 positions from floor(centre) - ceil(D/2) - 1: the tile's
@@ -741,14 +894,15 @@ struct StageMirror {
   // 2^-16), zero outside the rows; the CTAS words hold the two 16-bit
   // samples (v_a[k], v_b[k])
   static constexpr bool LIN = ST == ST_F32_LIN || ST == ST_F16_LIN || ST == ST_BF16_LIN;
-  using WordT = typename std::conditional<LIN, float4, uint32_t>::type;
+  using WordT = typename std::conditional<LIN, float4, typename MirrorWord<NS>::type>::type;
+  static_assert(!LIN || NS == 1, "a LINEAR word fills an LDS read");
   static constexpr size_t WIN = sizeof(WordT) * AC * L2;
   static constexpr size_t HALFBUF = WIN + sizeof(int) * AC * TAB;
   static constexpr size_t ANGS = 2 * HALFBUF;
   static constexpr size_t BYTES = ANGS + 2 * sizeof(SlotConsts) * AC;
   static_assert(TR % 4 == 0 && TC % 4 == 0, "16-byte table reads");
   static_assert(AC <= 64, "one lane of the deriving wave per slot");
-  typename std::conditional<LIN, float4, u16x2>::type v[EPT];  // the samples of word j
+  typename std::conditional<LIN, float4, u16x2>::type v[EPT][NS];  // the samples of word j
   int t[TPT];    // SY (rows) and CX (columns) entries of this thread
   SlotConsts k;  // constants of this thread's slot, pass being fetched
   MirrorSlot raw;  // deriving wave: the slot of its lane, pass after next
@@ -829,17 +983,20 @@ struct StageMirror {
         const int i1 = in1 ? kk : 0, i0 = in0 ? kk - 1 : 0;
         const float a0 = sample(k.ra + i0), a1 = sample(k.ra + i1);
         const float b0 = sample(rb + i0), b1 = sample(rb + i1);
-        v[j] = make_float4(in0 ? a0 : 0.0f, in1 ? a1 : 0.0f, (hb && in0) ? b0 : 0.0f, (hb && in1) ? b1 : 0.0f);
+        v[j][0] = make_float4(in0 ? a0 : 0.0f, in1 ? a1 : 0.0f, (hb && in0) ? b0 : 0.0f, (hb && in1) ? b1 : 0.0f);
       }
     } else {
-      const uint16_t *__restrict__ base16 = static_cast<const uint16_t *>(it.filt) - it.pad;
       const int mb = ~(k.rb >> 31);
 #pragma unroll
       for (int j = 0; j < EPT; ++j) {
         const int e = sub + j * TPA;  // word e of the slot: [0, L) window A, [L, 2L) window B
         const int kk = e < L ? window_pos(k.loA + e, k.exact & 1) : window_pos(k.loB + (e - L), k.exact & 2);
-        v[j].x = ldg32(base16, static_cast<unsigned>(k.ra + kk));
-        v[j].y = ldg32(base16, static_cast<unsigned>((k.rb + kk) & mb));
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+          const uint16_t *__restrict__ base16 = static_cast<const uint16_t *>((&it)[n].filt) - it.pad;
+          v[j][n].x = ldg32(base16, static_cast<unsigned>(k.ra + kk));
+          v[j][n].y = ldg32(base16, static_cast<unsigned>((k.rb + kk) & mb));
+        }
       }
     }
   }
@@ -855,15 +1012,23 @@ struct StageMirror {
       if constexpr (LIN) {
         // the differences scaled by 2^-16 (exact), so that the 16-bit
         // fraction of a coordinate weighs them as an integer
-        const float4 q = v[j];
+        const float4 q = v[j][0];
         win[a * L2 + e] = make_float4(q.x, (q.y - q.x) * 0x1p-16f, q.z, (q.w - q.z) * 0x1p-16f);
-      } else if constexpr (ST == ST_BF16_H) {
-        // BF16 -> FP32 (exact) -> FP16, rounded to nearest even
-        const half2v h = {static_cast<_Float16>(__uint_as_float(static_cast<uint32_t>(v[j].x) << 16)),
-                          static_cast<_Float16>(__uint_as_float(static_cast<uint32_t>(v[j].y) << 16))};
-        win[a * L2 + e] = __builtin_bit_cast(uint32_t, h);
       } else {
-        win[a * L2 + e] = __builtin_bit_cast(uint32_t, v[j]);
+        WordT word;
+        uint32_t *part = reinterpret_cast<uint32_t *>(&word);
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+          if constexpr (ST == ST_BF16_H) {
+            // BF16 -> FP32 (exact) -> FP16, rounded to nearest even
+            const half2v h = {static_cast<_Float16>(__uint_as_float(static_cast<uint32_t>(v[j][n].x) << 16)),
+                              static_cast<_Float16>(__uint_as_float(static_cast<uint32_t>(v[j][n].y) << 16))};
+            part[n] = __builtin_bit_cast(uint32_t, h);
+          } else {
+            part[n] = __builtin_bit_cast(uint32_t, v[j][n]);
+          }
+        }
+        win[a * L2 + e] = word;
       }
     }
     // word addresses are taken from the start of the LDS block
@@ -923,10 +1088,11 @@ __device__ __forceinline__ void run_passes_mirror(const Item &it, unsigned char 
   }
 }
 
-template <int KIND, int AC, int ST>
+template <int KIND, int AC, int ST, int NS>
 __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigned char *lds) {
   using G = KindGeo<KIND>;
-  using S = StageMirror<KIND, AC, ST>;
+  using S = StageMirror<KIND, AC, ST, NS>;
+  using WordT = typename S::WordT;
   constexpr int TR = G::TR, TC = G::TC, RT = G::RT, CT = G::CT;
   const float c = it.center;
   const int w = it.w, hp = w / 2;
@@ -944,15 +1110,20 @@ __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigne
     return col == hp ? w : 2 * hp - col;
   };
   if (tile_outside<KIND>(it, ty0, tx0) && tile_outside<KIND>(it, ty0, mx0)) {
-    zero_tile<TR, TC>(it, rowf, colf);
-    zero_tile<TR, TC>(it, rowf, colm);
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+      zero_tile<TR, TC>((&it)[n], rowf, colf);
+      zero_tile<TR, TC>((&it)[n], rowf, colm);
+    }
     return;
   }
-  float acc[TR][TC], accm[TR][TC];
+  float acc[NS][TR][TC], accm[NS][TR][TC];
 #pragma unroll
-  for (int r = 0; r < TR; ++r)
+  for (int n = 0; n < NS; ++n)
 #pragma unroll
-    for (int q = 0; q < TC; ++q) acc[r][q] = accm[r][q] = 0.0f;
+    for (int r = 0; r < TR; ++r)
+#pragma unroll
+      for (int q = 0; q < TC; ++q) acc[n][r][q] = accm[n][r][q] = 0.0f;
   const int wr0 = ty0 + (tid >> 6) * (4 * TR);
   const bool wskip = wave_outside(it, c, wr0, 4 * TR, tx0, CT) && wave_outside(it, c, wr0, 4 * TR, mx0, CT);
   // this lane's entries in the tables
@@ -977,16 +1148,17 @@ __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigne
       }
     };
     // the words of both windows for the pixel pairs of row r
-    auto words = [&](const int (&A)[TR], const int (&B)[TR], const int (&Cq)[TC], int r, uint32_t (&WA)[TC],
-                     uint32_t (&WB)[TC]) {
+    auto words = [&](const int (&A)[TR], const int (&B)[TR], const int (&Cq)[TC], int r, WordT (&WA)[TC],
+                     WordT (&WB)[TC]) {
 #pragma unroll
       for (int q = 0; q < TC; ++q) {
         const unsigned ua = static_cast<unsigned>(A[r] + Cq[q]);
         const unsigned ub = static_cast<unsigned>(B[r] - Cq[q]);
-        WA[q] = *reinterpret_cast<const uint32_t *>(lds0 + ((ua >> 16) << 2));
-        WB[q] = *reinterpret_cast<const uint32_t *>(lds0 + ((ub >> 16) << 2));
+        WA[q] = *reinterpret_cast<const WordT *>(lds0 + (ua >> 16) * sizeof(WordT));
+        WB[q] = *reinterpret_cast<const WordT *>(lds0 + (ub >> 16) * sizeof(WordT));
       }
     };
+    auto part = [](const WordT &w, int n) { return reinterpret_cast<const uint32_t *>(&w)[n]; };
     if constexpr (S::LIN) {
       // LINEAR: the word of window A at t_a(p) and of window B at t_a(p')
       // carry both angles' samples and differences; with their 16-bit
@@ -1011,10 +1183,11 @@ __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigne
           }
 #pragma unroll
           for (int q = 0; q < TC; ++q) {
-            acc[r][q] = fmaf(FA[q], WA[q].y, acc[r][q] + WA[q].x);
-            acc[r][q] = fmaf(FB[q], WB[q].w, acc[r][q] + WB[q].z);
-            accm[r][q] = fmaf(FB[q], WB[q].y, accm[r][q] + WB[q].x);
-            accm[r][q] = fmaf(FA[q], WA[q].w, accm[r][q] + WA[q].z);
+            float &p = acc[0][r][q], &pm = accm[0][r][q];
+            p = fmaf(FA[q], WA[q].y, p + WA[q].x);
+            p = fmaf(FB[q], WB[q].w, p + WB[q].z);
+            pm = fmaf(FB[q], WB[q].y, pm + WB[q].x);
+            pm = fmaf(FA[q], WA[q].w, pm + WA[q].z);
           }
         }
       }
@@ -1037,14 +1210,28 @@ __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigne
         terms(a + 1, A1, B1, C1);
 #pragma unroll
         for (int r = 0; r < TR; ++r) {
-          uint32_t WA0[TC], WB0[TC], WA1[TC], WB1[TC];
+          WordT WA0[TC], WB0[TC], WA1[TC], WB1[TC];
           words(A0, B0, C0, r, WA0, WB0);
           words(A1, B1, C1, r, WA1, WB1);
 #pragma unroll
-          for (int q = 0; q < TC; ++q) {
-            const half2v sum = pair_sum(WA0[q], WB0[q]) + pair_sum(WA1[q], WB1[q]);
-            acc[r][q] = __builtin_amdgcn_fdot2(sum, lo, acc[r][q], false);
-            accm[r][q] = __builtin_amdgcn_fdot2(sum, hi, accm[r][q], false);
+          for (int q = 0; q < TC; ++q)
+#pragma unroll
+            for (int n = 0; n < NS; ++n) {
+              const half2v sum = pair_sum(part(WA0[q], n), part(WB0[q], n)) + pair_sum(part(WA1[q], n), part(WB1[q], n));
+              acc[n][r][q] = __builtin_amdgcn_fdot2(sum, lo, acc[n][r][q], false);
+              accm[n][r][q] = __builtin_amdgcn_fdot2(sum, hi, accm[n][r][q], false);
+            }
+        }
+        if constexpr (NS == 4) {
+          // the 12 reads of the terms and the words of the first two pixel
+          // pairs, then a pixel pair's 28 VALU instructions per four reads:
+          // two waves per SIMD need the reads spread out (7.51 -> 7.24 ms
+          // for 32 slices of 2048 px x 1800 angles)
+          __builtin_amdgcn_sched_group_barrier(0x100, 12 + 8, 0);
+#pragma unroll
+          for (int i = 0; i < TR * TC; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x2, 28, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
           }
         }
       }
@@ -1053,14 +1240,16 @@ __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigne
         terms(a, A, B, Cq);
 #pragma unroll
         for (int r = 0; r < TR; ++r) {
-          uint32_t WA[TC], WB[TC];
+          WordT WA[TC], WB[TC];
           words(A, B, Cq, r, WA, WB);
 #pragma unroll
-          for (int q = 0; q < TC; ++q) {
-            const half2v sum = pair_sum(WA[q], WB[q]);
-            acc[r][q] = __builtin_amdgcn_fdot2(sum, lo, acc[r][q], false);
-            accm[r][q] = __builtin_amdgcn_fdot2(sum, hi, accm[r][q], false);
-          }
+          for (int q = 0; q < TC; ++q)
+#pragma unroll
+            for (int n = 0; n < NS; ++n) {
+              const half2v sum = pair_sum(part(WA[q], n), part(WB[q], n));
+              acc[n][r][q] = __builtin_amdgcn_fdot2(sum, lo, acc[n][r][q], false);
+              accm[n][r][q] = __builtin_amdgcn_fdot2(sum, hi, accm[n][r][q], false);
+            }
         }
       }
     } else {
@@ -1070,25 +1259,31 @@ __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigne
         terms(a, A, B, Cq);
 #pragma unroll
         for (int r = 0; r < TR; ++r) {
-          uint32_t WA[TC], WB[TC];
+          WordT WA[TC], WB[TC];
           words(A, B, Cq, r, WA, WB);
 #pragma unroll
-          for (int q = 0; q < TC; ++q) {
-            // the pixel's two samples (lo WA, hi WB) and the mirror pixel's
-            // (lo WB, hi WA), merged by bit-field inserts (the asm keeps them
-            // 32-bit merges) and each added by one dot2
-            uint32_t X = (WA[q] & 0xFFFFu) | (WB[q] & 0xFFFF0000u);
-            uint32_t Y = (WB[q] & 0xFFFFu) | (WA[q] & 0xFFFF0000u);
-            asm("" : "+v"(X), "+v"(Y));
-            acc[r][q] = add_pair<ST>(acc[r][q], X);
-            accm[r][q] = add_pair<ST>(accm[r][q], Y);
-          }
+          for (int q = 0; q < TC; ++q)
+#pragma unroll
+            for (int n = 0; n < NS; ++n) {
+              // the pixel's two samples (lo WA, hi WB) and the mirror pixel's
+              // (lo WB, hi WA), merged by bit-field inserts (the asm keeps them
+              // 32-bit merges) and each added by one dot2
+              const uint32_t wa = part(WA[q], n), wb = part(WB[q], n);
+              uint32_t X = (wa & 0xFFFFu) | (wb & 0xFFFF0000u);
+              uint32_t Y = (wb & 0xFFFFu) | (wa & 0xFFFF0000u);
+              asm("" : "+v"(X), "+v"(Y));
+              acc[n][r][q] = add_pair<ST>(acc[n][r][q], X);
+              accm[n][r][q] = add_pair<ST>(accm[n][r][q], Y);
+            }
         }
       }
     }
   });
-  store_tile<TR, TC>(it, acc, rowf, colf);
-  store_tile<TR, TC>(it, accm, rowf, colm);
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    store_tile<TR, TC>((&it)[n], acc[n], rowf, colf);
+    store_tile<TR, TC>((&it)[n], accm[n], rowf, colm);
+  }
 }
 
 // Grid-mapped launch: one workgroup per tile; blocks are remapped so that the
@@ -1139,12 +1334,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grid_waves<
 // Mirrored launch: AC slots (2 AC angles) per pass.
 template <int KIND, int AC, int ST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KindGeo<KIND>::WAVES, KindGeo<KIND>::WAVES))) void bp_mirror_kernel(const Item *__restrict__ items, int n_items) {
-  __shared__ __align__(16) unsigned char lds[StageMirror<KIND, AC, ST>::BYTES];
+  __shared__ __align__(16) unsigned char lds[StageMirror<KIND, AC, ST, 1>::BYTES];
   int b = blockIdx.x;
   const int q = gridDim.x >> 3;
   if (b < (q << 3)) b = (b & 7) * q + (b >> 3);
   const Item &it = items[find_item_by_tile(items, n_items, b)];
-  bp_tile_mirror<KIND, AC, ST>(it, b - it.tile_base, lds);
+  bp_tile_mirror<KIND, AC, ST, 1>(it, b - it.tile_base, lds);
+}
+
+// Launches of n_groups x NS slices, `tiles` tiles each: the workgroups of a
+// group come one after another, as a slice's do above. The samples of four
+// slices make 16-byte words, which the LDS gathers at 211 B/clk per CU
+// against 125 for 4- and 8-byte words, so two slices save VALU work only.
+// 32 slices of 2048 px x 1800 angles, one launch (one, two, four slices per
+// workgroup): FP32 17.5, 11.2, 9.3 ms (7.9 ms on a sinogram of zeros: with
+// four slices the chip lowers its clock from 2.4 to 2.0 GHz, and eight
+// slices, 8.9 ms, spend their gain on it); FP16 mirrored 10.0, 8.2, 7.2 ms.
+// LINEAR stays at one slice per workgroup: its 16-byte words leave the LDS
+// nothing to gain (18.5 ms against 18.3 with two).
+template <int NS> struct GroupShape;
+template <> struct GroupShape<2> { static constexpr int AC = 32, WAVES = 3, MIRROR_WAVES = 3; };
+template <> struct GroupShape<4> { static constexpr int AC = 16, WAVES = 3, MIRROR_WAVES = 2; };
+
+template <int NS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GroupShape<NS>::WAVES, GroupShape<NS>::WAVES))) void bp_group_kernel(const Item *__restrict__ items, int tiles) {
+  __shared__ __align__(16) unsigned char lds[StageGroup<TK_64x64, GroupShape<NS>::AC, NS>::BYTES];
+  int b = blockIdx.x;
+  const int q = gridDim.x >> 3;
+  if (b < (q << 3)) b = (b & 7) * q + (b >> 3);
+  const int g = b / tiles;
+  bp_tile_group<TK_64x64, GroupShape<NS>::AC, NS>(items[g * NS], b - g * tiles, lds);
+}
+
+template <int ST, int NS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GroupShape<NS>::MIRROR_WAVES, GroupShape<NS>::MIRROR_WAVES))) void bp_group_mirror_kernel(const Item *__restrict__ items, int tiles) {
+  __shared__ __align__(16) unsigned char lds[StageMirror<TK_64x64, 8, ST, NS>::BYTES];
+  int b = blockIdx.x;
+  const int q = gridDim.x >> 3;
+  if (b < (q << 3)) b = (b & 7) * q + (b >> 3);
+  const int g = b / tiles;
+  bp_tile_mirror<TK_64x64, 8, ST, NS>(items[g * NS], b - g * tiles, lds);
 }
 
 __global__ void reset_counter_kernel(unsigned *counter) { *counter = 0u; }
@@ -1185,9 +1414,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grid_waves<
 template <int KIND, int AC, int ST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KindGeo<KIND>::WAVES, KindGeo<KIND>::WAVES))) void bp_persistent_mirror_kernel(const Item *__restrict__ items, int n_items,
                                                                         int total_tiles, unsigned *counter) {
-  __shared__ __align__(16) unsigned char lds[StageMirror<KIND, AC, ST>::BYTES];
+  __shared__ __align__(16) unsigned char lds[StageMirror<KIND, AC, ST, 1>::BYTES];
   persistent_loop(items, n_items, total_tiles, counter,
-                  [&](const Item &it, int tile) { bp_tile_mirror<KIND, AC, ST>(it, tile, lds); });
+                  [&](const Item &it, int tile) { bp_tile_mirror<KIND, AC, ST, 1>(it, tile, lds); });
 }
 
 // Workgroups of a persistent launch: as many as the CUs hold at once, by the
@@ -1222,7 +1451,7 @@ hipError_t launch_persist_k(const Item *d_items, int n_items, int total_tiles, i
   if (mirror && mode == MODE_LINEAR) {
     // 64x64 tiles only (the 16-byte float words of both windows at 4 slots)
     if constexpr (KIND == TK_64x64) {
-      const int g = resident_workgroups(cus, KindGeo<KIND>::WAVES, StageMirror<KIND, 4, ST_F32_LIN>::BYTES);
+      const int g = resident_workgroups(cus, KindGeo<KIND>::WAVES, StageMirror<KIND, 4, ST_F32_LIN, 1>::BYTES);
       switch (store) {
         case ST_F32: hipLaunchKernelGGL((bp_persistent_mirror_kernel<KIND, 4, ST_F32_LIN>), dim3(g), dim3(256), 0, s, d_items, n_items, total_tiles, counter); break;
         case ST_F16: hipLaunchKernelGGL((bp_persistent_mirror_kernel<KIND, 4, ST_F16_LIN>), dim3(g), dim3(256), 0, s, d_items, n_items, total_tiles, counter); break;
@@ -1234,7 +1463,7 @@ hipError_t launch_persist_k(const Item *d_items, int n_items, int total_tiles, i
     }
   }
   if (mirror) {
-    const int g = resident_workgroups(cus, KindGeo<KIND>::WAVES, StageMirror<KIND, 8, ST_F16>::BYTES);
+    const int g = resident_workgroups(cus, KindGeo<KIND>::WAVES, StageMirror<KIND, 8, ST_F16, 1>::BYTES);
     if (store == ST_F16)
       hipLaunchKernelGGL((bp_persistent_mirror_kernel<KIND, 8, ST_F16>), dim3(g), dim3(256), 0, s, d_items, n_items,
                          total_tiles, counter);
@@ -1311,6 +1540,36 @@ hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles,
     case TK_64x64: return launch_k<TK_64x64>(d_items, n_items, total_tiles, angles_per_pass, mode, store, mirror, s);
     case TK_128x64: return launch_k<TK_128x64>(d_items, n_items, total_tiles, angles_per_pass, mode, store, mirror, s);
     default: return launch_k<TK_128x128>(d_items, n_items, total_tiles, angles_per_pass, mode, store, mirror, s);
+  }
+}
+
+namespace {
+
+template <int NS>
+hipError_t launch_group(const Item *d_items, int n_groups, int tiles, int store, bool mirror, hipStream_t s) {
+  const dim3 grid(n_groups * tiles), block(256);
+  if (!mirror) {
+    hipLaunchKernelGGL((bp_group_kernel<NS>), grid, block, 0, s, d_items, tiles);
+    return hipGetLastError();
+  }
+  switch (store) {
+    case ST_F16: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_F16, NS>), grid, block, 0, s, d_items, tiles); break;
+    case ST_BF16_H: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_BF16_H, NS>), grid, block, 0, s, d_items, tiles); break;
+    default: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_BF16, NS>), grid, block, 0, s, d_items, tiles); break;
+  }
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_backproject_groups(const Item *d_items, int n_groups, int group, int tiles, int store, bool mirror,
+                                     hipStream_t s) {
+  if (n_groups <= 0) return hipSuccess;
+  if (mirror ? store == ST_F32 : store != ST_F32) return hipErrorInvalidValue;
+  switch (group) {
+    case 2: return launch_group<2>(d_items, n_groups, tiles, store, mirror, s);
+    case 4: return launch_group<4>(d_items, n_groups, tiles, store, mirror, s);
+    default: return hipErrorInvalidValue;
   }
 }
 

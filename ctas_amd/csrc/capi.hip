@@ -13,6 +13,7 @@
 #include <condition_variable>
 #include <functional>
 #include <mutex>
+#include <numeric>
 #include <string>
 #include <thread>
 #include <tuple>
@@ -216,6 +217,80 @@ Item base_item(const ctas_fbp *h, int kind, bool mirror) {
   return it;
 }
 
+// One backprojection launch: `items` items from `first`, `group` slices per
+// workgroup, on tiles of `kind`.
+struct BpLaunch {
+  int first, items, group, kind;
+};
+
+// The launches that backproject S slices, and the order in which the item
+// table holds them (slices of a group lie back to back).
+//
+// Slices of one centre share their ray coordinates, so CTAS sampling of
+// float32 storage, and of 16-bit storage through mirrored angle pairs, takes
+// four or two of them per workgroup on 64x64 tiles, where that leaves enough
+// workgroups. Measured for 1 to 8 slices of 512 to 4096 px on 256 CUs, four
+// win from 448 workgroups (float32; 484 of 1400 px 445 us against 570 with
+// two and 768 alone, 288 of 768 px 274 against 258 and 353) and 484 (16-bit;
+// 544 of 2048 px 1111 us against 1387 and 1430, 288 of 1024 px 559 against
+// 513 and 454), two from 288 (float32; 183 us against 234, 256 workgroups 272
+// against 264) and 726 (16-bit; 571 us against 717, 576 workgroups 513
+// against 454). What remains is taken one by one. A tile kind
+// that the caller set is kept, for every slice.
+std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *centers, int S, std::vector<int> *order) {
+  order->resize(S);
+  std::iota(order->begin(), order->end(), 0);
+  const int kind = choose_kind(h);
+  const bool f32 = store_of(h->flags) == ST_F32, mirror = use_mirror(h);
+  if (h->tile_kind != TK_AUTO || mode_of(h->flags) != MODE_CTAS || (!f32 && !mirror) ||
+      static_cast<long long>(h->N) * h->w >= (1LL << 30))
+    return {{0, S, 1, kind}};
+  const long long rows = (h->w + 63) / 64, cols = mirror ? (h->w / 2 + 64) / 64 : rows;
+  const long long tiles = rows * cols, cus = h->cus;
+  const long long four = (mirror ? 15 : 14) * cus / 8, two = (mirror ? 20 : 9) * cus / 8;
+  std::map<uint32_t, std::vector<int>> by_centre;
+  for (int i = 0; i < S; ++i) {
+    uint32_t bits;
+    std::memcpy(&bits, centers + i, sizeof bits);
+    by_centre[bits].push_back(i);
+  }
+  std::vector<BpLaunch> launches;
+  std::vector<int> at;
+  for (const int group : {4, 2}) {
+    long long n = 0;
+    for (const auto &c : by_centre) n += static_cast<long long>(c.second.size()) / group;
+    if (n * tiles < (group == 4 ? four : two)) continue;
+    const int first = static_cast<int>(at.size());
+    for (auto &c : by_centre) {
+      const size_t take = c.second.size() / group * group;
+      at.insert(at.end(), c.second.begin(), c.second.begin() + take);
+      c.second.erase(c.second.begin(), c.second.begin() + take);
+    }
+    launches.push_back({first, static_cast<int>(at.size()) - first, group, TK_64x64});
+  }
+  if (launches.empty()) return {{0, S, 1, kind}};
+  const int first = static_cast<int>(at.size());
+  for (const auto &c : by_centre) at.insert(at.end(), c.second.begin(), c.second.end());
+  if (first < S) launches.push_back({first, S - first, 1, kind});
+  *order = at;
+  return launches;
+}
+
+int launch_planned(const ctas_fbp *h, const std::vector<BpLaunch> &launches, hipStream_t s) {
+  const std::vector<Item> &items = extra(h).resident;
+  for (const BpLaunch &l : launches) {
+    const int tiles = items[l.first].tiles, mode = mode_of(h->flags);
+    const bool mirror = use_mirror(h, l.kind);
+    const int st = bp_store(store_of(h->flags), h->contrast, mirror);
+    if (l.group > 1)
+      CTAS_HIP_TRY(launch_backproject_groups(h->d_items + l.first, l.items / l.group, l.group, tiles, st, mirror, s));
+    else
+      CTAS_HIP_TRY(launch_backproject(h->d_items + l.first, l.items, tiles * l.items, l.kind, choose_ac(h), mode, st,
+                                      mirror, s));
+  }
+  return CTAS_OK;
+}
+
 hipStream_t pick_stream(const ctas_fbp *h, void *stream) {
   return stream ? static_cast<hipStream_t>(stream) : h->stream;
 }
@@ -248,31 +323,34 @@ int enqueue_slices(ctas_fbp *h, const float *d_sino, float *d_out, float *d_f32,
   const size_t stride = slice_elems + 2 * static_cast<size_t>(pad);
   if (int rc = grow(h->d_filt, h->filt_cap, stride * S * store_bytes(st))) return rc;
   if (int rc = ensure_slices(h, S)) return rc;
-  const int kind = choose_kind(h);
-  const bool mirror = use_mirror(h, kind);
+  std::vector<int> order(S);
+  std::iota(order.begin(), order.end(), 0);
+  std::vector<BpLaunch> launches{{0, S, 1, choose_kind(h)}};
+  if (do_bp) launches = plan_backprojection(h, centers, S, &order);
   const int pairs = (h->N + 1) / 2;
   std::vector<Item> items(S);
-  for (int i = 0; i < S; ++i) {
-    Item it = base_item(h, kind, mirror);
-    it.sino = d_sino + slice_elems * i;
-    it.filt = static_cast<unsigned char *>(h->d_filt) + (stride * i + pad) * store_bytes(st);
-    it.pad = pad;
-    it.filt_f32 = d_f32 ? d_f32 + slice_elems * i : nullptr;
-    it.out = d_out ? d_out + static_cast<size_t>(h->w) * h->w * i : nullptr;
-    it.minmax = h->d_minmax + static_cast<size_t>(kMinMaxStride) * i;
-    it.status = h->d_status + i;
-    it.center = do_bp ? centers[i] : 0.0f;
-    it.tile_base = it.tiles * i;
-    it.pair_base = pairs * i;
-    items[i] = it;
-  }
+  for (const BpLaunch &l : launches)
+    for (int k = l.first; k < l.first + l.items; ++k) {
+      const int i = order[k];
+      Item it = base_item(h, l.kind, use_mirror(h, l.kind));
+      it.sino = d_sino + slice_elems * i;
+      it.filt = static_cast<unsigned char *>(h->d_filt) + (stride * i + pad) * store_bytes(st);
+      it.pad = pad;
+      it.filt_f32 = d_f32 ? d_f32 + slice_elems * i : nullptr;
+      it.out = d_out ? d_out + static_cast<size_t>(h->w) * h->w * i : nullptr;
+      it.minmax = h->d_minmax + static_cast<size_t>(kMinMaxStride) * i;
+      it.status = h->d_status + i;
+      it.center = do_bp ? centers[i] : 0.0f;
+      it.tile_base = it.tiles * (k - l.first);
+      it.pair_base = pairs * k;
+      items[k] = it;
+    }
   bool changed = false;
   if (int rc = upload_items(h, items, s, &changed, extra(h).resident)) return rc;
   if (pad) CTAS_HIP_TRY(launch_pad_zero(h->d_items, S, s));
   CTAS_HIP_TRY(launch_filter(h->d_items, S, pairs * S, h->logZ, h->logZ, h->contrast, st, s));
   if (do_bp)
-    CTAS_HIP_TRY(launch_backproject(h->d_items, S, items[0].tiles * S, kind, choose_ac(h),
-                                    mode_of(h->flags), bp_store(st, h->contrast, mirror), mirror, s));
+    if (int rc = launch_planned(h, launches, s)) return rc;
   h->last_S = S;
   return CTAS_OK;
 }
@@ -288,27 +366,27 @@ int enqueue_repeat(ctas_fbp *h, int slice, float *d_out, const float *centers, i
   for (int i = 0; i < n; ++i)
     if (int rc = check_center(h->w, centers[i])) return rc;
   const int st = store_of(h->flags);
-  const int kind = choose_kind(h);
-  const bool mirror = use_mirror(h, kind);
+  std::vector<int> order;
+  const std::vector<BpLaunch> launches = plan_backprojection(h, centers, n, &order);
   const size_t slice_elems = static_cast<size_t>(h->N) * h->w;
   const int pad = filt_pad_of(h);
   const size_t stride = slice_elems + 2 * static_cast<size_t>(pad);
   std::vector<Item> items(n);
-  for (int i = 0; i < n; ++i) {
-    Item it = base_item(h, kind, mirror);
-    it.filt = static_cast<unsigned char *>(h->d_filt) + (stride * (per_slice ? i : slice) + pad) * store_bytes(st);
-    it.pad = pad;
-    it.out = d_out + static_cast<size_t>(h->w) * h->w * i;
-    it.center = centers[i];
-    it.tile_base = it.tiles * i;
-    it.pair_base = 0;
-    items[i] = it;
-  }
+  for (const BpLaunch &l : launches)
+    for (int k = l.first; k < l.first + l.items; ++k) {
+      const int i = order[k];
+      Item it = base_item(h, l.kind, use_mirror(h, l.kind));
+      it.filt = static_cast<unsigned char *>(h->d_filt) + (stride * (per_slice ? i : slice) + pad) * store_bytes(st);
+      it.pad = pad;
+      it.out = d_out + static_cast<size_t>(h->w) * h->w * i;
+      it.center = centers[i];
+      it.tile_base = it.tiles * (k - l.first);
+      it.pair_base = 0;
+      items[k] = it;
+    }
   bool changed = false;
   if (int rc = upload_items(h, items, s, &changed, extra(h).resident)) return rc;
-  CTAS_HIP_TRY(launch_backproject(h->d_items, n, items[0].tiles * n, kind, choose_ac(h),
-                                  mode_of(h->flags), bp_store(st, h->contrast, mirror), mirror, s));
-  return CTAS_OK;
+  return launch_planned(h, launches, s);
 }
 
 // The status words carry deAbs (ABS contrast) and the FP16 range check (FP16
@@ -555,6 +633,7 @@ int ctas_fbp_create(ctas_fbp **ph, int w, int n_angles, int contrast, int filter
   while ((1 << h->logZ) < h->Z) ++h->logZ;
   hipDeviceProp_t prop;
   CTAS_HIP_TRY(hipGetDeviceProperties(&prop, h->device));
+  h->cus = std::max(prop.multiProcessorCount, 1);
   if (sizeof(float2) * static_cast<size_t>(h->Z) > prop.sharedMemPerBlock)
     return fail(CTAS_E_ARG, "width " + std::to_string(w) + " needs a padded line of " +
                                 std::to_string(h->Z) + " points, more than one workgroup's LDS holds");

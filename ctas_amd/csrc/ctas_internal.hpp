@@ -178,6 +178,11 @@ hipError_t launch_filter(const Item *d_items, int n_items, int total_pairs, int 
 // their tiles cover the columns up to w/2 together with the mirrored ones.
 hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles, int kind,
                               int angles_per_pass, int mode, int store, bool mirror, hipStream_t s);
+// CTAS sampling of n_groups groups of `group` (2 or 4) slices of one shape
+// and centre that lie back to back in d_items, on 64x64 tiles (`tiles` per
+// slice): float32 storage, or 16-bit storage through mirrored angle pairs.
+hipError_t launch_backproject_groups(const Item *d_items, int n_groups, int group, int tiles, int store, bool mirror,
+                                     hipStream_t s);
 // Same, one persistent launch with a work counter over the tiles of items of
 // one tile kind and pass length (widths and angle counts may differ); mirror:
 // FP16/BF16 items whose angles pair up (Item::slots). cus: compute units.
@@ -242,6 +247,7 @@ struct NullStreamJoin {
 // Handle (CTrec state). Defined here so that the C ABI units share it.
 struct ctas_fbp {
   int device = 0;
+  int cus = 1;  // compute units of the device
   int w = 0, N = 0, Z = 0, logZ = 0;
   int contrast = 0, filter = 0, flags = 0;
   float fparam = 0.f, anarc = 180.f;

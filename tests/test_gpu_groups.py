@@ -1,0 +1,77 @@
+"""Slices taken together by one workgroup, and launches on small tiles: bit
+for bit the slices of the one-slice kernel on 64x64 tiles, which the parity
+tests hold against the oracle. The same additions in the same order leave no
+room for a tolerance."""
+import numpy as np
+import pytest
+
+import ctas_amd as ca
+
+pytestmark = pytest.mark.gpu
+
+
+def _sinos(torch, S, N, w, contrast, seed):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    x = torch.rand((S, N, w), generator=g, device="cuda")
+    return 0.2 + 0.8 * x if contrast == ca.ABS else x - 0.4
+
+
+def _both(torch, w, N, centers, contrast, arc, store, seed=1):
+    """Slices by the handle's own choice of launches and by the one-slice
+    kernel, each also from the kept filtered sinograms."""
+    S = len(centers)
+    sino = _sinos(torch, S, N, w, contrast, seed)
+    out = []
+    for kind in (ca.TILE_AUTO, ca.TILE_64x64):
+        rec = ca.CTrec(w, N, contrast, "HANN", anarc=arc, store=store)
+        rec.set_tiles(kind, 0)
+        a = torch.full((S, w, w), np.nan, device="cuda")
+        b = torch.full((S, w, w), np.nan, device="cuda")
+        rec.reconstruct_dev(sino, a, centers)
+        rec.backproject_dev(b, centers)
+        torch.cuda.synchronize()
+        out += [a, b]
+    return out
+
+
+# 1400 px: 484 tiles a slice (242 mirrored), so four slices make a group from
+# one float32 or two 16-bit groups on, and two from one float32 or three
+# 16-bit pairs; centres repeat out of order and leave single slices.
+@pytest.mark.parametrize("store,contrast,centers", [
+    (ca.STORE_FP32, ca.ABS, [1.5, -2.25, 1.5, 1.5, -2.25, 1.5, 1.5, 0.0, 1.5, 1.5]),
+    (ca.STORE_FP32, ca.PHS, [-7.0] * 4),
+    (ca.STORE_FP32, ca.REF, [3.37] * 2),
+    (ca.STORE_FP16, ca.ABS, [1.5, -2.25] * 5),
+    (ca.STORE_FP16, ca.FLT, [3.0, 3.0, -4.5, 6.25, -4.5, 6.25]),
+    (ca.STORE_BF16, ca.ABS, [0.75] * 9),
+    (ca.STORE_BF16, ca.PHS, [-3.37] * 8),
+    (ca.STORE_BF16, ca.PHS, [2.0, 2.0, -4.5, 6.25, -4.5, 6.25, 1.0]),
+])
+@pytest.mark.parametrize("N,arc", [(37, 180.0), (50, 360.0)])
+def test_groups_equal_single_slices(torch_cuda, store, contrast, centers, N, arc):
+    torch = torch_cuda
+    auto, auto_kept, single, single_kept = _both(torch, 1400, N, centers, contrast, arc, store)
+    assert torch.equal(single, single_kept)
+    assert torch.equal(auto, single) and torch.equal(auto_kept, single)
+
+
+def test_groups_in_graph_replays(torch_cuda):
+    """The captured launches follow the data of each replay."""
+    torch = torch_cuda
+    w, N, centers = 1400, 40, [2.5] * 6
+    rec = ca.CTrec(w, N, ca.ABS, "RAMP")
+    one = rec.clone()
+    one.set_tiles(ca.TILE_64x64, 0)
+    sino = _sinos(torch, 6, N, w, ca.ABS, 0)
+    out, want = (torch.empty((6, w, w), device="cuda") for _ in range(2))
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    rec.graph_capture(sino, out, centers, stream)
+    for k in range(3):
+        sino.copy_(_sinos(torch, 6, N, w, ca.ABS, k))
+        one.reconstruct_dev(sino, want, centers)
+        torch.cuda.synchronize()
+        rec.graph_launch(stream)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
