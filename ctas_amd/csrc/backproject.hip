@@ -2,8 +2,9 @@
 // the fbp kernel of ct.cl:5-44).
 //
 // A 256-thread workgroup owns a tile of output pixels of one slice (64x64,
-// 128x64 or 128x128; each thread a 4x4, 8x4 or 8x8 lattice with stride 16),
-// or the same tile of two or four slices of one centre.
+// 128x64 or 128x128; each thread a 4x4, 8x4 or 8x8 lattice with stride 16;
+// 32x32 and 16x32 in launches of few tiles), or the same tile of two or four
+// slices of one centre.
 // The angles are taken in passes of AC. For each angle of a pass the
 // workgroup stages into LDS the window of the filtered row that the tile can
 // touch (a fixed length L >= the tile's diagonal + margin, placed around the
@@ -58,6 +59,8 @@ struct Geo {
 // Waves per SIMD the register budget of each tile kind is sized for.
 template <int KIND> struct KindGeo;
 template <> struct KindGeo<TK_64x64> : Geo<4, 4> { static constexpr int WAVES = 4; };
+template <> struct KindGeo<TK_32x32> : Geo<2, 2> { static constexpr int WAVES = 4; };
+template <> struct KindGeo<TK_16x32> : Geo<1, 2> { static constexpr int WAVES = 4; };
 template <> struct KindGeo<TK_128x64> : Geo<8, 4> { static constexpr int WAVES = 3; };
 template <> struct KindGeo<TK_128x128> : Geo<8, 8> { static constexpr int WAVES = 2; };
 
@@ -401,7 +404,9 @@ __device__ __forceinline__ void bp_tile(const Item &it, int tile, unsigned char 
 
   run_passes<S>(it, lds, AC, ycm, xcm, wskip, [&](const unsigned char *buf, int na) {
     const float4 *prm = reinterpret_cast<const float4 *>(buf + S::WIN);
-#pragma unroll 2
+    // small tiles leave few waves to hide the chain from an angle's constants
+    // to its samples: eight angles in flight
+#pragma unroll(TR * TC < 8 ? 8 : 2)
     for (int a = 0; a < na; ++a) {
       const float4 p = prm[a];
       const unsigned char *wb = buf + __float_as_int(p.w);
@@ -1536,6 +1541,19 @@ hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles,
     return hipGetLastError();
   }
   if (mirror && (mode != MODE_CTAS || store == ST_F32)) return hipErrorInvalidValue;
+  if (kind == TK_32x32 || kind == TK_16x32) {
+    // 64 angles per pass: a pass of fewer ends before its successor's
+    // windows arrive. One launch, 64x64 / 32x32 / 16x32 tiles: 256 px x 180
+    // angles 53 / 20 / 15 us, 512 x 360 98 / 34 / 28, 768 x 600 156 / 76 /
+    // 75, 1024 x 900 245 / 139 / 161, 1400 x 1000 296 / 254 / 288,
+    // 2048 x 1800 864 / 852 / 1039.
+    if (mode != MODE_CTAS || store != ST_F32) return hipErrorInvalidValue;
+    if (kind == TK_32x32)
+      hipLaunchKernelGGL((bp_grid_kernel<TK_32x32, 64, MODE_CTAS, ST_F32>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items);
+    else
+      hipLaunchKernelGGL((bp_grid_kernel<TK_16x32, 64, MODE_CTAS, ST_F32>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items);
+    return hipGetLastError();
+  }
   switch (kind) {
     case TK_64x64: return launch_k<TK_64x64>(d_items, n_items, total_tiles, angles_per_pass, mode, store, mirror, s);
     case TK_128x64: return launch_k<TK_128x64>(d_items, n_items, total_tiles, angles_per_pass, mode, store, mirror, s);

@@ -235,8 +235,10 @@ struct BpLaunch {
 // 544 of 2048 px 1111 us against 1387 and 1430, 288 of 1024 px 559 against
 // 513 and 454), two from 288 (float32; 183 us against 234, 256 workgroups 272
 // against 264) and 726 (16-bit; 571 us against 717, 576 workgroups 513
-// against 454). What remains is taken one by one. A tile kind
-// that the caller set is kept, for every slice.
+// against 454). What remains is taken one by one; float32 launches of less
+// than two 64x64 tiles per CU take 32x32 tiles, and 16x32 ones up to a
+// quarter of a tile per CU (backproject.hip). A tile kind that the caller
+// set is kept, for every slice.
 std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *centers, int S, std::vector<int> *order) {
   order->resize(S);
   std::iota(order->begin(), order->end(), 0);
@@ -248,6 +250,13 @@ std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *center
   const long long rows = (h->w + 63) / 64, cols = mirror ? (h->w / 2 + 64) / 64 : rows;
   const long long tiles = rows * cols, cus = h->cus;
   const long long four = (mirror ? 15 : 14) * cus / 8, two = (mirror ? 20 : 9) * cus / 8;
+  auto single = [&](int first, int n) {
+    BpLaunch l{first, n, 1, kind};
+    if (f32 && 4 * n * tiles <= cus) l.kind = TK_16x32;
+    else if (f32 && n * tiles < 2 * cus) l.kind = TK_32x32;
+    return l;
+  };
+  if (f32 && S * tiles < 2 * cus) return {single(0, S)};
   std::map<uint32_t, std::vector<int>> by_centre;
   for (int i = 0; i < S; ++i) {
     uint32_t bits;
@@ -268,10 +277,10 @@ std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *center
     }
     launches.push_back({first, static_cast<int>(at.size()) - first, group, TK_64x64});
   }
-  if (launches.empty()) return {{0, S, 1, kind}};
+  if (launches.empty()) return {single(0, S)};
   const int first = static_cast<int>(at.size());
   for (const auto &c : by_centre) at.insert(at.end(), c.second.begin(), c.second.end());
-  if (first < S) launches.push_back({first, S - first, 1, kind});
+  if (first < S) launches.push_back(single(first, S - first));
   *order = at;
   return launches;
 }

@@ -160,10 +160,12 @@ inline int store_of(int flags) {
 inline int mode_of(int flags) { return (flags & CTAS_INTERP_MASK) == CTAS_INTERP_LINEAR ? MODE_LINEAR : MODE_CTAS; }
 inline size_t store_bytes(int st) { return st == ST_F32 ? 4 : 2; }
 
-// Tile kinds: rows x cols of output per 256-thread workgroup.
-enum TileKind { TK_AUTO = 0, TK_64x64 = 1, TK_128x64 = 2, TK_128x128 = 3 };
-inline int tile_rows(int kind) { return kind == TK_64x64 ? 64 : 128; }
-inline int tile_cols(int kind) { return kind == TK_128x128 ? 128 : 64; }
+// Tile kinds: rows x cols of output per 256-thread workgroup. The two small
+// ones serve launches of CTAS sampling from float32 storage whose 64x64 tiles
+// would leave most of the chip idle; they are not among a caller's choices.
+enum TileKind { TK_AUTO = 0, TK_64x64 = 1, TK_128x64 = 2, TK_128x128 = 3, TK_32x32 = 4, TK_16x32 = 5 };
+inline int tile_rows(int kind) { return kind == TK_16x32 ? 16 : kind == TK_32x32 ? 32 : kind == TK_64x64 ? 64 : 128; }
+inline int tile_cols(int kind) { return kind >= TK_32x32 ? 32 : kind == TK_128x128 ? 128 : 64; }
 
 // ---- launchers (filter.hip, backproject.hip) ------------------------------
 // Zeros the pads around the filtered sinograms of the items (Item::pad).

@@ -75,3 +75,14 @@ def test_groups_in_graph_replays(torch_cuda):
         rec.graph_launch(stream)
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+# widths around the tiles' edges, the largest launch on 16x32 tiles (64 tiles
+# of 64x64) and launches on 32x32 tiles; angle counts around a pass of 64
+@pytest.mark.parametrize("w,S", [(2, 1), (15, 1), (16, 2), (17, 1), (33, 3), (64, 1), (65, 1), (512, 1), (513, 1),
+                                 (700, 2), (1439, 1)])
+@pytest.mark.parametrize("N,arc,c", [(1, 180.0, 0.0), (63, 180.0, 0.5), (64, 360.0, -0.25), (65, 150.0, 0.75)])
+def test_small_tiles_equal_64x64(torch_cuda, w, S, N, arc, c):
+    torch = torch_cuda
+    auto, auto_kept, single, _ = _both(torch, w, N, [c + 0.01 * k for k in range(S)], ca.PHS, arc, ca.STORE_FP32)
+    assert torch.equal(auto, single) and torch.equal(auto_kept, single)
