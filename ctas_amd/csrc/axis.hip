@@ -292,66 +292,147 @@ namespace {
 
 // ---- 0/180-degree registration (raxis(proj0, proj180, maxDev)) ----------
 // Column profile sum_r |p0 - 1| + |p180 - 1| (double terms added to a float
-// per column, rows in order), its centre of mass and the mean of the two
-// edge columns of the mirrored p180, each a sequential sum as in
-// lct.cpp:1226-1251; one workgroup, w <= 16384.
-__global__ __launch_bounds__(256) void pair_profile_kernel(const float *__restrict__ p0,
-                                                           const float *__restrict__ p180, int rows, int w,
-                                                           float *__restrict__ out) {
-  extern __shared__ float prof[];
-  for (int x = threadIdx.x; x < w; x += 256) {
-    float acc = 0.0f;
-    for (int r = 0; r < rows; ++r) {
-      const size_t i = static_cast<size_t>(r) * w + x;
-      acc = static_cast<float>(acc + (fabs(static_cast<double>(p0[i]) - 1.0) + fabs(static_cast<double>(p180[i]) - 1.0)));
+// per column, rows in order, lct.cpp:1226-1235). The sums are serial chains,
+// so a column is a lane, and one wave per workgroup spreads the columns over
+// the CUs; the rows of a chain are loaded 16 at a time. Bound by the chain:
+// 2048 rows of 2048 columns take 104 us (7.3 ms, the serial sums below
+// included, in one workgroup; those now take 38 us).
+__global__ __launch_bounds__(64) void pair_profile_kernel(const float *__restrict__ p0,
+                                                          const float *__restrict__ p180, int rows, int w,
+                                                          float *__restrict__ prof) {
+  const int x = blockIdx.x * 64 + threadIdx.x;
+  if (x >= w) return;
+  float acc = 0.0f;
+  auto add = [&](float a, float b) {
+    acc = static_cast<float>(acc + (fabs(static_cast<double>(a) - 1.0) + fabs(static_cast<double>(b) - 1.0)));
+  };
+  constexpr int U = 16;
+  int r = 0;
+  for (; r + U <= rows; r += U) {
+    float a[U], b[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const size_t i = static_cast<size_t>(r + j) * w + x;
+      a[j] = p0[i];
+      b[j] = p180[i];
     }
-    prof[x] = acc;
+#pragma unroll
+    for (int j = 0; j < U; ++j) add(a[j], b[j]);
   }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  double ssum = 0.0, wsum = 0.0;
-  for (int x = 0; x < w; ++x) {
-    ssum += prof[x];
-    wsum += static_cast<double>(static_cast<float>(x) * prof[x]);
+  for (; r < rows; ++r) {
+    const size_t i = static_cast<size_t>(r) * w + x;
+    add(p0[i], p180[i]);
   }
-  // p180 mirrored: its first column is p180's last and vice versa
-  double a0 = 0.0, a1 = 0.0;
-  for (int r = 0; r < rows; ++r) {
-    a0 += p180[static_cast<size_t>(r) * w + (w - 1)];
-    a1 += p180[static_cast<size_t>(r) * w];
-  }
-  out[0] = static_cast<float>(ssum == 0.0 ? 0.0 : 1.0);
-  out[1] = ssum == 0.0 ? 0.0f : static_cast<float>(wsum) / static_cast<float>(ssum);
-  out[2] = (static_cast<float>(a0) + static_cast<float>(a1)) / static_cast<float>(2 * rows);
+  prof[x] = acc;
 }
 
-// Registration error of trial shift x = shifts[blockIdx.x] (calcErr of
-// lct.cpp:1255-1270): sum over rows and columns of (p180r(col - sh) - p0)^2,
-// p180r the mirrored p180, `aver` outside the overlap, each square in float
-// and summed in double; the block's partial sums are reduced in a fixed order.
-__global__ __launch_bounds__(256) void pair_err_kernel(const float *__restrict__ p0, const float *__restrict__ p180,
-                                                       int rows, int w, const float *__restrict__ shifts, float aver,
-                                                       double *__restrict__ out) {
-  __shared__ double part[256];
-  const long sh = static_cast<long>(shifts[blockIdx.x]);
-  const long lo = sh > 0 ? sh : 0, hi = w - 1 + (sh < 0 ? sh : 0);
-  const size_t n = static_cast<size_t>(rows) * w;
-  double acc = 0.0;
-  for (size_t i = threadIdx.x; i < n; i += 256) {
-    const long col = static_cast<long>(i % w), r = static_cast<long>(i / w);
-    const long src = col - sh;
-    float d = aver;
-    if (col >= lo && col <= hi && src >= 0 && src < w) d = p180[r * w + (w - 1 - src)];
-    d = d - p0[i];
-    acc += static_cast<double>(d * d);
+// The serial sums of lct.cpp:1236-1251, each a workgroup whose first lane
+// adds what all lanes stage: block 0 the profile's sum and moment (out[0],
+// out[1]), blocks 1 and 2 the edge columns of the mirrored p180 (its first
+// column is p180's last and vice versa; out[2], out[3]).
+__global__ __launch_bounds__(256) void pair_sums_kernel(const float *__restrict__ prof,
+                                                        const float *__restrict__ p180, int rows, int w,
+                                                        double *__restrict__ out) {
+  constexpr int C = 1024;
+  __shared__ float stage[C];
+  const int what = blockIdx.x, n = what == 0 ? w : rows;
+  double sum = 0.0, moment = 0.0;
+  for (int i0 = 0; i0 < n; i0 += C) {
+    const int m = min(C, n - i0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < m; i += 256)
+      stage[i] = what == 0 ? prof[i0 + i] : p180[static_cast<size_t>(i0 + i) * w + (what == 1 ? w - 1 : 0)];
+    __syncthreads();
+    if (threadIdx.x != 0) continue;
+    if (what == 0) {
+#pragma unroll 8
+      for (int i = 0; i < m; ++i) {
+        sum += stage[i];
+        moment += static_cast<double>(static_cast<float>(i0 + i) * stage[i]);
+      }
+    } else {
+#pragma unroll 8
+      for (int i = 0; i < m; ++i) sum += stage[i];
+    }
   }
-  part[threadIdx.x] = acc;
+  if (threadIdx.x != 0) return;
+  if (what == 0) {
+    out[0] = sum;
+    out[1] = moment;
+  } else {
+    out[1 + what] = sum;
+  }
+}
+
+// Registration errors of k trial shifts (calcErr of lct.cpp:1255-1270): sum
+// over rows and columns of (p180r(col - sh) - p0)^2, p180r the mirrored p180,
+// `aver` outside the overlap, each square in float and summed in double.
+// Block (b, c) takes R rows and eight trials: the rows of p180 lie mirrored
+// in LDS, each sample of p0 is loaded once for the eight trials, and the
+// lanes' sums are reduced in a fixed order. part[t][b] receives the block's
+// sum of trial t. Bound by the conversions and double additions: the 65
+// trials of a sweep over 2048 x 2048 samples and the 33 of a bracket take
+// 77 us each on average; one workgroup per trial, reading both projections
+// from memory, took 8 ms for the sweep and as much for each probe of the
+// bisection.
+constexpr int kPairTrials = 8;
+__global__ __launch_bounds__(256) void pair_err_kernel(const float *__restrict__ p0, const float *__restrict__ p180,
+                                                       int rows, int w, int R, const int *__restrict__ shifts, int k,
+                                                       float aver, double *__restrict__ part) {
+  extern __shared__ float mirrored[];  // [R][w]
+  const int tid = threadIdx.x, r0 = blockIdx.x * R, nr = min(R, rows - r0), t0 = blockIdx.y * kPairTrials;
+  for (int r = 0; r < nr; ++r)
+    for (int x = tid; x < w; x += 256) mirrored[r * w + (w - 1 - x)] = p180[static_cast<size_t>(r0 + r) * w + x];
+  int sh[kPairTrials];
+  double acc[kPairTrials];
+#pragma unroll
+  for (int t = 0; t < kPairTrials; ++t) {
+    sh[t] = shifts[min(t0 + t, k - 1)];
+    acc[t] = 0.0;
+  }
+  __syncthreads();
+  for (int r = 0; r < nr; ++r) {
+    const float *line = mirrored + r * w;
+    const float *ref = p0 + static_cast<size_t>(r0 + r) * w;
+    for (int col = tid; col < w; col += 256) {
+      const float v = ref[col];
+#pragma unroll
+      for (int t = 0; t < kPairTrials; ++t) {
+        const int src = col - sh[t];
+        const bool in = static_cast<unsigned>(src) < static_cast<unsigned>(w);
+        const float s = line[in ? src : 0];
+        const float d = (in ? s : aver) - v;
+        acc[t] += static_cast<double>(d * d);
+      }
+    }
+  }
+  __shared__ double wave_sum[4][kPairTrials];
+#pragma unroll
+  for (int t = 0; t < kPairTrials; ++t) {
+    double a = acc[t];
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o);
+    if ((tid & 63) == 0) wave_sum[tid >> 6][t] = a;
+  }
+  __syncthreads();
+  if (tid < kPairTrials && t0 + tid < k)
+    part[static_cast<size_t>(t0 + tid) * gridDim.x + blockIdx.x] =
+        (wave_sum[0][tid] + wave_sum[1][tid]) + (wave_sum[2][tid] + wave_sum[3][tid]);
+}
+
+// Sum of trial blockIdx.x over the nb row blocks, in a fixed order.
+__global__ __launch_bounds__(256) void pair_err_sum_kernel(const double *__restrict__ part, int nb,
+                                                           double *__restrict__ out) {
+  __shared__ double red[256];
+  const double *p = part + static_cast<size_t>(blockIdx.x) * nb;
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < nb; i += 256) acc += p[i];
+  red[threadIdx.x] = acc;
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
-    if (static_cast<int>(threadIdx.x) < o) part[threadIdx.x] += part[threadIdx.x + o];
+    if (static_cast<int>(threadIdx.x) < o) red[threadIdx.x] += red[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = part[0];
+  if (threadIdx.x == 0) out[blockIdx.x] = red[0];
 }
 
 }  // namespace
@@ -376,39 +457,55 @@ extern "C" int ctas_raxis_pair(const float *p0, const float *p180, int rows, int
   const int kStep = 16;
   const int n_trials = static_cast<int>(1 + 2 * (maxDev == 0.0f ? 1.0f : maxDev * static_cast<float>(w) / kStep));
   // device: p0, p180, profile results, trial shifts, their sums
-  const int max_trials = std::max(n_trials, 8) + w / kStep + 4;
+  // the trial shifts of one evaluation: the sweep, a chunk of the walk, or the
+  // whole shifts of the bisection's bracket (2 kStep + 1 and a margin)
+  constexpr int kWalkChunk = 16;
+  const int max_trials = std::max(n_trials, 2 * kStep + 8);
+  // rows per workgroup: four where that leaves 256 of them, and within 64 KiB
+  // of LDS
+  const int R = std::max(1, std::min({4, rows / 256, 16384 / w}));
+  const int nb = (rows + R - 1) / R;
   struct Buf {
     void *p = nullptr;
     ~Buf() {
       if (p) (void)hipFree(p);
     }
   } buf;
-  const size_t off_res = 2 * n * sizeof(float), off_sh = off_res + 256, off_acc = off_sh + 4 * ((max_trials + 63) / 64 * 64);
-  if (hipMalloc(&buf.p, off_acc + sizeof(double) * max_trials) != hipSuccess)
+  auto up = [](size_t b) { return (b + 255) & ~static_cast<size_t>(255); };
+  const size_t off_prof = up(2 * n * sizeof(float)), off_sum = off_prof + up(sizeof(float) * w),
+               off_sh = off_sum + 256, off_acc = off_sh + up(sizeof(int) * max_trials),
+               off_part = off_acc + up(sizeof(double) * max_trials);
+  if (hipMalloc(&buf.p, off_part + sizeof(double) * max_trials * static_cast<size_t>(nb)) != hipSuccess)
     return fail(CTAS_E_NOMEM, "device allocation failed");
   char *base = static_cast<char *>(buf.p);
   float *d_p0 = reinterpret_cast<float *>(base), *d_p180 = d_p0 + n;
-  float *d_res = reinterpret_cast<float *>(base + off_res), *d_sh = reinterpret_cast<float *>(base + off_sh);
-  double *d_acc = reinterpret_cast<double *>(base + off_acc);
+  float *d_prof = reinterpret_cast<float *>(base + off_prof);
+  double *d_sum = reinterpret_cast<double *>(base + off_sum), *d_acc = reinterpret_cast<double *>(base + off_acc),
+         *d_part = reinterpret_cast<double *>(base + off_part);
+  int *d_sh = reinterpret_cast<int *>(base + off_sh);
   CTAS_HIP_TRY(hipMemcpy(d_p0, p0, n * sizeof(float), hipMemcpyHostToDevice));
   CTAS_HIP_TRY(hipMemcpy(d_p180, p180, n * sizeof(float), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(pair_profile_kernel, dim3(1), dim3(256), sizeof(float) * w, nullptr, d_p0, d_p180, rows, w,
-                     d_res);
+  hipLaunchKernelGGL(pair_profile_kernel, dim3((w + 63) / 64), dim3(64), 0, nullptr, d_p0, d_p180, rows, w, d_prof);
+  hipLaunchKernelGGL(pair_sums_kernel, dim3(3), dim3(256), 0, nullptr, d_prof, d_p180, rows, w, d_sum);
   CTAS_HIP_TRY(hipGetLastError());
-  float res[3];
-  CTAS_HIP_TRY(hipMemcpy(res, d_res, sizeof res, hipMemcpyDeviceToHost));
-  if (res[0] == 0.0f) return fail(CTAS_E_AXIS, "Impossible input projection averaging to zero.");
-  const float seed = res[1], mean_level = res[2];
+  double sums[4];
+  CTAS_HIP_TRY(hipMemcpy(sums, d_sum, sizeof sums, hipMemcpyDeviceToHost));
+  if (sums[0] == 0.0) return fail(CTAS_E_AXIS, "Impossible input projection averaging to zero.");
+  const float seed = static_cast<float>(sums[1]) / static_cast<float>(sums[0]);
+  const float mean_level = (static_cast<float>(sums[2]) + static_cast<float>(sums[3])) / static_cast<float>(2 * rows);
   int dev_rc = CTAS_OK;
-  // errors of trial shifts xs[0..k), one workgroup each
-  auto errs = [&](const float *xs, int k, float *e) {
+  // errors of the whole shifts sh[0..k)
+  auto whole_errs = [&](const std::vector<int> &sh, float *e) {
+    const int k = static_cast<int>(sh.size());
     if (dev_rc != CTAS_OK) return;
     std::vector<double> acc(k);
-    if (hipMemcpy(d_sh, xs, sizeof(float) * k, hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMemcpy(d_sh, sh.data(), sizeof(int) * k, hipMemcpyHostToDevice) != hipSuccess) {
       dev_rc = fail(CTAS_E_DEVICE, "registration: upload failed");
       return;
     }
-    hipLaunchKernelGGL(pair_err_kernel, dim3(k), dim3(256), 0, nullptr, d_p0, d_p180, rows, w, d_sh, mean_level, d_acc);
+    hipLaunchKernelGGL(pair_err_kernel, dim3(nb, (k + kPairTrials - 1) / kPairTrials), dim3(256),
+                       sizeof(float) * R * w, nullptr, d_p0, d_p180, rows, w, R, d_sh, k, mean_level, d_part);
+    hipLaunchKernelGGL(pair_err_sum_kernel, dim3(k), dim3(256), 0, nullptr, d_part, nb, d_acc);
     if (hipGetLastError() != hipSuccess ||
         hipMemcpy(acc.data(), d_acc, sizeof(double) * k, hipMemcpyDeviceToHost) != hipSuccess) {
       dev_rc = fail(CTAS_E_DEVICE, "registration: error sums failed on the device");
@@ -416,10 +513,22 @@ extern "C" int ctas_raxis_pair(const float *p0, const float *p180, int rows, int
     }
     for (int i = 0; i < k; ++i) e[i] = std::sqrt(static_cast<float>(acc[i]));
   };
-  auto calc_err = [&](float x) -> float {
-    float e = 0.0f;
-    errs(&x, 1, &e);
-    return e;
+  // a trial's error depends on its offset truncated to whole pixels
+  auto errs = [&](const float *xs, int k, float *e) {
+    std::vector<int> sh(k);
+    for (int i = 0; i < k; ++i) sh[i] = static_cast<int>(static_cast<long>(xs[i]));
+    whole_errs(sh, e);
+  };
+  // improveMe within the bracket [lo, hi]: its probes take at most
+  // 2 kStep + 1 whole shifts, evaluated together beforehand
+  auto refine = [&](const std::vector<float> &at, const std::vector<float> &e, int idx, int dir, int *rc) -> float {
+    const float a = at[idx - dir], b = at[idx + dir];
+    const int lo = static_cast<int>(static_cast<long>(std::min(a, b))), hi = static_cast<int>(static_cast<long>(std::max(a, b)));
+    std::vector<int> sh(hi - lo + 1);
+    for (size_t i = 0; i < sh.size(); ++i) sh[i] = lo + static_cast<int>(i);
+    std::vector<float> err(sh.size());
+    whole_errs(sh, err.data());
+    return improve_me(1.0f, at, e, idx, dir, [&](float x) { return err[static_cast<int>(static_cast<long>(x)) - lo]; }, rc);
   };
   std::vector<float> offsets(n_trials), errors(n_trials);
   for (int ii = 0; ii < n_trials; ++ii) offsets[ii] = 2 * (seed - mid) + static_cast<float>(kStep * (ii - (n_trials - 1) / 2));
@@ -431,7 +540,7 @@ extern "C" int ctas_raxis_pair(const float *p0, const float *p180, int rows, int
     if (errors[i] < errors[i - 1] && errors[i] < errors[i + 1] && errors[i] < best_error) best_error = errors[idx = i];
   int rc = CTAS_OK;
   if (idx >= 0) {
-    *result = mid + 0.5f * improve_me(1.0f, offsets, errors, idx, 1, calc_err, &rc);
+    *result = mid + 0.5f * refine(offsets, errors, idx, 1, &rc);
     return dev_rc != CTAS_OK ? dev_rc : rc;
   }
   idx = errors[0] < errors[n_trials - 1] ? 0 : n_trials - 1;
@@ -445,10 +554,12 @@ extern "C" int ctas_raxis_pair(const float *p0, const float *p180, int rows, int
   walk_errors[0] = errors[idx - dir];
   walk_errors[1] = errors[idx];
   int walk_best = 1;
+  for (int i = 0; i < walk_limit; ++i) walk_offsets[i + 2] = offsets[idx] + static_cast<float>(dir * (i + 1) * kStep);
   for (int i = 0; i < walk_limit; ++i) {
-    walk_offsets[i + 2] = offsets[idx] + static_cast<float>(dir * (i + 1) * kStep);
-    walk_errors[i + 2] = calc_err(walk_offsets[i + 2]);
-    if (dev_rc != CTAS_OK) return dev_rc;
+    if (i % kWalkChunk == 0) {
+      errs(walk_offsets.data() + i + 2, std::min(kWalkChunk, walk_limit - i), walk_errors.data() + i + 2);
+      if (dev_rc != CTAS_OK) return dev_rc;
+    }
     if (walk_errors[i + 2] < best_error) {
       best_error = walk_errors[i + 2];
       walk_best = i + 2;
@@ -457,7 +568,7 @@ extern "C" int ctas_raxis_pair(const float *p0, const float *p180, int rows, int
     }
   }
   if (walk_best == walk_limit + 1) return fail(CTAS_E_AXIS, "Failed to calculate rotation centre.");
-  *result = mid + 0.5f * improve_me(1.0f, walk_offsets, walk_errors, walk_best, dir, calc_err, &rc);
+  *result = mid + 0.5f * refine(walk_offsets, walk_errors, walk_best, dir, &rc);
   return dev_rc != CTAS_OK ? dev_rc : rc;
 }
 
