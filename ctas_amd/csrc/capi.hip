@@ -306,6 +306,39 @@ hipStream_t pick_stream(const ctas_fbp *h, void *stream) {
 
 }  // namespace
 
+namespace {
+std::mutex g_scratch_pool_mu;
+std::map<int, std::vector<void *>> g_scratch_pool;  // by device, kScratchBytes each
+}  // namespace
+
+Scratch::Scratch(size_t bytes) : bytes_(std::max<size_t>(bytes, 1)) {
+  if (hipGetDevice(&dev_) != hipSuccess) return;
+  if (bytes_ <= kScratchBytes) {
+    bytes_ = kScratchBytes;
+    std::lock_guard<std::mutex> lk(g_scratch_pool_mu);
+    auto &pool = g_scratch_pool[dev_];
+    if (!pool.empty()) {
+      p_ = pool.back();
+      pool.pop_back();
+      return;
+    }
+  }
+  if (hipMalloc(&p_, bytes_) != hipSuccess) p_ = nullptr;
+}
+
+Scratch::~Scratch() {
+  if (!p_) return;
+  if (done_ && bytes_ == kScratchBytes) {
+    std::lock_guard<std::mutex> lk(g_scratch_pool_mu);
+    auto &pool = g_scratch_pool[dev_];
+    if (pool.size() < static_cast<size_t>(kScratchKept)) {
+      pool.push_back(p_);
+      return;
+    }
+  }
+  (void)hipFree(p_);
+}
+
 int stream_wait(hipStream_t waiter, hipStream_t producer) {
   if (waiter == producer) return CTAS_OK;
   hipEvent_t e = nullptr;
@@ -1372,15 +1405,15 @@ int ctas_ring_filter_dev(float *d_sino, int S, int N, int w, int box, void *stre
   if (!d_sino || S <= 0 || N <= 0 || w <= 0 || box < 0) return fail(CTAS_E_ARG, "bad arguments");
   if (box == 0) return CTAS_OK;
   if (int rc = check_ring_box(box, w)) return rc;
-  // The column means need S*w floats of scratch; it is freed after the
-  // stream drains.
-  float *avg = nullptr;
-  if (hipMalloc(&avg, sizeof(float) * S * w) != hipSuccess) return fail(CTAS_E_NOMEM, "allocation failed");
+  // the column means, S*w floats
+  Scratch avg(sizeof(float) * S * w);
+  if (!avg.get()) return fail(CTAS_E_NOMEM, "allocation failed");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const hipError_t e = launch_ring(d_sino, avg, S, N, w, box, s);
-  (void)hipStreamSynchronize(s);
-  (void)hipFree(avg);
+  hipError_t e = launch_ring(d_sino, static_cast<float *>(avg.get()), S, N, w, box, s);
+  const hipError_t waited = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = waited;
   if (e != hipSuccess) return fail(CTAS_E_DEVICE, std::string("ring filter: ") + hipGetErrorString(e));
+  avg.done();
   return CTAS_OK;
 }
 
