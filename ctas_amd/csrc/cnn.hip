@@ -164,24 +164,10 @@ struct Im2col {  // B(k, n) = x[b][ci][y+dy][x+dx], k = ci*9 + r, n = (b*H + y)*
     return x[((static_cast<size_t>(b) * C + ci) * H + y2) * W + x2];
   }
 };
-struct Im2colT {  // B(n, k) = im2col(k, n): the pixel dimension is the reduction
-  Im2col f;
-  __device__ uint16_t operator()(int n, int k) const { return f(k, n); }
-};
 // gradient of the pre-activation: g = d(post) * (post > 0 ? 1 : kLeak), as bf16
 __device__ __forceinline__ uint16_t relu_grad(const float *d, const uint16_t *post, size_t i) {
   return bf16_rne(bf16_f(post[i]) > 0.0f ? d[i] : kLeak * d[i]);
 }
-struct GradA {  // A(co, n) = g[b][co][y][x], n = (b*H + y)*W + x
-  const float *d;
-  const uint16_t *post;
-  int C, H, W;
-  __device__ uint16_t operator()(int co, int n) const {
-    const int hw = H * W, b = n / hw, p = n - b * hw;
-    const size_t i = (static_cast<size_t>(b) * C + co) * hw + p;
-    return relu_grad(d, post, i);
-  }
-};
 struct WT {  // A(ci, k = co*9 + r) = W[co][ci*9 + r]
   const uint16_t *w;
   int Cin;
@@ -190,17 +176,15 @@ struct WT {  // A(ci, k = co*9 + r) = W[co][ci*9 + r]
     return w[static_cast<size_t>(co) * Cin * 9 + ci * 9 + r];
   }
 };
-struct ColG {  // B(k = co*9 + r, n) = g[b][co][y - dy][x - dx]
-  const float *d;
-  const uint16_t *post;
+struct ColG {  // B(k = co*9 + r, n) = g[b][co][y - dy][x - dx], g as bf16
+  const uint16_t *g;
   int C, H, W;
   __device__ uint16_t operator()(int k, int n) const {
     const int co = k / 9, r = k - co * 9;
     const int xx = n % W, t = n / W, yy = t % H, b = t / H;
     const int y2 = yy - (r / 3 - 1), x2 = xx - (r % 3 - 1);
     if (y2 < 0 || y2 >= H || x2 < 0 || x2 >= W) return 0;
-    const size_t i = ((static_cast<size_t>(b) * C + co) * H + y2) * W + x2;
-    return relu_grad(d, post, i);
+    return g[((static_cast<size_t>(b) * C + co) * H + y2) * W + x2];
   }
 };
 struct GradFlatA {  // A(o, b) = g[b][o] (fp32 gradient, ReLU-masked by post when given)
@@ -289,29 +273,258 @@ __global__ void maxpool_fwd(const uint16_t *__restrict__ x, uint16_t *__restrict
   }
 }
 
-// gradient to the first maximum of each window (rows/columns beyond the
-// pooled extent get zero)
-__global__ void maxpool_bwd(const uint16_t *__restrict__ x, const float *__restrict__ dy, float *__restrict__ dx,
-                            int BC, int H, int W) {
-  const int Ho = H / 2, Wo = W / 2;
-  const size_t total = static_cast<size_t>(BC) * H * W;
-  for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < total;
-       i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const int xx = static_cast<int>(i % W), yy = static_cast<int>((i / W) % H);
-    const size_t bc = i / (static_cast<size_t>(W) * H);
-    const int yo = yy / 2, xo = xx / 2;
-    float g = 0.0f;
-    if (yo < Ho && xo < Wo) {
-      const uint16_t *p = x + (bc * H + 2 * yo) * W + 2 * xo;
-      const float v[4] = {bf16_f(p[0]), bf16_f(p[1]), bf16_f(p[W]), bf16_f(p[W + 1])};
+// Backward of the pooling and of the leaky ReLU, and the bias gradient, in
+// one pass over a channel of a sample (block (co, b)): the pooled gradient dy
+// goes to the first maximum of its window, scaled by the slope of that
+// post-activation, as bf16 (the operand of the products that follow; every
+// other pixel gets zero, rows beyond the pooled extent too); part[co][b]
+// receives its sum before rounding. A thread takes four windows: two 16-byte
+// reads, one of dy, two writes. Bound by HBM: 28 us a layer on average for 64
+// samples (158 with the gradient in float32 and its bias sums apart).
+__global__ __launch_bounds__(256) void pool_bwd(const uint16_t *__restrict__ act, const float *__restrict__ dy,
+                                                uint16_t *__restrict__ g, float *__restrict__ part, int B, int C,
+                                                int H, int W) {
+  const int co = blockIdx.x, b = blockIdx.y;
+  const int Ho = H / 2, Wo = W / 2, Q = Wo / 4;  // W is a multiple of 8
+  const size_t plane = static_cast<size_t>(b) * C + co;
+  const uint16_t *a = act + plane * H * W;
+  uint16_t *gp = g + plane * H * W;
+  const float4 *d4 = reinterpret_cast<const float4 *>(dy + plane * Ho * Wo);
+  float s = 0.0f;
+  for (int i = threadIdx.x; i < Ho * Q; i += 256) {
+    const int yo = i / Q, q = i - yo * Q;
+    const size_t at = static_cast<size_t>(2 * yo) * W + 8 * q;
+    const u16x8 r0 = *reinterpret_cast<const u16x8 *>(a + at), r1 = *reinterpret_cast<const u16x8 *>(a + at + W);
+    const float4 d = d4[i];
+    const float dv[4] = {d.x, d.y, d.z, d.w};
+    u16x8 g0 = {}, g1 = {};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float v[4] = {bf16_f(r0[2 * j]), bf16_f(r0[2 * j + 1]), bf16_f(r1[2 * j]), bf16_f(r1[2 * j + 1])};
       int am = 0;
+      float best = v[0];
+#pragma unroll
       for (int k = 1; k < 4; ++k)
-        if (v[k] > v[am]) am = k;
-      const int mine = (yy - 2 * yo) * 2 + (xx - 2 * xo);
-      if (mine == am) g = dy[(bc * Ho + yo) * Wo + xo];
+        if (v[k] > best) {
+          best = v[k];
+          am = k;
+        }
+      const float gv = best > 0.0f ? dv[j] : kLeak * dv[j];
+      s += gv;
+      const uint16_t h = bf16_rne(gv);
+      g0[2 * j] = am == 0 ? h : 0;
+      g0[2 * j + 1] = am == 1 ? h : 0;
+      g1[2 * j] = am == 2 ? h : 0;
+      g1[2 * j + 1] = am == 3 ? h : 0;
     }
-    dx[i] = g;
+    *reinterpret_cast<u16x8 *>(gp + at) = g0;
+    *reinterpret_cast<u16x8 *>(gp + at + W) = g1;
   }
+  for (int i = 2 * Ho * (W / 8) + threadIdx.x; i < H * (W / 8); i += 256)
+    *reinterpret_cast<u16x8 *>(gp + static_cast<size_t>(8) * i) = u16x8{};
+  __shared__ float red[256];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[static_cast<size_t>(co) * B + b] = red[0];
+}
+
+// Weight gradient of a convolution, split over the pixels: ws[z][co][c] =
+// sum over the pixels of split z of g[co][pixel] x[ci][pixel + tap], c = ci*9
+// + tap, 32 pixels per matrix instruction in pixel order. Both operands of
+// the instruction are eight consecutive pixels of one row per lane, which a
+// lane loads by itself, the next 32 pixels while the current ones are
+// multiplied: no LDS and no barrier. Bound by the L1, which takes a cycle per
+// line that a load touches, and 16 rows of g or x are 16 lines or more, so a
+// wave takes all output channels and all nine taps of 16 input channels: of a
+// row it reads the aligned octets and the two pixels beside the 32, and forms
+// the octets of the three horizontal taps in registers. 64 samples, layers
+// one to four: 75 (its own kernel below), 64, 33 and 30 us; 380 us on average
+// through the general product, 142 for the second layer with an unaligned
+// load per tap.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// octet d moved one pixel right (lo: the pixel before it in the upper half)
+// or left (hi: the pixel after it in the lower half)
+__device__ __forceinline__ u32x4 octet_right(u32x4 d, uint32_t lo) {
+  return u32x4{(d.x << 16) | (lo >> 16), (d.y << 16) | (d.x >> 16), (d.z << 16) | (d.y >> 16), (d.w << 16) | (d.z >> 16)};
+}
+__device__ __forceinline__ u32x4 octet_left(u32x4 d, uint32_t hi) {
+  return u32x4{(d.x >> 16) | (d.y << 16), (d.y >> 16) | (d.z << 16), (d.z >> 16) | (d.w << 16), (d.w >> 16) | (hi << 16)};
+}
+
+template <int CIN, int COUT, int H, int W>
+__global__ __launch_bounds__(64) void wgrad_kernel(const uint16_t *__restrict__ g, const uint16_t *__restrict__ x,
+                                                   float *__restrict__ ws, int K, int chunk) {
+  constexpr int N = CIN * 9, MT = COUT / 16, HW = H * W;
+  static_assert(W % 32 == 0 && CIN % 16 == 0, "32 pixels of one row and 16 channels per step");
+  const int lane = threadIdx.x, r16 = lane & 15, g8 = (lane >> 4) * 8;
+  const int z = blockIdx.x, ci = blockIdx.y * 16 + r16;
+  const int kb = z * chunk, ke = min(K, kb + chunk);
+  // steps of loads in flight: a wave has 32 or so, and each would wait out a
+  // memory latency
+  constexpr int U = 4;
+  struct Step {
+    u32x4 a[MT], b[3];
+    uint32_t edge[3];  // first and last quarter of the lanes: the pixels before and after the 32
+    uint32_t row[3], end, live;  // masks of what lies inside the image and the split
+  } st[U];
+  // Branch-free, and masked when used: a branch would wait for its loads.
+  auto load = [&](int pn, Step &s) {
+    const bool live = pn < ke;
+    const int p = live ? pn : ke - 32;  // past the end the last step again, masked
+    const int b = p / HW, q = p - b * HW, y = q / W, x0 = q - y * W;  // uniform
+    const uint16_t *ga = g + static_cast<size_t>(b) * COUT * HW + q;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) s.a[m] = *reinterpret_cast<const u32x4 *>(ga + (16 * m + r16) * HW + g8);
+    const uint16_t *xb = x + (static_cast<size_t>(b) * CIN + blockIdx.y * 16) * HW;
+    const int xs = x0 + g8;
+    const int beside = g8 == 0 ? (xs > 0 ? -2 : 0) : g8 == 24 ? (xs < W - 8 ? 8 : 0) : 0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int yy = y + d - 1;
+      const bool row = yy >= 0 && yy < H;
+      const int at = r16 * HW + (row ? yy : y) * W + xs;
+      s.b[d] = *reinterpret_cast<const u32x4 *>(xb + at);
+      s.edge[d] = *reinterpret_cast<const uint32_t *>(xb + at + beside);
+      s.row[d] = row && live ? ~0u : 0u;
+    }
+    s.live = live ? ~0u : 0u;
+    s.end = beside ? ~0u : 0u;
+  };
+  f4 acc[MT][9];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < 9; ++t) acc[m][t] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < U; ++u) load(kb + 32 * u, st[u]);
+  for (int p0 = kb; p0 < ke; p0 += 32 * U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + 32 * u;
+      bf16x8 a[MT], bb[9];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, st[u].a[m] & st[u].live);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const u32x4 o = st[u].b[d] & st[u].row[d];
+        // the pixels beside an octet are the neighbouring lanes' octets'
+        const uint32_t edge = st[u].edge[d] & (st[u].row[d] & st[u].end);
+        const uint32_t before = __shfl(o.w, lane - 16), after = __shfl(o.x, lane + 16);
+        bb[3 * d] = __builtin_bit_cast(bf16x8, octet_right(o, g8 == 0 ? edge : before));
+        bb[3 * d + 1] = __builtin_bit_cast(bf16x8, o);
+        bb[3 * d + 2] = __builtin_bit_cast(bf16x8, octet_left(o, g8 == 24 ? edge : after));
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < 9; ++t) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bb[t], acc[m][t], 0, 0, 0);
+      // the next step's operands are not waited for before these products
+      __builtin_amdgcn_sched_barrier(0);
+      // two steps are one 128-byte line of each row: loaded together
+      if (u & 1) {
+        load(p + 32 * (U - 1), st[u - 1]);
+        load(p + 32 * U, st[u]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        ws[(static_cast<size_t>(z) * COUT + 16 * m + (lane >> 4) * 4 + r) * N + ci * 9 + t] = acc[m][t][r];
+}
+
+// The same for the network's two-channel input: its 18 columns (channel and
+// tap) are two tiles of lanes, and a lane loads the octet of its own tap,
+// which starts a pixel to the left or right (the row's ends are shifted in as
+// zeros).
+typedef uint16_t u16x8u __attribute__((ext_vector_type(8), aligned(2)));
+template <int CIN, int COUT, int H, int W>
+__global__ __launch_bounds__(64) void wgrad_taps_kernel(const uint16_t *__restrict__ g, const uint16_t *__restrict__ x,
+                                                        float *__restrict__ ws, int K, int chunk) {
+  constexpr int N = CIN * 9, MT = COUT / 16, NT = (N + 15) / 16, HW = H * W;
+  static_assert(W % 32 == 0, "32 pixels of one row per step");
+  const int lane = threadIdx.x, r16 = lane & 15, g8 = (lane >> 4) * 8;
+  const int z = blockIdx.x, kb = z * chunk, ke = min(K, kb + chunk);
+  int coff[NT], dyc[NT], dxc[NT];
+  bool use[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int c = t * 16 + r16;
+    use[t] = c < N;
+    const int cc = use[t] ? c : 0, ci = cc / 9, r = cc - 9 * ci;
+    dyc[t] = r / 3 - 1;
+    dxc[t] = r % 3 - 1;
+    coff[t] = ci * HW;
+  }
+  constexpr int U = 4;  // steps of loads in flight
+  u32x4 av[U][MT], bv[U][NT];
+  auto load = [&](int p, u32x4 (&av)[MT], u32x4 (&bv)[NT]) {
+    const int b = p / HW, q = p - b * HW, y = q / W, x0 = q - y * W;  // uniform
+    const uint16_t *ga = g + static_cast<size_t>(b) * COUT * HW + q;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) av[m] = *reinterpret_cast<const u32x4 *>(ga + (16 * m + r16) * HW + g8);
+    const uint16_t *xb = x + static_cast<size_t>(b) * CIN * HW;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int yy = y + dyc[t], xs = x0 + g8 + dxc[t];
+      const bool row = use[t] && yy >= 0 && yy < H;
+      const int at = coff[t] + (row ? yy : y) * W + min(max(xs, 0), W - 8);
+      bv[t] = __builtin_bit_cast(u32x4, *reinterpret_cast<const u16x8u *>(xb + at));
+    }
+  };
+  // masked and shifted when used: a branch would wait for its loads
+  auto operand = [&](int p, const u32x4 &v, int t) {  // zero past the split
+    const int q = p % HW, y = q / W, x0 = q - y * W;
+    const int yy = y + dyc[t], xs = x0 + g8 + dxc[t];
+    const u32x4 e = xs < 0 ? octet_right(v, 0) : xs > W - 8 ? octet_left(v, 0) : v;
+    return e & (use[t] && yy >= 0 && yy < H && p < ke ? ~0u : 0u);
+  };
+  f4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[m][t] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < U; ++u) load(min(kb + 32 * u, ke - 32), av[u], bv[u]);
+  for (int p0 = kb; p0 < ke; p0 += 32 * U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + 32 * u;
+      bf16x8 a[MT], bb[NT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, av[u][m] & (p < ke ? ~0u : 0u));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) bb[t] = __builtin_bit_cast(bf16x8, operand(p, bv[u][t], t));
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bb[t], acc[m][t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (u & 1) {  // past the end the last step again
+        load(min(p + 32 * (U - 1), ke - 32), av[u - 1], bv[u - 1]);
+        load(min(p + 32 * U, ke - 32), av[u], bv[u]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int c = t * 16 + r16;
+      if (c >= N) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        ws[(static_cast<size_t>(z) * COUT + 16 * m + (lane >> 4) * 4 + r) * N + c] = acc[m][t][r];
+    }
 }
 
 // Sum of the split-K partials (fixed order) into the weight gradient.
@@ -369,29 +582,7 @@ __global__ void bias_grad(const float *__restrict__ d, const uint16_t *__restric
   if (threadIdx.x == 0) db[co] = red[0];
 }
 
-// Bias gradient of a convolution layer in two fixed-order steps that fill
-// the chip: block (co, b) sums the slope-scaled gradient over the pixels of
-// one channel of one sample (contiguous, coalesced) into part[co][b], then
-// bias_grad_sum adds the samples in order.
-__global__ __launch_bounds__(256) void bias_grad_part(const float *__restrict__ d, const uint16_t *__restrict__ post,
-                                                      float *__restrict__ part, int B, int C, int HW) {
-  const int co = blockIdx.x, b = blockIdx.y;
-  const size_t base = (static_cast<size_t>(b) * C + co) * HW;
-  float s = 0.0f;
-  for (int p = threadIdx.x; p < HW; p += blockDim.x) {
-    const size_t i = base + p;
-    s += bf16_f(post[i]) > 0.0f ? d[i] : kLeak * d[i];
-  }
-  __shared__ float red[256];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[static_cast<size_t>(co) * B + b] = red[0];
-}
-
+// Bias gradient of a convolution layer: the samples' sums of pool_bwd in order.
 __global__ void bias_grad_sum(const float *__restrict__ part, float *__restrict__ db, int B, int C) {
   const int co = blockIdx.x * blockDim.x + threadIdx.x;
   if (co >= C) return;
@@ -571,7 +762,8 @@ struct ctas_cnn {
   int step = 0;
   int cap = 0;  // batch capacity of the activation buffers
   uint16_t *act[4] = {}, *pool[4] = {}, *h1 = nullptr;
-  float *out = nullptr, *gout = nullptr, *gh1 = nullptr, *gf = nullptr, *gbig = nullptr, *gbig2 = nullptr;
+  uint16_t *gact = nullptr;  // bf16 gradient of a layer's pre-activation
+  float *out = nullptr, *gout = nullptr, *gh1 = nullptr, *gf = nullptr, *gbig2 = nullptr;
   float *ws = nullptr;
   size_t ws_cap = 0;
   float *loss = nullptr;
@@ -596,11 +788,12 @@ void release_batch(ctas_cnn *n) {
     if (n->pool[l]) (void)hipFree(n->pool[l]);
     n->act[l] = n->pool[l] = nullptr;
   }
-  void *ptrs[] = {n->h1, n->out, n->gout, n->gh1, n->gf, n->gbig, n->gbig2};
+  void *ptrs[] = {n->h1, n->out, n->gout, n->gh1, n->gf, n->gact, n->gbig2};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   n->h1 = nullptr;
-  n->out = n->gout = n->gh1 = n->gf = n->gbig = n->gbig2 = nullptr;
+  n->gact = nullptr;
+  n->out = n->gout = n->gh1 = n->gf = n->gbig2 = nullptr;
   n->cap = 0;
 }
 
@@ -623,7 +816,7 @@ int ensure_batch(ctas_cnn *n, int B) {
   if (int rc = alloc(reinterpret_cast<void **>(&n->gout), static_cast<size_t>(B) * kOut * 4)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->gh1), static_cast<size_t>(B) * kH1 * 4)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->gf), static_cast<size_t>(B) * kF * 4)) return rc;
-  if (int rc = alloc(reinterpret_cast<void **>(&n->gbig), big * 4)) return rc;
+  if (int rc = alloc(reinterpret_cast<void **>(&n->gact), big * 2)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->gbig2), big * 4)) return rc;
   n->cap = B;
   return CTAS_OK;
@@ -710,6 +903,28 @@ int weight_grad(ctas_cnn *n, FA fa, FB fb, int M, int Ncols, int K, float *dst) 
   return CTAS_OK;
 }
 
+// The same of a convolution layer on B samples.
+template <int CIN, int COUT, int H, int W>
+int conv_weight_grad(ctas_cnn *n, const uint16_t *g, const uint16_t *in, int B, float *dst) {
+  constexpr int N = CIN * 9;
+  const int K = B * H * W;
+  int splits = std::max(1, std::min(2048, K / 1024));
+  int chunk = (K + splits - 1) / splits;
+  chunk = (chunk + kKS - 1) & ~(kKS - 1);
+  splits = (K + chunk - 1) / chunk;
+  if (int rc = ensure_ws(n, static_cast<size_t>(splits) * COUT * N)) return rc;
+  if constexpr (CIN % 16 == 0)
+    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, H, W>), dim3(splits, CIN / 16), dim3(64), 0, n->stream, g, in, n->ws, K,
+                       chunk);
+  else
+    hipLaunchKernelGGL((wgrad_taps_kernel<CIN, COUT, H, W>), dim3(splits), dim3(64), 0, n->stream, g, in, n->ws, K,
+                       chunk);
+  CTAS_HIP_TRY(hipGetLastError());
+  hipLaunchKernelGGL(reduce_splits, dim3((COUT * N + 15) / 16), dim3(256), 0, n->stream, n->ws, dst, splits,
+                     COUT * N);
+  return CTAS_OK;
+}
+
 int backward(ctas_cnn *n, const uint16_t *x, int B) {
   hipStream_t s = n->stream;
   // fc2: dW[o][k] = sum_b gout[b][o] h1[b][k]; dh1[b][k] = sum_o W[o][k] gout[b][o]
@@ -724,27 +939,26 @@ int backward(ctas_cnn *n, const uint16_t *x, int B) {
   CTAS_HIP_TRY(gemm(DenseAT{W16(n, 8), kF}, GradFlatB{GradFlatA{n->gh1, n->h1, kH1}}, StoreFlatDX{n->gf, kF}, kF, B,
                     kH1, s));
   // conv layers, last to first. gpool = gradient of the layer's pooled
-  // output; gact (buffer gbig) = gradient of its post-activation; the
-  // gradient of its input (= the previous pooled output) goes to gbig2.
+  // output; gact = bf16 gradient of its pre-activation; the gradient of its
+  // input (= the previous pooled output) goes to gbig2.
   const float *gpool = n->gf;
-  float *gact = n->gbig;
+  uint16_t *gact = n->gact;
   for (int l = 3; l >= 0; --l) {
     const Layer &L = kConv[l];
     const int HW = L.H * L.W;
-    const size_t a = static_cast<size_t>(B) * L.cout * HW;
-    hipLaunchKernelGGL(maxpool_bwd, dim3(blocks_for(a)), dim3(256), 0, s, n->act[l], gpool, gact, B * L.cout, L.H,
-                       L.W);
-    const uint16_t *in = l ? n->pool[l - 1] : x;
-    if (int rc = weight_grad(n, GradA{gact, n->act[l], L.cout, L.H, L.W}, Im2colT{Im2col{in, L.cin, L.H, L.W}},
-                             L.cout, L.cin * 9, B * HW, G32(n, 2 * l)))
-      return rc;
-    // the workspace's split partials were reduced by weight_grad on this stream
     if (int rc = ensure_ws(n, static_cast<size_t>(L.cout) * B)) return rc;
-    hipLaunchKernelGGL(bias_grad_part, dim3(L.cout, B), dim3(256), 0, s, gact, n->act[l], n->ws, B, L.cout, HW);
+    hipLaunchKernelGGL(pool_bwd, dim3(L.cout, B), dim3(256), 0, s, n->act[l], gpool, gact, n->ws, B, L.cout, L.H, L.W);
     hipLaunchKernelGGL(bias_grad_sum, dim3(1), dim3(64), 0, s, n->ws, G32(n, 2 * l + 1), B, L.cout);
+    // the workspace's bias partials were summed on this stream
+    const uint16_t *in = l ? n->pool[l - 1] : x;
+    if (int rc = l == 0   ? conv_weight_grad<2, 32, 180, 256>(n, gact, in, B, G32(n, 0))
+                 : l == 1 ? conv_weight_grad<32, 32, 90, 128>(n, gact, in, B, G32(n, 2))
+                 : l == 2 ? conv_weight_grad<32, 64, 45, 64>(n, gact, in, B, G32(n, 4))
+                          : conv_weight_grad<64, 64, 22, 32>(n, gact, in, B, G32(n, 6)))
+      return rc;
     if (l > 0) {
-      CTAS_HIP_TRY(gemm(WT{W16(n, 2 * l), L.cin}, ColG{gact, n->act[l], L.cout, L.H, L.W},
-                        StoreDX{n->gbig2, L.cin, L.H, L.W}, L.cin, B * HW, L.cout * 9, s));
+      CTAS_HIP_TRY(gemm(WT{W16(n, 2 * l), L.cin}, ColG{gact, L.cout, L.H, L.W}, StoreDX{n->gbig2, L.cin, L.H, L.W},
+                        L.cin, B * HW, L.cout * 9, s));
       gpool = n->gbig2;
     }
   }
