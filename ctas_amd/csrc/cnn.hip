@@ -153,40 +153,10 @@ struct DenseAT {  // A(m, k) = P[k][m] bf16 (transposed), row stride ld
   int ld;
   __device__ uint16_t operator()(int m, int k) const { return p[static_cast<size_t>(k) * ld + m]; }
 };
-struct Im2col {  // B(k, n) = x[b][ci][y+dy][x+dx], k = ci*9 + r, n = (b*H + y)*W + x
-  const uint16_t *x;
-  int C, H, W;
-  __device__ uint16_t operator()(int k, int n) const {
-    const int ci = k / 9, r = k - ci * 9;
-    const int xx = n % W, t = n / W, yy = t % H, b = t / H;
-    const int y2 = yy + r / 3 - 1, x2 = xx + r % 3 - 1;
-    if (y2 < 0 || y2 >= H || x2 < 0 || x2 >= W) return 0;
-    return x[((static_cast<size_t>(b) * C + ci) * H + y2) * W + x2];
-  }
-};
 // gradient of the pre-activation: g = d(post) * (post > 0 ? 1 : kLeak), as bf16
 __device__ __forceinline__ uint16_t relu_grad(const float *d, const uint16_t *post, size_t i) {
   return bf16_rne(bf16_f(post[i]) > 0.0f ? d[i] : kLeak * d[i]);
 }
-struct WT {  // A(ci, k = co*9 + r) = W[co][ci*9 + r]
-  const uint16_t *w;
-  int Cin;
-  __device__ uint16_t operator()(int ci, int k) const {
-    const int co = k / 9, r = k - co * 9;
-    return w[static_cast<size_t>(co) * Cin * 9 + ci * 9 + r];
-  }
-};
-struct ColG {  // B(k = co*9 + r, n) = g[b][co][y - dy][x - dx], g as bf16
-  const uint16_t *g;
-  int C, H, W;
-  __device__ uint16_t operator()(int k, int n) const {
-    const int co = k / 9, r = k - co * 9;
-    const int xx = n % W, t = n / W, yy = t % H, b = t / H;
-    const int y2 = yy - (r / 3 - 1), x2 = xx - (r % 3 - 1);
-    if (y2 < 0 || y2 >= H || x2 < 0 || x2 >= W) return 0;
-    return g[((static_cast<size_t>(b) * C + co) * H + y2) * W + x2];
-  }
-};
 struct GradFlatA {  // A(o, b) = g[b][o] (fp32 gradient, ReLU-masked by post when given)
   const float *d;
   const uint16_t *post;
@@ -257,22 +227,6 @@ struct StoreFlatDX {  // dx[b][f] fp32 from C(f, b)
 };
 
 // ---- elementwise kernels -------------------------------------------------------------
-__global__ void maxpool_fwd(const uint16_t *__restrict__ x, uint16_t *__restrict__ y, int BC, int H, int W) {
-  const int Ho = H / 2, Wo = W / 2;
-  const size_t total = static_cast<size_t>(BC) * Ho * Wo;
-  for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < total;
-       i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const int xo = static_cast<int>(i % Wo), yo = static_cast<int>((i / Wo) % Ho);
-    const size_t bc = i / (static_cast<size_t>(Wo) * Ho);
-    const uint16_t *p = x + (bc * H + 2 * yo) * W + 2 * xo;
-    float m = bf16_f(p[0]);
-    m = fmaxf(m, bf16_f(p[1]));
-    m = fmaxf(m, bf16_f(p[W]));
-    m = fmaxf(m, bf16_f(p[W + 1]));
-    y[i] = bf16_rne(m);
-  }
-}
-
 // Backward of the pooling and of the leaky ReLU, and the bias gradient, in
 // one pass over a channel of a sample (block (co, b)): the pooled gradient dy
 // goes to the first maximum of its window, scaled by the slope of that
@@ -527,6 +481,185 @@ __global__ __launch_bounds__(64) void wgrad_taps_kernel(const uint16_t *__restri
     }
 }
 
+// 3x3 convolution of a layer as a product over k = channel*9 + tap (padding
+// 1): forward (BWD false; bias, leaky ReLU, bf16 output y and its 2x2 maximum
+// `pool`) or the gradient of the layer's input (BWD true: CI the layer's
+// output channels, x their bf16 gradients, the stencil mirrored, float32
+// output dx). Four waves share a patch of the input in LDS, with its border
+// (zeros outside the image); each takes all output channels of 2 rows x 32
+// columns. A lane gathers its pixel's eight operands of a matrix instruction
+// from the patch, at offsets (in elements) that a table in LDS holds for
+// every k, and reads the weights [CO][K] as the instruction takes them. The
+// gathers bind it: eight 2-byte LDS reads per 16 pixels and 32 k serve CO/16
+// instructions. 64 samples, layers one to four forward with the pooling:
+// 86, 51, 41 and 22 us; backward, layers two to four: 42, 28 and 15 (181 and
+// 147 us a layer through the general product, which forms every element's
+// index anew, and a pooling of its own).
+// `per` matrix instructions in a row make a partial sum, and the partial sums
+// are added in order: the sums of a product split over k.
+template <int CI, int CO, int H, int W>
+struct ConvGeo {
+  static constexpr int K = CI * 9, STEPS = (K + 31) / 32, MT = CO / 16;
+  static constexpr int COLS = W < 128 ? W : 128, WX = COLS / 32, RB = 2 * (4 / WX);
+  static constexpr int XB = W / COLS, YB = (H + RB - 1) / RB;
+  static constexpr int PR = RB + 2, STRIDE = COLS + 16;  // patch rows; columns with eight on either side
+  static constexpr int OUT = 4 * CO * 2 * 32;            // elements of the block's output tile
+  static constexpr int ELEMS = CI * PR * STRIDE > OUT ? CI * PR * STRIDE : OUT;
+};
+
+template <int CI, int CO, int H, int W, bool BWD>
+__global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
+                                                   const float *__restrict__ bias, uint16_t *__restrict__ y,
+                                                   uint16_t *__restrict__ pool, float *__restrict__ dx, int per) {
+  using G = ConvGeo<CI, CO, H, W>;
+  constexpr int K = G::K, MT = G::MT, HW = H * W;
+  __shared__ __align__(16) uint16_t patch[G::ELEMS];
+  __shared__ __align__(16) uint16_t offs[G::STEPS * 32];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g8 = (lane >> 4) * 8;
+  const int x0 = (blockIdx.x % G::XB) * G::COLS, y0 = (blockIdx.x / G::XB) * G::RB;
+  const size_t b = blockIdx.y;
+  for (int k = tid; k < G::STEPS * 32; k += 256) {
+    const int kk = k < K ? k : 0, ci = kk / 9, r = kk - 9 * ci;
+    const int row = BWD ? 2 - r / 3 : r / 3, col = BWD ? 1 - r % 3 : r % 3 - 1;
+    offs[k] = static_cast<uint16_t>((ci * G::PR + row) * G::STRIDE + col + 8);
+  }
+  {
+    constexpr int OCT = G::STRIDE / 8, ITEMS = CI * G::PR * OCT, PT = (ITEMS + 255) / 256;
+    const uint16_t *xb = x + b * CI * HW;
+    u32x4 v[PT];
+    bool in[PT];
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      const int i = min(tid + 256 * j, ITEMS - 1), o = i % OCT, t = i / OCT, pr = t % G::PR, ci = t / G::PR;
+      const int xx = x0 + 8 * (o - 1), yy = y0 - 1 + pr;
+      in[j] = xx >= 0 && xx < W && yy >= 0 && yy < H;
+      // the network's input is the caller's, aligned to its elements only
+      v[j] = __builtin_bit_cast(u32x4, *reinterpret_cast<const u16x8u *>(xb + (in[j] ? ci * HW + yy * W + xx : 0)));
+    }
+#pragma unroll
+    for (int j = 0; j < PT; ++j)
+      if (tid + 256 * j < ITEMS) *reinterpret_cast<u32x4 *>(patch + 8 * (tid + 256 * j)) = in[j] ? v[j] : u32x4{};
+  }
+  __syncthreads();
+  const int wx = (wave % G::WX) * 32, wy = (wave / G::WX) * 2;  // the wave's pixels within the block
+  f4 acc[4][MT], sum[4][MT];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = sum[t][m] = f4{0.f, 0.f, 0.f, 0.f};
+  const uint16_t *base[4];  // tile t: row t / 2, columns 16 (t % 2) ...
+#pragma unroll
+  for (int t = 0; t < 4; ++t) base[t] = patch + (wy + (t >> 1)) * G::STRIDE + wx + 16 * (t & 1) + r16;
+  int left = per;
+  u16x8 next[MT];  // the weights of the next 32 k, in flight during a step
+  auto weights = [&](int c) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const uint16_t *row = w + (16 * m + r16) * K + 32 * c + g8;
+      if constexpr (K % 32 == 0) {
+        next[m] = *reinterpret_cast<const u16x8 *>(row);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) next[m][j] = 32 * c + g8 + j < K ? row[j] : static_cast<uint16_t>(0);
+      }
+    }
+  };
+  weights(0);
+  for (int c = 0; c < G::STEPS; ++c) {
+    bf16x8 a[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, next[m]);
+    if (G::STEPS > 1) weights(min(c + 1, G::STEPS - 1));
+    const u16x8 o = *reinterpret_cast<const u16x8 *>(offs + 32 * c + g8);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      u16x8 e;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        e[j] = base[t][o[j]];
+        if (K % 32 != 0 && 32 * c + g8 + j >= K) e[j] = 0;
+      }
+      const bf16x8 bv = __builtin_bit_cast(bf16x8, e);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bv, acc[t][m], 0, 0, 0);
+    }
+    if (--left == 0) {
+      left = per;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          sum[t][m] += acc[t][m];
+          acc[t][m] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+  if (left != per)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) sum[t][m] += acc[t][m];
+  const int row4 = (lane >> 4) * 4;
+  if constexpr (BWD) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int yy = y0 + wy + (t >> 1), xx = x0 + wx + 16 * (t & 1) + r16;
+      if (yy >= H) continue;
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dx[(b * CO + 16 * m + row4 + r) * HW + yy * W + xx] = sum[t][m][r];
+    }
+  } else {
+    // the tile through LDS, so that the stores and the pooling take octets
+    __syncthreads();
+    uint16_t *out = patch + wave * (CO * 64);  // [CO][2][32]
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int co = 16 * m + row4 + r;
+          out[co * 64 + 32 * (t >> 1) + 16 * (t & 1) + r16] = bf16_rne(leaky(sum[t][m][r] + bias[co]));
+        }
+    __syncthreads();
+    const int yy = y0 + wy, xx = x0 + wx + 8 * (lane & 3);
+#pragma unroll
+    for (int i = 0; i < CO / 16; ++i) {
+      const int co = 16 * i + (lane >> 2);
+      const u16x8 top = *reinterpret_cast<const u16x8 *>(out + co * 64 + 8 * (lane & 3));
+      const u16x8 low = *reinterpret_cast<const u16x8 *>(out + co * 64 + 32 + 8 * (lane & 3));
+      const size_t plane = b * CO + co;
+      if (yy < H) *reinterpret_cast<u16x8 *>(y + plane * HW + yy * W + xx) = top;
+      if (yy + 1 < H) {
+        *reinterpret_cast<u16x8 *>(y + plane * HW + (yy + 1) * W + xx) = low;
+        typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+        u16x4 mx;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float v = bf16_f(top[2 * j]);
+          v = fmaxf(v, bf16_f(top[2 * j + 1]));
+          v = fmaxf(v, bf16_f(low[2 * j]));
+          v = fmaxf(v, bf16_f(low[2 * j + 1]));
+          mx[j] = bf16_rne(v);
+        }
+        *reinterpret_cast<u16x4 *>(pool + plane * (H / 2) * (W / 2) + (yy / 2) * (W / 2) + xx / 2) = mx;
+      }
+    }
+  }
+}
+
+// The weights of layers two to four as the input gradients' products take
+// them: wt[ci][co*9 + tap] = w[co][ci*9 + tap], layer l at its own offset.
+__global__ __launch_bounds__(256) void transpose_weights(const uint16_t *__restrict__ w, uint16_t *__restrict__ wt,
+                                                         int cout, int cin) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= cout * cin * 9) return;
+  const int co = i / (cin * 9), q = i - co * cin * 9, ci = q / 9, r = q - 9 * ci;
+  wt[(ci * cout + co) * 9 + r] = w[i];
+}
+
 // Sum of the split-K partials (fixed order) into the weight gradient.
 // Sum over the splits of a K-split product, in a fixed order: 16 outputs per
 // block, each summed by 16 threads over interleaved splits (z = g, g + 16,
@@ -758,7 +891,7 @@ struct ctas_cnn {
   std::vector<ctas::cnn::Param> prm;  // w1 b1 w2 b2 w3 b3 w4 b4 wf1 bf1 wf2 bf2
   size_t nparam = 0;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
-  uint16_t *p16 = nullptr;
+  uint16_t *p16 = nullptr, *wt = nullptr;  // bf16 weights; a layer's, transposed
   int step = 0;
   int cap = 0;  // batch capacity of the activation buffers
   uint16_t *act[4] = {}, *pool[4] = {}, *h1 = nullptr;
@@ -866,19 +999,34 @@ int product_act(ctas_cnn *n, FA fa, FB fb, int M, int Ncols, int K, const float 
   return CTAS_OK;
 }
 
+// Convolution layer l with its pooling. The sums are those of a product
+// split over k where one of 64x64 tiles would not fill the chip.
+template <int L, int CI, int CO, int H, int W>
+hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B) {
+  using G = ConvGeo<CI, CO, H, W>;
+  const int splits = forward_splits(CO, B * H * W, G::K), per = (G::STEPS + splits - 1) / splits;
+  hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, x,
+                     W16(n, 2 * L), P32(n, 2 * L + 1), n->act[L], n->pool[L], nullptr, per);
+  return hipGetLastError();
+}
+
+// Gradient of the input of layer l (its weights transposed first) into gbig2.
+template <int L, int CIN, int COUT, int H, int W>
+hipError_t conv_input_grad(ctas_cnn *n, const uint16_t *g, int B) {
+  using G = ConvGeo<COUT, CIN, H, W>;
+  hipLaunchKernelGGL(transpose_weights, dim3((COUT * CIN * 9 + 255) / 256), dim3(256), 0, n->stream, W16(n, 2 * L),
+                     n->wt, COUT, CIN);
+  hipLaunchKernelGGL((conv_kernel<COUT, CIN, H, W, true>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, g, n->wt,
+                     nullptr, nullptr, nullptr, n->gbig2, G::STEPS);
+  return hipGetLastError();
+}
+
 int forward(ctas_cnn *n, const uint16_t *x, int B) {
   hipStream_t s = n->stream;
-  const uint16_t *in = x;
-  for (int l = 0; l < 4; ++l) {
-    const Layer &L = kConv[l];
-    const int HW = L.H * L.W;
-    if (int rc = product_act(n, DenseA{W16(n, 2 * l), L.cin * 9}, Im2col{in, L.cin, L.H, L.W}, L.cout, B * HW,
-                             L.cin * 9, P32(n, 2 * l + 1), n->act[l], HW))
-      return rc;
-    const size_t q = static_cast<size_t>(B) * L.cout * (L.H / 2) * (L.W / 2);
-    hipLaunchKernelGGL(maxpool_fwd, dim3(blocks_for(q)), dim3(256), 0, s, n->act[l], n->pool[l], B * L.cout, L.H, L.W);
-    in = n->pool[l];
-  }
+  CTAS_HIP_TRY((conv_forward<0, 2, 32, 180, 256>(n, x, B)));
+  CTAS_HIP_TRY((conv_forward<1, 32, 32, 90, 128>(n, n->pool[0], B)));
+  CTAS_HIP_TRY((conv_forward<2, 32, 64, 45, 64>(n, n->pool[1], B)));
+  CTAS_HIP_TRY((conv_forward<3, 64, 64, 22, 32>(n, n->pool[2], B)));
   if (int rc = product_act(n, DenseA{W16(n, 8), kF}, ActB{n->pool[3], kF}, kH1, B, kF, P32(n, 9), n->h1, 1))
     return rc;
   CTAS_HIP_TRY(gemm(DenseA{W16(n, 10), kH1}, ActB{n->h1, kH1}, StoreFC{nullptr, n->out, P32(n, 11), kOut, false},
@@ -945,7 +1093,6 @@ int backward(ctas_cnn *n, const uint16_t *x, int B) {
   uint16_t *gact = n->gact;
   for (int l = 3; l >= 0; --l) {
     const Layer &L = kConv[l];
-    const int HW = L.H * L.W;
     if (int rc = ensure_ws(n, static_cast<size_t>(L.cout) * B)) return rc;
     hipLaunchKernelGGL(pool_bwd, dim3(L.cout, B), dim3(256), 0, s, n->act[l], gpool, gact, n->ws, B, L.cout, L.H, L.W);
     hipLaunchKernelGGL(bias_grad_sum, dim3(1), dim3(64), 0, s, n->ws, G32(n, 2 * l + 1), B, L.cout);
@@ -957,8 +1104,10 @@ int backward(ctas_cnn *n, const uint16_t *x, int B) {
                           : conv_weight_grad<64, 64, 22, 32>(n, gact, in, B, G32(n, 6)))
       return rc;
     if (l > 0) {
-      CTAS_HIP_TRY(gemm(WT{W16(n, 2 * l), L.cin}, ColG{gact, L.cout, L.H, L.W}, StoreDX{n->gbig2, L.cin, L.H, L.W},
-                        L.cin, B * HW, L.cout * 9, s));
+      const hipError_t e = l == 1   ? conv_input_grad<1, 32, 32, 90, 128>(n, gact, B)
+                           : l == 2 ? conv_input_grad<2, 32, 64, 45, 64>(n, gact, B)
+                                    : conv_input_grad<3, 64, 64, 22, 32>(n, gact, B);
+      CTAS_HIP_TRY(e);
       gpool = n->gbig2;
     }
   }
@@ -1006,6 +1155,7 @@ extern "C" int ctas_cnn_create(ctas_cnn **pn, uint64_t seed) {
   if (int rc = alloc(reinterpret_cast<void **>(&n->m), off * 4)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->v), off * 4)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->p16), off * 2)) return rc;
+  if (int rc = alloc(reinterpret_cast<void **>(&n->wt), 64 * 64 * 9 * 2)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->loss), 256)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->norm), sizeof(float) * (kNormBlocks + 2))) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->ftmp), sizeof(float) * kFeatA * kFeatW)) return rc;
@@ -1024,7 +1174,7 @@ extern "C" int ctas_cnn_destroy(ctas_cnn *n) {
   if (!n) return CTAS_OK;
   (void)hipStreamSynchronize(n->stream);
   release_batch(n);
-  void *ptrs[] = {n->p, n->g, n->m, n->v, n->p16, n->ws, n->loss, n->ftmp, n->xin, n->norm};
+  void *ptrs[] = {n->p, n->g, n->m, n->v, n->p16, n->wt, n->ws, n->loss, n->ftmp, n->xin, n->norm};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   (void)hipStreamDestroy(n->stream);
