@@ -682,37 +682,63 @@ __global__ __launch_bounds__(256) void reduce_splits(const float *__restrict__ w
 }
 
 // Epilogue of a split forward product: y[b][m][p] = bf16(leaky(sum over
-// splits of ws[z][m][n] + bias[m])), n = b*HW + p.
-__global__ void finish_act(const float *__restrict__ ws, int splits, int M, int N, const float *__restrict__ bias,
-                           uint16_t *__restrict__ y, int HW) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M * N) return;
-  const int m = i / N, n = i - m * N;
+// splits of ws[z][m][n] + bias[m])), n = b*HW + p, 16 outputs per workgroup.
+// The sum runs over the splits in order, so 256 threads stage 64 splits at a
+// time for the 16 that add them: 176 splits of one sample's first fully
+// connected layer take 3.6 us (29 with each thread's loads one after another),
+// those of 64 samples 5.3 (42).
+__global__ __launch_bounds__(256) void finish_act(const float *__restrict__ ws, int splits, int M, int N,
+                                                  const float *__restrict__ bias, uint16_t *__restrict__ y, int HW) {
+  constexpr int C = 64;
+  __shared__ float stage[C][17];
+  const int o = threadIdx.x & 15, g = threadIdx.x >> 4, i = blockIdx.x * 16 + o;
+  const int at = min(i, M * N - 1);
   float v = 0.0f;
-  for (int z = 0; z < splits; ++z) v += ws[static_cast<size_t>(z) * M * N + i];
-  const int b = n / HW, p = n - b * HW;
+  for (int z0 = 0; z0 < splits; z0 += C) {
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < C / 16; ++j) {
+      const int z = z0 + g + 16 * j;
+      stage[g + 16 * j][o] = ws[static_cast<size_t>(min(z, splits - 1)) * M * N + at];
+    }
+    __syncthreads();
+    if (g == 0) {
+      const int n = min(C, splits - z0);
+      if (n == C) {
+#pragma unroll
+        for (int z = 0; z < C; ++z) v += stage[z][o];
+      } else {
+        for (int z = 0; z < n; ++z) v += stage[z][o];
+      }
+    }
+  }
+  if (g != 0 || i >= M * N) return;
+  const int m = i / N, n = i - m * N, b = n / HW, p = n - b * HW;
   y[(static_cast<size_t>(b) * M + m) * HW + p] = bf16_rne(leaky(v + bias[m]));
 }
 
-// Bias gradient: sum of the slope-scaled gradient over batch and pixels (one
-// block per channel, fixed-order tree reduction).
-__global__ void bias_grad(const float *__restrict__ d, const uint16_t *__restrict__ post, float *__restrict__ db,
-                          int B, int C, int HW) {
+// Bias gradient of a fully connected layer: sum of the slope-scaled gradient
+// over the batch in order, one workgroup per channel, 256 samples staged at a
+// time.
+__global__ __launch_bounds__(256) void bias_grad(const float *__restrict__ d, const uint16_t *__restrict__ post,
+                                                 float *__restrict__ db, int B, int C) {
+  __shared__ float stage[256];
   const int co = blockIdx.x;
   float s = 0.0f;
-  for (int b = 0; b < B; ++b)
-    for (int p = threadIdx.x; p < HW; p += blockDim.x) {
-      const size_t i = (static_cast<size_t>(b) * C + co) * HW + p;
-      s += (!post || bf16_f(post[i]) > 0.0f) ? d[i] : kLeak * d[i];
-    }
-  __shared__ float red[256];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+  for (int b0 = 0; b0 < B; b0 += 256) {
+    const int n = min(256, B - b0);
     __syncthreads();
+    if (static_cast<int>(threadIdx.x) < n) {
+      const size_t i = static_cast<size_t>(b0 + threadIdx.x) * C + co;
+      stage[threadIdx.x] = (!post || bf16_f(post[i]) > 0.0f) ? d[i] : kLeak * d[i];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll 16
+      for (int b = 0; b < n; ++b) s += stage[b];
+    }
   }
-  if (threadIdx.x == 0) db[co] = red[0];
+  if (threadIdx.x == 0) db[co] = s;
 }
 
 // Bias gradient of a convolution layer: the samples' sums of pool_bwd in order.
@@ -814,41 +840,75 @@ __global__ void to_bf16(const float *__restrict__ p, uint16_t *__restrict__ q, i
 // (detector and angle order reversed), which puts the projections that
 // mirror each other across the 0/180 degree seam (P(theta + pi, s) =
 // P(theta, -s)) in the same rows of the two channels, shifted by twice
-// the axis offset. Grid (1, 180): one block per angle cell, one thread per
-// detector bin.
-__global__ __launch_bounds__(256) void features_kernel(const float *__restrict__ sino, int N, int w,
-                                                       float *__restrict__ tmp) {
+// the axis offset. Grid (1, 180): one block per angle cell.
+// The cells' sums run row by row and column by column, a cell per thread, so
+// a block of 1024 takes the logarithms of a row coalesced into LDS, 4096
+// columns at a time, and the 256 owners add their columns from there. One
+// thread per cell, reading its columns from memory, took 13.5 us for 1800 x
+// 2048, bound by the logarithms of three waves per CU; this takes 8.9.
+constexpr int kFeatCols = 4096, kFeatT = 1024;
+__global__ __launch_bounds__(kFeatT) void features_kernel(const float *__restrict__ sino, int N, int w,
+                                                          float *__restrict__ tmp) {
+  __shared__ float line[2][kFeatCols];
   const int a = blockIdx.y;
   const int x = threadIdx.x;
   const int r0 = static_cast<int>(static_cast<long long>(a) * N / kFeatA);
   const int r1 = max(r0 + 1, static_cast<int>(static_cast<long long>(a + 1) * N / kFeatA));
   const int c0 = static_cast<int>(static_cast<long long>(x) * w / kFeatW);
   const int c1 = max(c0 + 1, static_cast<int>(static_cast<long long>(x + 1) * w / kFeatW));
+  constexpr int PT = kFeatCols / kFeatT;
+  const int nseg = (w + kFeatCols - 1) / kFeatCols, steps = (r1 - r0) * nseg;
+  float v[PT];
+  auto fetch = [&](int k) {
+    const int r = r0 + k / nseg, b = (k % nseg) * kFeatCols;
+    const float *row = sino + static_cast<size_t>(r) * w;
+#pragma unroll
+    for (int j = 0; j < PT; ++j) v[j] = row[min(b + x + kFeatT * j, w - 1)];
+  };
+  fetch(0);
   float s = 0.0f;
-  for (int r = r0; r < r1; ++r)
-    for (int c = c0; c < c1; ++c) s += -logf(fmaxf(sino[static_cast<size_t>(r) * w + c], 1e-6f));
-  tmp[a * kFeatW + x] = s / static_cast<float>((r1 - r0) * (c1 - c0));
+  for (int k = 0; k < steps; ++k) {
+    const int b = (k % nseg) * kFeatCols;
+    float *buf = line[k & 1];
+#pragma unroll
+    for (int j = 0; j < PT; ++j)
+      if (b + x + kFeatT * j < w) buf[x + kFeatT * j] = -logf(fmaxf(v[j], 1e-6f));
+    if (k + 1 < steps) fetch(k + 1);
+    __syncthreads();
+    if (x < kFeatW)
+      for (int c = max(c0, b); c < min(c1, b + kFeatCols); ++c) s += buf[c - b];
+  }
+  if (x < kFeatW) tmp[a * kFeatW + x] = s / static_cast<float>((r1 - r0) * (c1 - c0));
 }
 
 // Mean and standard deviation of the 180 x 256 features, then the two
-// standardised bf16 channels. One block of 1024 threads (a few float4 loads
-// each), partial sums reduced in a fixed order.
+// standardised bf16 channels. Every block of 1024 threads forms the sums for
+// itself (a thread's 12 float4 loads in flight together, partial sums reduced
+// in a fixed order) and writes 1024 features: one block doing all of it, a
+// load at a time, took 16 us; this takes 4.6.
 __global__ __launch_bounds__(1024) void standardise_kernel(const float *__restrict__ tmp, uint16_t *__restrict__ feat) {
   __shared__ float red[1024], red2[1024];
-  constexpr int n = kFeatA * kFeatW;
-  static_assert(n % 4 == 0, "float4 loads");
+  constexpr int n = kFeatA * kFeatW, Q = n / 4, PT = (Q + 1023) / 1024;
+  static_assert(n % 1024 == 0, "whole blocks of features");
   const float4 *t4 = reinterpret_cast<const float4 *>(tmp);
+  float4 q[PT];
+#pragma unroll
+  for (int j = 0; j < PT; ++j) q[j] = t4[min(static_cast<int>(threadIdx.x) + 1024 * j, Q - 1)];
+  const int i = blockIdx.x * 1024 + threadIdx.x;
+  const float mine = tmp[i];
   float s = 0.0f, s2 = 0.0f;
-  for (int i = threadIdx.x; i < n / 4; i += 1024) {
-    const float4 v = t4[i];
-    s += (v.x + v.y) + (v.z + v.w);
-    s2 += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
-  }
+#pragma unroll
+  for (int j = 0; j < PT; ++j)
+    if (static_cast<int>(threadIdx.x) + 1024 * j < Q) {
+      const float4 v = q[j];
+      s += (v.x + v.y) + (v.z + v.w);
+      s2 += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+    }
   red[threadIdx.x] = s;
   red2[threadIdx.x] = s2;
   __syncthreads();
   for (int o = 512; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
+    if (static_cast<int>(threadIdx.x) < o) {
       red[threadIdx.x] += red[threadIdx.x + o];
       red2[threadIdx.x] += red2[threadIdx.x + o];
     }
@@ -857,17 +917,15 @@ __global__ __launch_bounds__(1024) void standardise_kernel(const float *__restri
   const float mean = red[0] / n;
   const float var = fmaxf(red2[0] / n - mean * mean, 1e-12f);
   const float inv = 1.0f / sqrtf(var);
-  for (int i = threadIdx.x; i < n; i += 1024) {
-    const int a = i / kFeatW, x = i - a * kFeatW;
-    const float v = (tmp[i] - mean) * inv;
-    feat[i] = bf16_rne(v);
-    feat[n + (kFeatA - 1 - a) * kFeatW + (kFeatW - 1 - x)] = bf16_rne(v);
-  }
+  const int a = i / kFeatW, x = i - a * kFeatW;
+  const float v = (mine - mean) * inv;
+  feat[i] = bf16_rne(v);
+  feat[n + (kFeatA - 1 - a) * kFeatW + (kFeatW - 1 - x)] = bf16_rne(v);
 }
 
 hipError_t launch_features(const float *d_sino, int N, int w, float *d_tmp, uint16_t *d_x, hipStream_t s) {
-  hipLaunchKernelGGL(features_kernel, dim3(1, kFeatA), dim3(kFeatW), 0, s, d_sino, N, w, d_tmp);
-  hipLaunchKernelGGL(standardise_kernel, dim3(1), dim3(1024), 0, s, d_tmp, d_x);
+  hipLaunchKernelGGL(features_kernel, dim3(1, kFeatA), dim3(kFeatT), 0, s, d_sino, N, w, d_tmp);
+  hipLaunchKernelGGL(standardise_kernel, dim3(kFeatA * kFeatW / 1024), dim3(1024), 0, s, d_tmp, d_x);
   return hipGetLastError();
 }
 
@@ -995,7 +1053,7 @@ int product_act(ctas_cnn *n, FA fa, FB fb, int M, int Ncols, int K, const float 
   chunk = (chunk + kKS - 1) & ~(kKS - 1);
   const int real = (K + chunk - 1) / chunk;
   CTAS_HIP_TRY(gemm(fa, fb, StorePartial{n->ws, M, Ncols}, M, Ncols, K, s, splits));
-  hipLaunchKernelGGL(finish_act, dim3((M * Ncols + 255) / 256), dim3(256), 0, s, n->ws, real, M, Ncols, bias, y, HW);
+  hipLaunchKernelGGL(finish_act, dim3((M * Ncols + 15) / 16), dim3(256), 0, s, n->ws, real, M, Ncols, bias, y, HW);
   return CTAS_OK;
 }
 
@@ -1078,12 +1136,12 @@ int backward(ctas_cnn *n, const uint16_t *x, int B) {
   // fc2: dW[o][k] = sum_b gout[b][o] h1[b][k]; dh1[b][k] = sum_o W[o][k] gout[b][o]
   if (int rc = weight_grad(n, GradFlatA{n->gout, nullptr, kOut}, ActBT{n->h1, kH1}, kOut, kH1, B, G32(n, 10)))
     return rc;
-  hipLaunchKernelGGL(bias_grad, dim3(kOut), dim3(256), 0, s, n->gout, nullptr, G32(n, 11), B, kOut, 1);
+  hipLaunchKernelGGL(bias_grad, dim3(kOut), dim3(256), 0, s, n->gout, nullptr, G32(n, 11), B, kOut);
   CTAS_HIP_TRY(gemm(DenseAT{W16(n, 10), kH1}, GradFlatB{GradFlatA{n->gout, nullptr, kOut}}, StoreFlatDX{n->gh1, kH1},
                     kH1, B, kOut, s));
   // fc1 (ReLU on h1)
   if (int rc = weight_grad(n, GradFlatA{n->gh1, n->h1, kH1}, ActBT{n->pool[3], kF}, kH1, kF, B, G32(n, 8))) return rc;
-  hipLaunchKernelGGL(bias_grad, dim3(kH1), dim3(256), 0, s, n->gh1, n->h1, G32(n, 9), B, kH1, 1);
+  hipLaunchKernelGGL(bias_grad, dim3(kH1), dim3(256), 0, s, n->gh1, n->h1, G32(n, 9), B, kH1);
   CTAS_HIP_TRY(gemm(DenseAT{W16(n, 8), kF}, GradFlatB{GradFlatA{n->gh1, n->h1, kH1}}, StoreFlatDX{n->gf, kF}, kF, B,
                     kH1, s));
   // conv layers, last to first. gpool = gradient of the layer's pooled

@@ -34,3 +34,18 @@ def test_gradients_of_small_batches(torch_cuda, B):
     for k, n in enumerate(co.SIZES):
         a, b = got[starts[k]:starts[k] + n], gref[starts[k]:starts[k] + n]
         assert rel_rms(a, b) < 3e-2, k
+
+
+@pytest.mark.parametrize("N,w", [(1, 2), (7, 255), (180, 256), (181, 257), (360, 1024), (900, 4096), (365, 4097)])
+def test_features_at_cell_edges(torch_cuda, N, w):
+    """Cells of one sample, of uneven sizes and across the staged columns:
+    within a bf16 rounding of the oracle's maps."""
+    torch = torch_cuda
+    rng = np.random.default_rng(N + w)
+    P = rng.uniform(0.0, 1.0, (N, w)).astype(np.float32)
+    d_x = torch.zeros((2, 180, 256), dtype=torch.int16, device="cuda")
+    ca.cnn_features_dev(torch.from_numpy(P).cuda(), d_x)
+    got = co.from_bf16_bits(d_x.cpu().numpy().view(np.uint16))
+    ref = co.features(P)
+    # one rounding of values up to 10 in magnitude, and one more flipped by the float32 sums
+    assert np.abs(got - ref).max() <= 2 * 2.0 ** -8 * np.abs(ref).max()
