@@ -5,7 +5,7 @@
 // Score of one trial slice: the one-sided Gaussian smoothing of
 // lct.cpp:837-843 / 878-884 is the circular convolution with
 // g[u]*g[v], g[n] = exp(-n^2 / (2 sigma^2)), evaluated separably with the
-// taps above 1e-9 (a row pass through LDS, then a column pass); then the
+// taps above 1e-9 (a row pass, then a column pass, both in LDS); then the
 // rows [r, w-r) with r = ceil|c| are Sobel-filtered into the matching rows
 // of zeroed full-size derivative arrays, and the magnitude is read from the
 // top w-2r rows of those arrays (the shape mismatch of lct.cpp:905), the
@@ -48,104 +48,146 @@ Taps make_taps(float sigma) {
   return t;
 }
 
-// i mod w for i >= -kMaxTaps: one addition unless the taps outnumber w.
+// i mod w for i >= -(kMaxTaps + 1); w - 1 past the end, which no valid
+// derivative reads.
 __device__ __forceinline__ int wrap_index(int i, int w) {
+  if (i >= w) return w - 1;
   if (i >= 0) return i;
   i += w;
   return i >= 0 ? i : ((i % w) + w) % w;
 }
 
-// Row pass: dst[u][v] = sum_n g[n] src[u][(v - n) mod w]. Grid (w, n).
-__global__ __launch_bounds__(256) void smooth_rows_kernel(const float *__restrict__ src, float *__restrict__ dst,
-                                                          int w, Taps taps) {
-  extern __shared__ float row[];
-  const size_t base = (static_cast<size_t>(blockIdx.y) * w + blockIdx.x) * w;
-  for (int v = threadIdx.x; v < w; v += blockDim.x) row[v] = src[base + v];
-  __syncthreads();
-  for (int v = threadIdx.x; v < w; v += blockDim.x) {
-    float a = 0.0f;
-    for (int n = 0; n < taps.nt; ++n) {
-      a = a + taps.g[n] * row[wrap_index(v - n, w)];
-    }
-    dst[base + v] = a;
+// dst[k] = sum_n g[n] src[k - n] (n ascending) for the four outputs k = 0..3
+// of a line with element stride `st`; src points at output 0.
+__device__ __forceinline__ float4 smooth4(const float *src, int st, const Taps &taps) {
+  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+  float x0 = src[0], x1 = src[st], x2 = src[2 * st], x3 = src[3 * st];
+#pragma unroll 4
+  for (int n = 0; n < taps.nt; ++n) {
+    const float g = taps.g[n];
+    a0 = a0 + g * x0;
+    a1 = a1 + g * x1;
+    a2 = a2 + g * x2;
+    a3 = a3 + g * x3;
+    x3 = x2;
+    x2 = x1;
+    x1 = x0;
+    x0 = src[-min(n + 1, taps.nt - 1) * st];
   }
+  return make_float4(a0, a1, a2, a3);
 }
 
-// Column pass: dst[u][v] = sum_m g[m] src[(u - m) mod w][v]. Grid (w, n).
-__global__ __launch_bounds__(256) void smooth_cols_kernel(const float *__restrict__ src, float *__restrict__ dst,
-                                                          int w, Taps taps) {
-  const int u = blockIdx.x;
-  const size_t sl = static_cast<size_t>(blockIdx.y) * w * w;
-  for (int v = threadIdx.x; v < w; v += blockDim.x) {
-    float a = 0.0f;
-    for (int m = 0; m < taps.nt; ++m) {
-      a = a + taps.g[m] * src[sl + static_cast<size_t>(wrap_index(u - m, w)) * w + v];
-    }
-    dst[sl + static_cast<size_t>(u) * w + v] = a;
-  }
+// Partial sums of the score of slice k = blockIdx.y over the derivative
+// rows and columns of tile blockIdx.x: partial[(k nb + tile) 2 + {0, 1}] =
+// {sum of cS, #(cS > 0)}, nb = gridDim.x. The tile of the slice, with the
+// rows above and the columns to the left that the one-sided smoothing
+// reaches (circularly) and a border of one for the Sobel operator, is read
+// into LDS once; smoothing along rows, along columns and the derivatives
+// follow there, four outputs per thread in the smoothing so that each LDS read
+// serves up to four taps. Bound by LDS reads: nine slices of 2048 px, 8
+// taps, 165 us (628 in three passes over memory).
+constexpr int kScoreTH = 32, kScoreTW = 64;      // derivatives of a tile
+constexpr int kScoreSH = kScoreTH + 4, kScoreSW = kScoreTW + 4;  // smoothed rows and columns: 34 and 66, rounded up to fours
+
+__host__ __device__ inline int score_reach(int nt) { return nt > 0 ? nt - 1 : 0; }
+inline size_t score_lds(int nt) {
+  const int e = score_reach(nt), rows = kScoreSH + e;
+  return sizeof(float) * (static_cast<size_t>(rows) * (kScoreSW + e) + static_cast<size_t>(rows) * kScoreSW);
 }
 
-// Sobel derivative of the cropped slice cs (h x w) at (yy, x), accumulated
-// in the statement order of lct.cpp:887-902; (dy, dx, coefficient) terms.
-__device__ __forceinline__ float sobel_term(const float *cs, int h, int w, int yy, int x, int a, int b, float k,
-                                            float acc) {
-  const int sy = yy - a, sx = x - b;
-  if (sy >= 0 && sy < h && sx >= 0 && sx < w) acc = acc + k * cs[static_cast<size_t>(sy) * w + sx];
-  return acc;
-}
-
-// Partial sums of the score of slice k (blockIdx.y) over the derivative rows
-// y = 1 + blockIdx.x, 1 + blockIdx.x + nb, ... (nb = gridDim.x), lanes over
-// the columns; partial[(k nb + b) 2 + {0, 1}] = {sum of cS, #(cS > 0)}.
-__global__ __launch_bounds__(256) void sobel_score_kernel(const float *__restrict__ slices,
-                                                          const float *__restrict__ centres, int w,
-                                                          int smoothed, double *__restrict__ partial) {
-  const int k = blockIdx.y, nb = gridDim.x;
+__global__ __launch_bounds__(256) void score_kernel(const float *__restrict__ slices, const float *__restrict__ centres,
+                                                    int w, int tiles_x, Taps taps, double *__restrict__ partial) {
+  extern __shared__ float score_buf[];
+  const int e = score_reach(taps.nt), rows = kScoreSH + e, cols = kScoreSW + e;
+  float *src = score_buf;            // [rows][cols], then the smoothed tile [kScoreSH][kScoreSW]
+  float *mid = src + rows * cols;    // [rows][kScoreSW]: smoothed along rows
+  const int tid = threadIdx.x, k = blockIdx.y, nb = gridDim.x;
   const float c = centres[k];
   const int r = static_cast<int>(ceilf(fabsf(c)));
   const int h = w - 2 * r;
-  const float *cs = slices + static_cast<size_t>(k) * w * w + static_cast<size_t>(r) * w;
+  // the full-array row y of lct.cpp:887-912 holds cropped-derivative row
+  // y - r (zero above r): rows y = max(1, r) .. h - 2, columns 1 .. w - 2
+  const int yy0 = blockIdx.x / tiles_x * kScoreTH, x0 = 1 + blockIdx.x % tiles_x * kScoreTW;
+  const int yy_lo = r < 1 ? 1 - r : 0, yy_hi = h - 2 - r;
   double sm = 0.0, cnt = 0.0;
-  // full-array row y holds cropped-derivative row y - r (zero above r):
-  // rows y = max(1, r) .. h - 2, columns 1 .. w - 2
-  for (int y = 1 + blockIdx.x; y <= h - 2; y += nb) {
-    const int yy = y - r;
-    if (yy < 0) continue;
-    for (int x = 1 + threadIdx.x; x <= w - 2; x += blockDim.x) {
+  if (yy0 <= yy_hi) {
+    const float *sl = slices + static_cast<size_t>(k) * w * w;
+    // slice rows r + yy0 - 1 - e .., columns x0 - 1 - e ..
+    for (int b = tid & 63; b < cols; b += 64) {
+      const float *column = sl + wrap_index(x0 - 1 - e + b, w);
+      for (int a0 = tid >> 6; a0 < rows; a0 += 32) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = column[static_cast<size_t>(wrap_index(r + yy0 - 1 - e + a0 + 4 * j, w)) * w];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (a0 + 4 * j < rows) src[(a0 + 4 * j) * cols + b] = v[j];
+      }
+    }
+    __syncthreads();
+    if (taps.nt > 0) {
+      for (int i = tid; i < rows * (kScoreSW / 4); i += 256) {
+        const int a = i / (kScoreSW / 4), b = 4 * (i - a * (kScoreSW / 4));
+        *reinterpret_cast<float4 *>(mid + a * kScoreSW + b) = smooth4(src + a * cols + e + b, 1, taps);
+      }
+      __syncthreads();
+      for (int i = tid; i < (kScoreSH / 4) * kScoreSW; i += 256) {
+        const int a = 4 * (i / kScoreSW), b = i % kScoreSW;
+        const float4 v = smooth4(mid + (e + a) * kScoreSW + b, kScoreSW, taps);
+        float *d = src + a * kScoreSW + b;
+        d[0] = v.x;
+        d[kScoreSW] = v.y;
+        d[2 * kScoreSW] = v.z;
+        d[3 * kScoreSW] = v.w;
+      }
+      __syncthreads();
+    }
+    // rows above the cropped slice count as zero (those below are not reached)
+    auto at = [&](int yy, int x) {
+      return yy < 0 ? 0.0f : src[(yy - yy0 + 1) * kScoreSW + (x - x0 + 1)];
+    };
+    const int x = x0 + (tid & 63);
+    for (int j = tid >> 6; j < kScoreTH; j += 4) {
+      const int yy = yy0 + j;
+      if (yy < yy_lo || yy > yy_hi || x > w - 2) continue;
+      // the statement order of lct.cpp:887-902
+      const float a = at(yy - 1, x - 1), b = at(yy - 1, x), d = at(yy - 1, x + 1);
+      const float p = at(yy, x - 1), q = at(yy, x + 1);
+      const float u = at(yy + 1, x - 1), v = at(yy + 1, x), z = at(yy + 1, x + 1);
       float dH = 0.0f, dV = 0.0f;
-      dH = sobel_term(cs, h, w, yy, x, -1, -1, -1.0f, dH);
-      dH = sobel_term(cs, h, w, yy, x, -1, 0, -2.0f, dH);
-      dH = sobel_term(cs, h, w, yy, x, -1, 1, -1.0f, dH);
-      dH = sobel_term(cs, h, w, yy, x, 1, -1, 1.0f, dH);
-      dH = sobel_term(cs, h, w, yy, x, 1, 0, 2.0f, dH);
-      dH = sobel_term(cs, h, w, yy, x, 1, 1, 1.0f, dH);
-      dV = sobel_term(cs, h, w, yy, x, -1, -1, -1.0f, dV);
-      dV = sobel_term(cs, h, w, yy, x, 0, -1, -2.0f, dV);
-      dV = sobel_term(cs, h, w, yy, x, 1, -1, -1.0f, dV);
-      dV = sobel_term(cs, h, w, yy, x, -1, 1, 1.0f, dV);
-      dV = sobel_term(cs, h, w, yy, x, 0, 1, 2.0f, dV);
-      dV = sobel_term(cs, h, w, yy, x, 1, 1, 1.0f, dV);
+      dH = dH + -1.0f * z;
+      dH = dH + -2.0f * v;
+      dH = dH + -1.0f * u;
+      dH = dH + 1.0f * d;
+      dH = dH + 2.0f * b;
+      dH = dH + 1.0f * a;
+      dV = dV + -1.0f * z;
+      dV = dV + -2.0f * q;
+      dV = dV + -1.0f * d;
+      dV = dV + 1.0f * u;
+      dV = dV + 2.0f * p;
+      dV = dV + 1.0f * a;
       const float m = sqrtf(dH * dH + dV * dV);
       sm += m;
       // #(cS > 0) of lct.cpp:912: the reference's float-FFT smoothing leaves
       // round-off in every pixel, so then every derivative pixel counts.
-      cnt += (smoothed || m > 0.0f) ? 1.0 : 0.0;
+      cnt += (taps.nt > 0 || m > 0.0f) ? 1.0 : 0.0;
     }
   }
-  __shared__ double ps[256], pc[256];
-  ps[threadIdx.x] = sm;
-  pc[threadIdx.x] = cnt;
+  for (int o = 32; o > 0; o >>= 1) {
+    sm += __shfl_xor(sm, o);
+    cnt += __shfl_xor(cnt, o);
+  }
+  __shared__ double ps[4], pc[4];
+  if ((tid & 63) == 0) {
+    ps[tid >> 6] = sm;
+    pc[tid >> 6] = cnt;
+  }
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      ps[threadIdx.x] += ps[threadIdx.x + o];
-      pc[threadIdx.x] += pc[threadIdx.x + o];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    partial[(static_cast<size_t>(k) * nb + blockIdx.x) * 2] = ps[0];
-    partial[(static_cast<size_t>(k) * nb + blockIdx.x) * 2 + 1] = pc[0];
+  if (tid == 0) {
+    double *out = partial + (static_cast<size_t>(k) * nb + blockIdx.x) * 2;
+    out[0] = (ps[0] + ps[1]) + (ps[2] + ps[3]);
+    out[1] = (pc[0] + pc[1]) + (pc[2] + pc[3]);
   }
 }
 
@@ -177,18 +219,18 @@ __global__ __launch_bounds__(256) void score_finish_kernel(const double *__restr
 
 }  // namespace
 
-hipError_t launch_ag_scores(float *d_slices, int n, int w, const float *d_centres, float sigma, float *d_tmp,
+int score_tiles(int w) {
+  return ((w + kScoreTW - 1) / kScoreTW) * ((w + kScoreTH - 1) / kScoreTH);
+}
+
+hipError_t launch_ag_scores(const float *d_slices, int n, int w, const float *d_centres, float sigma,
                             double *d_partial, float *d_scores, hipStream_t s) {
-  if (sigma > 1.0f) {
-    const Taps taps = make_taps(sigma);
-    hipLaunchKernelGGL(smooth_rows_kernel, dim3(w, n), dim3(256), sizeof(float) * w, s, d_slices, d_tmp, w, taps);
-    hipLaunchKernelGGL(smooth_cols_kernel, dim3(w, n), dim3(256), 0, s, d_tmp, d_slices, w, taps);
-  }
-  // as many row blocks per slice as fill the chip, within the partial
-  // buffer's kScoreBlocks x kScoreChunk pairs
-  const int nb = std::max(1, std::min(1024, kScoreBlocks * kScoreChunk / std::max(n, 1)));
-  hipLaunchKernelGGL(sobel_score_kernel, dim3(nb, n), dim3(256), 0, s, d_slices, d_centres, w,
-                     sigma > 1.0f ? 1 : 0, d_partial);
+  Taps taps{};
+  if (sigma > 1.0f) taps = make_taps(sigma);
+  const int nb = score_tiles(w);
+  hipLaunchKernelGGL(score_kernel, dim3(nb, n), dim3(256), score_lds(taps.nt), s, d_slices, d_centres, w,
+                     (w + kScoreTW - 1) / kScoreTW, taps, d_partial);
+  if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   hipLaunchKernelGGL(score_finish_kernel, dim3(n), dim3(256), 0, s, d_partial, d_scores, nb);
   return hipGetLastError();
 }
@@ -267,9 +309,7 @@ extern "C" int ctas_axis_scores(ctas_fbp *h, const float *axisR, int n, float *s
     for (int i = 0; i < m; ++i)
       centres[i] = static_cast<float>(static_cast<double>(axisR[k0 + i]) - 0.5 * (w - 1));
     if (int rc = grow_buf(h->d_out, h->out_cap, sizeof(float) * ww * m)) return rc;
-    if (int rc = grow_buf(h->d_tmp, h->score_cap, sizeof(float) * ww * m)) return rc;
-    size_t pcap = h->d_partial ? sizeof(double) * 2 * kScoreBlocks * kScoreChunk : 0;
-    if (int rc = grow_buf(h->d_partial, pcap, sizeof(double) * 2 * kScoreBlocks * kScoreChunk)) return rc;
+    if (int rc = grow_buf(h->d_partial, h->score_cap, sizeof(double) * 2 * score_tiles(w) * m)) return rc;
     if (!h->d_centres) {
       if (hipMalloc(&h->d_centres, sizeof(float) * kScoreChunk) != hipSuccess ||
           hipMalloc(&h->d_scores, sizeof(float) * kScoreChunk) != hipSuccess)
@@ -279,8 +319,7 @@ extern "C" int ctas_axis_scores(ctas_fbp *h, const float *axisR, int n, float *s
     // scores and their download, then one wait (centres outlives it)
     CTAS_HIP_TRY(hipMemcpyAsync(h->d_centres, centres.data(), sizeof(float) * m, hipMemcpyHostToDevice, h->stream));
     if (int rc = ctas_fbp_repeat_dev(h, 0, h->d_out, centres.data(), m, h->stream)) return rc;
-    CTAS_HIP_TRY(launch_ag_scores(h->d_out, m, w, h->d_centres, sigma, h->d_tmp, h->d_partial, h->d_scores,
-                                  h->stream));
+    CTAS_HIP_TRY(launch_ag_scores(h->d_out, m, w, h->d_centres, sigma, h->d_partial, h->d_scores, h->stream));
     CTAS_HIP_TRY(hipMemcpyAsync(scores + k0, h->d_scores, sizeof(float) * m, hipMemcpyDeviceToHost, h->stream));
     CTAS_HIP_TRY(hipStreamSynchronize(h->stream));
   }

@@ -725,7 +725,7 @@ int ctas_fbp_destroy(ctas_fbp *h) {
   if (h->graph_exec) (void)hipGraphExecDestroy(h->graph_exec);
   if (h->graph) (void)hipGraphDestroy(h->graph);
   void *ptrs[] = {h->d_W, h->d_sincos, h->d_sincos64, h->d_slots, h->d_slot_tab, h->d_tw, h->d_filt, h->d_io, h->d_out, h->d_minmax,
-                  h->d_status, h->d_items, h->d_centres, h->d_partial, h->d_tmp, h->d_scores};
+                  h->d_status, h->d_items, h->d_centres, h->d_partial, h->d_scores};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (h->stream) (void)hipStreamDestroy(h->stream);

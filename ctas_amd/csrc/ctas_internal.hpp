@@ -213,11 +213,10 @@ hipError_t launch_ts(const float *proj, long long proj_stride, int n_proj, const
 bool ts_odd_basis(int filter, float param, int n, int Z, std::vector<float2> &uv, float &gain);
 // Axis-score kernels (axis.hip).
 // AverageGradient::apply scores of n slices [n][w][w] reconstructed at the
-// given centres (n <= kScoreChunk); d_tmp holds n*w*w floats, d_partial
-// kScoreBlocks*kScoreChunk*2 doubles.
-hipError_t launch_ag_scores(float *d_slices, int n, int w, const float *d_centres, float sigma,
-                            float *d_tmp, double *d_partial, float *d_scores, hipStream_t s);
-constexpr int kScoreBlocks = 128;
+// given centres (n <= kScoreChunk); d_partial holds 2 n score_tiles(w) doubles.
+hipError_t launch_ag_scores(const float *d_slices, int n, int w, const float *d_centres, float sigma,
+                            double *d_partial, float *d_scores, hipStream_t s);
+int score_tiles(int w);
 constexpr int kScoreChunk = 64;  // centres per scoring batch (bounds the scratch slices)
 // Phantom projector (phantom.hip).
 hipError_t launch_phantom(int N, int w, double c, int n_ell, const double *d_ell, double N0,
@@ -297,7 +296,7 @@ struct ctas_fbp {
   float2 *d_minmax = nullptr; int *d_status = nullptr; int mm_cap = 0;  // slices
   ctas::Item *d_items = nullptr; int items_cap = 0;
   float *d_centres = nullptr; int centres_cap = 0;
-  double *d_partial = nullptr; float *d_tmp = nullptr; size_t score_cap = 0;
+  double *d_partial = nullptr; size_t score_cap = 0;
   float *d_scores = nullptr;
   int kept_slices = 0;         // filtered slices held for repeat()
   int last_S = 0;
