@@ -1291,9 +1291,20 @@ __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigne
   }
 }
 
-// Grid-mapped launch: one workgroup per tile; blocks are remapped so that the
-// round-robin dispatch over the 8 XCDs gives each XCD a contiguous range of
-// tiles (neighbouring tiles share sinogram windows in that XCD's L2).
+// Grid-mapped launches: one workgroup per tile. Blocks go to the 8 XCDs in
+// turn; they are remapped so that an XCD gets whole rows of `row` tiles
+// (neighbouring tiles share sinogram windows in its L2), every eighth row of
+// the launch. With one contiguous range of tiles per XCD, a launch of few
+// slices gave some XCDs the rows across the middle of the disc and others
+// those at its top and bottom, where most tiles are outside: 8 slices of
+// 4096 px x 3000 angles, float16, four per workgroup, 14.0 -> 12.0 ms.
+__device__ __forceinline__ int tile_of_block(int row) {
+  const int b = blockIdx.x, n = gridDim.x;
+  if (b >= n - n % (8 * row)) return b;  // the rows left over, in turn
+  const int xcd = b & 7, at = b >> 3;
+  return (at / row * 8 + xcd) * row + at % row;
+}
+
 template <int KIND, int AC, int MODE, int ST>
 constexpr bool use_fx() {
   return MODE == MODE_CTAS && ST != ST_F32;
@@ -1323,12 +1334,10 @@ constexpr int grid_waves() {
 }
 
 template <int KIND, int AC, int MODE, int ST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grid_waves<KIND, AC, MODE, ST>(), grid_waves<KIND, AC, MODE, ST>()))) void bp_grid_kernel(const Item *__restrict__ items, int n_items) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grid_waves<KIND, AC, MODE, ST>(), grid_waves<KIND, AC, MODE, ST>()))) void bp_grid_kernel(const Item *__restrict__ items, int n_items, int row) {
   constexpr int A = eff_ac<KIND, AC, MODE, ST>();
   __shared__ __align__(16) unsigned char lds[stage_bytes<KIND, A, MODE, ST>()];
-  int b = blockIdx.x;
-  const int q = gridDim.x >> 3;
-  if (b < (q << 3)) b = (b & 7) * q + (b >> 3);
+  const int b = tile_of_block(row);
   const Item &it = items[find_item_by_tile(items, n_items, b)];
   if constexpr (use_fx<KIND, A, MODE, ST>())
     bp_tile_px2<KIND, A, ST>(it, b - it.tile_base, lds);
@@ -1338,11 +1347,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grid_waves<
 
 // Mirrored launch: AC slots (2 AC angles) per pass.
 template <int KIND, int AC, int ST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KindGeo<KIND>::WAVES, KindGeo<KIND>::WAVES))) void bp_mirror_kernel(const Item *__restrict__ items, int n_items) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KindGeo<KIND>::WAVES, KindGeo<KIND>::WAVES))) void bp_mirror_kernel(const Item *__restrict__ items, int n_items, int row) {
   __shared__ __align__(16) unsigned char lds[StageMirror<KIND, AC, ST, 1>::BYTES];
-  int b = blockIdx.x;
-  const int q = gridDim.x >> 3;
-  if (b < (q << 3)) b = (b & 7) * q + (b >> 3);
+  const int b = tile_of_block(row);
   const Item &it = items[find_item_by_tile(items, n_items, b)];
   bp_tile_mirror<KIND, AC, ST, 1>(it, b - it.tile_base, lds);
 }
@@ -1362,21 +1369,17 @@ template <> struct GroupShape<2> { static constexpr int AC = 32, WAVES = 3, MIRR
 template <> struct GroupShape<4> { static constexpr int AC = 16, WAVES = 3, MIRROR_WAVES = 2; };
 
 template <int NS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GroupShape<NS>::WAVES, GroupShape<NS>::WAVES))) void bp_group_kernel(const Item *__restrict__ items, int tiles) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GroupShape<NS>::WAVES, GroupShape<NS>::WAVES))) void bp_group_kernel(const Item *__restrict__ items, int tiles, int row) {
   __shared__ __align__(16) unsigned char lds[StageGroup<TK_64x64, GroupShape<NS>::AC, NS>::BYTES];
-  int b = blockIdx.x;
-  const int q = gridDim.x >> 3;
-  if (b < (q << 3)) b = (b & 7) * q + (b >> 3);
+  const int b = tile_of_block(row);
   const int g = b / tiles;
   bp_tile_group<TK_64x64, GroupShape<NS>::AC, NS>(items[g * NS], b - g * tiles, lds);
 }
 
 template <int ST, int NS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GroupShape<NS>::MIRROR_WAVES, GroupShape<NS>::MIRROR_WAVES))) void bp_group_mirror_kernel(const Item *__restrict__ items, int tiles) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GroupShape<NS>::MIRROR_WAVES, GroupShape<NS>::MIRROR_WAVES))) void bp_group_mirror_kernel(const Item *__restrict__ items, int tiles, int row) {
   __shared__ __align__(16) unsigned char lds[StageMirror<TK_64x64, 8, ST, NS>::BYTES];
-  int b = blockIdx.x;
-  const int q = gridDim.x >> 3;
-  if (b < (q << 3)) b = (b & 7) * q + (b >> 3);
+  const int b = tile_of_block(row);
   const int g = b / tiles;
   bp_tile_mirror<TK_64x64, 8, ST, NS>(items[g * NS], b - g * tiles, lds);
 }
@@ -1489,54 +1492,55 @@ hipError_t launch_persist_k(const Item *d_items, int n_items, int total_tiles, i
 }
 
 template <int KIND, int AC, int MODE>
-hipError_t launch_kas(const Item *d_items, int n_items, int total_tiles, int store, hipStream_t s) {
+hipError_t launch_kas(const Item *d_items, int n_items, int total_tiles, int row, int store, hipStream_t s) {
   switch (store) {
-    case ST_F32: hipLaunchKernelGGL((bp_grid_kernel<KIND, AC, MODE, ST_F32>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items); break;
-    case ST_F16: hipLaunchKernelGGL((bp_grid_kernel<KIND, AC, MODE, ST_F16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items); break;
-    default: hipLaunchKernelGGL((bp_grid_kernel<KIND, AC, MODE, ST_BF16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items); break;
+    case ST_F32: hipLaunchKernelGGL((bp_grid_kernel<KIND, AC, MODE, ST_F32>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
+    case ST_F16: hipLaunchKernelGGL((bp_grid_kernel<KIND, AC, MODE, ST_F16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
+    default: hipLaunchKernelGGL((bp_grid_kernel<KIND, AC, MODE, ST_BF16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
   }
   return hipGetLastError();
 }
 
 template <int KIND, int MODE>
-hipError_t launch_km(const Item *d_items, int n_items, int total_tiles, int ac, int store, hipStream_t s) {
-  if (ac == 16) return launch_kas<KIND, 16, MODE>(d_items, n_items, total_tiles, store, s);
-  return launch_kas<KIND, 32, MODE>(d_items, n_items, total_tiles, store, s);
+hipError_t launch_km(const Item *d_items, int n_items, int total_tiles, int row, int ac, int store, hipStream_t s) {
+  if (ac == 16) return launch_kas<KIND, 16, MODE>(d_items, n_items, total_tiles, row, store, s);
+  return launch_kas<KIND, 32, MODE>(d_items, n_items, total_tiles, row, store, s);
 }
 
 template <int KIND, int AC>
-hipError_t launch_mirror(const Item *d_items, int n_items, int total_tiles, int store, hipStream_t s) {
+hipError_t launch_mirror(const Item *d_items, int n_items, int total_tiles, int row, int store, hipStream_t s) {
   if (store == ST_F16)
-    hipLaunchKernelGGL((bp_mirror_kernel<KIND, AC, ST_F16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items);
+    hipLaunchKernelGGL((bp_mirror_kernel<KIND, AC, ST_F16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
   else if (store == ST_BF16_H)
-    hipLaunchKernelGGL((bp_mirror_kernel<KIND, AC, ST_BF16_H>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items);
+    hipLaunchKernelGGL((bp_mirror_kernel<KIND, AC, ST_BF16_H>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
   else
-    hipLaunchKernelGGL((bp_mirror_kernel<KIND, AC, ST_BF16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items);
+    hipLaunchKernelGGL((bp_mirror_kernel<KIND, AC, ST_BF16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
   return hipGetLastError();
 }
 
 template <int KIND>
-hipError_t launch_k(const Item *d_items, int n_items, int total_tiles, int ac, int mode, int store, bool mirror,
-                    hipStream_t s) {
+hipError_t launch_k(const Item *d_items, int n_items, int total_tiles, int row, int ac, int mode, int store,
+                    bool mirror, hipStream_t s) {
   // 8 slots (16 angles) per pass: the staging registers of 16 slots spill
-  if (mirror) return launch_mirror<KIND, 8>(d_items, n_items, total_tiles, store, s);
-  if (mode == MODE_LINEAR) return launch_km<KIND, MODE_LINEAR>(d_items, n_items, total_tiles, ac, store, s);
-  return launch_km<KIND, MODE_CTAS>(d_items, n_items, total_tiles, ac, store, s);
+  if (mirror) return launch_mirror<KIND, 8>(d_items, n_items, total_tiles, row, store, s);
+  if (mode == MODE_LINEAR) return launch_km<KIND, MODE_LINEAR>(d_items, n_items, total_tiles, row, ac, store, s);
+  return launch_km<KIND, MODE_CTAS>(d_items, n_items, total_tiles, row, ac, store, s);
 }
 
 }  // namespace
 
-hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles, int kind,
+hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles, int row, int kind,
                               int angles_per_pass, int mode, int store, bool mirror, hipStream_t s) {
   if (total_tiles <= 0) return hipSuccess;
+  if (row < 1) return hipErrorInvalidValue;
   if (mirror && mode == MODE_LINEAR) {
     // 64x64 tiles: the 16-byte float words of both windows (16-bit samples
     // converted when staged) fill the static LDS of a workgroup at 4 slots
     if (kind != TK_64x64) return hipErrorInvalidValue;
     switch (store) {
-      case ST_F32: hipLaunchKernelGGL((bp_mirror_kernel<TK_64x64, 4, ST_F32_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items); break;
-      case ST_F16: hipLaunchKernelGGL((bp_mirror_kernel<TK_64x64, 4, ST_F16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items); break;
-      default: hipLaunchKernelGGL((bp_mirror_kernel<TK_64x64, 4, ST_BF16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items); break;
+      case ST_F32: hipLaunchKernelGGL((bp_mirror_kernel<TK_64x64, 4, ST_F32_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
+      case ST_F16: hipLaunchKernelGGL((bp_mirror_kernel<TK_64x64, 4, ST_F16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
+      default: hipLaunchKernelGGL((bp_mirror_kernel<TK_64x64, 4, ST_BF16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
     }
     return hipGetLastError();
   }
@@ -1549,44 +1553,45 @@ hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles,
     // 2048 x 1800 864 / 852 / 1039.
     if (mode != MODE_CTAS || store != ST_F32) return hipErrorInvalidValue;
     if (kind == TK_32x32)
-      hipLaunchKernelGGL((bp_grid_kernel<TK_32x32, 64, MODE_CTAS, ST_F32>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items);
+      hipLaunchKernelGGL((bp_grid_kernel<TK_32x32, 64, MODE_CTAS, ST_F32>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
     else
-      hipLaunchKernelGGL((bp_grid_kernel<TK_16x32, 64, MODE_CTAS, ST_F32>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items);
+      hipLaunchKernelGGL((bp_grid_kernel<TK_16x32, 64, MODE_CTAS, ST_F32>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
     return hipGetLastError();
   }
   switch (kind) {
-    case TK_64x64: return launch_k<TK_64x64>(d_items, n_items, total_tiles, angles_per_pass, mode, store, mirror, s);
-    case TK_128x64: return launch_k<TK_128x64>(d_items, n_items, total_tiles, angles_per_pass, mode, store, mirror, s);
-    default: return launch_k<TK_128x128>(d_items, n_items, total_tiles, angles_per_pass, mode, store, mirror, s);
+    case TK_64x64: return launch_k<TK_64x64>(d_items, n_items, total_tiles, row, angles_per_pass, mode, store, mirror, s);
+    case TK_128x64: return launch_k<TK_128x64>(d_items, n_items, total_tiles, row, angles_per_pass, mode, store, mirror, s);
+    default: return launch_k<TK_128x128>(d_items, n_items, total_tiles, row, angles_per_pass, mode, store, mirror, s);
   }
 }
 
 namespace {
 
 template <int NS>
-hipError_t launch_group(const Item *d_items, int n_groups, int tiles, int store, bool mirror, hipStream_t s) {
+hipError_t launch_group(const Item *d_items, int n_groups, int tiles, int row, int store, bool mirror, hipStream_t s) {
   const dim3 grid(n_groups * tiles), block(256);
   if (!mirror) {
-    hipLaunchKernelGGL((bp_group_kernel<NS>), grid, block, 0, s, d_items, tiles);
+    hipLaunchKernelGGL((bp_group_kernel<NS>), grid, block, 0, s, d_items, tiles, row);
     return hipGetLastError();
   }
   switch (store) {
-    case ST_F16: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_F16, NS>), grid, block, 0, s, d_items, tiles); break;
-    case ST_BF16_H: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_BF16_H, NS>), grid, block, 0, s, d_items, tiles); break;
-    default: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_BF16, NS>), grid, block, 0, s, d_items, tiles); break;
+    case ST_F16: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_F16, NS>), grid, block, 0, s, d_items, tiles, row); break;
+    case ST_BF16_H: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_BF16_H, NS>), grid, block, 0, s, d_items, tiles, row); break;
+    default: hipLaunchKernelGGL((bp_group_mirror_kernel<ST_BF16, NS>), grid, block, 0, s, d_items, tiles, row); break;
   }
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_backproject_groups(const Item *d_items, int n_groups, int group, int tiles, int store, bool mirror,
-                                     hipStream_t s) {
+hipError_t launch_backproject_groups(const Item *d_items, int n_groups, int group, int tiles, int row, int store,
+                                     bool mirror, hipStream_t s) {
   if (n_groups <= 0) return hipSuccess;
+  if (row < 1) return hipErrorInvalidValue;
   if (mirror ? store == ST_F32 : store != ST_F32) return hipErrorInvalidValue;
   switch (group) {
-    case 2: return launch_group<2>(d_items, n_groups, tiles, store, mirror, s);
-    case 4: return launch_group<4>(d_items, n_groups, tiles, store, mirror, s);
+    case 2: return launch_group<2>(d_items, n_groups, tiles, row, store, mirror, s);
+    case 4: return launch_group<4>(d_items, n_groups, tiles, row, store, mirror, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -288,13 +288,13 @@ std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *center
 int launch_planned(const ctas_fbp *h, const std::vector<BpLaunch> &launches, hipStream_t s) {
   const std::vector<Item> &items = extra(h).resident;
   for (const BpLaunch &l : launches) {
-    const int tiles = items[l.first].tiles, mode = mode_of(h->flags);
+    const int tiles = items[l.first].tiles, row = items[l.first].tiles_x, mode = mode_of(h->flags);
     const bool mirror = use_mirror(h, l.kind);
     const int st = bp_store(store_of(h->flags), h->contrast, mirror);
     if (l.group > 1)
-      CTAS_HIP_TRY(launch_backproject_groups(h->d_items + l.first, l.items / l.group, l.group, tiles, st, mirror, s));
+      CTAS_HIP_TRY(launch_backproject_groups(h->d_items + l.first, l.items / l.group, l.group, tiles, row, st, mirror, s));
     else
-      CTAS_HIP_TRY(launch_backproject(h->d_items + l.first, l.items, tiles * l.items, l.kind, choose_ac(h), mode, st,
+      CTAS_HIP_TRY(launch_backproject(h->d_items + l.first, l.items, tiles * l.items, row, l.kind, choose_ac(h), mode, st,
                                       mirror, s));
   }
   return CTAS_OK;

@@ -178,13 +178,14 @@ hipError_t launch_filter(const Item *d_items, int n_items, int total_pairs, int 
 // Backprojection of all tiles of all items (grid-mapped).
 // mirror: FP16/BF16 storage with CTAS sampling, items carry mirror slots and
 // their tiles cover the columns up to w/2 together with the mirrored ones.
-hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles, int kind,
+// row: tiles in a row of an item (Item::tiles_x, the same for all).
+hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles, int row, int kind,
                               int angles_per_pass, int mode, int store, bool mirror, hipStream_t s);
 // CTAS sampling of n_groups groups of `group` (2 or 4) slices of one shape
 // and centre that lie back to back in d_items, on 64x64 tiles (`tiles` per
 // slice): float32 storage, or 16-bit storage through mirrored angle pairs.
-hipError_t launch_backproject_groups(const Item *d_items, int n_groups, int group, int tiles, int store, bool mirror,
-                                     hipStream_t s);
+hipError_t launch_backproject_groups(const Item *d_items, int n_groups, int group, int tiles, int row, int store,
+                                     bool mirror, hipStream_t s);
 // Same, one persistent launch with a work counter over the tiles of items of
 // one tile kind and pass length (widths and angle counts may differ); mirror:
 // FP16/BF16 items whose angles pair up (Item::slots). cus: compute units.
