@@ -1390,7 +1390,7 @@ __global__ void reset_counter_kernel(unsigned *counter) { *counter = 0u; }
 // pull tiles from a global counter until every tile of every item is done.
 // One launch serves items of uneven width that share a tile kind and pass
 // length; each variant keeps the register budget of its grid kernel. The
-// items come costliest first, so the launch ends with the small tiles.
+// items come with the most angles first, so the launch ends with cheap tiles.
 template <class Tile>
 __device__ __forceinline__ void persistent_loop(const Item *__restrict__ items, int n_items, int total_tiles,
                                                 unsigned *counter, Tile tile) {

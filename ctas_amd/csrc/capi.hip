@@ -1059,7 +1059,7 @@ int ctas_fbp_batch_uneven(const ctas_batch_item *items, int n, int contrast, int
   struct Entry {
     int src, kind, ac;
     bool mirror;
-    double cost;
+    int cost;  // of a tile: its angles
     GeomRes g;
   };
   std::vector<Entry> ents(n);
@@ -1073,10 +1073,12 @@ int ctas_fbp_batch_uneven(const ctas_batch_item *items, int n, int contrast, int
     e.ac = pk.second;
     e.mirror = mirror_applies(flags, bi.n_angles, bi.w, e.g.n_paired) ||
                mirror_linear_applies(flags, bi.n_angles, bi.w, e.g.n_paired, e.kind);
-    e.cost = static_cast<double>(bi.w) * bi.w * bi.n_angles;
+    e.cost = bi.n_angles;
   }
-  // One persistent launch per (tile kind, pass length, mirrored) group, its
-  // items costliest first, so that each launch ends with the small tiles.
+  // One persistent launch per (tile kind, pass length, mirrored) group, the
+  // items of the most angles first: a tile costs its angles whatever the width
+  // of its item, and the launch ends with the cheap ones (16 items of 512 to
+  // 2048 px: 2250 us by the items' cost, 2116 by the tiles').
   std::stable_sort(ents.begin(), ents.end(), [](const Entry &a, const Entry &b) {
     if (a.mirror != b.mirror) return a.mirror < b.mirror;
     if (a.kind != b.kind) return a.kind < b.kind;
