@@ -142,6 +142,13 @@ hipError_t gemm(FA fa, FB fb, FC fc, int M, int N, int K, hipStream_t s, int spl
   return hipGetLastError();
 }
 
+// ---- the network -----------------------------------------------------------------
+struct Layer {
+  int cin, cout, H, W;  // conv: input channels, output channels, spatial size
+};
+constexpr Layer kConv[4] = {{2, 32, 180, 256}, {32, 32, 90, 128}, {32, 64, 45, 64}, {64, 64, 22, 32}};
+constexpr int kF = 64 * 11 * 16, kH1 = 16, kOut = 2;
+
 // ---- operand functors ---------------------------------------------------------
 struct DenseA {  // A[m][k] bf16, row stride ld
   const uint16_t *p;
@@ -182,15 +189,6 @@ struct ActBT {  // B(n, k) = act[n][k]
 };
 
 // ---- store functors -------------------------------------------------------------
-struct StoreConvAct {  // y[b][co][y][x] = leaky(acc + bias[co]) as bf16
-  uint16_t *y;
-  const float *bias;
-  int C, H, W;
-  __device__ void operator()(int co, int n, float v, int) const {
-    const int hw = H * W, b = n / hw, p = n - b * hw;
-    y[(static_cast<size_t>(b) * C + co) * hw + p] = bf16_rne(leaky(v + bias[co]));
-  }
-};
 struct StoreDX {  // dx[b][ci][y][x] (fp32)
   float *dx;
   int C, H, W;
@@ -204,20 +202,6 @@ struct StorePartial {  // ws[split][m][n]
   int M, N;
   __device__ void operator()(int m, int n, float v, int z) const {
     ws[(static_cast<size_t>(z) * M + m) * N + n] = v;
-  }
-};
-struct StoreFC {  // out[b][o] = acc + bias[o] (leaky ReLU optional), bf16 and/or fp32
-  uint16_t *y16;
-  float *y32;
-  const float *bias;
-  int O;
-  bool relu;
-  __device__ void operator()(int o, int b, float v, int) const {
-    float r = v + bias[o];
-    if (relu) r = leaky(r);
-    const size_t i = static_cast<size_t>(b) * O + o;
-    if (y16) y16[i] = bf16_rne(r);
-    if (y32) y32[i] = r;
   }
 };
 struct StoreFlatDX {  // dx[b][f] fp32 from C(f, b)
@@ -565,12 +549,14 @@ __global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ 
     }
   };
   weights(0);
+  u16x8 o_next = *reinterpret_cast<const u16x8 *>(offs + g8);
   for (int c = 0; c < G::STEPS; ++c) {
     bf16x8 a[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, next[m]);
     if (G::STEPS > 1) weights(min(c + 1, G::STEPS - 1));
-    const u16x8 o = *reinterpret_cast<const u16x8 *>(offs + 32 * c + g8);
+    const u16x8 o = o_next;
+    o_next = *reinterpret_cast<const u16x8 *>(offs + 32 * min(c + 1, G::STEPS - 1) + g8);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       u16x8 e;
@@ -650,6 +636,61 @@ __global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ 
   }
 }
 
+// End of the network, 16 samples per workgroup: h = leaky(sum over splits of
+// ws[z][unit][sample] + b1) as bf16 (the first fully connected layer's
+// product, split over k), out = w2 h + b2. The sum runs over the splits in
+// order, so 1024 threads stage 64 splits at a time for the 256 that add them.
+// One sample 6.4 us, 64 samples 8.6 (9.1 and 9.8 with the second layer apart).
+__global__ __launch_bounds__(1024) void head_kernel(const float *__restrict__ ws, int splits,
+                                                    const float *__restrict__ b1, const uint16_t *__restrict__ w2,
+                                                    const float *__restrict__ b2, uint16_t *__restrict__ h1,
+                                                    float *__restrict__ out, int B) {
+  constexpr int C = 64;  // splits at a time
+  __shared__ float part[C][256];  // [unit][sample] of a split
+  __shared__ __align__(16) uint16_t hs[16][16];  // [sample][unit]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g8 = (lane >> 4) * 8;
+  const int s0 = blockIdx.x * 16;
+  const int o = tid & 255, g = tid >> 8;  // output (unit o / 16, sample o % 16), quarter of the splits
+  const size_t at = static_cast<size_t>(o >> 4) * B + min(s0 + (o & 15), B - 1);
+  float v = 0.0f;
+  for (int z0 = 0; z0 < splits; z0 += C) {
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < C / 4; ++j)
+      part[g + 4 * j][o] = ws[static_cast<size_t>(min(z0 + g + 4 * j, splits - 1)) * kH1 * B + at];
+    __syncthreads();
+    if (tid < 256) {
+      const int n = min(C, splits - z0);
+      if (n == C) {
+#pragma unroll
+        for (int z = 0; z < C; ++z) v += part[z][tid];
+      } else {
+        for (int z = 0; z < n; ++z) v += part[z][tid];
+      }
+    }
+  }
+  if (tid < 256) {
+    const int u = tid >> 4, smp = tid & 15;
+    const uint16_t h = bf16_rne(leaky(v + b1[u]));
+    hs[smp][u] = h;
+    if (s0 + smp < B) h1[static_cast<size_t>(s0 + smp) * kH1 + u] = h;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  // out[o][sample]: 16 units of the 32 a matrix instruction multiplies
+  u16x8 a = {}, b = {};
+  if (g8 < 16) {
+    if (r16 < kOut) a = *reinterpret_cast<const u16x8 *>(w2 + r16 * kH1 + g8);
+    b = *reinterpret_cast<const u16x8 *>(&hs[r16][g8]);
+  }
+  f4 acc = {0.f, 0.f, 0.f, 0.f};
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+  if (lane < 16 && s0 + r16 < B) {
+#pragma unroll
+    for (int o = 0; o < kOut; ++o) out[static_cast<size_t>(s0 + r16) * kOut + o] = acc[o] + b2[o];
+  }
+}
+
 // The weights of layers two to four as the input gradients' products take
 // them: wt[ci][co*9 + tap] = w[co][ci*9 + tap], layer l at its own offset.
 __global__ __launch_bounds__(256) void transpose_weights(const uint16_t *__restrict__ w, uint16_t *__restrict__ wt,
@@ -679,42 +720,6 @@ __global__ __launch_bounds__(256) void reduce_splits(const float *__restrict__ w
     for (int k = 1; k < 16; ++k) t += part[k][o];
     out[i] = t;
   }
-}
-
-// Epilogue of a split forward product: y[b][m][p] = bf16(leaky(sum over
-// splits of ws[z][m][n] + bias[m])), n = b*HW + p, 16 outputs per workgroup.
-// The sum runs over the splits in order, so 256 threads stage 64 splits at a
-// time for the 16 that add them: 176 splits of one sample's first fully
-// connected layer take 3.6 us (29 with each thread's loads one after another),
-// those of 64 samples 5.3 (42).
-__global__ __launch_bounds__(256) void finish_act(const float *__restrict__ ws, int splits, int M, int N,
-                                                  const float *__restrict__ bias, uint16_t *__restrict__ y, int HW) {
-  constexpr int C = 64;
-  __shared__ float stage[C][17];
-  const int o = threadIdx.x & 15, g = threadIdx.x >> 4, i = blockIdx.x * 16 + o;
-  const int at = min(i, M * N - 1);
-  float v = 0.0f;
-  for (int z0 = 0; z0 < splits; z0 += C) {
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < C / 16; ++j) {
-      const int z = z0 + g + 16 * j;
-      stage[g + 16 * j][o] = ws[static_cast<size_t>(min(z, splits - 1)) * M * N + at];
-    }
-    __syncthreads();
-    if (g == 0) {
-      const int n = min(C, splits - z0);
-      if (n == C) {
-#pragma unroll
-        for (int z = 0; z < C; ++z) v += stage[z][o];
-      } else {
-        for (int z = 0; z < n; ++z) v += stage[z][o];
-      }
-    }
-  }
-  if (g != 0 || i >= M * N) return;
-  const int m = i / N, n = i - m * N, b = n / HW, p = n - b * HW;
-  y[(static_cast<size_t>(b) * M + m) * HW + p] = bf16_rne(leaky(v + bias[m]));
 }
 
 // Bias gradient of a fully connected layer: sum of the slope-scaled gradient
@@ -857,26 +862,36 @@ __global__ __launch_bounds__(kFeatT) void features_kernel(const float *__restric
   const int c0 = static_cast<int>(static_cast<long long>(x) * w / kFeatW);
   const int c1 = max(c0 + 1, static_cast<int>(static_cast<long long>(x + 1) * w / kFeatW));
   constexpr int PT = kFeatCols / kFeatT;
-  const int nseg = (w + kFeatCols - 1) / kFeatCols, steps = (r1 - r0) * nseg;
+  // a step takes as many whole rows as fit, or a part of one row
+  const int rps = max(1, kFeatCols / w), nseg = (w + kFeatCols - 1) / kFeatCols;
+  const int steps = nseg > 1 ? (r1 - r0) * nseg : (r1 - r0 + rps - 1) / rps;
+  const size_t last = static_cast<size_t>(r1) * w - 1;  // of the cell's samples
   float v[PT];
   auto fetch = [&](int k) {
-    const int r = r0 + k / nseg, b = (k % nseg) * kFeatCols;
-    const float *row = sino + static_cast<size_t>(r) * w;
+    const size_t at = static_cast<size_t>(r0 + (nseg > 1 ? k / nseg : k * rps)) * w + (nseg > 1 ? (k % nseg) * kFeatCols : 0);
 #pragma unroll
-    for (int j = 0; j < PT; ++j) v[j] = row[min(b + x + kFeatT * j, w - 1)];
+    for (int j = 0; j < PT; ++j) {
+      const size_t i = at + x + kFeatT * j;
+      v[j] = sino[i < last ? i : last];
+    }
   };
   fetch(0);
   float s = 0.0f;
   for (int k = 0; k < steps; ++k) {
-    const int b = (k % nseg) * kFeatCols;
     float *buf = line[k & 1];
 #pragma unroll
-    for (int j = 0; j < PT; ++j)
-      if (b + x + kFeatT * j < w) buf[x + kFeatT * j] = -logf(fmaxf(v[j], 1e-6f));
+    for (int j = 0; j < PT; ++j) buf[x + kFeatT * j] = -logf(fmaxf(v[j], 1e-6f));
     if (k + 1 < steps) fetch(k + 1);
     __syncthreads();
-    if (x < kFeatW)
+    if (x >= kFeatW) continue;
+    if (nseg > 1) {
+      const int b = (k % nseg) * kFeatCols;
       for (int c = max(c0, b); c < min(c1, b + kFeatCols); ++c) s += buf[c - b];
+    } else {
+      const int rows = min(rps, r1 - r0 - k * rps);
+      for (int r = 0; r < rows; ++r)
+        for (int c = c0; c < c1; ++c) s += buf[r * w + c];
+    }
   }
   if (x < kFeatW) tmp[a * kFeatW + x] = s / static_cast<float>((r1 - r0) * (c1 - c0));
 }
@@ -928,13 +943,6 @@ hipError_t launch_features(const float *d_sino, int N, int w, float *d_tmp, uint
   hipLaunchKernelGGL(standardise_kernel, dim3(kFeatA * kFeatW / 1024), dim3(1024), 0, s, d_tmp, d_x);
   return hipGetLastError();
 }
-
-// ---- the network -----------------------------------------------------------------
-struct Layer {
-  int cin, cout, H, W;  // conv: input channels, output channels, spatial size
-};
-constexpr Layer kConv[4] = {{2, 32, 180, 256}, {32, 32, 90, 128}, {32, 64, 45, 64}, {64, 64, 22, 32}};
-constexpr int kF = 64 * 11 * 16, kH1 = 16, kOut = 2;
 
 struct Param {
   size_t off, n;
@@ -1037,26 +1045,6 @@ int forward_splits(int M, int N, int K) {
   return std::max(1, std::min((256 + tiles - 1) / tiles, K / 64));
 }
 
-// A product with bias + ReLU + bf16 epilogue: direct store when it fills
-// the chip, else split over K into the workspace and finished in a fixed
-// order.
-template <class FA, class FB>
-int product_act(ctas_cnn *n, FA fa, FB fb, int M, int Ncols, int K, const float *bias, uint16_t *y, int HW) {
-  hipStream_t s = n->stream;
-  const int splits = forward_splits(M, Ncols, K);
-  if (splits == 1) {
-    CTAS_HIP_TRY(gemm(fa, fb, StoreConvAct{y, bias, M, 1, HW}, M, Ncols, K, s));
-    return CTAS_OK;
-  }
-  if (int rc = ensure_ws(n, static_cast<size_t>(splits) * M * Ncols)) return rc;
-  int chunk = (K + splits - 1) / splits;
-  chunk = (chunk + kKS - 1) & ~(kKS - 1);
-  const int real = (K + chunk - 1) / chunk;
-  CTAS_HIP_TRY(gemm(fa, fb, StorePartial{n->ws, M, Ncols}, M, Ncols, K, s, splits));
-  hipLaunchKernelGGL(finish_act, dim3((M * Ncols + 15) / 16), dim3(256), 0, s, n->ws, real, M, Ncols, bias, y, HW);
-  return CTAS_OK;
-}
-
 // Convolution layer l with its pooling. The sums are those of a product
 // split over k where one of 64x64 tiles would not fill the chip.
 template <int L, int CI, int CO, int H, int W>
@@ -1085,10 +1073,14 @@ int forward(ctas_cnn *n, const uint16_t *x, int B) {
   CTAS_HIP_TRY((conv_forward<1, 32, 32, 90, 128>(n, n->pool[0], B)));
   CTAS_HIP_TRY((conv_forward<2, 32, 64, 45, 64>(n, n->pool[1], B)));
   CTAS_HIP_TRY((conv_forward<3, 64, 64, 22, 32>(n, n->pool[2], B)));
-  if (int rc = product_act(n, DenseA{W16(n, 8), kF}, ActB{n->pool[3], kF}, kH1, B, kF, P32(n, 9), n->h1, 1))
-    return rc;
-  CTAS_HIP_TRY(gemm(DenseA{W16(n, 10), kH1}, ActB{n->h1, kH1}, StoreFC{nullptr, n->out, P32(n, 11), kOut, false},
-                    kOut, B, kH1, s));
+  int splits = forward_splits(kH1, B, kF);
+  const int chunk = ((kF + splits - 1) / splits + kKS - 1) & ~(kKS - 1);
+  if (int rc = ensure_ws(n, static_cast<size_t>(splits) * kH1 * B)) return rc;
+  CTAS_HIP_TRY(gemm(DenseA{W16(n, 8), kF}, ActB{n->pool[3], kF}, StorePartial{n->ws, kH1, B}, kH1, B, kF, s, splits));
+  splits = (kF + chunk - 1) / chunk;  // those that hold any k
+  hipLaunchKernelGGL(head_kernel, dim3((B + 15) / 16), dim3(1024), 0, s, n->ws, splits, P32(n, 9), W16(n, 10),
+                     P32(n, 11), n->h1, n->out, B);
+  CTAS_HIP_TRY(hipGetLastError());
   return CTAS_OK;
 }
 
