@@ -211,44 +211,53 @@ struct StoreFlatDX {  // dx[b][f] fp32 from C(f, b)
 };
 
 // ---- elementwise kernels -------------------------------------------------------------
+// What the backward pass has to know of a window of the pooling: its first
+// maximum's place (two bits: row, column) and whether that is positive.
+__device__ __forceinline__ uint32_t pool_code(uint16_t a, uint16_t b, uint16_t c, uint16_t d) {
+  const float v[4] = {bf16_f(a), bf16_f(b), bf16_f(c), bf16_f(d)};
+  uint32_t at = 0;
+  float best = v[0];
+#pragma unroll
+  for (int k = 1; k < 4; ++k)
+    if (v[k] > best) {
+      best = v[k];
+      at = k;
+    }
+  return at | (best > 0.0f ? 4u : 0u);
+}
+
 // Backward of the pooling and of the leaky ReLU, and the bias gradient, in
 // one pass over a channel of a sample (block (co, b)): the pooled gradient dy
 // goes to the first maximum of its window, scaled by the slope of that
 // post-activation, as bf16 (the operand of the products that follow; every
 // other pixel gets zero, rows beyond the pooled extent too); part[co][b]
-// receives its sum before rounding. A thread takes four windows: two 16-byte
-// reads, one of dy, two writes. Bound by HBM: 28 us a layer on average for 64
-// samples (158 with the gradient in float32 and its bias sums apart).
-__global__ __launch_bounds__(256) void pool_bwd(const uint16_t *__restrict__ act, const float *__restrict__ dy,
+// receives its sum before rounding. A thread takes four windows: one read of
+// their codes, one of dy, two writes. Bound by HBM, whose bytes are the
+// writes and half as many reads: 20 us a layer on average for 64 samples, 51
+// for the first (31 from activations of full size, which the forward pass then
+// has to write; 158 with the gradient in float32 and its bias sums apart).
+__global__ __launch_bounds__(256) void pool_bwd(const uint8_t *__restrict__ code, const float *__restrict__ dy,
                                                 uint16_t *__restrict__ g, float *__restrict__ part, int B, int C,
                                                 int H, int W) {
   const int co = blockIdx.x, b = blockIdx.y;
   const int Ho = H / 2, Wo = W / 2, Q = Wo / 4;  // W is a multiple of 8
   const size_t plane = static_cast<size_t>(b) * C + co;
-  const uint16_t *a = act + plane * H * W;
   uint16_t *gp = g + plane * H * W;
   const float4 *d4 = reinterpret_cast<const float4 *>(dy + plane * Ho * Wo);
+  const uint32_t *c4 = reinterpret_cast<const uint32_t *>(code + plane * Ho * Wo);
   float s = 0.0f;
   for (int i = threadIdx.x; i < Ho * Q; i += 256) {
     const int yo = i / Q, q = i - yo * Q;
     const size_t at = static_cast<size_t>(2 * yo) * W + 8 * q;
-    const u16x8 r0 = *reinterpret_cast<const u16x8 *>(a + at), r1 = *reinterpret_cast<const u16x8 *>(a + at + W);
+    const uint32_t c = c4[i];
     const float4 d = d4[i];
     const float dv[4] = {d.x, d.y, d.z, d.w};
-    u16x8 g0 = {}, g1 = {};
+    u16x8 g0, g1;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float v[4] = {bf16_f(r0[2 * j]), bf16_f(r0[2 * j + 1]), bf16_f(r1[2 * j]), bf16_f(r1[2 * j + 1])};
-      int am = 0;
-      float best = v[0];
-#pragma unroll
-      for (int k = 1; k < 4; ++k)
-        if (v[k] > best) {
-          best = v[k];
-          am = k;
-        }
-      const float gv = best > 0.0f ? dv[j] : kLeak * dv[j];
+      const float gv = c & (4u << (8 * j)) ? dv[j] : kLeak * dv[j];
       s += gv;
+      const uint32_t am = c >> (8 * j) & 3u;
       const uint16_t h = bf16_rne(gv);
       g0[2 * j] = am == 0 ? h : 0;
       g0[2 * j + 1] = am == 1 ? h : 0;
@@ -466,8 +475,8 @@ __global__ __launch_bounds__(64) void wgrad_taps_kernel(const uint16_t *__restri
 }
 
 // 3x3 convolution of a layer as a product over k = channel*9 + tap (padding
-// 1): forward (BWD false; bias, leaky ReLU, bf16 output y and its 2x2 maximum
-// `pool`) or the gradient of the layer's input (BWD true: CI the layer's
+// 1): forward (BWD false; bias, leaky ReLU, of the bf16 output its 2x2 maximum
+// `pool` and, where a backward pass follows, the windows' codes) or the gradient of the layer's input (BWD true: CI the layer's
 // output channels, x their bf16 gradients, the stencil mirrored, float32
 // output dx). Four waves share a patch of the input in LDS, with its border
 // (zeros outside the image); each takes all output channels of 2 rows x 32
@@ -476,7 +485,7 @@ __global__ __launch_bounds__(64) void wgrad_taps_kernel(const uint16_t *__restri
 // every k, and reads the weights [CO][K] as the instruction takes them. The
 // gathers bind it: eight 2-byte LDS reads per 16 pixels and 32 k serve CO/16
 // instructions. 64 samples, layers one to four forward with the pooling:
-// 86, 51, 41 and 22 us; backward, layers two to four: 42, 28 and 15 (181 and
+// 84, 53, 41 and 22 us; backward, layers two to four: 42, 28 and 15 (181 and
 // 147 us a layer through the general product, which forms every element's
 // index anew, and a pooling of its own).
 // `per` matrix instructions in a row make a partial sum, and the partial sums
@@ -493,8 +502,8 @@ struct ConvGeo {
 
 template <int CI, int CO, int H, int W, bool BWD>
 __global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-                                                   const float *__restrict__ bias, uint16_t *__restrict__ y,
-                                                   uint16_t *__restrict__ pool, float *__restrict__ dx, int per) {
+                                                   const float *__restrict__ bias, uint16_t *__restrict__ pool,
+                                                   uint8_t *__restrict__ code, float *__restrict__ dx, int per) {
   using G = ConvGeo<CI, CO, H, W>;
   constexpr int K = G::K, MT = G::MT, HW = H * W;
   __shared__ __align__(16) uint16_t patch[G::ELEMS];
@@ -616,22 +625,22 @@ __global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ 
       const int co = 16 * i + (lane >> 2);
       const u16x8 top = *reinterpret_cast<const u16x8 *>(out + co * 64 + 8 * (lane & 3));
       const u16x8 low = *reinterpret_cast<const u16x8 *>(out + co * 64 + 32 + 8 * (lane & 3));
-      const size_t plane = b * CO + co;
-      if (yy < H) *reinterpret_cast<u16x8 *>(y + plane * HW + yy * W + xx) = top;
-      if (yy + 1 < H) {
-        *reinterpret_cast<u16x8 *>(y + plane * HW + (yy + 1) * W + xx) = low;
-        typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-        u16x4 mx;
+      if (yy + 1 >= H) continue;
+      const size_t at = (b * CO + co) * (H / 2) * (W / 2) + (yy / 2) * (W / 2) + xx / 2;
+      typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+      u16x4 mx;
+      uint32_t codes = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float v = bf16_f(top[2 * j]);
-          v = fmaxf(v, bf16_f(top[2 * j + 1]));
-          v = fmaxf(v, bf16_f(low[2 * j]));
-          v = fmaxf(v, bf16_f(low[2 * j + 1]));
-          mx[j] = bf16_rne(v);
-        }
-        *reinterpret_cast<u16x4 *>(pool + plane * (H / 2) * (W / 2) + (yy / 2) * (W / 2) + xx / 2) = mx;
+      for (int j = 0; j < 4; ++j) {
+        float v = bf16_f(top[2 * j]);
+        v = fmaxf(v, bf16_f(top[2 * j + 1]));
+        v = fmaxf(v, bf16_f(low[2 * j]));
+        v = fmaxf(v, bf16_f(low[2 * j + 1]));
+        mx[j] = bf16_rne(v);
+        codes |= pool_code(top[2 * j], top[2 * j + 1], low[2 * j], low[2 * j + 1]) << (8 * j);
       }
+      *reinterpret_cast<u16x4 *>(pool + at) = mx;
+      if (code) *reinterpret_cast<uint32_t *>(code + at) = codes;
     }
   }
 }
@@ -960,7 +969,8 @@ struct ctas_cnn {
   uint16_t *p16 = nullptr, *wt = nullptr;  // bf16 weights; a layer's, transposed
   int step = 0;
   int cap = 0;  // batch capacity of the activation buffers
-  uint16_t *act[4] = {}, *pool[4] = {}, *h1 = nullptr;
+  uint16_t *pool[4] = {}, *h1 = nullptr;
+  uint8_t *code[4] = {};  // of the pooling's windows, for the backward pass
   uint16_t *gact = nullptr;  // bf16 gradient of a layer's pre-activation
   float *out = nullptr, *gout = nullptr, *gh1 = nullptr, *gf = nullptr, *gbig2 = nullptr;
   float *ws = nullptr;
@@ -983,9 +993,10 @@ int alloc(void **p, size_t bytes) {
 
 void release_batch(ctas_cnn *n) {
   for (int l = 0; l < 4; ++l) {
-    if (n->act[l]) (void)hipFree(n->act[l]);
     if (n->pool[l]) (void)hipFree(n->pool[l]);
-    n->act[l] = n->pool[l] = nullptr;
+    if (n->code[l]) (void)hipFree(n->code[l]);
+    n->pool[l] = nullptr;
+    n->code[l] = nullptr;
   }
   void *ptrs[] = {n->h1, n->out, n->gout, n->gh1, n->gf, n->gact, n->gbig2};
   for (void *q : ptrs)
@@ -1005,8 +1016,8 @@ int ensure_batch(ctas_cnn *n, int B) {
     const Layer &L = kConv[l];
     const size_t a = static_cast<size_t>(B) * L.cout * L.H * L.W;
     const size_t q = static_cast<size_t>(B) * L.cout * (L.H / 2) * (L.W / 2);
-    if (int rc = alloc(reinterpret_cast<void **>(&n->act[l]), a * 2)) return rc;
     if (int rc = alloc(reinterpret_cast<void **>(&n->pool[l]), q * 2)) return rc;
+    if (int rc = alloc(reinterpret_cast<void **>(&n->code[l]), q)) return rc;
     big = std::max(big, a);
     big = std::max(big, static_cast<size_t>(B) * L.cin * L.H * L.W);
   }
@@ -1046,13 +1057,14 @@ int forward_splits(int M, int N, int K) {
 }
 
 // Convolution layer l with its pooling. The sums are those of a product
-// split over k where one of 64x64 tiles would not fill the chip.
+// split over k where one of 64x64 tiles would not fill the chip. `codes`: a
+// backward pass follows.
 template <int L, int CI, int CO, int H, int W>
-hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B) {
+hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
   using G = ConvGeo<CI, CO, H, W>;
   const int splits = forward_splits(CO, B * H * W, G::K), per = (G::STEPS + splits - 1) / splits;
   hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, x,
-                     W16(n, 2 * L), P32(n, 2 * L + 1), n->act[L], n->pool[L], nullptr, per);
+                     W16(n, 2 * L), P32(n, 2 * L + 1), n->pool[L], codes ? n->code[L] : nullptr, nullptr, per);
   return hipGetLastError();
 }
 
@@ -1067,12 +1079,12 @@ hipError_t conv_input_grad(ctas_cnn *n, const uint16_t *g, int B) {
   return hipGetLastError();
 }
 
-int forward(ctas_cnn *n, const uint16_t *x, int B) {
+int forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
   hipStream_t s = n->stream;
-  CTAS_HIP_TRY((conv_forward<0, 2, 32, 180, 256>(n, x, B)));
-  CTAS_HIP_TRY((conv_forward<1, 32, 32, 90, 128>(n, n->pool[0], B)));
-  CTAS_HIP_TRY((conv_forward<2, 32, 64, 45, 64>(n, n->pool[1], B)));
-  CTAS_HIP_TRY((conv_forward<3, 64, 64, 22, 32>(n, n->pool[2], B)));
+  CTAS_HIP_TRY((conv_forward<0, 2, 32, 180, 256>(n, x, B, codes)));
+  CTAS_HIP_TRY((conv_forward<1, 32, 32, 90, 128>(n, n->pool[0], B, codes)));
+  CTAS_HIP_TRY((conv_forward<2, 32, 64, 45, 64>(n, n->pool[1], B, codes)));
+  CTAS_HIP_TRY((conv_forward<3, 64, 64, 22, 32>(n, n->pool[2], B, codes)));
   int splits = forward_splits(kH1, B, kF);
   const int chunk = ((kF + splits - 1) / splits + kKS - 1) & ~(kKS - 1);
   if (int rc = ensure_ws(n, static_cast<size_t>(splits) * kH1 * B)) return rc;
@@ -1144,7 +1156,7 @@ int backward(ctas_cnn *n, const uint16_t *x, int B) {
   for (int l = 3; l >= 0; --l) {
     const Layer &L = kConv[l];
     if (int rc = ensure_ws(n, static_cast<size_t>(L.cout) * B)) return rc;
-    hipLaunchKernelGGL(pool_bwd, dim3(L.cout, B), dim3(256), 0, s, n->act[l], gpool, gact, n->ws, B, L.cout, L.H, L.W);
+    hipLaunchKernelGGL(pool_bwd, dim3(L.cout, B), dim3(256), 0, s, n->code[l], gpool, gact, n->ws, B, L.cout, L.H, L.W);
     hipLaunchKernelGGL(bias_grad_sum, dim3(1), dim3(64), 0, s, n->ws, G32(n, 2 * l + 1), B, L.cout);
     // the workspace's bias partials were summed on this stream
     const uint16_t *in = l ? n->pool[l - 1] : x;
@@ -1281,7 +1293,7 @@ extern "C" int ctas_cnn_forward_dev(ctas_cnn *n, const uint16_t *d_x, int B, flo
   if (!n || !d_x || !d_out || B <= 0) return fail(CTAS_E_ARG, "bad arguments");
   if (int rc = stream_wait(n->stream, static_cast<hipStream_t>(stream))) return rc;
   if (int rc = ensure_batch(n, B)) return rc;
-  if (int rc = forward(n, d_x, B)) return rc;
+  if (int rc = forward(n, d_x, B, false)) return rc;
   CTAS_HIP_TRY(hipMemcpyAsync(d_out, n->out, sizeof(float) * kOut * B, hipMemcpyDeviceToDevice, n->stream));
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
   return CTAS_OK;
@@ -1293,7 +1305,7 @@ extern "C" int ctas_cnn_gradients_dev(ctas_cnn *n, const uint16_t *d_x, const fl
   if (!n || !d_x || !d_target || B <= 0) return fail(CTAS_E_ARG, "bad arguments");
   if (int rc = stream_wait(n->stream, static_cast<hipStream_t>(stream))) return rc;
   if (int rc = ensure_batch(n, B)) return rc;
-  if (int rc = forward(n, d_x, B)) return rc;
+  if (int rc = forward(n, d_x, B, true)) return rc;
   hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, n->stream, n->out, d_target, n->gout, n->loss, B);
   if (int rc = backward(n, d_x, B)) return rc;
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
@@ -1478,7 +1490,7 @@ extern "C" int ctas_cnn_predict_dev(ctas_cnn *n, const float *d_sino, int N, int
   if (int rc = ensure_batch(n, 1)) return rc;
   if (!n->xin && alloc(reinterpret_cast<void **>(&n->xin), 2 * kFeatA * kFeatW * 2)) return CTAS_E_NOMEM;
   CTAS_HIP_TRY(launch_features(d_sino, N, w, n->ftmp, n->xin, n->stream));
-  if (int rc = forward(n, n->xin, 1)) return rc;
+  if (int rc = forward(n, n->xin, 1, false)) return rc;
   float o[2];
   CTAS_HIP_TRY(hipMemcpyAsync(o, n->out, sizeof(o), hipMemcpyDeviceToHost, n->stream));
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
