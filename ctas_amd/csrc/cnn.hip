@@ -230,15 +230,15 @@ __device__ __forceinline__ uint32_t pool_code(uint16_t a, uint16_t b, uint16_t c
 // one pass over a channel of a sample (block (co, b)): the pooled gradient dy
 // goes to the first maximum of its window, scaled by the slope of that
 // post-activation, as bf16 (the operand of the products that follow; every
-// other pixel gets zero, rows beyond the pooled extent too); part[co][b]
+// other pixel gets zero, rows beyond the pooled extent too); part[b][co]
 // receives its sum before rounding. A thread takes four windows: one read of
 // their codes, one of dy, two writes. Bound by HBM, whose bytes are the
 // writes and half as many reads: 20 us a layer on average for 64 samples, 51
 // for the first (31 from activations of full size, which the forward pass then
 // has to write; 158 with the gradient in float32 and its bias sums apart).
 __global__ __launch_bounds__(256) void pool_bwd(const uint8_t *__restrict__ code, const float *__restrict__ dy,
-                                                uint16_t *__restrict__ g, float *__restrict__ part, int B, int C,
-                                                int H, int W) {
+                                                uint16_t *__restrict__ g, float *__restrict__ part, int C, int H,
+                                                int W) {
   const int co = blockIdx.x, b = blockIdx.y;
   const int Ho = H / 2, Wo = W / 2, Q = Wo / 4;  // W is a multiple of 8
   const size_t plane = static_cast<size_t>(b) * C + co;
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(256) void pool_bwd(const uint8_t *__restrict__ code
     if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[static_cast<size_t>(co) * B + b] = red[0];
+  if (threadIdx.x == 0) part[static_cast<size_t>(b) * C + co] = red[0];
 }
 
 // Weight gradient of a convolution, split over the pixels: ws[z][co][c] =
@@ -701,74 +701,78 @@ __global__ __launch_bounds__(1024) void head_kernel(const float *__restrict__ ws
 }
 
 // The weights of layers two to four as the input gradients' products take
-// them: wt[ci][co*9 + tap] = w[co][ci*9 + tap], layer l at its own offset.
-__global__ __launch_bounds__(256) void transpose_weights(const uint16_t *__restrict__ w, uint16_t *__restrict__ wt,
-                                                         int cout, int cin) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= cout * cin * 9) return;
+// them, wt[ci][co*9 + tap] = w[co][ci*9 + tap], one layer after the other.
+constexpr int kWtAt[5] = {0, 0, 32 * 32 * 9, 32 * 32 * 9 + 32 * 64 * 9, 32 * 32 * 9 + 32 * 64 * 9 + 64 * 64 * 9};
+__global__ __launch_bounds__(256) void transpose_weights(const uint16_t *__restrict__ w2,
+                                                         const uint16_t *__restrict__ w3,
+                                                         const uint16_t *__restrict__ w4, uint16_t *__restrict__ wt) {
+  int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= kWtAt[4]) return;
+  const int l = i < kWtAt[2] ? 1 : i < kWtAt[3] ? 2 : 3;
+  const int cout = kConv[l].cout, cin = kConv[l].cin;
+  const uint16_t *w = l == 1 ? w2 : l == 2 ? w3 : w4;
+  wt += kWtAt[l];
+  i -= kWtAt[l];
   const int co = i / (cin * 9), q = i - co * cin * 9, ci = q / 9, r = q - 9 * ci;
   wt[(ci * cout + co) * 9 + r] = w[i];
 }
 
-// Sum of the split-K partials (fixed order) into the weight gradient.
-// Sum over the splits of a K-split product, in a fixed order: 16 outputs per
-// block, each summed by 16 threads over interleaved splits (z = g, g + 16,
-// ...) and their 16 partials added in order.
-__global__ __launch_bounds__(256) void reduce_splits(const float *__restrict__ ws, float *__restrict__ out,
-                                                     int splits, int MN) {
-  const int o = threadIdx.x & 15, g = threadIdx.x >> 4;
-  const int i = blockIdx.x * 16 + o;
+// Sums over the splits of a product, in a fixed order, of two products in one
+// launch: 16 outputs per block, each summed by G threads over interleaved
+// splits (z = g, g + G, ...) and their G partials added in order. Bound by the
+// latency of a thread's loads, which are independent: 64 threads per output
+// from 256 splits on (2002 splits of 576 outputs 5 us, 720 of 9216 11 us; 38 and
+// 16 with 16 threads), 16 below, where most of 64 would find none (180 and 44
+// splits: 5.5 us, a launch).
+struct Partials {
+  const float *ws;  // [splits][MN]
+  float *out;
+  int splits, MN;
+};
+template <int G>
+__global__ __launch_bounds__(16 * G) void reduce_splits(Partials a, Partials b) {
+  const int o = threadIdx.x & 15, g = threadIdx.x >> 4, blocks_a = (a.MN + 15) / 16;
+  const Partials p = static_cast<int>(blockIdx.x) < blocks_a ? a : b;
+  const int i = (blockIdx.x - (static_cast<int>(blockIdx.x) < blocks_a ? 0 : blocks_a)) * 16 + o;
   float s = 0.0f;
-  if (i < MN)
-    for (int z = g; z < splits; z += 16) s += ws[static_cast<size_t>(z) * MN + i];
-  __shared__ float part[16][17];
+  if (i < p.MN) {
+#pragma unroll 8
+    for (int z = g; z < p.splits; z += G) s += p.ws[static_cast<size_t>(z) * p.MN + i];
+  }
+  __shared__ float part[G][17];
   part[g][o] = s;
   __syncthreads();
-  if (g == 0 && i < MN) {
+  if (g == 0 && i < p.MN) {
     float t = part[0][o];
-    for (int k = 1; k < 16; ++k) t += part[k][o];
-    out[i] = t;
-  }
-}
-
-// Bias gradient of a fully connected layer: sum of the slope-scaled gradient
-// over the batch in order, one workgroup per channel, 256 samples staged at a
-// time.
-__global__ __launch_bounds__(256) void bias_grad(const float *__restrict__ d, const uint16_t *__restrict__ post,
-                                                 float *__restrict__ db, int B, int C) {
-  __shared__ float stage[256];
-  const int co = blockIdx.x;
-  float s = 0.0f;
-  for (int b0 = 0; b0 < B; b0 += 256) {
-    const int n = min(256, B - b0);
-    __syncthreads();
-    if (static_cast<int>(threadIdx.x) < n) {
-      const size_t i = static_cast<size_t>(b0 + threadIdx.x) * C + co;
-      stage[threadIdx.x] = (!post || bf16_f(post[i]) > 0.0f) ? d[i] : kLeak * d[i];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
 #pragma unroll 16
-      for (int b = 0; b < n; ++b) s += stage[b];
-    }
+    for (int k = 1; k < G; ++k) t += part[k][o];
+    p.out[i] = t;
   }
-  if (threadIdx.x == 0) db[co] = s;
 }
-
-// Bias gradient of a convolution layer: the samples' sums of pool_bwd in order.
-__global__ void bias_grad_sum(const float *__restrict__ part, float *__restrict__ db, int B, int C) {
-  const int co = blockIdx.x * blockDim.x + threadIdx.x;
-  if (co >= C) return;
-  float s = 0.0f;
-  for (int b = 0; b < B; ++b) s += part[static_cast<size_t>(co) * B + b];
-  db[co] = s;
+hipError_t launch_reduce(Partials a, Partials b, hipStream_t s) {
+  const dim3 grid((a.MN + 15) / 16 + (b.MN + 15) / 16);
+  if (std::max(a.splits, b.splits) >= 256)
+    hipLaunchKernelGGL(reduce_splits<64>, grid, dim3(1024), 0, s, a, b);
+  else
+    hipLaunchKernelGGL(reduce_splits<16>, grid, dim3(256), 0, s, a, b);
+  return hipGetLastError();
 }
 
 // Loss over targets t[b] = {offset, tolerance} (output units):
-// Huber(offset error, delta 0.25) + 0.2 * BCE(confidence logit, |error| < tolerance).
-// g_out = dL/d(out) / B; loss = mean over the batch.
-__global__ void loss_kernel(const float *__restrict__ out, const float *__restrict__ tgt, float *__restrict__ g,
-                            float *__restrict__ loss, int B) {
+// Huber(offset error, delta 0.25) + 0.2 * BCE(confidence logit, |error| < tolerance),
+// mean over the batch, with its gradient g = dL/d(out) / B, and the backward
+// pass of the second fully connected layer: the gradients of its weights w
+// (dw, operands rounded to bf16 as in the other layers' products) and bias
+// (db), of its input h (gh) and of the first layer's bias (db1, with the slope
+// of h). One workgroup: the sums run over a batch of tens of samples, and what
+// it costs is its launch: 4.7 us, 29 with a kernel for the loss, each product,
+// its split sum and each bias sum.
+__global__ __launch_bounds__(256) void loss_kernel(const float *__restrict__ out, const float *__restrict__ tgt,
+                                                   const uint16_t *__restrict__ h, const uint16_t *__restrict__ w,
+                                                   float *g, float *__restrict__ loss, float *__restrict__ dw,
+                                                   float *__restrict__ db, float *__restrict__ gh,
+                                                   float *__restrict__ db1, int B) {
+  static_assert(kH1 == 16 && kOut == 2, "a thread per unit and sixteenth of the batch");
   __shared__ float red[256];
   float l = 0.0f;
   for (int b = threadIdx.x; b < B; b += blockDim.x) {
@@ -792,6 +796,31 @@ __global__ void loss_kernel(const float *__restrict__ out, const float *__restri
     __syncthreads();
   }
   if (threadIdx.x == 0) *loss = red[0] / B;
+  const int k = threadIdx.x & 15, q = threadIdx.x >> 4;
+  const float w0 = bf16_f(w[k]), w1 = bf16_f(w[kH1 + k]);
+  float s[5] = {};  // dw of the two outputs, db1; db of the two outputs
+  for (int b = q; b < B; b += 16) {
+    const float d0 = g[2 * b], d1 = g[2 * b + 1];
+    const float q0 = bf16_f(bf16_rne(d0)), q1 = bf16_f(bf16_rne(d1)), hv = bf16_f(h[b * kH1 + k]);
+    const float v = w0 * q0 + w1 * q1;
+    gh[b * kH1 + k] = v;
+    s[0] += q0 * hv;
+    s[1] += q1 * hv;
+    s[2] += hv > 0.0f ? v : kLeak * v;
+    s[3] += d0;
+    s[4] += d1;
+  }
+  __shared__ float part[5][16][17];
+#pragma unroll
+  for (int j = 0; j < 5; ++j) part[j][q][k] = s[j];
+  __syncthreads();
+  if (q >= 5 || (q >= 3 && k > 0)) return;
+  float t = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) t += part[q][i][k];
+  if (q < 2) dw[q * kH1 + k] = t;
+  else if (q == 2) db1[k] = t;
+  else db[q - 3] = t;
 }
 
 // Global gradient norm: per-block sums of squares, then one block sums them
@@ -966,7 +995,7 @@ struct ctas_cnn {
   std::vector<ctas::cnn::Param> prm;  // w1 b1 w2 b2 w3 b3 w4 b4 wf1 bf1 wf2 bf2
   size_t nparam = 0;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
-  uint16_t *p16 = nullptr, *wt = nullptr;  // bf16 weights; a layer's, transposed
+  uint16_t *p16 = nullptr, *wt = nullptr;  // bf16 weights; those of layers two to four, transposed
   int step = 0;
   int cap = 0;  // batch capacity of the activation buffers
   uint16_t *pool[4] = {}, *h1 = nullptr;
@@ -1068,14 +1097,12 @@ hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
   return hipGetLastError();
 }
 
-// Gradient of the input of layer l (its weights transposed first) into gbig2.
+// Gradient of the input of layer l into gbig2.
 template <int L, int CIN, int COUT, int H, int W>
 hipError_t conv_input_grad(ctas_cnn *n, const uint16_t *g, int B) {
   using G = ConvGeo<COUT, CIN, H, W>;
-  hipLaunchKernelGGL(transpose_weights, dim3((COUT * CIN * 9 + 255) / 256), dim3(256), 0, n->stream, W16(n, 2 * L),
-                     n->wt, COUT, CIN);
-  hipLaunchKernelGGL((conv_kernel<COUT, CIN, H, W, true>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, g, n->wt,
-                     nullptr, nullptr, nullptr, n->gbig2, G::STEPS);
+  hipLaunchKernelGGL((conv_kernel<COUT, CIN, H, W, true>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, g,
+                     n->wt + kWtAt[L], nullptr, nullptr, nullptr, n->gbig2, G::STEPS);
   return hipGetLastError();
 }
 
@@ -1096,84 +1123,69 @@ int forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
   return CTAS_OK;
 }
 
-// weight gradient of a GEMM whose reduction runs over K (split, reduced in a
-// fixed order)
-template <class FA, class FB>
-int weight_grad(ctas_cnn *n, FA fa, FB fb, int M, int Ncols, int K, float *dst) {
-  // enough K splits that the few output tiles of a weight gradient still
-  // put several workgroups on every CU
-  const int splits = std::max(1, std::min(2048, K / 1024));
-  if (int rc = ensure_ws(n, static_cast<size_t>(splits) * M * Ncols)) return rc;
-  int chunk = (K + splits - 1) / splits;
-  chunk = (chunk + kKS - 1) & ~(kKS - 1);
-  const int real = (K + chunk - 1) / chunk;
-  CTAS_HIP_TRY(gemm(fa, fb, StorePartial{n->ws, M, Ncols}, M, Ncols, K, n->stream, splits));
-  hipLaunchKernelGGL(reduce_splits, dim3((M * Ncols + 15) / 16), dim3(256), 0, n->stream, n->ws, dst, real,
-                     M * Ncols);
+// Weight gradient of the first fully connected layer on B samples: K is split
+// (and the splits summed in a fixed order) only where the batch is large.
+int dense_weight_grad(ctas_cnn *n, int B, float *dst) {
+  const GradFlatA fa{n->gh1, n->h1, kH1};
+  const ActBT fb{n->pool[3], kF};
+  int splits = std::max(1, std::min(2048, B / 1024));
+  if (splits == 1) {
+    CTAS_HIP_TRY(gemm(fa, fb, StorePartial{dst, kH1, kF}, kH1, kF, B, n->stream));
+    return CTAS_OK;
+  }
+  if (int rc = ensure_ws(n, static_cast<size_t>(splits) * kH1 * kF)) return rc;
+  const int chunk = ((B + splits - 1) / splits + kKS - 1) & ~(kKS - 1);
+  CTAS_HIP_TRY(gemm(fa, fb, StorePartial{n->ws, kH1, kF}, kH1, kF, B, n->stream, splits));
+  splits = (B + chunk - 1) / chunk;
+  CTAS_HIP_TRY(launch_reduce({n->ws, dst, splits, kH1 * kF}, {}, n->stream));
   return CTAS_OK;
 }
 
-// The same of a convolution layer on B samples.
-template <int CIN, int COUT, int H, int W>
-int conv_weight_grad(ctas_cnn *n, const uint16_t *g, const uint16_t *in, int B, float *dst) {
+// Gradients of a convolution layer's weights and bias on B samples, and of its
+// pre-activation (gact), from that of its pooled output.
+template <int L, int CIN, int COUT, int H, int W>
+int conv_weight_grad(ctas_cnn *n, const float *gpool, const uint16_t *in, int B) {
   constexpr int N = CIN * 9;
   const int K = B * H * W;
   int splits = std::max(1, std::min(2048, K / 1024));
   int chunk = (K + splits - 1) / splits;
   chunk = (chunk + kKS - 1) & ~(kKS - 1);
   splits = (K + chunk - 1) / chunk;
-  if (int rc = ensure_ws(n, static_cast<size_t>(splits) * COUT * N)) return rc;
+  const size_t bias_at = static_cast<size_t>(splits) * COUT * N;
+  if (int rc = ensure_ws(n, bias_at + static_cast<size_t>(B) * COUT)) return rc;
+  hipLaunchKernelGGL(pool_bwd, dim3(COUT, B), dim3(256), 0, n->stream, n->code[L], gpool, n->gact, n->ws + bias_at,
+                     COUT, H, W);
   if constexpr (CIN % 16 == 0)
-    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, H, W>), dim3(splits, CIN / 16), dim3(64), 0, n->stream, g, in, n->ws, K,
-                       chunk);
+    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, H, W>), dim3(splits, CIN / 16), dim3(64), 0, n->stream, n->gact, in,
+                       n->ws, K, chunk);
   else
-    hipLaunchKernelGGL((wgrad_taps_kernel<CIN, COUT, H, W>), dim3(splits), dim3(64), 0, n->stream, g, in, n->ws, K,
-                       chunk);
+    hipLaunchKernelGGL((wgrad_taps_kernel<CIN, COUT, H, W>), dim3(splits), dim3(64), 0, n->stream, n->gact, in, n->ws,
+                       K, chunk);
   CTAS_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(reduce_splits, dim3((COUT * N + 15) / 16), dim3(256), 0, n->stream, n->ws, dst, splits,
-                     COUT * N);
+  CTAS_HIP_TRY(launch_reduce({n->ws, G32(n, 2 * L), splits, COUT * N}, {n->ws + bias_at, G32(n, 2 * L + 1), B, COUT},
+                             n->stream));
   return CTAS_OK;
 }
 
+// From the loss's backward pass of the second fully connected layer on.
 int backward(ctas_cnn *n, const uint16_t *x, int B) {
   hipStream_t s = n->stream;
-  // fc2: dW[o][k] = sum_b gout[b][o] h1[b][k]; dh1[b][k] = sum_o W[o][k] gout[b][o]
-  if (int rc = weight_grad(n, GradFlatA{n->gout, nullptr, kOut}, ActBT{n->h1, kH1}, kOut, kH1, B, G32(n, 10)))
-    return rc;
-  hipLaunchKernelGGL(bias_grad, dim3(kOut), dim3(256), 0, s, n->gout, nullptr, G32(n, 11), B, kOut);
-  CTAS_HIP_TRY(gemm(DenseAT{W16(n, 10), kH1}, GradFlatB{GradFlatA{n->gout, nullptr, kOut}}, StoreFlatDX{n->gh1, kH1},
-                    kH1, B, kOut, s));
+  hipLaunchKernelGGL(transpose_weights, dim3((kWtAt[4] + 255) / 256), dim3(256), 0, s, W16(n, 2), W16(n, 4), W16(n, 6),
+                     n->wt);
   // fc1 (ReLU on h1)
-  if (int rc = weight_grad(n, GradFlatA{n->gh1, n->h1, kH1}, ActBT{n->pool[3], kF}, kH1, kF, B, G32(n, 8))) return rc;
-  hipLaunchKernelGGL(bias_grad, dim3(kH1), dim3(256), 0, s, n->gh1, n->h1, G32(n, 9), B, kH1);
+  if (int rc = dense_weight_grad(n, B, G32(n, 8))) return rc;
   CTAS_HIP_TRY(gemm(DenseAT{W16(n, 8), kF}, GradFlatB{GradFlatA{n->gh1, n->h1, kH1}}, StoreFlatDX{n->gf, kF}, kF, B,
                     kH1, s));
-  // conv layers, last to first. gpool = gradient of the layer's pooled
-  // output; gact = bf16 gradient of its pre-activation; the gradient of its
-  // input (= the previous pooled output) goes to gbig2.
-  const float *gpool = n->gf;
-  uint16_t *gact = n->gact;
-  for (int l = 3; l >= 0; --l) {
-    const Layer &L = kConv[l];
-    if (int rc = ensure_ws(n, static_cast<size_t>(L.cout) * B)) return rc;
-    hipLaunchKernelGGL(pool_bwd, dim3(L.cout, B), dim3(256), 0, s, n->code[l], gpool, gact, n->ws, B, L.cout, L.H, L.W);
-    hipLaunchKernelGGL(bias_grad_sum, dim3(1), dim3(64), 0, s, n->ws, G32(n, 2 * l + 1), B, L.cout);
-    // the workspace's bias partials were summed on this stream
-    const uint16_t *in = l ? n->pool[l - 1] : x;
-    if (int rc = l == 0   ? conv_weight_grad<2, 32, 180, 256>(n, gact, in, B, G32(n, 0))
-                 : l == 1 ? conv_weight_grad<32, 32, 90, 128>(n, gact, in, B, G32(n, 2))
-                 : l == 2 ? conv_weight_grad<32, 64, 45, 64>(n, gact, in, B, G32(n, 4))
-                          : conv_weight_grad<64, 64, 22, 32>(n, gact, in, B, G32(n, 6)))
-      return rc;
-    if (l > 0) {
-      const hipError_t e = l == 1   ? conv_input_grad<1, 32, 32, 90, 128>(n, gact, B)
-                           : l == 2 ? conv_input_grad<2, 32, 64, 45, 64>(n, gact, B)
-                                    : conv_input_grad<3, 64, 64, 22, 32>(n, gact, B);
-      CTAS_HIP_TRY(e);
-      gpool = n->gbig2;
-    }
-  }
-  return CTAS_OK;
+  // conv layers, last to first. gf = gradient of the last layer's pooled
+  // output; gact = bf16 gradient of a layer's pre-activation; the gradient of
+  // its input (= the previous pooled output) goes to gbig2.
+  if (int rc = conv_weight_grad<3, 64, 64, 22, 32>(n, n->gf, n->pool[2], B)) return rc;
+  CTAS_HIP_TRY((conv_input_grad<3, 64, 64, 22, 32>(n, n->gact, B)));
+  if (int rc = conv_weight_grad<2, 32, 64, 45, 64>(n, n->gbig2, n->pool[1], B)) return rc;
+  CTAS_HIP_TRY((conv_input_grad<2, 32, 64, 45, 64>(n, n->gact, B)));
+  if (int rc = conv_weight_grad<1, 32, 32, 90, 128>(n, n->gbig2, n->pool[0], B)) return rc;
+  CTAS_HIP_TRY((conv_input_grad<1, 32, 32, 90, 128>(n, n->gact, B)));
+  return conv_weight_grad<0, 2, 32, 180, 256>(n, n->gbig2, x, B);
 }
 
 }  // namespace
@@ -1217,7 +1229,7 @@ extern "C" int ctas_cnn_create(ctas_cnn **pn, uint64_t seed) {
   if (int rc = alloc(reinterpret_cast<void **>(&n->m), off * 4)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->v), off * 4)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->p16), off * 2)) return rc;
-  if (int rc = alloc(reinterpret_cast<void **>(&n->wt), 64 * 64 * 9 * 2)) return rc;
+  if (int rc = alloc(reinterpret_cast<void **>(&n->wt), kWtAt[4] * 2)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->loss), 256)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->norm), sizeof(float) * (kNormBlocks + 2))) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->ftmp), sizeof(float) * kFeatA * kFeatW)) return rc;
@@ -1306,7 +1318,8 @@ extern "C" int ctas_cnn_gradients_dev(ctas_cnn *n, const uint16_t *d_x, const fl
   if (int rc = stream_wait(n->stream, static_cast<hipStream_t>(stream))) return rc;
   if (int rc = ensure_batch(n, B)) return rc;
   if (int rc = forward(n, d_x, B, true)) return rc;
-  hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, n->stream, n->out, d_target, n->gout, n->loss, B);
+  hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, n->stream, n->out, d_target, n->h1, W16(n, 10), n->gout,
+                     n->loss, G32(n, 10), G32(n, 11), n->gh1, G32(n, 9), B);
   if (int rc = backward(n, d_x, B)) return rc;
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
   if (loss) CTAS_HIP_TRY(hipMemcpy(loss, n->loss, sizeof(float), hipMemcpyDeviceToHost));

@@ -36,6 +36,13 @@ def test_gradients_of_small_batches(torch_cuda, B):
         assert rel_rms(a, b) < 3e-2, k
 
 
+@pytest.mark.parametrize("B", [6, 23])
+def test_gradients_across_the_widths_of_the_sums(torch_cuda, B):
+    """Split counts on either side of where a sum takes more threads: 270 and
+    67 in the first two layers, 1035 and 258, and bias sums of 17 or more."""
+    test_gradients_of_small_batches(torch_cuda, B)
+
+
 @pytest.mark.parametrize("N,w", [(1, 2), (7, 255), (180, 256), (181, 257), (360, 1024), (900, 4096), (365, 4097)])
 def test_features_at_cell_edges(torch_cuda, N, w):
     """Cells of one sample, of uneven sizes and across the staged columns:
