@@ -388,90 +388,129 @@ __global__ __launch_bounds__(64) void wgrad_kernel(const uint16_t *__restrict__ 
         ws[(static_cast<size_t>(z) * COUT + 16 * m + (lane >> 4) * 4 + r) * N + ci * 9 + t] = acc[m][t][r];
 }
 
-// The same for the network's two-channel input: its 18 columns (channel and
-// tap) are two tiles of lanes, and a lane loads the octet of its own tap,
-// which starts a pixel to the left or right (the row's ends are shifted in as
-// zeros).
+// The same for the network's two-channel input, which has no gradient of its
+// own: nothing else reads the gradient of the layer's pre-activation, so it is
+// formed here, from the pooled gradient dy and the windows' codes, a pair of
+// rows at a time, and never stored; ws[z][COUT*18 + co] receives its sum before
+// rounding (bias). The input's 18 columns (channel and tap) are two tiles of
+// lanes; a step's octets of it are loaded once, one per lane, with the image's
+// border as zeros, and each lane takes those of its own taps from LDS (read
+// from memory at a pixel's shift they bound the kernel: 66 us). K counts steps
+// of two rows' 32 pixels. Bound by the latency of a step with two in flight
+// (four: 48 us). 64 samples: 45 us, where pooling backward and the product took
+// 51 and 79 and wrote and read 190 MB between them.
 typedef uint16_t u16x8u __attribute__((ext_vector_type(8), aligned(2)));
 template <int CIN, int COUT, int H, int W>
-__global__ __launch_bounds__(64) void wgrad_taps_kernel(const uint16_t *__restrict__ g, const uint16_t *__restrict__ x,
-                                                        float *__restrict__ ws, int K, int chunk) {
-  constexpr int N = CIN * 9, MT = COUT / 16, NT = (N + 15) / 16, HW = H * W;
-  static_assert(W % 32 == 0, "32 pixels of one row per step");
+__global__ __launch_bounds__(64) void wgrad_taps_kernel(const uint8_t *__restrict__ code, const float *__restrict__ dy,
+                                                        const uint16_t *__restrict__ x, float *__restrict__ ws, int K,
+                                                        int chunk) {
+  constexpr int N = CIN * 9, MT = COUT / 16, NT = (N + 15) / 16, HW = H * W, PW = W / 2, PHW = HW / 4;
+  constexpr int SR = 4 * CIN, SW = 48, OCT = SW / 8;  // rows and columns of a step's input: its border and octets
+  static_assert(W % 32 == 0 && H % 2 == 0, "32 pixels of two rows of one window row per step");
+  static_assert(SR * OCT <= 64, "one octet of the input per lane");
+  __shared__ __align__(16) uint16_t rows[2][SR * SW];
   const int lane = threadIdx.x, r16 = lane & 15, g8 = (lane >> 4) * 8;
   const int z = blockIdx.x, kb = z * chunk, ke = min(K, kb + chunk);
-  int coff[NT], dyc[NT], dxc[NT];
-  bool use[NT];
+  int at0[NT], edge[NT], dxc[NT];  // the lane's octet in `rows`, the pair beside it, its shift
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int c = t * 16 + r16;
-    use[t] = c < N;
-    const int cc = use[t] ? c : 0, ci = cc / 9, r = cc - 9 * ci;
-    dyc[t] = r / 3 - 1;
+    const int c = t * 16 + r16, cc = c < N ? c : 0, ci = cc / 9, r = cc - 9 * ci;
     dxc[t] = r % 3 - 1;
-    coff[t] = ci * HW;
+    at0[t] = (4 * ci + r / 3) * SW + 8 + g8;
+    edge[t] = at0[t] + (dxc[t] < 0 ? -2 : 8);
   }
-  constexpr int U = 4;  // steps of loads in flight
-  u32x4 av[U][MT], bv[U][NT];
-  auto load = [&](int p, u32x4 (&av)[MT], u32x4 (&bv)[NT]) {
-    const int b = p / HW, q = p - b * HW, y = q / W, x0 = q - y * W;  // uniform
-    const uint16_t *ga = g + static_cast<size_t>(b) * COUT * HW + q;
+  const int sr = min(lane / OCT, SR - 1), sci = sr >> 2, sy = (sr & 3) - 1, sx = 8 * (lane % OCT) - 8;  // staged octet
+  constexpr int U = 2;  // steps of loads in flight
+  struct Step {
+    float4 d[MT];
+    uint32_t c[MT];
+    u32x4 x;
+    uint32_t in;
+  } st[U];
+  auto load = [&](int pn, Step &s) {  // step p: 32 columns of window row yo of sample b
+    const int p = min(pn, ke - 1);    // past the end the last step again, masked
+    const int i = 32 * p, b = i / (H / 2 * W), q = i - b * (H / 2 * W), yo = q / W, x0 = q - yo * W;  // uniform
+    const size_t at = static_cast<size_t>(b) * COUT * PHW + yo * PW + x0 / 2;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) av[m] = *reinterpret_cast<const u32x4 *>(ga + (16 * m + r16) * HW + g8);
-    const uint16_t *xb = x + static_cast<size_t>(b) * CIN * HW;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int yy = y + dyc[t], xs = x0 + g8 + dxc[t];
-      const bool row = use[t] && yy >= 0 && yy < H;
-      const int at = coff[t] + (row ? yy : y) * W + min(max(xs, 0), W - 8);
-      bv[t] = __builtin_bit_cast(u32x4, *reinterpret_cast<const u16x8u *>(xb + at));
+    for (int m = 0; m < MT; ++m) {
+      const int o = (16 * m + r16) * PHW + g8 / 2;
+      s.d[m] = *reinterpret_cast<const float4 *>(dy + at + o);
+      s.c[m] = *reinterpret_cast<const uint32_t *>(code + at + o);
     }
-  };
-  // masked and shifted when used: a branch would wait for its loads
-  auto operand = [&](int p, const u32x4 &v, int t) {  // zero past the split
-    const int q = p % HW, y = q / W, x0 = q - y * W;
-    const int yy = y + dyc[t], xs = x0 + g8 + dxc[t];
-    const u32x4 e = xs < 0 ? octet_right(v, 0) : xs > W - 8 ? octet_left(v, 0) : v;
-    return e & (use[t] && yy >= 0 && yy < H && p < ke ? ~0u : 0u);
+    const int yy = 2 * yo + sy, xx = x0 + sx;
+    const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
+    // the caller's input is aligned to its elements only
+    s.x = __builtin_bit_cast(u32x4, *reinterpret_cast<const u16x8u *>(
+                                        x + static_cast<size_t>(b) * CIN * HW + (in ? sci * HW + yy * W + xx : 0)));
+    s.in = in && pn < ke ? ~0u : 0u;
   };
   f4 acc[MT][NT];
+  float bias[MT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int m = 0; m < MT; ++m) {
+    bias[m] = 0.0f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[m][t] = f4{0.f, 0.f, 0.f, 0.f};
+  }
 #pragma unroll
-  for (int u = 0; u < U; ++u) load(min(kb + 32 * u, ke - 32), av[u], bv[u]);
-  for (int p0 = kb; p0 < ke; p0 += 32 * U) {
+  for (int u = 0; u < U; ++u) load(kb + u, st[u]);
+  for (int p0 = kb; p0 < ke; p0 += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int p = p0 + 32 * u;
-      bf16x8 a[MT], bb[NT];
+      const int p = p0 + u;
+      uint16_t *buf = rows[u & 1];  // one wave: the step before last has read it
+      if (lane < SR * OCT) *reinterpret_cast<u32x4 *>(buf + 8 * lane) = st[u].x & st[u].in;
+      u32x4 a[2][MT];
 #pragma unroll
-      for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, av[u][m] & (p < ke ? ~0u : 0u));
+      for (int m = 0; m < MT; ++m) {
+        const float dv[4] = {st[u].d[m].x, st[u].d[m].y, st[u].d[m].z, st[u].d[m].w};
+        const uint32_t c = st[u].c[m];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) bb[t] = __builtin_bit_cast(bf16x8, operand(p, bv[u][t], t));
+        for (int j = 0; j < 4; ++j) {
+          const float v = p < ke ? (c & (4u << (8 * j)) ? dv[j] : kLeak * dv[j]) : 0.0f;
+          bias[m] += v;
+          // at its column, in the row of the window that held the maximum
+          const uint32_t w = static_cast<uint32_t>(bf16_rne(v)) << (c >> (8 * j) & 1u) * 16;
+          const bool low = c & (2u << (8 * j));
+          a[0][m][j] = low ? 0u : w;
+          a[1][m][j] = low ? w : 0u;
+        }
+      }
+      __syncthreads();
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bb[t], acc[m][t], 0, 0, 0);
+        for (int t = 0; t < NT; ++t) {
+          const u32x4 o = *reinterpret_cast<const u32x4 *>(buf + at0[t] + h * SW);
+          const uint32_t e = *reinterpret_cast<const uint32_t *>(buf + edge[t] + h * SW);
+          const u32x4 right = octet_right(o, e), left = octet_left(o, e);
+          const bf16x8 bb = __builtin_bit_cast(bf16x8, dxc[t] < 0 ? right : dxc[t] > 0 ? left : o);
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[h][m]), bb, acc[m][t], 0, 0, 0);
+        }
       __builtin_amdgcn_sched_barrier(0);
-      if (u & 1) {  // past the end the last step again
-        load(min(p + 32 * (U - 1), ke - 32), av[u - 1], bv[u - 1]);
-        load(min(p + 32 * U, ke - 32), av[u], bv[u]);
+      if (u & 1) {  // a line of each row of dy
+        load(p + U - 1, st[u - 1]);
+        load(p + U, st[u]);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
+  float *out = ws + static_cast<size_t>(z) * COUT * (N + 1);
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int m = 0; m < MT; ++m) {
+    bias[m] += __shfl_xor(bias[m], 16);
+    bias[m] += __shfl_xor(bias[m], 32);
+    if (lane < 16) out[COUT * N + 16 * m + r16] = bias[m];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int c = t * 16 + r16;
       if (c >= N) continue;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        ws[(static_cast<size_t>(z) * COUT + 16 * m + (lane >> 4) * 4 + r) * N + c] = acc[m][t][r];
+      for (int r = 0; r < 4; ++r) out[(16 * m + (lane >> 4) * 4 + r) * N + c] = acc[m][t][r];
     }
+  }
 }
 
 // 3x3 convolution of a layer as a product over k = channel*9 + tap (padding
@@ -725,9 +764,9 @@ __global__ __launch_bounds__(256) void transpose_weights(const uint16_t *__restr
 // 16 with 16 threads), 16 below, where most of 64 would find none (180 and 44
 // splits: 5.5 us, a launch).
 struct Partials {
-  const float *ws;  // [splits][MN]
+  const float *ws;  // [splits][MN], `stride` from one split to the next
   float *out;
-  int splits, MN;
+  int splits, MN, stride;
 };
 template <int G>
 __global__ __launch_bounds__(16 * G) void reduce_splits(Partials a, Partials b) {
@@ -737,7 +776,7 @@ __global__ __launch_bounds__(16 * G) void reduce_splits(Partials a, Partials b) 
   float s = 0.0f;
   if (i < p.MN) {
 #pragma unroll 8
-    for (int z = g; z < p.splits; z += G) s += p.ws[static_cast<size_t>(z) * p.MN + i];
+    for (int z = g; z < p.splits; z += G) s += p.ws[static_cast<size_t>(z) * p.stride + i];
   }
   __shared__ float part[G][17];
   part[g][o] = s;
@@ -1000,7 +1039,7 @@ struct ctas_cnn {
   int cap = 0;  // batch capacity of the activation buffers
   uint16_t *pool[4] = {}, *h1 = nullptr;
   uint8_t *code[4] = {};  // of the pooling's windows, for the backward pass
-  uint16_t *gact = nullptr;  // bf16 gradient of a layer's pre-activation
+  uint16_t *gact = nullptr;  // bf16 gradient of a layer's pre-activation (layers two to four)
   float *out = nullptr, *gout = nullptr, *gh1 = nullptr, *gf = nullptr, *gbig2 = nullptr;
   float *ws = nullptr;
   size_t ws_cap = 0;
@@ -1043,12 +1082,10 @@ int ensure_batch(ctas_cnn *n, int B) {
   size_t big = 0;
   for (int l = 0; l < 4; ++l) {
     const Layer &L = kConv[l];
-    const size_t a = static_cast<size_t>(B) * L.cout * L.H * L.W;
     const size_t q = static_cast<size_t>(B) * L.cout * (L.H / 2) * (L.W / 2);
     if (int rc = alloc(reinterpret_cast<void **>(&n->pool[l]), q * 2)) return rc;
     if (int rc = alloc(reinterpret_cast<void **>(&n->code[l]), q)) return rc;
-    big = std::max(big, a);
-    big = std::max(big, static_cast<size_t>(B) * L.cin * L.H * L.W);
+    if (l > 0) big = std::max(big, static_cast<size_t>(B) * std::max(L.cin, L.cout) * L.H * L.W);
   }
   if (int rc = alloc(reinterpret_cast<void **>(&n->h1), static_cast<size_t>(B) * kH1 * 2)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->out), static_cast<size_t>(B) * kOut * 4)) return rc;
@@ -1137,7 +1174,7 @@ int dense_weight_grad(ctas_cnn *n, int B, float *dst) {
   const int chunk = ((B + splits - 1) / splits + kKS - 1) & ~(kKS - 1);
   CTAS_HIP_TRY(gemm(fa, fb, StorePartial{n->ws, kH1, kF}, kH1, kF, B, n->stream, splits));
   splits = (B + chunk - 1) / chunk;
-  CTAS_HIP_TRY(launch_reduce({n->ws, dst, splits, kH1 * kF}, {}, n->stream));
+  CTAS_HIP_TRY(launch_reduce({n->ws, dst, splits, kH1 * kF, kH1 * kF}, {}, n->stream));
   return CTAS_OK;
 }
 
@@ -1155,15 +1192,28 @@ int conv_weight_grad(ctas_cnn *n, const float *gpool, const uint16_t *in, int B)
   if (int rc = ensure_ws(n, bias_at + static_cast<size_t>(B) * COUT)) return rc;
   hipLaunchKernelGGL(pool_bwd, dim3(COUT, B), dim3(256), 0, n->stream, n->code[L], gpool, n->gact, n->ws + bias_at,
                      COUT, H, W);
-  if constexpr (CIN % 16 == 0)
-    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, H, W>), dim3(splits, CIN / 16), dim3(64), 0, n->stream, n->gact, in,
-                       n->ws, K, chunk);
-  else
-    hipLaunchKernelGGL((wgrad_taps_kernel<CIN, COUT, H, W>), dim3(splits), dim3(64), 0, n->stream, n->gact, in, n->ws,
-                       K, chunk);
+  hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, H, W>), dim3(splits, CIN / 16), dim3(64), 0, n->stream, n->gact, in,
+                     n->ws, K, chunk);
   CTAS_HIP_TRY(hipGetLastError());
-  CTAS_HIP_TRY(launch_reduce({n->ws, G32(n, 2 * L), splits, COUT * N}, {n->ws + bias_at, G32(n, 2 * L + 1), B, COUT},
-                             n->stream));
+  CTAS_HIP_TRY(launch_reduce({n->ws, G32(n, 2 * L), splits, COUT * N, COUT * N},
+                             {n->ws + bias_at, G32(n, 2 * L + 1), B, COUT, COUT}, n->stream));
+  return CTAS_OK;
+}
+
+// The same of the first layer, without the gradient of its pre-activation.
+template <int L, int CIN, int COUT, int H, int W>
+int conv_taps_grad(ctas_cnn *n, const float *gpool, const uint16_t *in, int B) {
+  constexpr int MN = COUT * CIN * 9, S = MN + COUT;
+  const int K = B * (H * W / 64);  // a wave takes some 1500 pixels, as in the other layers
+  int splits = std::max(1, std::min(2048, K / 16));
+  const int chunk = (K + splits - 1) / splits;
+  splits = (K + chunk - 1) / chunk;
+  if (int rc = ensure_ws(n, static_cast<size_t>(splits) * S)) return rc;
+  hipLaunchKernelGGL((wgrad_taps_kernel<CIN, COUT, H, W>), dim3(splits), dim3(64), 0, n->stream, n->code[L], gpool, in,
+                     n->ws, K, chunk);
+  CTAS_HIP_TRY(hipGetLastError());
+  CTAS_HIP_TRY(launch_reduce({n->ws, G32(n, 2 * L), splits, MN, S},
+                             {n->ws + MN, G32(n, 2 * L + 1), splits, COUT, S}, n->stream));
   return CTAS_OK;
 }
 
@@ -1185,7 +1235,7 @@ int backward(ctas_cnn *n, const uint16_t *x, int B) {
   CTAS_HIP_TRY((conv_input_grad<2, 32, 64, 45, 64>(n, n->gact, B)));
   if (int rc = conv_weight_grad<1, 32, 32, 90, 128>(n, n->gbig2, n->pool[0], B)) return rc;
   CTAS_HIP_TRY((conv_input_grad<1, 32, 32, 90, 128>(n, n->gact, B)));
-  return conv_weight_grad<0, 2, 32, 180, 256>(n, n->gbig2, x, B);
+  return conv_taps_grad<0, 2, 32, 180, 256>(n, n->gbig2, x, B);
 }
 
 }  // namespace
