@@ -911,6 +911,22 @@ __global__ void adam_kernel(float *__restrict__ p, uint16_t *__restrict__ p16, c
   p16[i] = bf16_rne(pi);
 }
 
+// The parameters, each at its aligned offset, one after the other.
+constexpr int kParams = 12;
+struct Packing {
+  int off[kParams], at[kParams];  // of parameter i in p and in out
+};
+__global__ __launch_bounds__(256) void pack_params(const float *__restrict__ p, float *__restrict__ out, Packing pk,
+                                                   int count) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= count) return;
+  int from = i;
+#pragma unroll
+  for (int k = 0; k < kParams; ++k)
+    if (i >= pk.at[k]) from = pk.off[k] + i - pk.at[k];
+  out[i] = p[from];
+}
+
 __global__ void to_bf16(const float *__restrict__ p, uint16_t *__restrict__ q, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) q[i] = bf16_rne(p[i]);
@@ -1103,6 +1119,7 @@ int ensure_ws(ctas_cnn *n, size_t floats) {
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
   if (n->ws) (void)hipFree(n->ws);
   n->ws = nullptr;
+  n->ws_cap = 0;
   if (int rc = alloc(reinterpret_cast<void **>(&n->ws), floats * 4)) return rc;
   n->ws_cap = floats;
   return CTAS_OK;
@@ -1317,6 +1334,24 @@ extern "C" int ctas_cnn_num_params(const ctas_cnn *n, int *count) {
 }
 
 static int copy_params(ctas_cnn *n, float *host, const float *dev, bool to_host) {
+  size_t count = 0;
+  for (const auto &p : n->prm) count += p.n;
+  // one after the other on the device first: most of the twelve are small, and
+  // each copy has its own latency (gradients of 64 samples and their values on
+  // the host: 842 us with twelve copies, 702 with one)
+  if (to_host && ensure_ws(n, count) == CTAS_OK) {
+    ctas::cnn::Packing pk;
+    for (size_t i = 0, at = 0; i < n->prm.size(); at += n->prm[i++].n) {
+      pk.off[i] = static_cast<int>(n->prm[i].off);
+      pk.at[i] = static_cast<int>(at);
+    }
+    hipLaunchKernelGGL(pack_params, dim3((count + 255) / 256), dim3(256), 0, n->stream, dev, n->ws, pk,
+                       static_cast<int>(count));
+    CTAS_HIP_TRY(hipGetLastError());
+    CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
+    CTAS_HIP_TRY(hipMemcpy(host, n->ws, count * 4, hipMemcpyDeviceToHost));
+    return CTAS_OK;
+  }
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
   size_t at = 0;
   for (const auto &p : n->prm) {
