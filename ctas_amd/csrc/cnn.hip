@@ -47,11 +47,9 @@ namespace cnn {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 
+// to nearest even, one conversion instruction (bits by hand take seven)
 __device__ __forceinline__ uint16_t bf16_rne(float v) {
-  uint32_t u = __float_as_uint(v);
-  if ((u & 0x7f800000u) == 0x7f800000u) return static_cast<uint16_t>((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));
 }
 __device__ __forceinline__ float bf16_f(uint16_t h) { return __uint_as_float(static_cast<uint32_t>(h) << 16); }
 
