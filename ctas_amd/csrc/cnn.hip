@@ -286,10 +286,12 @@ __global__ __launch_bounds__(256) void pool_bwd(const uint8_t *__restrict__ code
 // line that a load touches, and 16 rows of g or x are 16 lines or more, so a
 // wave takes all output channels and all nine taps of 16 input channels: of a
 // row it reads the aligned octets and the two pixels beside the 32, and forms
-// the octets of the three horizontal taps in registers. 64 samples, layers
-// one to four: 75 (its own kernel below), 64, 33 and 30 us; 380 us on average
-// through the general product, 142 for the second layer with an unaligned
-// load per tap.
+// the octets of the three horizontal taps in registers. Four waves of a
+// workgroup take a quarter of its pixels each and add their sums through LDS:
+// a wave per SIMD with a quarter of the splits to write and to reduce, whatever
+// the layer's size. 64 samples, layers two to four: 51, 21 and 15 us (55, 33
+// and 26 with a split per wave, 704 to 44 of them; 380 on average through the
+// general product).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // octet d moved one pixel right (lo: the pixel before it in the upper half)
 // or left (hi: the pixel after it in the lower half)
@@ -301,16 +303,17 @@ __device__ __forceinline__ u32x4 octet_left(u32x4 d, uint32_t hi) {
 }
 
 template <int CIN, int COUT, int H, int W>
-__global__ __launch_bounds__(64) void wgrad_kernel(const uint16_t *__restrict__ g, const uint16_t *__restrict__ x,
+__global__ __launch_bounds__(256, 2) void wgrad_kernel(const uint16_t *__restrict__ g, const uint16_t *__restrict__ x,
                                                    float *__restrict__ ws, int K, int chunk) {
   constexpr int N = CIN * 9, MT = COUT / 16, HW = H * W;
   static_assert(W % 32 == 0 && CIN % 16 == 0, "32 pixels of one row and 16 channels per step");
-  const int lane = threadIdx.x, r16 = lane & 15, g8 = (lane >> 4) * 8;
-  const int z = blockIdx.x, ci = blockIdx.y * 16 + r16;
-  const int kb = z * chunk, ke = min(K, kb + chunk);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g8 = (lane >> 4) * 8;
+  const int z = blockIdx.x;
+  const int kb = __builtin_amdgcn_readfirstlane(z * chunk + wave * (chunk / 4)), ke = min(K, kb + chunk / 4);
+  const int before_at = g8 == 0 ? -2 : 0, after_at = g8 == 24 ? 8 : 0;
   // steps of loads in flight: a wave has 32 or so, and each would wait out a
   // memory latency
-  constexpr int U = 4;
+  constexpr int U = MT > 2 ? 2 : 4;
   struct Step {
     u32x4 a[MT], b[3];
     uint32_t edge[3];  // first and last quarter of the lanes: the pixels before and after the 32
@@ -326,7 +329,7 @@ __global__ __launch_bounds__(64) void wgrad_kernel(const uint16_t *__restrict__ 
     for (int m = 0; m < MT; ++m) s.a[m] = *reinterpret_cast<const u32x4 *>(ga + (16 * m + r16) * HW + g8);
     const uint16_t *xb = x + (static_cast<size_t>(b) * CIN + blockIdx.y * 16) * HW;
     const int xs = x0 + g8;
-    const int beside = g8 == 0 ? (xs > 0 ? -2 : 0) : g8 == 24 ? (xs < W - 8 ? 8 : 0) : 0;
+    const int beside = (x0 > 0 ? before_at : 0) + (x0 < W - 32 ? after_at : 0);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       const int yy = y + d - 1;
@@ -377,13 +380,24 @@ __global__ __launch_bounds__(64) void wgrad_kernel(const uint16_t *__restrict__ 
       }
     }
   }
+  // the four waves' sums, 16 output channels at a time
+  constexpr int RS = 16 * 9 + 4;  // padded row: 16 input channels and their taps
+  __shared__ float part[4][16 * RS];
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int m = 0; m < MT; ++m) {
+    if (m > 0) __syncthreads();
 #pragma unroll
     for (int t = 0; t < 9; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        ws[(static_cast<size_t>(z) * COUT + 16 * m + (lane >> 4) * 4 + r) * N + ci * 9 + t] = acc[m][t][r];
+      for (int r = 0; r < 4; ++r) part[wave][((lane >> 4) * 4 + r) * RS + r16 * 9 + t] = acc[m][t][r];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+      const int i = threadIdx.x + 256 * j, co = i / 144, c = i - co * 144, at = co * RS + c;
+      ws[(static_cast<size_t>(z) * COUT + 16 * m + co) * N + blockIdx.y * 144 + c] =
+          ((part[0][at] + part[1][at]) + part[2][at]) + part[3][at];
+    }
+  }
 }
 
 // The same for the network's two-channel input, which has no gradient of its
@@ -399,7 +413,7 @@ __global__ __launch_bounds__(64) void wgrad_kernel(const uint16_t *__restrict__ 
 // 51 and 79 and wrote and read 190 MB between them.
 typedef uint16_t u16x8u __attribute__((ext_vector_type(8), aligned(2)));
 template <int CIN, int COUT, int H, int W>
-__global__ __launch_bounds__(64) void wgrad_taps_kernel(const uint8_t *__restrict__ code, const float *__restrict__ dy,
+__global__ __launch_bounds__(64, 2) void wgrad_taps_kernel(const uint8_t *__restrict__ code, const float *__restrict__ dy,
                                                         const uint16_t *__restrict__ x, float *__restrict__ ws, int K,
                                                         int chunk) {
   constexpr int N = CIN * 9, MT = COUT / 16, NT = (N + 15) / 16, HW = H * W, PW = W / 2, PHW = HW / 4;
@@ -521,12 +535,15 @@ __global__ __launch_bounds__(64) void wgrad_taps_kernel(const uint8_t *__restric
 // from the patch, at offsets (in elements) that a table in LDS holds for
 // every k, and reads the weights [CO][K] as the instruction takes them. The
 // gathers bind it: eight 2-byte LDS reads per 16 pixels and 32 k serve CO/16
-// instructions. 64 samples, layers one to four forward with the pooling:
-// 84, 53, 41 and 22 us; backward, layers two to four: 42, 28 and 15 (181 and
+// instructions. Accumulators stay in vector registers (two waves per SIMD
+// asked for: with one, the compiler keeps them in the other half of the file
+// and moves them for every addition). 64 samples, layers one to four forward
+// with the pooling: 48, 41, 19 and 19 us; backward, layers two to four: 40, 27
+// and 14 (181 and
 // 147 us a layer through the general product, which forms every element's
 // index anew, and a pooling of its own).
-// `per` matrix instructions in a row make a partial sum, and the partial sums
-// are added in order: the sums of a product split over k.
+// SPLIT: `per` matrix instructions in a row make a partial sum, and the partial
+// sums are added in order: the sums of a product split over k.
 template <int CI, int CO, int H, int W>
 struct ConvGeo {
   static constexpr int K = CI * 9, STEPS = (K + 31) / 32, MT = CO / 16;
@@ -537,8 +554,8 @@ struct ConvGeo {
   static constexpr int ELEMS = CI * PR * STRIDE > OUT ? CI * PR * STRIDE : OUT;
 };
 
-template <int CI, int CO, int H, int W, bool BWD>
-__global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
+template <int CI, int CO, int H, int W, bool BWD, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void conv_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
                                                    const float *__restrict__ bias, uint16_t *__restrict__ pool,
                                                    uint8_t *__restrict__ code, float *__restrict__ dx, int per) {
   using G = ConvGeo<CI, CO, H, W>;
@@ -572,11 +589,11 @@ __global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ 
   }
   __syncthreads();
   const int wx = (wave % G::WX) * 32, wy = (wave / G::WX) * 2;  // the wave's pixels within the block
-  f4 acc[4][MT], sum[4][MT];
+  f4 acc[4][MT], sum[SPLIT ? 4 : 1][MT];
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[t][m] = sum[t][m] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MT; ++m) acc[t][m] = sum[SPLIT ? t : 0][m] = f4{0.f, 0.f, 0.f, 0.f};
   const uint16_t *base[4];  // tile t: row t / 2, columns 16 (t % 2) ...
 #pragma unroll
   for (int t = 0; t < 4; ++t) base[t] = patch + (wy + (t >> 1)) * G::STRIDE + wx + 16 * (t & 1) + r16;
@@ -615,22 +632,22 @@ __global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ 
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bv, acc[t][m], 0, 0, 0);
     }
-    if (--left == 0) {
+    if (SPLIT && --left == 0) {
       left = per;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-          sum[t][m] += acc[t][m];
+          sum[SPLIT ? t : 0][m] += acc[t][m];
           acc[t][m] = f4{0.f, 0.f, 0.f, 0.f};
         }
     }
   }
-  if (left != per)
+  if (SPLIT)
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) sum[t][m] += acc[t][m];
+      for (int m = 0; m < MT; ++m) acc[t][m] = left != per ? sum[SPLIT ? t : 0][m] + acc[t][m] : sum[SPLIT ? t : 0][m];
   const int row4 = (lane >> 4) * 4;
   if constexpr (BWD) {
 #pragma unroll
@@ -640,7 +657,7 @@ __global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ 
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) dx[(b * CO + 16 * m + row4 + r) * HW + yy * W + xx] = sum[t][m][r];
+        for (int r = 0; r < 4; ++r) dx[(b * CO + 16 * m + row4 + r) * HW + yy * W + xx] = acc[t][m][r];
     }
   } else {
     // the tile through LDS, so that the stores and the pooling take octets
@@ -653,7 +670,7 @@ __global__ __launch_bounds__(256) void conv_kernel(const uint16_t *__restrict__ 
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int co = 16 * m + row4 + r;
-          out[co * 64 + 32 * (t >> 1) + 16 * (t & 1) + r16] = bf16_rne(leaky(sum[t][m][r] + bias[co]));
+          out[co * 64 + 32 * (t >> 1) + 16 * (t & 1) + r16] = bf16_rne(leaky(acc[t][m][r] + bias[co]));
         }
     __syncthreads();
     const int yy = y0 + wy, xx = x0 + wx + 8 * (lane & 3);
@@ -1144,8 +1161,14 @@ template <int L, int CI, int CO, int H, int W>
 hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
   using G = ConvGeo<CI, CO, H, W>;
   const int splits = forward_splits(CO, B * H * W, G::K), per = (G::STEPS + splits - 1) / splits;
-  hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, x,
-                     W16(n, 2 * L), P32(n, 2 * L + 1), n->pool[L], codes ? n->code[L] : nullptr, nullptr, per);
+  const dim3 grid(G::XB * G::YB, B);
+  uint8_t *code = codes ? n->code[L] : nullptr;
+  if (per < G::STEPS)
+    hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, true>), grid, dim3(256), 0, n->stream, x, W16(n, 2 * L),
+                       P32(n, 2 * L + 1), n->pool[L], code, nullptr, per);
+  else
+    hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, false>), grid, dim3(256), 0, n->stream, x, W16(n, 2 * L),
+                       P32(n, 2 * L + 1), n->pool[L], code, nullptr, per);
   return hipGetLastError();
 }
 
@@ -1153,7 +1176,7 @@ hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
 template <int L, int CIN, int COUT, int H, int W>
 hipError_t conv_input_grad(ctas_cnn *n, const uint16_t *g, int B) {
   using G = ConvGeo<COUT, CIN, H, W>;
-  hipLaunchKernelGGL((conv_kernel<COUT, CIN, H, W, true>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, g,
+  hipLaunchKernelGGL((conv_kernel<COUT, CIN, H, W, true, false>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, g,
                      n->wt + kWtAt[L], nullptr, nullptr, nullptr, n->gbig2, G::STEPS);
   return hipGetLastError();
 }
@@ -1198,16 +1221,17 @@ int dense_weight_grad(ctas_cnn *n, int B, float *dst) {
 template <int L, int CIN, int COUT, int H, int W>
 int conv_weight_grad(ctas_cnn *n, const float *gpool, const uint16_t *in, int B) {
   constexpr int N = CIN * 9;
+  // a workgroup per CU, with four steps or more for each wave (second layer 51
+  // us; 55 with two workgroups per CU, 62 with four)
   const int K = B * H * W;
-  int splits = std::max(1, std::min(2048, K / 1024));
-  int chunk = (K + splits - 1) / splits;
-  chunk = (chunk + kKS - 1) & ~(kKS - 1);
+  int splits = std::max(1, std::min(256 / (CIN / 16), K / 512));
+  const int chunk = ((K + splits - 1) / splits + 127) & ~127;
   splits = (K + chunk - 1) / chunk;
   const size_t bias_at = static_cast<size_t>(splits) * COUT * N;
   if (int rc = ensure_ws(n, bias_at + static_cast<size_t>(B) * COUT)) return rc;
   hipLaunchKernelGGL(pool_bwd, dim3(COUT, B), dim3(256), 0, n->stream, n->code[L], gpool, n->gact, n->ws + bias_at,
                      COUT, H, W);
-  hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, H, W>), dim3(splits, CIN / 16), dim3(64), 0, n->stream, n->gact, in,
+  hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, H, W>), dim3(splits, CIN / 16), dim3(256), 0, n->stream, n->gact, in,
                      n->ws, K, chunk);
   CTAS_HIP_TRY(hipGetLastError());
   CTAS_HIP_TRY(launch_reduce({n->ws, G32(n, 2 * L), splits, COUT * N, COUT * N},
