@@ -280,18 +280,18 @@ __global__ __launch_bounds__(256) void pool_bwd(const uint8_t *__restrict__ code
 // Weight gradient of a convolution, split over the pixels: ws[z][co][c] =
 // sum over the pixels of split z of g[co][pixel] x[ci][pixel + tap], c = ci*9
 // + tap, 32 pixels per matrix instruction in pixel order. Both operands of
-// the instruction are eight consecutive pixels of one row per lane, which a
-// lane loads by itself, the next 32 pixels while the current ones are
-// multiplied: no LDS and no barrier. Bound by the L1, which takes a cycle per
-// line that a load touches, and 16 rows of g or x are 16 lines or more, so a
-// wave takes all output channels and all nine taps of 16 input channels: of a
-// row it reads the aligned octets and the two pixels beside the 32, and forms
-// the octets of the three horizontal taps in registers. Four waves of a
-// workgroup take a quarter of its pixels each and add their sums through LDS:
-// a wave per SIMD with a quarter of the splits to write and to reduce, whatever
-// the layer's size. 64 samples, layers two to four: 51, 21 and 15 us (55, 33
-// and 26 with a split per wave, 704 to 44 of them; 380 on average through the
-// general product).
+// the instruction are eight consecutive pixels of one row per lane, and
+// neighbouring lanes take 16 rows: loaded so, a load touches 64 pieces of
+// memory and not 16, and the L1 binds. A wave therefore loads its rows of 32
+// pixels as they lie, the next steps' while the current one is multiplied, and
+// takes its operands from LDS, which also gives the pixels beside an octet for
+// the horizontal taps. It takes all output channels and all nine taps of 16
+// input channels. Four waves of a workgroup take a quarter of its pixels each
+// and add their sums through LDS: a wave per SIMD with a quarter of the splits
+// to write and to reduce, whatever the layer's size. Bound by the latency of a
+// step. 64 samples, layers two to four: 43, 21 and 14 us (51, 21 and 15 with
+// operands loaded by their lanes; 55, 33 and 26 so with a split per wave, 704 to
+// 44 of them; 380 on average through the general product).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // octet d moved one pixel right (lo: the pixel before it in the upper half)
 // or left (hi: the pixel after it in the lower half)
@@ -310,14 +310,20 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const uint16_t *__restric
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g8 = (lane >> 4) * 8;
   const int z = blockIdx.x;
   const int kb = __builtin_amdgcn_readfirstlane(z * chunk + wave * (chunk / 4)), ke = min(K, kb + chunk / 4);
-  const int before_at = g8 == 0 ? -2 : 0, after_at = g8 == 24 ? 8 : 0;
-  // steps of loads in flight: a wave has 32 or so, and each would wait out a
-  // memory latency
-  constexpr int U = MT > 2 ? 2 : 4;
+  // A wave's operands in LDS: rows of 32 pixels, g's of 16*MT channels, and x's
+  // of three lines and 16 channels with a pair of pixels on either side
+  // (elements 6 and 40); pitches whose 16 rows fall into different banks.
+  constexpr int PA = 40, PB = 56, STAGE = MT * 16 * PA + 48 * PB;
+  constexpr int RS = 16 * 9 + 4;  // padded row of the sums: 16 input channels and their taps
+  __shared__ __align__(16) uint16_t lds[4 * (STAGE > 2 * 16 * RS ? STAGE : 2 * 16 * RS)];
+  uint16_t *sa = lds + wave * STAGE, *sb = sa + MT * 16 * PA;
+  const int lr = lane >> 2, lo = 8 * (lane & 3);                        // the octet a lane loads: row, column
+  const int ed = lane >> 5, eside = lane >> 4 & 1, eat = eside ? 40 : 6;  // its pairs: line ed and line 2 of channel r16
+  constexpr int U = MT > 2 ? 2 : 4;  // steps of loads in flight
   struct Step {
     u32x4 a[MT], b[3];
-    uint32_t edge[3];  // first and last quarter of the lanes: the pixels before and after the 32
-    uint32_t row[3], end, live;  // masks of what lies inside the image and the split
+    uint32_t edge[2];
+    uint32_t row[3], beside, live;  // masks of what lies inside the image and the split
   } st[U];
   // Branch-free, and masked when used: a branch would wait for its loads.
   auto load = [&](int pn, Step &s) {
@@ -326,21 +332,22 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const uint16_t *__restric
     const int b = p / HW, q = p - b * HW, y = q / W, x0 = q - y * W;  // uniform
     const uint16_t *ga = g + static_cast<size_t>(b) * COUT * HW + q;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) s.a[m] = *reinterpret_cast<const u32x4 *>(ga + (16 * m + r16) * HW + g8);
-    const uint16_t *xb = x + (static_cast<size_t>(b) * CIN + blockIdx.y * 16) * HW;
-    const int xs = x0 + g8;
-    const int beside = (x0 > 0 ? before_at : 0) + (x0 < W - 32 ? after_at : 0);
+    for (int m = 0; m < MT; ++m) s.a[m] = *reinterpret_cast<const u32x4 *>(ga + (16 * m + lr) * HW + lo);
+    const uint16_t *xb = x + (static_cast<size_t>(b) * CIN + blockIdx.y * 16) * HW + x0;
+    int line[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       const int yy = y + d - 1;
       const bool row = yy >= 0 && yy < H;
-      const int at = r16 * HW + (row ? yy : y) * W + xs;
-      s.b[d] = *reinterpret_cast<const u32x4 *>(xb + at);
-      s.edge[d] = *reinterpret_cast<const uint32_t *>(xb + at + beside);
+      line[d] = (row ? yy : y) * W;
+      s.b[d] = *reinterpret_cast<const u32x4 *>(xb + lr * HW + line[d] + lo);
       s.row[d] = row && live ? ~0u : 0u;
     }
+    const int left = x0 > 0 ? -2 : 0, right = x0 < W - 32 ? 32 : 0, beside = eside ? right : left;
+    s.edge[0] = *reinterpret_cast<const uint32_t *>(xb + r16 * HW + (ed ? line[1] : line[0]) + beside);
+    s.edge[1] = *reinterpret_cast<const uint32_t *>(xb + r16 * HW + line[2] + beside);
+    s.beside = beside ? ~0u : 0u;
     s.live = live ? ~0u : 0u;
-    s.end = beside ? ~0u : 0u;
   };
   f4 acc[MT][9];
 #pragma unroll
@@ -353,19 +360,32 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const uint16_t *__restric
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int p = p0 + 32 * u;
+#pragma unroll
+      for (int m = 0; m < MT; ++m) *reinterpret_cast<u32x4 *>(sa + (16 * m + lr) * PA + lo) = st[u].a[m] & st[u].live;
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+        *reinterpret_cast<u32x4 *>(sb + (16 * d + lr) * PB + 8 + lo) = st[u].b[d] & st[u].row[d];
+      *reinterpret_cast<uint32_t *>(sb + (16 * ed + r16) * PB + eat) =
+          st[u].edge[0] & (st[u].beside & (ed ? st[u].row[1] : st[u].row[0]));
+      if (ed == 0) *reinterpret_cast<uint32_t *>(sb + (32 + r16) * PB + eat) = st[u].edge[1] & (st[u].beside & st[u].row[2]);
+      // one wave: its LDS operations are in order, only the compiler's are not
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       bf16x8 a[MT], bb[9];
 #pragma unroll
-      for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, st[u].a[m] & st[u].live);
+      for (int m = 0; m < MT; ++m) a[m] = *reinterpret_cast<const bf16x8 *>(sa + (16 * m + r16) * PA + g8);
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const u32x4 o = st[u].b[d] & st[u].row[d];
-        // the pixels beside an octet are the neighbouring lanes' octets'
-        const uint32_t edge = st[u].edge[d] & (st[u].row[d] & st[u].end);
-        const uint32_t before = __shfl(o.w, lane - 16), after = __shfl(o.x, lane + 16);
-        bb[3 * d] = __builtin_bit_cast(bf16x8, octet_right(o, g8 == 0 ? edge : before));
+        const uint16_t *at = sb + (16 * d + r16) * PB + 8 + g8;
+        const u32x4 o = *reinterpret_cast<const u32x4 *>(at);
+        bb[3 * d] = __builtin_bit_cast(bf16x8, octet_right(o, *reinterpret_cast<const uint32_t *>(at - 2)));
         bb[3 * d + 1] = __builtin_bit_cast(bf16x8, o);
-        bb[3 * d + 2] = __builtin_bit_cast(bf16x8, octet_left(o, g8 == 24 ? edge : after));
+        bb[3 * d + 2] = __builtin_bit_cast(bf16x8, octet_left(o, *reinterpret_cast<const uint32_t *>(at + 8)));
       }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -381,21 +401,20 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const uint16_t *__restric
     }
   }
   // the four waves' sums, 16 output channels at a time
-  constexpr int RS = 16 * 9 + 4;  // padded row: 16 input channels and their taps
-  __shared__ float part[4][16 * RS];
+  float *part = reinterpret_cast<float *>(lds);
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    if (m > 0) __syncthreads();
+    __syncthreads();
 #pragma unroll
     for (int t = 0; t < 9; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) part[wave][((lane >> 4) * 4 + r) * RS + r16 * 9 + t] = acc[m][t][r];
+      for (int r = 0; r < 4; ++r) part[(wave * 16 + (lane >> 4) * 4 + r) * RS + r16 * 9 + t] = acc[m][t][r];
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < 9; ++j) {
       const int i = threadIdx.x + 256 * j, co = i / 144, c = i - co * 144, at = co * RS + c;
       ws[(static_cast<size_t>(z) * COUT + 16 * m + co) * N + blockIdx.y * 144 + c] =
-          ((part[0][at] + part[1][at]) + part[2][at]) + part[3][at];
+          ((part[at] + part[16 * RS + at]) + part[32 * RS + at]) + part[48 * RS + at];
     }
   }
 }
@@ -1221,8 +1240,8 @@ int dense_weight_grad(ctas_cnn *n, int B, float *dst) {
 template <int L, int CIN, int COUT, int H, int W>
 int conv_weight_grad(ctas_cnn *n, const float *gpool, const uint16_t *in, int B) {
   constexpr int N = CIN * 9;
-  // a workgroup per CU, with four steps or more for each wave (second layer 51
-  // us; 55 with two workgroups per CU, 62 with four)
+  // a workgroup per CU, with four steps or more for each wave (second layer 43
+  // us; 49 with two workgroups per CU)
   const int K = B * H * W;
   int splits = std::max(1, std::min(256 / (CIN / 16), K / 512));
   const int chunk = ((K + splits - 1) / splits + 127) & ~127;
