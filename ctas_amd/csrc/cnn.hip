@@ -561,42 +561,48 @@ __global__ __launch_bounds__(64, 2) void wgrad_taps_kernel(const uint8_t *__rest
 // and 14 (181 and
 // 147 us a layer through the general product, which forms every element's
 // index anew, and a pooling of its own).
-// SPLIT: `per` matrix instructions in a row make a partial sum, and the partial
-// sums are added in order: the sums of a product split over k.
-template <int CI, int CO, int H, int W>
+// SPLIT, for a batch whose pixels and channels are fewer than 256 tiles of 64 x
+// 64: `per` matrix instructions in a row make a partial sum, and the partial
+// sums are added in order (the sums of a product split over k). As most CUs
+// would have no block of four waves, a block is a wave with 2 rows x 16 columns:
+// its gathers do not queue behind three others'. One sample, layers two to
+// four: 5.4, 6.1 and 10.3 us (7.4, 10.4 and 14.3 as four waves of 2 x 32).
+template <int CI, int CO, int H, int W, bool SPLIT>
 struct ConvGeo {
   static constexpr int K = CI * 9, STEPS = (K + 31) / 32, MT = CO / 16;
-  static constexpr int COLS = W < 128 ? W : 128, WX = COLS / 32, RB = 2 * (4 / WX);
+  static constexpr int WAVES = SPLIT ? 1 : 4, TC = SPLIT ? 1 : 2, WC = 16 * TC;  // a wave's columns
+  static constexpr int COLS = SPLIT ? WC : W < 128 ? W : 128, WX = COLS / WC, RB = 2 * (WAVES / WX);
   static constexpr int XB = W / COLS, YB = (H + RB - 1) / RB;
   static constexpr int PR = RB + 2, STRIDE = COLS + 16;  // patch rows; columns with eight on either side
-  static constexpr int OUT = 4 * CO * 2 * 32;            // elements of the block's output tile
+  static constexpr int OUT = WAVES * CO * 2 * WC;        // elements of the block's output tile
   static constexpr int ELEMS = CI * PR * STRIDE > OUT ? CI * PR * STRIDE : OUT;
+  static constexpr int DEPTH = SPLIT && STEPS % 3 == 0 ? 3 : 1;  // steps of weights in flight
 };
 
 template <int CI, int CO, int H, int W, bool BWD, bool SPLIT>
-__global__ __launch_bounds__(256, 2) void conv_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
+__global__ __launch_bounds__(SPLIT ? 64 : 256, 2) void conv_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
                                                    const float *__restrict__ bias, uint16_t *__restrict__ pool,
                                                    uint8_t *__restrict__ code, float *__restrict__ dx, int per) {
-  using G = ConvGeo<CI, CO, H, W>;
-  constexpr int K = G::K, MT = G::MT, HW = H * W;
+  using G = ConvGeo<CI, CO, H, W, SPLIT>;
+  constexpr int K = G::K, MT = G::MT, HW = H * W, NT = 64 * G::WAVES, T = 2 * G::TC, WC = G::WC;
   __shared__ __align__(16) uint16_t patch[G::ELEMS];
   __shared__ __align__(16) uint16_t offs[G::STEPS * 32];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g8 = (lane >> 4) * 8;
   const int x0 = (blockIdx.x % G::XB) * G::COLS, y0 = (blockIdx.x / G::XB) * G::RB;
   const size_t b = blockIdx.y;
-  for (int k = tid; k < G::STEPS * 32; k += 256) {
+  for (int k = tid; k < G::STEPS * 32; k += NT) {
     const int kk = k < K ? k : 0, ci = kk / 9, r = kk - 9 * ci;
     const int row = BWD ? 2 - r / 3 : r / 3, col = BWD ? 1 - r % 3 : r % 3 - 1;
     offs[k] = static_cast<uint16_t>((ci * G::PR + row) * G::STRIDE + col + 8);
   }
   {
-    constexpr int OCT = G::STRIDE / 8, ITEMS = CI * G::PR * OCT, PT = (ITEMS + 255) / 256;
+    constexpr int OCT = G::STRIDE / 8, ITEMS = CI * G::PR * OCT, PT = (ITEMS + NT - 1) / NT;
     const uint16_t *xb = x + b * CI * HW;
     u32x4 v[PT];
     bool in[PT];
 #pragma unroll
     for (int j = 0; j < PT; ++j) {
-      const int i = min(tid + 256 * j, ITEMS - 1), o = i % OCT, t = i / OCT, pr = t % G::PR, ci = t / G::PR;
+      const int i = min(tid + NT * j, ITEMS - 1), o = i % OCT, t = i / OCT, pr = t % G::PR, ci = t / G::PR;
       const int xx = x0 + 8 * (o - 1), yy = y0 - 1 + pr;
       in[j] = xx >= 0 && xx < W && yy >= 0 && yy < H;
       // the network's input is the caller's, aligned to its elements only
@@ -604,21 +610,23 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(const uint16_t *__restrict
     }
 #pragma unroll
     for (int j = 0; j < PT; ++j)
-      if (tid + 256 * j < ITEMS) *reinterpret_cast<u32x4 *>(patch + 8 * (tid + 256 * j)) = in[j] ? v[j] : u32x4{};
+      if (tid + NT * j < ITEMS) *reinterpret_cast<u32x4 *>(patch + 8 * (tid + NT * j)) = in[j] ? v[j] : u32x4{};
   }
   __syncthreads();
-  const int wx = (wave % G::WX) * 32, wy = (wave / G::WX) * 2;  // the wave's pixels within the block
-  f4 acc[4][MT], sum[SPLIT ? 4 : 1][MT];
+  const int wx = (wave % G::WX) * WC, wy = (wave / G::WX) * 2;  // the wave's pixels within the block
+  f4 acc[T][MT], sum[SPLIT ? T : 1][MT];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < T; ++t)
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[t][m] = sum[SPLIT ? t : 0][m] = f4{0.f, 0.f, 0.f, 0.f};
-  const uint16_t *base[4];  // tile t: row t / 2, columns 16 (t % 2) ...
+  const uint16_t *base[T];  // tile t: row t / TC, columns 16 (t % TC) ...
 #pragma unroll
-  for (int t = 0; t < 4; ++t) base[t] = patch + (wy + (t >> 1)) * G::STRIDE + wx + 16 * (t & 1) + r16;
+  for (int t = 0; t < T; ++t) base[t] = patch + (wy + t / G::TC) * G::STRIDE + wx + 16 * (t % G::TC) + r16;
   int left = per;
-  u16x8 next[MT];  // the weights of the next 32 k, in flight during a step
-  auto weights = [&](int c) {
+  // the weights of the next D times 32 k, in flight during a step
+  constexpr int D = G::DEPTH;
+  u16x8 ahead[D][MT];
+  auto weights = [&](int c, u16x8 (&next)[MT]) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const uint16_t *row = w + (16 * m + r16) * K + 32 * c + g8;
@@ -630,48 +638,53 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(const uint16_t *__restrict
       }
     }
   };
-  weights(0);
+#pragma unroll
+  for (int d = 0; d < D; ++d) weights(d, ahead[d]);
   u16x8 o_next = *reinterpret_cast<const u16x8 *>(offs + g8);
-  for (int c = 0; c < G::STEPS; ++c) {
-    bf16x8 a[MT];
+  for (int c0 = 0; c0 < G::STEPS; c0 += D) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, next[m]);
-    if (G::STEPS > 1) weights(min(c + 1, G::STEPS - 1));
-    const u16x8 o = o_next;
-    o_next = *reinterpret_cast<const u16x8 *>(offs + 32 * min(c + 1, G::STEPS - 1) + g8);
+    for (int d = 0; d < D; ++d) {
+      const int c = c0 + d;
+      bf16x8 a[MT];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      u16x8 e;
+      for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, ahead[d][m]);
+      if (G::STEPS > 1) weights(min(c + D, G::STEPS - 1), ahead[d]);
+      const u16x8 o = o_next;
+      o_next = *reinterpret_cast<const u16x8 *>(offs + 32 * min(c + 1, G::STEPS - 1) + g8);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        e[j] = base[t][o[j]];
-        if (K % 32 != 0 && 32 * c + g8 + j >= K) e[j] = 0;
-      }
-      const bf16x8 bv = __builtin_bit_cast(bf16x8, e);
+      for (int t = 0; t < T; ++t) {
+        u16x8 e;
 #pragma unroll
-      for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bv, acc[t][m], 0, 0, 0);
-    }
-    if (SPLIT && --left == 0) {
-      left = per;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          sum[SPLIT ? t : 0][m] += acc[t][m];
-          acc[t][m] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 8; ++j) {
+          e[j] = base[t][o[j]];
+          if (K % 32 != 0 && 32 * c + g8 + j >= K) e[j] = 0;
         }
+        const bf16x8 bv = __builtin_bit_cast(bf16x8, e);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bv, acc[t][m], 0, 0, 0);
+      }
+      if (SPLIT && --left == 0) {
+        left = per;
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            sum[SPLIT ? t : 0][m] += acc[t][m];
+            acc[t][m] = f4{0.f, 0.f, 0.f, 0.f};
+          }
+      }
     }
   }
   if (SPLIT)
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < T; ++t)
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[t][m] = left != per ? sum[SPLIT ? t : 0][m] + acc[t][m] : sum[SPLIT ? t : 0][m];
   const int row4 = (lane >> 4) * 4;
   if constexpr (BWD) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int yy = y0 + wy + (t >> 1), xx = x0 + wx + 16 * (t & 1) + r16;
+    for (int t = 0; t < T; ++t) {
+      const int yy = y0 + wy + t / G::TC, xx = x0 + wx + 16 * (t % G::TC) + r16;
       if (yy >= H) continue;
 #pragma unroll
       for (int m = 0; m < MT; ++m)
@@ -681,23 +694,23 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(const uint16_t *__restrict
   } else {
     // the tile through LDS, so that the stores and the pooling take octets
     __syncthreads();
-    uint16_t *out = patch + wave * (CO * 64);  // [CO][2][32]
+    uint16_t *out = patch + wave * (CO * 2 * WC);  // [CO][2][WC]
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < T; ++t)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int co = 16 * m + row4 + r;
-          out[co * 64 + 32 * (t >> 1) + 16 * (t & 1) + r16] = bf16_rne(leaky(acc[t][m][r] + bias[co]));
+          out[co * 2 * WC + WC * (t / G::TC) + 16 * (t % G::TC) + r16] = bf16_rne(leaky(acc[t][m][r] + bias[co]));
         }
     __syncthreads();
-    const int yy = y0 + wy, xx = x0 + wx + 8 * (lane & 3);
+    const int yy = y0 + wy, col = 8 * (lane % (WC / 8)), xx = x0 + wx + col;
 #pragma unroll
-    for (int i = 0; i < CO / 16; ++i) {
-      const int co = 16 * i + (lane >> 2);
-      const u16x8 top = *reinterpret_cast<const u16x8 *>(out + co * 64 + 8 * (lane & 3));
-      const u16x8 low = *reinterpret_cast<const u16x8 *>(out + co * 64 + 32 + 8 * (lane & 3));
+    for (int i = 0; i < CO / (512 / WC); ++i) {
+      const int co = 512 / WC * i + lane / (WC / 8);
+      const u16x8 top = *reinterpret_cast<const u16x8 *>(out + co * 2 * WC + col);
+      const u16x8 low = *reinterpret_cast<const u16x8 *>(out + co * 2 * WC + WC + col);
       if (yy + 1 >= H) continue;
       const size_t at = (b * CO + co) * (H / 2) * (W / 2) + (yy / 2) * (W / 2) + xx / 2;
       typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
@@ -1178,15 +1191,15 @@ int forward_splits(int M, int N, int K) {
 // backward pass follows.
 template <int L, int CI, int CO, int H, int W>
 hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
-  using G = ConvGeo<CI, CO, H, W>;
+  using G = ConvGeo<CI, CO, H, W, false>;
+  using S = ConvGeo<CI, CO, H, W, true>;
   const int splits = forward_splits(CO, B * H * W, G::K), per = (G::STEPS + splits - 1) / splits;
-  const dim3 grid(G::XB * G::YB, B);
   uint8_t *code = codes ? n->code[L] : nullptr;
   if (per < G::STEPS)
-    hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, true>), grid, dim3(256), 0, n->stream, x, W16(n, 2 * L),
+    hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, true>), dim3(S::XB * S::YB, B), dim3(64), 0, n->stream, x, W16(n, 2 * L),
                        P32(n, 2 * L + 1), n->pool[L], code, nullptr, per);
   else
-    hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, false>), grid, dim3(256), 0, n->stream, x, W16(n, 2 * L),
+    hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, false>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, x, W16(n, 2 * L),
                        P32(n, 2 * L + 1), n->pool[L], code, nullptr, per);
   return hipGetLastError();
 }
@@ -1194,7 +1207,7 @@ hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
 // Gradient of the input of layer l into gbig2.
 template <int L, int CIN, int COUT, int H, int W>
 hipError_t conv_input_grad(ctas_cnn *n, const uint16_t *g, int B) {
-  using G = ConvGeo<COUT, CIN, H, W>;
+  using G = ConvGeo<COUT, CIN, H, W, false>;
   hipLaunchKernelGGL((conv_kernel<COUT, CIN, H, W, true, false>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, g,
                      n->wt + kWtAt[L], nullptr, nullptr, nullptr, n->gbig2, G::STEPS);
   return hipGetLastError();
