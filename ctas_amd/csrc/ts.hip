@@ -69,40 +69,38 @@ __device__ __forceinline__ int ts_column(int x, float cs, float pc, float rc, in
 // `odd` holds (u[x], v[x]), x < n, for odd n >= 3 and is null otherwise.
 //
 // Sums S_u, S_v of the rows r0 and r1 of one projection (after -log for
-// ABS): thread lt of a group of 256, reduced over its wave; lane 0 of wave
-// w leaves {S_u row 0, S_u row 1, S_v row 0, S_v row 1} at stash[4 w].
-__device__ __forceinline__ void odd_sums(const float *r0, const float *r1, bool has0, bool has1, int n,
-                                         bool absorb, const float2 *__restrict__ odd, int lt, float *stash) {
-  float su0 = 0.0f, su1 = 0.0f, sv0 = 0.0f, sv1 = 0.0f;
-  for (int x = lt; x < n; x += 256) {
-    float a = has0 ? r0[x] : 1.0f, c = has1 ? r1[x] : 1.0f;
-    if (absorb) {
-      a = -__logf(a);
-      c = -__logf(c);
-    }
-    a = has0 ? a : 0.0f;
-    c = has1 ? c : 0.0f;
-    const float2 uv = odd[x];
-    su0 += a * uv.x;
-    su1 += c * uv.x;
-    sv0 += a * uv.y;
-    sv1 += c * uv.y;
+// ABS): a thread adds the points that it holds for the transform, and their
+// sums over a wave go to the wave's place among 16 floats, {S_u row 0, S_u row 1,
+// S_v row 0, S_v row 1}. Read anew in a loop of their own, and with a branch
+// around each of the terms' table reads, they cost more than the transforms: 16
+// kept projections of 2048 rows of 777, 1437, 2047 and 3001 points 176, 567, 638
+// and 1615 us, now 146, 285, 300 and 1197 (the middle two with two waves per SIMD
+// asked for; 463 and 480 without).
+struct OddSums {
+  float u0 = 0.0f, u1 = 0.0f, v0 = 0.0f, v1 = 0.0f;
+  __device__ __forceinline__ void add(float a, float c, float2 uv) {
+    u0 += a * uv.x;
+    u1 += c * uv.x;
+    v0 += a * uv.y;
+    v1 += c * uv.y;
   }
+  __device__ __forceinline__ void leave(int lt, float *stash) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    su0 += __shfl_xor(su0, o);
-    su1 += __shfl_xor(su1, o);
-    sv0 += __shfl_xor(sv0, o);
-    sv1 += __shfl_xor(sv1, o);
+    for (int o = 32; o > 0; o >>= 1) {
+      u0 += __shfl_xor(u0, o);
+      u1 += __shfl_xor(u1, o);
+      v0 += __shfl_xor(v0, o);
+      v1 += __shfl_xor(v1, o);
+    }
+    if ((lt & 63) == 0) {
+      float *d = stash + 4 * (lt >> 6);
+      d[0] = u0;
+      d[1] = u1;
+      d[2] = v0;
+      d[3] = v1;
+    }
   }
-  if ((lt & 63) == 0) {
-    float *d = stash + 4 * (lt >> 6);
-    d[0] = su0;
-    d[1] = su1;
-    d[2] = sv0;
-    d[3] = sv1;
-  }
-}
+};
 
 // The four waves' stashes summed: {S_u row 0, S_u row 1, S_v row 0, S_v row 1}.
 __device__ __forceinline__ float4 odd_total(const float *stash) {
@@ -178,6 +176,7 @@ __global__ __launch_bounds__(256 * K) void ts_kernel(const float *proj, long lon
     const float *r0 = proj + static_cast<size_t>(p) * proj_stride + row0;
     const float *r1 = r0 + n;
     // The row pair at positions s0..s0+n-1 of the zeroed line, bit-reversed.
+    OddSums sums;
     for (int m = lt; m < Z; m += 256) {
       const int x = m - s0;
       float a = 0.0f, c = 0.0f;
@@ -188,10 +187,11 @@ __global__ __launch_bounds__(256 * K) void ts_kernel(const float *proj, long lon
           c = r1[x];
           if (absorb) c = -__logf(c);
         }
+        if (odd) sums.add(a, c, odd[x]);
       }
       buf[lds_pad(__brev(static_cast<unsigned>(m)) >> rsh, psh)] = make_float2(a, c);
     }
-    if (odd) odd_sums(r0, r1, live, live && has1, n, absorb, odd, lt, ostash);
+    if (odd) sums.leave(lt, ostash);
     __syncthreads();
     line_filter(buf, twp, Wp, Z, logZ, lt, psh);
     if (odd) {
@@ -353,13 +353,6 @@ __global__ __launch_bounds__(256, ODD ? 1 : 2) void ts2048_kernel(const float *p
   fetch(0);
 
   for (int p = 0; p < n_proj; ++p) {
-    if (ODD) {
-      const float *base = proj + static_cast<size_t>(p) * proj_stride;
-#pragma unroll
-      for (int l = 0; l < 2; ++l)
-        odd_sums(base + static_cast<size_t>(rr[2 * l]) * n, base + static_cast<size_t>(rr[2 * l + 1]) * n,
-                 rv[2 * l], rv[2 * l + 1], n, absorb, odd, tid, ostash + 16 * l);
-    }
     // pass 1: thread t, both lines, x[t + 256 j]
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
@@ -377,6 +370,12 @@ __global__ __launch_bounds__(256, ODD ? 1 : 2) void ts2048_kernel(const float *p
           }
         }
         v[j] = make_float2(rv[2 * l] ? a : 0.0f, rv[2 * l + 1] ? c : 0.0f);
+      }
+      if (ODD) {
+        OddSums sums;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sums.add(v[j].x, v[j].y, odd[min(max(tid + 256 * j - s0, 0), n - 1)]);
+        sums.leave(tid, ostash + 16 * l);
       }
       dft8<false>(v);
 #pragma unroll
@@ -441,13 +440,10 @@ __global__ __launch_bounds__(256, ODD ? 1 : 2) void ts2048_kernel(const float *p
       for (int l = 0; l < 2; ++l) {
         const float4 t = odd_total(ostash + 16 * l);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int x = tid + 256 * j - s0;
-          if (x >= 0 && x < n) {
-            const float2 d = odd_term(odd, odd_g, t, x);
-            y[l][j].x += d.x;
-            y[l][j].y += d.y;
-          }
+        for (int j = 0; j < 8; ++j) {  // points outside the row are not read
+          const float2 d = odd_term(odd, odd_g, t, min(max(tid + 256 * j - s0, 0), n - 1));
+          y[l][j].x += d.x;
+          y[l][j].y += d.y;
         }
       }
     }
@@ -545,7 +541,7 @@ constexpr int kP16 = 17;  // padded row length of the exchanges
 constexpr size_t kTs4096Lds = sizeof(float2) * 256 * kP16 + sizeof(float) * 16;  // + odd sums
 
 template <int J, bool ODD>
-__global__ __launch_bounds__(256) void ts4096_kernel(const float *proj, long long proj_stride, int n_proj,
+__global__ __launch_bounds__(256, 2) void ts4096_kernel(const float *proj, long long proj_stride, int n_proj,
                                                      TsConsts consts, float *filtered,
                                                      float *__restrict__ result, const float *__restrict__ W,
                                                      const float2 *__restrict__ tw, int rows, int n, int contrast,
@@ -594,9 +590,6 @@ __global__ __launch_bounds__(256) void ts4096_kernel(const float *proj, long lon
 
   for (int p = 0; p < n_proj; ++p) {
     if (!kPrefetch) fetch(p);
-    if (ODD)
-      odd_sums(proj + static_cast<size_t>(p) * proj_stride + row0, proj + static_cast<size_t>(p) * proj_stride + row1c,
-               true, has1, n, absorb, odd, tid, ostash);
     float2 v[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -611,6 +604,12 @@ __global__ __launch_bounds__(256) void ts4096_kernel(const float *proj, long lon
         }
       }
       v[j] = make_float2(a, has1 ? c : 0.0f);
+    }
+    if (ODD) {
+      OddSums sums;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) sums.add(v[j].x, v[j].y, odd[min(max(tid + 256 * j - s0, 0), n - 1)]);
+      sums.leave(tid, ostash);
     }
     if (kPrefetch && p + 1 < n_proj) fetch(p + 1);
 
@@ -658,13 +657,10 @@ __global__ __launch_bounds__(256) void ts4096_kernel(const float *proj, long lon
     if (ODD) {
       const float4 t = odd_total(ostash);
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int x = tid + 256 * j - s0;
-        if (x >= 0 && x < n) {
-          const float2 d = odd_term(odd, odd_g, t, x);
-          v[j].x += d.x;
-          v[j].y += d.y;
-        }
+      for (int j = 0; j < 16; ++j) {  // points outside the row are not read
+        const float2 d = odd_term(odd, odd_g, t, min(max(tid + 256 * j - s0, 0), n - 1));
+        v[j].x += d.x;
+        v[j].y += d.y;
       }
     }
     __syncthreads();  // the exchange is read; the line goes in its place
@@ -752,7 +748,6 @@ __global__ __launch_bounds__(256) void ts8192_kernel(const float *proj, long lon
   for (int p = 0; p < n_proj; ++p) {
     const float *r0 = proj + static_cast<size_t>(p) * proj_stride + row0;
     const float *r1 = proj + static_cast<size_t>(p) * proj_stride + row1c;
-    if (ODD) odd_sums(r0, r1, true, has1, n, absorb, odd, tid, ostash);
     float2 v[32];
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
@@ -767,6 +762,12 @@ __global__ __launch_bounds__(256) void ts8192_kernel(const float *proj, long lon
         }
       }
       v[j] = make_float2(a, has1 ? c : 0.0f);
+    }
+    if (ODD) {
+      OddSums sums;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) sums.add(v[j].x, v[j].y, odd[min(max(tid + 256 * j - s0, 0), n - 1)]);
+      sums.leave(tid, ostash);
     }
     dft32<false>(v);
 #pragma unroll
@@ -834,13 +835,10 @@ __global__ __launch_bounds__(256) void ts8192_kernel(const float *proj, long lon
     if (ODD) {
       const float4 t = odd_total(ostash);
 #pragma unroll
-      for (int j = 0; j < 32; ++j) {
-        const int x = tid + 256 * j - s0;
-        if (x >= 0 && x < n) {
-          const float2 d = odd_term(odd, odd_g, t, x);
-          v[j].x += d.x;
-          v[j].y += d.y;
-        }
+      for (int j = 0; j < 32; ++j) {  // points outside the row are not read
+        const float2 d = odd_term(odd, odd_g, t, min(max(tid + 256 * j - s0, 0), n - 1));
+        v[j].x += d.x;
+        v[j].y += d.y;
       }
     }
     __syncthreads();  // the exchange is read; the line goes in its place
