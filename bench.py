@@ -8,8 +8,8 @@ one hipGraph-captured launch sequence (deAbs + filter -> backprojection).
 One step = one reconstruction of the whole stack with the inputs already in
 HBM. Prints one JSON line. The roofline object prices the backprojection's
 LDS sample bytes (4 per voxel-update) against the LDS read peak measured in
-this run (ds_read_b128, the widest read; the b32 peak of the reads the
-kernel issues is reported beside it), and carries the VALU issue roof:
+this run (ds_read_b128, the read of four slices' words that the kernel
+issues; the b32 peak is reported beside it), and carries the VALU issue roof:
 VALU instructions per voxel-update counted by rocprofv3 (SQ_INSTS_VALU) in
 a child run of the same launch, against the measured v_add_f32 issue rate.
 HBM traffic per launch comes from rocprofv3 FETCH_SIZE / WRITE_SIZE child
@@ -85,7 +85,7 @@ def measure_peaks() -> dict:
             "lds_bytes_per_workgroup": int(out[11])}
 
 
-def _pmc_pass(args, counters, kernel_re, kind, ac, store, interp):
+def _pmc_pass(args, counters, kernel_re, store, interp):
     """One rocprofv3 --pmc pass over a child run of the launch; returns
     {kernel substring: {counter: value}} for the bp kernel and the copy."""
     import csv
@@ -99,7 +99,7 @@ def _pmc_pass(args, counters, kernel_re, kind, ac, store, interp):
                "-d", d, "-o", "pmc", "-f", "csv", "--", sys.executable, str(Path(__file__).resolve()),
                "--pmc-child", "--slices", str(args.slices), "--width", str(args.width),
                "--angles", str(args.angles), "--center", str(args.center),
-               "--child-tiles", f"{kind},{ac},{store},{interp}"]
+               "--child-store", f"{store},{interp}"]
         env = dict(os.environ, TMPDIR="/tmp")
         with open(os.path.join(d, "log.txt"), "w") as log:
             subprocess.run(cmd, cwd="/tmp", env=env, stdout=log, stderr=subprocess.STDOUT, timeout=300)
@@ -124,13 +124,13 @@ def _pmc_pass(args, counters, kernel_re, kind, ac, store, interp):
         shutil.rmtree(d, ignore_errors=True)
 
 
-def pmc_measure(args, kernel_name, kind, ac, store, interp, updates, bp_ms, peaks):
+def pmc_measure(args, kernel_name, store, interp, updates, bp_ms, peaks):
     """HBM traffic and VALU instructions of one backprojection launch from
     two rocprofv3 --pmc passes over a child run of the same launch."""
     print("[bench] rocprofv3 --pmc passes (FETCH_SIZE, WRITE_SIZE, SQ_INSTS_VALU)", file=sys.stderr, flush=True)
     a = _pmc_pass(args, ["FETCH_SIZE", "SQ_INSTS_VALU", "SQ_INSTS_LDS", "SQ_ACTIVE_INST_VALU2", "SQ_LDS_IDX_ACTIVE"],
-                  kernel_name, kind, ac, store, interp)
-    b = _pmc_pass(args, ["WRITE_SIZE", "SQ_WAVES"], kernel_name, kind, ac, store, interp)
+                  kernel_name, store, interp)
+    b = _pmc_pass(args, ["WRITE_SIZE", "SQ_WAVES"], kernel_name, store, interp)
     bp_a, bp_b, cp_a, cp_b = a.get("bp", {}), b.get("bp", {}), a.get("copy", {}), b.get("copy", {})
     need = [(bp_a, "FETCH_SIZE"), (bp_a, "SQ_INSTS_VALU"), (bp_b, "WRITE_SIZE"), (cp_a, "FETCH_SIZE"),
             (cp_b, "WRITE_SIZE")]
@@ -168,15 +168,16 @@ def binding_of(pmc):
 
 
 def lds_issue(insts, bp_ms, clk_cu, updates, peaks, idx_active=None):
-    """LDS wave instructions of the launch against the measured ds_read_b32
-    issue rate (the kernels' sample reads are b32), and the fraction of the
-    launch's CU cycles in which the LDS was busy (SQ_LDS_IDX_ACTIVE)."""
+    """LDS wave instructions of the launch against the measured ds_read_b128
+    issue rate (the kernels' sample reads take four slices' words at once), and
+    the fraction of the launch's CU cycles in which the LDS was busy
+    (SQ_LDS_IDX_ACTIVE)."""
     if not insts:
         return None
     achieved = insts / (bp_ms * 1e-3) / clk_cu
-    peak = peaks["lds_instr_per_clk_cu"]["b32"]
+    peak = peaks["lds_instr_per_clk_cu"]["b128"]
     return {"sq_insts_lds": insts, "instr_per_update": round(insts * 64 / updates, 3),
-            "achieved": round(achieved, 3), "peak_b32": peak, "unit": "wave instructions/clk/CU",
+            "achieved": round(achieved, 3), "peak_b128": peak, "unit": "wave instructions/clk/CU",
             "frac": round(achieved / peak, 4),
             "lds_busy_frac": round(idx_active / (bp_ms * 1e-3) / clk_cu, 4) if idx_active else None}
 
@@ -187,13 +188,12 @@ def pmc_child(args) -> int:
     import ctypes
     import torch
     import ctas_amd as ca
-    kind, ac, store, interp = (int(x) for x in args.child_tiles.split(","))
+    store, interp = (int(x) for x in args.child_store.split(","))
     S, w, N, c = args.slices, args.width, args.angles, args.center
     d_sino = make_inputs(torch, ca, S, N, w, c)
     d_out = torch.empty((S, w, w), dtype=torch.float32, device="cuda")
     stream = torch.cuda.Stream()
     rec = ca.CTrec(w, N, ca.ABS, "HANN", interp=interp, store=store)
-    rec.set_tiles(kind, ac)
     rec.prepare_dev(d_sino, stream)
     src = torch.ones(COPY_BYTES // 4, dtype=torch.float32, device="cuda")
     dst = torch.empty_like(src)
@@ -476,7 +476,7 @@ def main() -> int:
     ap.add_argument("--no-4096", action="store_true")
     ap.add_argument("--no-pmc", action="store_true", help="skip the rocprofv3 counter passes")
     ap.add_argument("--pmc-child", action="store_true", help=argparse.SUPPRESS)
-    ap.add_argument("--child-tiles", default="1,32,0,0", help=argparse.SUPPRESS)
+    ap.add_argument("--child-store", default="0,0", help=argparse.SUPPRESS)
     args = ap.parse_args()
     if args.pmc_child:
         return pmc_child(args)
@@ -532,7 +532,7 @@ def main() -> int:
     frac_in = in_mask_fraction(w, c)
     pmc = None
     if not args.no_pmc:
-        pmc = pmc_measure(args, "bp_grid_kernel", kind, ac, ca.STORE_FP32, ca.INTERP_CTAS, updates, bp_ms, peaks)
+        pmc = pmc_measure(args, "bp_group_kernel", ca.STORE_FP32, ca.INTERP_CTAS, updates, bp_ms, peaks)
     result = {
         "metric": "Gvoxel-updates/s FBP 2048^2x1800 FP32 vs FP16; axis-find ms CNN vs sweep",
         "value": round(value, 2),
@@ -553,13 +553,13 @@ def main() -> int:
         "roofline": {"bound": "lds", "achieved": round(achieved, 1), "peak": lds_peak,
                      "unit": "GB/s", "frac": round(achieved / lds_peak, 4),
                      "traffic": (round(pmc["traffic"]) if pmc and "traffic" in pmc else None),
-                     "kernel": "bp_grid_kernel", "kernel_ms": round(bp_ms, 3),
+                     "kernel": "bp_group_kernel", "kernel_ms": round(bp_ms, 3),
                      "bytes_per_update": 4,
                      "peak_b32": lds_peak32, "frac_b32": round(achieved / lds_peak32, 4),
                      "binding": binding_of(pmc) if pmc else "valu_issue",
                      "valu": (pmc["valu"] if pmc and "valu" in pmc else None),
                      "lds_issue": (pmc.get("lds_issue") if pmc else None),
-                     "note": "LDS sample bytes per full-grid voxel-update (one ds_read_b32 each) over the "
+                     "note": "LDS sample bytes per full-grid voxel-update (a ds_read_b128 for four slices) over the "
                              "kernel's HIP-event time; peak = ds_read_b128 bytes/clk/CU x CUs x clock "
                              "measured in this run (peak_b32: the same for ds_read_b32); binding: the "
                              "instruction-issue roof nearest to full (valu.frac, lds_issue.frac)"},
@@ -576,20 +576,19 @@ def main() -> int:
         var = {}
         for name, store in (("fp16", ca.STORE_FP16), ("bf16", ca.STORE_BF16)):
             print(f"[bench] {name} CTAS", file=sys.stderr, flush=True)
-            vrec, vms, vbp, _ = run_variant(store, ca.INTERP_CTAS, max(2, args.steps // 2), 1)
+            _, vms, vbp, _ = run_variant(store, ca.INTERP_CTAS, max(2, args.steps // 2), 1)
             var[name] = {"value": round(updates / (vms / 1e3) / 1e9, 2), "ms_per_step": round(vms, 3),
                          "bp_kernel_ms": round(vbp, 3), "speedup_vs_fp32": round(ms / vms, 3)}
             if name == "fp16" and not args.no_pmc:
                 # the mirrored kernel: 2 B of LDS sample words per voxel-update
-                vk, vac = vrec.tiles()
-                vp = pmc_measure(args, "bp_mirror_kernel", vk, vac, store, ca.INTERP_CTAS, updates, vbp, peaks)
+                vp = pmc_measure(args, "bp_group_mirror_kernel", store, ca.INTERP_CTAS, updates, vbp, peaks)
                 a16 = updates * 2.0 / (vbp / 1e3) / 1e9
                 var[name]["roofline"] = {"bound": "lds", "achieved": round(a16, 1), "peak": lds_peak, "unit": "GB/s",
                                          "frac": round(a16 / lds_peak, 4),
                                          "traffic": round(vp["traffic"]) if "traffic" in vp else None,
                                          "binding": binding_of(vp), "valu": vp.get("valu"),
                                          "lds_issue": vp.get("lds_issue"),
-                                         "kernel": "bp_mirror_kernel", "bytes_per_update": 2}
+                                         "kernel": "bp_group_mirror_kernel", "bytes_per_update": 2}
         for name, store in (("fp32_linear", ca.STORE_FP32), ("fp16_linear", ca.STORE_FP16)):
             print(f"[bench] {name}", file=sys.stderr, flush=True)
             _, lms, lbp, _ = run_variant(store, ca.INTERP_LINEAR, max(2, args.steps // 2), 1)

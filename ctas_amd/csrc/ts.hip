@@ -291,7 +291,7 @@ constexpr int kLineB = 128 * kB;             // [k * 16 + m2][t1]
 constexpr size_t kTs2048Lds = sizeof(float2) * (2 * kLineA + 2 * kLineB) + sizeof(float) * 32;  // + odd sums
 
 template <int J, bool ODD>
-__global__ __launch_bounds__(256, ODD ? 1 : 2) void ts2048_kernel(const float *proj, long long proj_stride, int n_proj,
+__global__ __launch_bounds__(256, 2) void ts2048_kernel(const float *proj, long long proj_stride, int n_proj,
                                                      TsConsts consts, float *filtered,
                                                      float *__restrict__ result, const float *__restrict__ W,
                                                      const float2 *__restrict__ tw, int rows, int n, int contrast,
@@ -541,7 +541,7 @@ constexpr int kP16 = 17;  // padded row length of the exchanges
 constexpr size_t kTs4096Lds = sizeof(float2) * 256 * kP16 + sizeof(float) * 16;  // + odd sums
 
 template <int J, bool ODD>
-__global__ __launch_bounds__(256, 2) void ts4096_kernel(const float *proj, long long proj_stride, int n_proj,
+__global__ __launch_bounds__(256, ODD ? 2 : 1) void ts4096_kernel(const float *proj, long long proj_stride, int n_proj,
                                                      TsConsts consts, float *filtered,
                                                      float *__restrict__ result, const float *__restrict__ W,
                                                      const float2 *__restrict__ tw, int rows, int n, int contrast,
