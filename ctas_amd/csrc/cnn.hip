@@ -546,9 +546,9 @@ __global__ __launch_bounds__(64, 2) void wgrad_taps_kernel(const uint8_t *__rest
 
 // 3x3 convolution of a layer as a product over k = channel*9 + tap (padding
 // 1): forward (BWD false; bias, leaky ReLU, of the bf16 output its 2x2 maximum
-// `pool` and, where a backward pass follows, the windows' codes) or the gradient of the layer's input (BWD true: CI the layer's
-// output channels, x their bf16 gradients, the stencil mirrored, float32
-// output dx). Four waves share a patch of the input in LDS, with its border
+// `pool` and, where a backward pass follows, the windows' codes) or the
+// gradient of the layer's input (BWD true: CI the layer's output channels, x
+// their bf16 gradients, the stencil mirrored, float32 output dx). Four waves share a patch of the input in LDS, with its border
 // (zeros outside the image); each takes all output channels of 2 rows x 32
 // columns. A lane gathers its pixel's eight operands of a matrix instruction
 // from the patch, at offsets (in elements) that a table in LDS holds for
@@ -558,33 +558,33 @@ __global__ __launch_bounds__(64, 2) void wgrad_taps_kernel(const uint8_t *__rest
 // asked for: with one, the compiler keeps them in the other half of the file
 // and moves them for every addition). 64 samples, layers one to four forward
 // with the pooling: 48, 41, 19 and 19 us; backward, layers two to four: 40, 27
-// and 14 (181 and
-// 147 us a layer through the general product, which forms every element's
-// index anew, and a pooling of its own).
+// and 14 (181 and 147 us a layer through the general product, which forms every
+// element's index anew, and a pooling of its own).
 // SPLIT, for a batch whose pixels and channels are fewer than 256 tiles of 64 x
 // 64: `per` matrix instructions in a row make a partial sum, and the partial
 // sums are added in order (the sums of a product split over k). As most CUs
-// would have no block of four waves, a block is a wave with 2 rows x 16 columns:
-// its gathers do not queue behind three others'. One sample, layers two to
-// four: 5.4, 6.1 and 10.3 us (7.4, 10.4 and 14.3 as four waves of 2 x 32).
+// would have no block, a block takes 2 rows x 16 columns, and its four waves
+// every fourth partial sum. One sample, layers two to four: 5.1, 4.8 and
+// 7.4 us (5.4, 6.1 and 10.4 with one wave for all of them; 7.4, 10.4 and 14.3 as
+// blocks of four waves' 2 x 32 pixels).
 template <int CI, int CO, int H, int W, bool SPLIT>
 struct ConvGeo {
   static constexpr int K = CI * 9, STEPS = (K + 31) / 32, MT = CO / 16;
-  static constexpr int WAVES = SPLIT ? 1 : 4, TC = SPLIT ? 1 : 2, WC = 16 * TC;  // a wave's columns
+  static constexpr int WAVES = SPLIT ? 1 : 4, TC = SPLIT ? 1 : 2, WC = 16 * TC;  // waves side by side; a wave's columns
   static constexpr int COLS = SPLIT ? WC : W < 128 ? W : 128, WX = COLS / WC, RB = 2 * (WAVES / WX);
   static constexpr int XB = W / COLS, YB = (H + RB - 1) / RB;
   static constexpr int PR = RB + 2, STRIDE = COLS + 16;  // patch rows; columns with eight on either side
   static constexpr int OUT = WAVES * CO * 2 * WC;        // elements of the block's output tile
   static constexpr int ELEMS = CI * PR * STRIDE > OUT ? CI * PR * STRIDE : OUT;
-  static constexpr int DEPTH = SPLIT && STEPS % 3 == 0 ? 3 : 1;  // steps of weights in flight
+  static constexpr int PS = 2 * WC + 4;                  // floats of a channel in a partial sum's tile
 };
 
 template <int CI, int CO, int H, int W, bool BWD, bool SPLIT>
-__global__ __launch_bounds__(SPLIT ? 64 : 256, 2) void conv_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
+__global__ __launch_bounds__(256, 2) void conv_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
                                                    const float *__restrict__ bias, uint16_t *__restrict__ pool,
                                                    uint8_t *__restrict__ code, float *__restrict__ dx, int per) {
   using G = ConvGeo<CI, CO, H, W, SPLIT>;
-  constexpr int K = G::K, MT = G::MT, HW = H * W, NT = 64 * G::WAVES, T = 2 * G::TC, WC = G::WC;
+  constexpr int K = G::K, MT = G::MT, HW = H * W, NT = 256, T = 2 * G::TC, WC = G::WC;
   __shared__ __align__(16) uint16_t patch[G::ELEMS];
   __shared__ __align__(16) uint16_t offs[G::STEPS * 32];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g8 = (lane >> 4) * 8;
@@ -613,20 +613,20 @@ __global__ __launch_bounds__(SPLIT ? 64 : 256, 2) void conv_kernel(const uint16_
       if (tid + NT * j < ITEMS) *reinterpret_cast<u32x4 *>(patch + 8 * (tid + NT * j)) = in[j] ? v[j] : u32x4{};
   }
   __syncthreads();
-  const int wx = (wave % G::WX) * WC, wy = (wave / G::WX) * 2;  // the wave's pixels within the block
-  f4 acc[T][MT], sum[SPLIT ? T : 1][MT];
+  const int sw = SPLIT ? 0 : wave, wx = (sw % G::WX) * WC, wy = (sw / G::WX) * 2;  // the wave's pixels in the block
+  f4 acc[T][MT];
+  auto clear = [&] {
 #pragma unroll
-  for (int t = 0; t < T; ++t)
+    for (int t = 0; t < T; ++t)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[t][m] = sum[SPLIT ? t : 0][m] = f4{0.f, 0.f, 0.f, 0.f};
+      for (int m = 0; m < MT; ++m) acc[t][m] = f4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
   const uint16_t *base[T];  // tile t: row t / TC, columns 16 (t % TC) ...
 #pragma unroll
   for (int t = 0; t < T; ++t) base[t] = patch + (wy + t / G::TC) * G::STRIDE + wx + 16 * (t % G::TC) + r16;
-  int left = per;
-  // the weights of the next D times 32 k, in flight during a step
-  constexpr int D = G::DEPTH;
-  u16x8 ahead[D][MT];
-  auto weights = [&](int c, u16x8 (&next)[MT]) {
+  u16x8 next[MT];  // the weights of the next 32 k, in flight during a step
+  auto weights = [&](int c) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const uint16_t *row = w + (16 * m + r16) * K + 32 * c + g8;
@@ -638,49 +638,61 @@ __global__ __launch_bounds__(SPLIT ? 64 : 256, 2) void conv_kernel(const uint16_
       }
     }
   };
+  u16x8 o_next;
+  auto ahead = [&](int c) {
+    weights(min(c, G::STEPS - 1));
+    o_next = *reinterpret_cast<const u16x8 *>(offs + 32 * min(c, G::STEPS - 1) + g8);
+  };
+  auto step = [&](int c, int then) {  // step c, its operands in flight; `then` is the wave's next
+    bf16x8 a[MT];
 #pragma unroll
-  for (int d = 0; d < D; ++d) weights(d, ahead[d]);
-  u16x8 o_next = *reinterpret_cast<const u16x8 *>(offs + g8);
-  for (int c0 = 0; c0 < G::STEPS; c0 += D) {
+    for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, next[m]);
+    const u16x8 o = o_next;
+    if (G::STEPS > 1) ahead(then);
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int c = c0 + d;
-      bf16x8 a[MT];
+    for (int t = 0; t < T; ++t) {
+      u16x8 e;
 #pragma unroll
-      for (int m = 0; m < MT; ++m) a[m] = __builtin_bit_cast(bf16x8, ahead[d][m]);
-      if (G::STEPS > 1) weights(min(c + D, G::STEPS - 1), ahead[d]);
-      const u16x8 o = o_next;
-      o_next = *reinterpret_cast<const u16x8 *>(offs + 32 * min(c + 1, G::STEPS - 1) + g8);
-#pragma unroll
-      for (int t = 0; t < T; ++t) {
-        u16x8 e;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          e[j] = base[t][o[j]];
-          if (K % 32 != 0 && 32 * c + g8 + j >= K) e[j] = 0;
-        }
-        const bf16x8 bv = __builtin_bit_cast(bf16x8, e);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bv, acc[t][m], 0, 0, 0);
+      for (int j = 0; j < 8; ++j) {
+        e[j] = base[t][o[j]];
+        if (K % 32 != 0 && 32 * c + g8 + j >= K) e[j] = 0;
       }
-      if (SPLIT && --left == 0) {
-        left = per;
+      const bf16x8 bv = __builtin_bit_cast(bf16x8, e);
 #pragma unroll
-        for (int t = 0; t < T; ++t)
-#pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            sum[SPLIT ? t : 0][m] += acc[t][m];
-            acc[t][m] = f4{0.f, 0.f, 0.f, 0.f};
-          }
-      }
+      for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], bv, acc[t][m], 0, 0, 0);
     }
-  }
-  if (SPLIT)
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) acc[t][m] = left != per ? sum[SPLIT ? t : 0][m] + acc[t][m] : sum[SPLIT ? t : 0][m];
+  };
   const int row4 = (lane >> 4) * 4;
+  constexpr int E = SPLIT ? CO * 2 * WC / NT : 1;  // outputs that a thread adds up
+  float total[E] = {};
+  if constexpr (SPLIT) {
+    __shared__ float part[4][CO * G::PS];  // a wave's partial sum: [channel][2][WC]
+    ahead(wave * per);
+    for (int c0 = 0; c0 < G::STEPS; c0 += 4 * per) {
+      const int cb = c0 + wave * per, ce = min(cb + per, G::STEPS);
+      clear();
+      for (int c = cb; c < ce; ++c) step(c, c + 1 < ce ? c + 1 : cb + 4 * per);
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) part[wave][(16 * m + row4 + r) * G::PS + WC * t + r16] = acc[t][m][r];
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (c0 + k * per < G::STEPS)
+#pragma unroll
+          for (int i = 0; i < E; ++i) {
+            const int at = tid + NT * i;
+            total[i] += part[k][at / (2 * WC) * G::PS + at % (2 * WC)];
+          }
+      __syncthreads();
+    }
+  } else {
+    ahead(0);
+    for (int c = 0; c < G::STEPS; ++c) step(c, c + 1);
+  }
   if constexpr (BWD) {
 #pragma unroll
     for (int t = 0; t < T; ++t) {
@@ -694,20 +706,29 @@ __global__ __launch_bounds__(SPLIT ? 64 : 256, 2) void conv_kernel(const uint16_
   } else {
     // the tile through LDS, so that the stores and the pooling take octets
     __syncthreads();
-    uint16_t *out = patch + wave * (CO * 2 * WC);  // [CO][2][WC]
+    uint16_t *out = patch + sw * (CO * 2 * WC);  // [CO][2][WC]
+    if constexpr (SPLIT) {
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+      for (int i = 0; i < E; ++i) {
+        const int at = tid + NT * i;
+        out[at] = bf16_rne(leaky(total[i] + bias[at / (2 * WC)]));
+      }
+    } else {
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
+      for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int co = 16 * m + row4 + r;
-          out[co * 2 * WC + WC * (t / G::TC) + 16 * (t % G::TC) + r16] = bf16_rne(leaky(acc[t][m][r] + bias[co]));
-        }
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int co = 16 * m + row4 + r;
+            out[co * 2 * WC + WC * (t / G::TC) + 16 * (t % G::TC) + r16] = bf16_rne(leaky(acc[t][m][r] + bias[co]));
+          }
+    }
     __syncthreads();
     const int yy = y0 + wy, col = 8 * (lane % (WC / 8)), xx = x0 + wx + col;
 #pragma unroll
     for (int i = 0; i < CO / (512 / WC); ++i) {
+      if (SPLIT && i != wave) continue;
       const int co = 512 / WC * i + lane / (WC / 8);
       const u16x8 top = *reinterpret_cast<const u16x8 *>(out + co * 2 * WC + col);
       const u16x8 low = *reinterpret_cast<const u16x8 *>(out + co * 2 * WC + WC + col);
@@ -1195,12 +1216,15 @@ hipError_t conv_forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
   using S = ConvGeo<CI, CO, H, W, true>;
   const int splits = forward_splits(CO, B * H * W, G::K), per = (G::STEPS + splits - 1) / splits;
   uint8_t *code = codes ? n->code[L] : nullptr;
-  if (per < G::STEPS)
-    hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, true>), dim3(S::XB * S::YB, B), dim3(64), 0, n->stream, x, W16(n, 2 * L),
-                       P32(n, 2 * L + 1), n->pool[L], code, nullptr, per);
-  else
-    hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, false>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, x, W16(n, 2 * L),
-                       P32(n, 2 * L + 1), n->pool[L], code, nullptr, per);
+  if constexpr (G::STEPS > 1) {
+    if (per < G::STEPS) {
+      hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, true>), dim3(S::XB * S::YB, B), dim3(256), 0, n->stream, x,
+                         W16(n, 2 * L), P32(n, 2 * L + 1), n->pool[L], code, nullptr, per);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((conv_kernel<CI, CO, H, W, false, false>), dim3(G::XB * G::YB, B), dim3(256), 0, n->stream, x, W16(n, 2 * L),
+                     P32(n, 2 * L + 1), n->pool[L], code, nullptr, per);
   return hipGetLastError();
 }
 
