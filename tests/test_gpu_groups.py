@@ -86,3 +86,22 @@ def test_small_tiles_equal_64x64(torch_cuda, w, S, N, arc, c):
     torch = torch_cuda
     auto, auto_kept, single, _ = _both(torch, w, N, [c + 0.01 * k for k in range(S)], ca.PHS, arc, ca.STORE_FP32)
     assert torch.equal(auto, single) and torch.equal(auto_kept, single)
+
+
+@pytest.mark.parametrize("S", [7, 8, 9, 19])
+@pytest.mark.parametrize("interp,store", [(ca.INTERP_LINEAR, ca.STORE_FP32), (ca.INTERP_CTAS, ca.STORE_FP16)])
+@pytest.mark.parametrize("w", [200, 330])
+def test_every_tile_of_many_slices_once(torch_cuda, S, interp, store, w):
+    """Whole slices per XCD, and the rows of those left over: each slice as
+    if it were alone."""
+    torch = torch_cuda
+    sino = _sinos(torch, S, 24, w, ca.ABS, S)
+    rec = ca.CTrec(w, 24, ca.ABS, "HANN", store=store, interp=interp)
+    rec.set_tiles(ca.TILE_64x64, 0)
+    got = torch.full((S, w, w), np.nan, device="cuda")
+    want = torch.empty((w, w), device="cuda")
+    rec.reconstruct_dev(sino, got, [1.25] * S)
+    for s in range(S):
+        rec.reconstruct_dev(sino[s:s + 1], want.view(1, w, w), [1.25])
+        torch.cuda.synchronize()
+        assert torch.equal(got[s], want), s
