@@ -905,8 +905,19 @@ struct StageMirror {
   static constexpr size_t HALFBUF = WIN + sizeof(int) * AC * TAB;
   static constexpr size_t ANGS = 2 * HALFBUF;
   static constexpr size_t BYTES = ANGS + 2 * sizeof(SlotConsts) * AC;
-  static_assert(TR % 4 == 0 && TC % 4 == 0, "16-byte table reads");
+  static_assert(TR % 2 == 0 && TC % 2 == 0, "8- or 16-byte table reads");
   static_assert(AC <= 64, "one lane of the deriving wave per slot");
+  // A 32x32 tile is a quarter of the 64x64 tile at (ty0 - dy, tx0 - dx) and
+  // takes that tile's bases and its entries of that tile's tables, so that
+  // the coordinates are bit for bit the same.
+  static constexpr bool QUARTER = KIND == TK_32x32;
+  int dy = 0, dx = 0;
+  __device__ __forceinline__ void place(const Item &it, int ty0, int tx0) {
+    if constexpr (QUARTER) {
+      dy = ty0 & 32;
+      dx = ((it.w / 2 + 1 - tx0 + 63) & ~63) - (it.w / 2 + 1 - tx0);
+    }
+  }
   typename std::conditional<LIN, float4, u16x2>::type v[EPT][NS];  // the samples of word j
   int t[TPT];    // SY (rows) and CX (columns) entries of this thread
   SlotConsts k;  // constants of this thread's slot, pass being fetched
@@ -931,12 +942,13 @@ struct StageMirror {
     const int l = threadIdx.x & 63;
     const int w = it.w, hp = w / 2;
     const double cd = static_cast<double>(it.center), s = raw.s, co = raw.c;
-    const double rowterm = cd + hp * ((1.0 - s) - co) + s * (ty0 - cd);
+    const int by0 = ty0 - dy, bx0 = tx0 - dx;
+    const double rowterm = cd + hp * ((1.0 - s) - co) + s * (by0 - cd);
     // LINEAR interpolates between bin centres: word floor(t + 1/2)
     const double half = LIN ? 0.5 : 0.0;
-    const double TA = rowterm + co * tx0 + half;             // pixel (ty0, tx0)
-    const double TB = rowterm + co * (2 * hp - tx0) + half;  // its mirror
-    const double hy = s * (0.5 * (RT - 1)), hx = co * (0.5 * (CT - 1));
+    const double TA = rowterm + co * bx0 + half;             // pixel (by0, bx0)
+    const double TB = rowterm + co * (2 * hp - bx0) + half;  // its mirror
+    const double hy = s * (dy + 0.5 * (RT - 1)), hx = co * (dx + 0.5 * (CT - 1));
     SlotConsts c;
     c.loA = static_cast<int>(floor(TA + hy + hx)) - LO;
     c.loB = static_cast<int>(floor(TB + hy - hx)) - LO;
@@ -958,9 +970,18 @@ struct StageMirror {
     const int tid = threadIdx.x, sub = tid - (tid / TPA) * TPA;
     // the slot's row terms (lattice order of this tile kind), then its
     // column terms (lattice order)
-    const int *st = it.slot_tab + (a0 + min(tid / TPA, na - 1)) * kSlotTab + lattice_offset(KIND);
+    const int *st = it.slot_tab + (a0 + min(tid / TPA, na - 1)) * kSlotTab + lattice_offset(QUARTER ? TK_64x64 : KIND);
 #pragma unroll
-    for (int j = 0; j < TPT; ++j) t[j] = ldg32(st, static_cast<unsigned>(min(sub + j * TPA, RT + CT - 1)));
+    for (int j = 0; j < TPT; ++j) {
+      int e = min(sub + j * TPA, RT + CT - 1);
+      if constexpr (QUARTER) {  // row or column of this lattice position, and its place in the 64x64 tables
+        if (e < RT)
+          e = lattice_row(dy + e / (4 * TR) * (4 * TR) + e % TR * 4 + (e / TR & 3), 4);
+        else
+          e = 64 + lattice_col(dx + (e - RT) / TC + 16 * ((e - RT) % TC), 4);
+      }
+      t[j] = ldg32(st, static_cast<unsigned>(e));
+    }
     // offsets from the start of the zero pad before the sinogram; a slot
     // without a partner reads its second samples from the pad's first element
     if constexpr (LIN) {
@@ -1061,6 +1082,7 @@ __device__ __forceinline__ void run_passes_mirror(const Item &it, unsigned char 
                                                   bool wskip, Compute compute) {
   Stage st;
   st.base = lds;
+  st.place(it, ty0, tx0);
   const bool first = threadIdx.x < 64;
   const int N = it.n_slots;
   const int P = (N + AC - 1) / AC;
@@ -1139,17 +1161,25 @@ __device__ __forceinline__ void bp_tile_mirror(const Item &it, int tile, unsigne
     // slot a's row terms (window A, window B) and column terms of this lane
     auto terms = [&](int a, int (&A)[TR], int (&B)[TR], int (&Cq)[TC]) {
       const int *tab = reinterpret_cast<const int *>(buf + S::WIN) + a * S::TAB;
+      if constexpr (TR == 2) {
+        const int2 va = *reinterpret_cast<const int2 *>(tab + rbase), vb = *reinterpret_cast<const int2 *>(tab + RT + rbase);
+        const int2 vc = *reinterpret_cast<const int2 *>(tab + cbase);
+        A[0] = va.x; A[1] = va.y;
+        B[0] = vb.x; B[1] = vb.y;
+        Cq[0] = vc.x; Cq[1] = vc.y;
+      } else {
 #pragma unroll
-      for (int r = 0; r < TR; r += 4) {
-        const int4 va = *reinterpret_cast<const int4 *>(tab + rbase + r);
-        const int4 vb = *reinterpret_cast<const int4 *>(tab + RT + rbase + r);
-        A[r] = va.x; A[r + 1] = va.y; A[r + 2] = va.z; A[r + 3] = va.w;
-        B[r] = vb.x; B[r + 1] = vb.y; B[r + 2] = vb.z; B[r + 3] = vb.w;
-      }
+        for (int r = 0; r < TR; r += 4) {
+          const int4 va = *reinterpret_cast<const int4 *>(tab + rbase + r);
+          const int4 vb = *reinterpret_cast<const int4 *>(tab + RT + rbase + r);
+          A[r] = va.x; A[r + 1] = va.y; A[r + 2] = va.z; A[r + 3] = va.w;
+          B[r] = vb.x; B[r + 1] = vb.y; B[r + 2] = vb.z; B[r + 3] = vb.w;
+        }
 #pragma unroll
-      for (int q = 0; q < TC; q += 4) {
-        const int4 vc = *reinterpret_cast<const int4 *>(tab + cbase + q);
-        Cq[q] = vc.x; Cq[q + 1] = vc.y; Cq[q + 2] = vc.z; Cq[q + 3] = vc.w;
+        for (int q = 0; q < TC; q += 4) {
+          const int4 vc = *reinterpret_cast<const int4 *>(tab + cbase + q);
+          Cq[q] = vc.x; Cq[q + 1] = vc.y; Cq[q + 2] = vc.z; Cq[q + 3] = vc.w;
+        }
       }
     };
     // the words of both windows for the pixel pairs of row r
@@ -1524,6 +1554,10 @@ hipError_t launch_mirror(const Item *d_items, int n_items, int total_tiles, int 
   return hipGetLastError();
 }
 
+// Slots per pass on quarter tiles (50 KB of LDS): with a workgroup or two per
+// CU a pass has to outlast its successor's windows.
+constexpr int kSmallLin = 16, kSmall16 = 32;
+
 template <int KIND>
 hipError_t launch_k(const Item *d_items, int n_items, int total_tiles, int row, int ac, int mode, int store,
                     bool mirror, hipStream_t s) {
@@ -1539,6 +1573,26 @@ hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles,
                               int angles_per_pass, int mode, int store, bool mirror, hipStream_t s) {
   if (total_tiles <= 0) return hipSuccess;
   if (row < 1) return hipErrorInvalidValue;
+  if (mirror && kind == TK_32x32) {
+    switch (store) {
+      case ST_F32:
+        if (mode != MODE_LINEAR) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, kSmallLin, ST_F32_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
+        return hipGetLastError();
+      case ST_F16:
+        if (mode == MODE_LINEAR)
+          hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, kSmallLin, ST_F16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
+        else
+          hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, kSmall16, ST_F16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
+        return hipGetLastError();
+      default:
+        if (mode == MODE_LINEAR) {
+          hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, kSmallLin, ST_BF16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
+          return hipGetLastError();
+        }
+        return launch_mirror<TK_32x32, kSmall16>(d_items, n_items, total_tiles, row, store, s);
+    }
+  }
   if (mirror && mode == MODE_LINEAR) {
     // 64x64 tiles: the 16-byte float words of both windows (16-bit samples
     // converted when staged) fill the static LDS of a workgroup at 4 slots

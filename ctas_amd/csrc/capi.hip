@@ -183,7 +183,7 @@ bool use_mirror(const ctas_fbp *h) { return mirror_applies(h->flags, h->N, h->w,
 // float words of its two windows fill the static LDS of a workgroup).
 bool mirror_linear_applies(int flags, int N, int w, int n_paired, int kind) {
   const int pad = store_of(flags) == ST_F32 ? 0 : filt_pad(w);
-  return mode_of(flags) == MODE_LINEAR && kind == TK_64x64 && 4 * n_paired >= N &&
+  return mode_of(flags) == MODE_LINEAR && (kind == TK_64x64 || kind == TK_32x32) && 4 * n_paired >= N &&
          static_cast<long long>(N) * w + 2LL * pad < (1LL << 31);
 }
 bool use_mirror(const ctas_fbp *h, int kind) {
@@ -237,25 +237,31 @@ struct BpLaunch {
 // against 264) and 726 (16-bit; 571 us against 717, 576 workgroups 513
 // against 454). What remains is taken one by one; float32 launches of less
 // than two 64x64 tiles per CU take 32x32 tiles, and 16x32 ones up to a
-// quarter of a tile per CU (backproject.hip). A tile kind that the caller
-// set is kept, for every slice.
+// quarter of a tile per CU (backproject.hip). Mirrored launches of few tile
+// pairs take quarters of them: LINEAR below 448 (432 of 1024 px 425 us against
+// 479, 484 of 1400 px 554 against 530, 144 of 1024 px 162 against 389), 16-bit
+// below 512 (484 of 1400 px 307 against 316, 144 of 1024 px 113 against 215). A
+// tile kind that the caller set is kept, for every slice.
 std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *centers, int S, std::vector<int> *order) {
   order->resize(S);
   std::iota(order->begin(), order->end(), 0);
   const int kind = choose_kind(h);
-  const bool f32 = store_of(h->flags) == ST_F32, mirror = use_mirror(h);
-  if (h->tile_kind != TK_AUTO || mode_of(h->flags) != MODE_CTAS || (!f32 && !mirror) ||
-      static_cast<long long>(h->N) * h->w >= (1LL << 30))
+  const bool linear = mode_of(h->flags) == MODE_LINEAR, f32 = store_of(h->flags) == ST_F32 && !linear;
+  const bool mirror = use_mirror(h, kind);
+  if (h->tile_kind != TK_AUTO || (!f32 && !mirror) || static_cast<long long>(h->N) * h->w >= (1LL << 30))
     return {{0, S, 1, kind}};
   const long long rows = (h->w + 63) / 64, cols = mirror ? (h->w / 2 + 64) / 64 : rows;
   const long long tiles = rows * cols, cus = h->cus;
   const long long four = (mirror ? 15 : 14) * cus / 8, two = (mirror ? 20 : 9) * cus / 8;
+  const long long small = (linear ? 14 : 16) * cus / 8;
   auto single = [&](int first, int n) {
     BpLaunch l{first, n, 1, kind};
     if (f32 && 4 * n * tiles <= cus) l.kind = TK_16x32;
     else if (f32 && n * tiles < 2 * cus) l.kind = TK_32x32;
+    else if (mirror && kind == TK_64x64 && n * tiles < small) l.kind = TK_32x32;
     return l;
   };
+  if (linear) return {single(0, S)};
   if (f32 && S * tiles < 2 * cus) return {single(0, S)};
   std::map<uint32_t, std::vector<int>> by_centre;
   for (int i = 0; i < S; ++i) {

@@ -1417,7 +1417,9 @@ static int copy_params(ctas_cnn *n, float *host, const float *dev, bool to_host)
   // one after the other on the device first: most of the twelve are small, and
   // each copy has its own latency (gradients of 64 samples and their values on
   // the host: 842 us with twelve copies, 702 with one)
-  if (to_host && ensure_ws(n, count) == CTAS_OK) {
+  // (from the network's own device; copies take any)
+  int dev_now = -1;
+  if (to_host && hipGetDevice(&dev_now) == hipSuccess && dev_now == n->device && ensure_ws(n, count) == CTAS_OK) {
     ctas::cnn::Packing pk;
     for (size_t i = 0, at = 0; i < n->prm.size(); at += n->prm[i++].n) {
       pk.off[i] = static_cast<int>(n->prm[i].off);

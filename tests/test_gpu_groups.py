@@ -105,3 +105,26 @@ def test_every_tile_of_many_slices_once(torch_cuda, S, interp, store, w):
         rec.reconstruct_dev(sino[s:s + 1], want.view(1, w, w), [1.25])
         torch.cuda.synchronize()
         assert torch.equal(got[s], want), s
+
+
+# Mirrored launches of few tile pairs: widths at the edges of the quarter
+# tiles, odd ones, a table with angles that have no partner, and both sides of
+# the tile count where the whole ones take over (448 and 512 at 256 CUs).
+@pytest.mark.parametrize("interp,store", [(ca.INTERP_LINEAR, ca.STORE_FP32), (ca.INTERP_LINEAR, ca.STORE_FP16),
+                                          (ca.INTERP_LINEAR, ca.STORE_BF16), (ca.INTERP_CTAS, ca.STORE_FP16),
+                                          (ca.INTERP_CTAS, ca.STORE_BF16)])
+@pytest.mark.parametrize("S,w,N,c", [(1, 31, 40, 0.0), (1, 33, 37, 1.5), (2, 64, 50, -2.0), (1, 127, 91, 5.5),
+                                     (3, 130, 36, -4.25), (1, 513, 180, 3.37), (3, 1024, 20, 1.0), (4, 1024, 20, 1.0)])
+@pytest.mark.parametrize("contrast,arc", [(ca.ABS, 180.0), (ca.PHS, 360.0)])
+def test_quarter_tiles_equal_whole_ones(torch_cuda, interp, store, S, w, N, c, contrast, arc):
+    torch = torch_cuda
+    sino = _sinos(torch, S, N, w, contrast, w)
+    got = []
+    for kind in (ca.TILE_AUTO, ca.TILE_64x64):
+        rec = ca.CTrec(w, N, contrast, "HANN", anarc=arc, store=store, interp=interp)
+        rec.set_tiles(kind, 0)
+        out = torch.full((S, w, w), np.nan, device="cuda")
+        rec.reconstruct_dev(sino, out, [c + 0.5 * s for s in range(S)])
+        torch.cuda.synchronize()
+        got.append(out)
+    assert torch.equal(got[0], got[1])
