@@ -1197,8 +1197,6 @@ const uint16_t *W16(const ctas_cnn *n, int i) { return n->p16 + n->prm[i].off; }
 const float *P32(const ctas_cnn *n, int i) { return n->p + n->prm[i].off; }
 float *G32(const ctas_cnn *n, int i) { return n->g + n->prm[i].off; }
 
-int blocks_for(size_t n) { return static_cast<int>(std::min<size_t>((n + 255) / 256, 65535)); }
-
 // Splits of the reduction for a product whose C tiles alone would not fill
 // the chip (inference on a single sinogram); 1 when they do.
 int forward_splits(int M, int N, int K) {
