@@ -1554,9 +1554,20 @@ hipError_t launch_mirror(const Item *d_items, int n_items, int total_tiles, int 
   return hipGetLastError();
 }
 
-// Slots per pass on quarter tiles (50 KB of LDS): with a workgroup or two per
-// CU a pass has to outlast its successor's windows.
-constexpr int kSmallLin = 16, kSmall16 = 32;
+// Quarter tiles, LIN slots per pass LINEAR and twice as many of 16-bit data.
+template <int LIN>
+hipError_t launch_quarters(const Item *d_items, int n_items, int total_tiles, int row, int mode, int store, hipStream_t s) {
+  if (mode != MODE_LINEAR) {
+    if (store == ST_F32) return hipErrorInvalidValue;
+    return launch_mirror<TK_32x32, 2 * LIN>(d_items, n_items, total_tiles, row, store, s);
+  }
+  switch (store) {
+    case ST_F32: hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, LIN, ST_F32_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
+    case ST_F16: hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, LIN, ST_F16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
+    default: hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, LIN, ST_BF16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row); break;
+  }
+  return hipGetLastError();
+}
 
 template <int KIND>
 hipError_t launch_k(const Item *d_items, int n_items, int total_tiles, int row, int ac, int mode, int store,
@@ -1574,24 +1585,12 @@ hipError_t launch_backproject(const Item *d_items, int n_items, int total_tiles,
   if (total_tiles <= 0) return hipSuccess;
   if (row < 1) return hipErrorInvalidValue;
   if (mirror && kind == TK_32x32) {
-    switch (store) {
-      case ST_F32:
-        if (mode != MODE_LINEAR) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, kSmallLin, ST_F32_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
-        return hipGetLastError();
-      case ST_F16:
-        if (mode == MODE_LINEAR)
-          hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, kSmallLin, ST_F16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
-        else
-          hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, kSmall16, ST_F16>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
-        return hipGetLastError();
-      default:
-        if (mode == MODE_LINEAR) {
-          hipLaunchKernelGGL((bp_mirror_kernel<TK_32x32, kSmallLin, ST_BF16_LIN>), dim3(total_tiles), dim3(256), 0, s, d_items, n_items, row);
-          return hipGetLastError();
-        }
-        return launch_mirror<TK_32x32, kSmall16>(d_items, n_items, total_tiles, row, store, s);
-    }
+    // With a workgroup or two per CU a pass has to outlast its successor's
+    // windows (50 KB of LDS); with more than the three that fit so, half the
+    // slots: LINEAR, 144 tile pairs of 1024 px 163 us with all and 184 with
+    // half, 288 of them 296 and 263
+    if (angles_per_pass == 32) return launch_quarters<16>(d_items, n_items, total_tiles, row, mode, store, s);
+    return launch_quarters<8>(d_items, n_items, total_tiles, row, mode, store, s);
   }
   if (mirror && mode == MODE_LINEAR) {
     // 64x64 tiles: the 16-byte float words of both windows (16-bit samples

@@ -238,9 +238,10 @@ struct BpLaunch {
 // against 454). What remains is taken one by one; float32 launches of less
 // than two 64x64 tiles per CU take 32x32 tiles, and 16x32 ones up to a
 // quarter of a tile per CU (backproject.hip). Mirrored launches of few tile
-// pairs take quarters of them: LINEAR below 448 (432 of 1024 px 425 us against
-// 479, 484 of 1400 px 554 against 530, 144 of 1024 px 162 against 389), 16-bit
-// below 512 (484 of 1400 px 307 against 316, 144 of 1024 px 113 against 215). A
+// pairs take quarters of them: LINEAR below four per CU, where whole ones do not
+// fill the chip once (144 of 1024 px 165 us against 389, 484 of 1400 px 485
+// against 532, 1008 of 1024 px 750 against 773, 1088 of 2048 px 1541 against
+// 1520), 16-bit below three (144 113 against 215, 726 of 1400 px 394 against 410). A
 // tile kind that the caller set is kept, for every slice.
 std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *centers, int S, std::vector<int> *order) {
   order->resize(S);
@@ -253,7 +254,7 @@ std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *center
   const long long rows = (h->w + 63) / 64, cols = mirror ? (h->w / 2 + 64) / 64 : rows;
   const long long tiles = rows * cols, cus = h->cus;
   const long long four = (mirror ? 15 : 14) * cus / 8, two = (mirror ? 20 : 9) * cus / 8;
-  const long long small = (linear ? 14 : 16) * cus / 8;
+  const long long small = (linear ? 4 : 3) * cus;
   auto single = [&](int first, int n) {
     BpLaunch l{first, n, 1, kind};
     if (f32 && 4 * n * tiles <= cus) l.kind = TK_16x32;
@@ -297,10 +298,13 @@ int launch_planned(const ctas_fbp *h, const std::vector<BpLaunch> &launches, hip
     const int tiles = items[l.first].tiles, row = items[l.first].tiles_x, mode = mode_of(h->flags);
     const bool mirror = use_mirror(h, l.kind);
     const int st = bp_store(store_of(h->flags), h->contrast, mirror);
+    // quarter tiles: as many angles per pass as leave every workgroup resident
+    const bool quarters = mirror && l.kind == TK_32x32;
+    const int ac = !quarters ? choose_ac(h) : static_cast<long long>(tiles) * l.items <= 3 * h->cus ? 32 : 16;
     if (l.group > 1)
       CTAS_HIP_TRY(launch_backproject_groups(h->d_items + l.first, l.items / l.group, l.group, tiles, row, st, mirror, s));
     else
-      CTAS_HIP_TRY(launch_backproject(h->d_items + l.first, l.items, tiles * l.items, row, l.kind, choose_ac(h), mode, st,
+      CTAS_HIP_TRY(launch_backproject(h->d_items + l.first, l.items, tiles * l.items, row, l.kind, ac, mode, st,
                                       mirror, s));
   }
   return CTAS_OK;

@@ -128,3 +128,11 @@ def test_quarter_tiles_equal_whole_ones(torch_cuda, interp, store, S, w, N, c, c
         torch.cuda.synchronize()
         got.append(out)
     assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("interp,store", [(ca.INTERP_LINEAR, ca.STORE_FP32), (ca.INTERP_CTAS, ca.STORE_BF16)])
+@pytest.mark.parametrize("S", [5, 6, 7, 8])
+def test_quarter_tiles_where_whole_ones_take_over(torch_cuda, interp, store, S):
+    """720, 864, 1008 and 1152 tile pairs: the last counts on quarters are 720
+    of 16-bit storage and 1008 LINEAR at 256 CUs."""
+    test_quarter_tiles_equal_whole_ones(torch_cuda, interp, store, S, 1024, 20, 1.0, ca.ABS, 180.0)
