@@ -64,10 +64,22 @@ int grow(T *&ptr, size_t &cap, size_t bytes) {
   return CTAS_OK;
 }
 
+// Room for the filtered slices and for the slices' extrema and status; what a
+// captured graph uses is left to it.
+int ensure_filt(ctas_fbp *h, size_t bytes) {
+  if (bytes > h->filt_cap && h->d_filt == h->graph.filt) {
+    h->d_filt = nullptr;
+    h->filt_cap = 0;
+  }
+  return grow(h->d_filt, h->filt_cap, bytes);
+}
+
 int ensure_slices(ctas_fbp *h, int S) {
   if (S <= h->mm_cap && h->d_minmax) return CTAS_OK;
-  if (h->d_minmax) (void)hipFree(h->d_minmax);
-  if (h->d_status) (void)hipFree(h->d_status);
+  if (h->d_minmax != h->graph.minmax) {
+    if (h->d_minmax) (void)hipFree(h->d_minmax);
+    if (h->d_status) (void)hipFree(h->d_status);
+  }
   h->d_minmax = nullptr;
   h->d_status = nullptr;
   h->mm_cap = 0;
@@ -292,8 +304,9 @@ std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *center
   return launches;
 }
 
-int launch_planned(const ctas_fbp *h, const std::vector<BpLaunch> &launches, hipStream_t s) {
-  const std::vector<Item> &items = extra(h).resident;
+// items: the host's copy of d_items
+int launch_planned(const ctas_fbp *h, const Item *d_items, const std::vector<Item> &items,
+                   const std::vector<BpLaunch> &launches, hipStream_t s) {
   for (const BpLaunch &l : launches) {
     const int tiles = items[l.first].tiles, row = items[l.first].tiles_x, mode = mode_of(h->flags);
     const bool mirror = use_mirror(h, l.kind);
@@ -302,10 +315,10 @@ int launch_planned(const ctas_fbp *h, const std::vector<BpLaunch> &launches, hip
     const bool quarters = mirror && l.kind == TK_32x32;
     const int ac = !quarters ? choose_ac(h) : static_cast<long long>(tiles) * l.items <= 3 * h->cus ? 32 : 16;
     if (l.group > 1)
-      CTAS_HIP_TRY(launch_backproject_groups(h->d_items + l.first, l.items / l.group, l.group, tiles, row, st, mirror, s));
+      CTAS_HIP_TRY(launch_backproject_groups(d_items + l.first, l.items / l.group, l.group, tiles, row, st, mirror, s));
     else
-      CTAS_HIP_TRY(launch_backproject(h->d_items + l.first, l.items, tiles * l.items, row, l.kind, ac, mode, st,
-                                      mirror, s));
+      CTAS_HIP_TRY(launch_backproject(d_items + l.first, l.items, tiles * l.items, row, l.kind, ac, mode, st, mirror,
+                                      s));
   }
   return CTAS_OK;
 }
@@ -512,10 +525,10 @@ int stream_wait(hipStream_t waiter, hipStream_t producer) {
 
 namespace {
 
-// Enqueue prepare (+ optional backprojection) for S slices of device data;
-// `filtered` (optional) is recorded between the two.
-int enqueue_slices(ctas_fbp *h, const float *d_sino, float *d_out, float *d_f32,
-                   const float *centers, int S, bool do_bp, hipStream_t s, hipEvent_t filtered = nullptr) {
+// The items and launches of prepare (+ optional backprojection) for S slices
+// of device data, and room for what they write on the device.
+int plan_slices(ctas_fbp *h, const float *d_sino, float *d_out, float *d_f32, const float *centers, int S, bool do_bp,
+                std::vector<Item> &items, std::vector<BpLaunch> &launches) {
   if (S <= 0) return fail(CTAS_E_ARG, "number of slices must be positive");
   if (do_bp)
     for (int i = 0; i < S; ++i)
@@ -524,14 +537,14 @@ int enqueue_slices(ctas_fbp *h, const float *d_sino, float *d_out, float *d_f32,
   const size_t slice_elems = static_cast<size_t>(h->N) * h->w;
   const int pad = filt_pad_of(h);
   const size_t stride = slice_elems + 2 * static_cast<size_t>(pad);
-  if (int rc = grow(h->d_filt, h->filt_cap, stride * S * store_bytes(st))) return rc;
+  if (int rc = ensure_filt(h, stride * S * store_bytes(st))) return rc;
   if (int rc = ensure_slices(h, S)) return rc;
   std::vector<int> order(S);
   std::iota(order.begin(), order.end(), 0);
-  std::vector<BpLaunch> launches{{0, S, 1, choose_kind(h)}};
+  launches = {{0, S, 1, choose_kind(h)}};
   if (do_bp) launches = plan_backprojection(h, centers, S, &order);
   const int pairs = (h->N + 1) / 2;
-  std::vector<Item> items(S);
+  items.assign(S, Item{});
   for (const BpLaunch &l : launches)
     for (int k = l.first; k < l.first + l.items; ++k) {
       const int i = order[k];
@@ -548,13 +561,29 @@ int enqueue_slices(ctas_fbp *h, const float *d_sino, float *d_out, float *d_f32,
       it.pair_base = pairs * k;
       items[k] = it;
     }
+  return CTAS_OK;
+}
+
+// The kernels of planned slices, whose table `items` lies at d_items;
+// `filtered` (optional) is recorded between the two stages.
+int launch_slices(const ctas_fbp *h, const Item *d_items, const std::vector<Item> &items,
+                  const std::vector<BpLaunch> &launches, bool do_bp, hipStream_t s, hipEvent_t filtered = nullptr) {
+  const int S = static_cast<int>(items.size()), st = store_of(h->flags);
+  if (filt_pad_of(h)) CTAS_HIP_TRY(launch_pad_zero(d_items, S, s));
+  CTAS_HIP_TRY(launch_filter(d_items, S, (h->N + 1) / 2 * S, h->logZ, h->logZ, h->contrast, st, s));
+  if (filtered) CTAS_HIP_TRY(hipEventRecord(filtered, s));
+  return do_bp ? launch_planned(h, d_items, items, launches, s) : CTAS_OK;
+}
+
+// Enqueue prepare (+ optional backprojection) for S slices of device data.
+int enqueue_slices(ctas_fbp *h, const float *d_sino, float *d_out, float *d_f32,
+                   const float *centers, int S, bool do_bp, hipStream_t s, hipEvent_t filtered = nullptr) {
+  std::vector<Item> items;
+  std::vector<BpLaunch> launches;
+  if (int rc = plan_slices(h, d_sino, d_out, d_f32, centers, S, do_bp, items, launches)) return rc;
   bool changed = false;
   if (int rc = upload_items(h, items, s, &changed, extra(h).resident)) return rc;
-  if (pad) CTAS_HIP_TRY(launch_pad_zero(h->d_items, S, s));
-  CTAS_HIP_TRY(launch_filter(h->d_items, S, pairs * S, h->logZ, h->logZ, h->contrast, st, s));
-  if (filtered) CTAS_HIP_TRY(hipEventRecord(filtered, s));
-  if (do_bp)
-    if (int rc = launch_planned(h, launches, s)) return rc;
+  if (int rc = launch_slices(h, h->d_items, items, launches, do_bp, s, filtered)) return rc;
   h->last_S = S;
   return CTAS_OK;
 }
@@ -590,7 +619,40 @@ int enqueue_repeat(ctas_fbp *h, int slice, float *d_out, const float *centers, i
     }
   bool changed = false;
   if (int rc = upload_items(h, items, s, &changed, extra(h).resident)) return rc;
-  return launch_planned(h, launches, s);
+  return launch_planned(h, h->d_items, items, launches, s);
+}
+
+// Frees the captured graph, its table and the buffers that only it holds.
+// Nothing of it may be running.
+void drop_graph(ctas_fbp *h) {
+  if (h->graph.exec) (void)hipGraphExecDestroy(h->graph.exec);
+  if (h->graph.graph) (void)hipGraphDestroy(h->graph.graph);
+  if (h->graph.d_items) (void)hipFree(h->graph.d_items);
+  if (h->graph.filt && h->graph.filt != h->d_filt) (void)hipFree(h->graph.filt);
+  if (h->graph.minmax && h->graph.minmax != h->d_minmax) {
+    (void)hipFree(h->graph.minmax);
+    (void)hipFree(h->graph.status);
+  }
+  h->graph = {};
+}
+
+// The buffers of a replay are the handle's own again (a call after the capture
+// may have needed larger ones): ctas_fbp_status and the filtered slices for
+// repeat are the replay's.
+void take_graph_buffers(ctas_fbp *h) {
+  if (h->d_filt != h->graph.filt) {
+    if (h->d_filt) (void)hipFree(h->d_filt);
+    h->d_filt = h->graph.filt;
+    h->filt_cap = h->graph.filt_cap;
+    h->kept_slices = std::min(h->kept_slices, static_cast<int>(h->graph.items.size()));
+  }
+  if (h->d_minmax != h->graph.minmax) {
+    if (h->d_minmax) (void)hipFree(h->d_minmax);
+    if (h->d_status) (void)hipFree(h->d_status);
+    h->d_minmax = h->graph.minmax;
+    h->d_status = h->graph.status;
+    h->mm_cap = h->graph.mm_cap;
+  }
 }
 
 // The status words carry deAbs (ABS contrast) and the FP16 range check (FP16
@@ -884,8 +946,7 @@ int ctas_fbp_clone(const ctas_fbp *src, ctas_fbp **ph) {
 int ctas_fbp_destroy(ctas_fbp *h) {
   if (!h) return CTAS_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  if (h->graph_exec) (void)hipGraphExecDestroy(h->graph_exec);
-  if (h->graph) (void)hipGraphDestroy(h->graph);
+  drop_graph(h);
   void *ptrs[] = {h->d_W, h->d_sincos, h->d_sincos64, h->d_slots, h->d_slot_tab, h->d_tw, h->d_filt, h->d_io, h->d_out, h->d_minmax,
                   h->d_status, h->d_items, h->d_centres, h->d_partial, h->d_scores};
   for (void *p : ptrs)
@@ -946,7 +1007,16 @@ int ctas_fbp_set_angles(ctas_fbp *h, const float *sincos) {
   std::vector<double> sc64(h->sincos.begin(), h->sincos.end());
   h->neg_sin = any_negative_sine(sc64);
   CTAS_HIP_TRY(hipMemcpy(h->d_sincos64, sc64.data(), sizeof(double) * sc64.size(), hipMemcpyHostToDevice));
-  return upload_slots(h, sc64);
+  if (int rc = upload_slots(h, sc64)) return rc;
+  // a captured graph reads the same tables; its items count their entries
+  auto &g = h->graph;
+  if (g.items.empty()) return CTAS_OK;
+  for (Item &it : g.items) {
+    it.neg_sin = h->neg_sin;
+    if (it.slots) it.n_slots = h->n_slots;
+  }
+  CTAS_HIP_TRY(hipMemcpy(g.d_items, g.items.data(), sizeof(Item) * g.items.size(), hipMemcpyHostToDevice));
+  return CTAS_OK;
 }
 
 int ctas_fbp_get_angles(const ctas_fbp *h, float *sincos) {
@@ -1088,44 +1158,49 @@ int ctas_fbp_graph_capture(ctas_fbp *h, const float *d_sino, float *d_out, const
                            void *stream) {
   if (!h || !d_sino || !d_out || !centers) return fail(CTAS_E_ARG, "bad arguments");
   hipStream_t s = pick_stream(h, stream);
-  if (h->graph_exec) {
-    (void)hipGraphExecDestroy(h->graph_exec);
-    h->graph_exec = nullptr;
-  }
-  if (h->graph) {
-    (void)hipGraphDestroy(h->graph);
-    h->graph = nullptr;
-  }
-  // Make the item table resident before capture so that no copy is recorded.
-  if (!stream) CTAS_HIP_TRY(hipDeviceSynchronize());
+  // what an earlier graph of this handle still runs uses its table and buffers
   CTAS_HIP_TRY(hipStreamSynchronize(s));
-  extra(h).resident.clear();
-  {
-    // first enqueue uploads the table; it also runs the work once
-    if (int rc = enqueue_slices(h, d_sino, d_out, nullptr, centers, S, true, s)) return rc;
-    CTAS_HIP_TRY(hipStreamSynchronize(s));
+  CTAS_HIP_TRY(hipStreamSynchronize(h->stream));
+  drop_graph(h);
+  if (!stream) CTAS_HIP_TRY(hipDeviceSynchronize());
+  // the work once, uncaptured: it loads the kernels
+  if (int rc = enqueue_slices(h, d_sino, d_out, nullptr, centers, S, true, s)) return rc;
+  CTAS_HIP_TRY(hipStreamSynchronize(s));
+  // a table of the graph's own, which later calls on the handle leave alone
+  auto &gr = h->graph;
+  std::vector<BpLaunch> launches;
+  int rc = plan_slices(h, d_sino, d_out, nullptr, centers, S, true, gr.items, launches);
+  if (!rc && hipMalloc(&gr.d_items, sizeof(Item) * S) != hipSuccess)
+    rc = fail(CTAS_E_NOMEM, "device allocation of the item table failed");
+  hipError_t e = hipSuccess;
+  if (!rc) e = hipMemcpy(gr.d_items, gr.items.data(), sizeof(Item) * S, hipMemcpyHostToDevice);
+  if (!rc && e == hipSuccess) e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+  if (!rc && e == hipSuccess) {
+    rc = launch_slices(h, gr.d_items, gr.items, launches, true, s);
+    e = hipStreamEndCapture(s, &gr.graph);
   }
-  CTAS_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-  const int rc = enqueue_slices(h, d_sino, d_out, nullptr, centers, S, true, s);
-  hipGraph_t g = nullptr;
-  const hipError_t e = hipStreamEndCapture(s, &g);
+  if (!rc && e == hipSuccess) e = hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0);
+  if (!rc && e != hipSuccess) rc = fail(CTAS_E_DEVICE, std::string("graph capture: ") + hipGetErrorString(e));
   if (rc) {
-    if (g) (void)hipGraphDestroy(g);
+    drop_graph(h);
     return rc;
   }
-  if (e != hipSuccess) return fail(CTAS_E_DEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-  h->graph = g;
-  CTAS_HIP_TRY(hipGraphInstantiate(&h->graph_exec, g, nullptr, nullptr, 0));
+  gr.filt = h->d_filt;
+  gr.filt_cap = h->filt_cap;
+  gr.minmax = h->d_minmax;
+  gr.status = h->d_status;
+  gr.mm_cap = h->mm_cap;
   h->kept_slices = S;
   return CTAS_OK;
 }
 
 int ctas_fbp_graph_launch(ctas_fbp *h, void *stream) {
   if (!h) return fail(CTAS_E_ARG, "null handle");
-  if (!h->graph_exec) return fail(CTAS_E_STATE, "no captured graph: call ctas_fbp_graph_capture first");
+  if (!h->graph.exec) return fail(CTAS_E_STATE, "no captured graph: call ctas_fbp_graph_capture first");
   NullStreamJoin join(h->stream, stream);
   if (join.rc) return join.rc;
-  CTAS_HIP_TRY(hipGraphLaunch(h->graph_exec, pick_stream(h, stream)));
+  take_graph_buffers(h);
+  CTAS_HIP_TRY(hipGraphLaunch(h->graph.exec, pick_stream(h, stream)));
   return CTAS_OK;
 }
 

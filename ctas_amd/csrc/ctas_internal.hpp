@@ -305,6 +305,15 @@ struct ctas_fbp {
   int tile_kind = ctas::TK_AUTO;
   int angles_per_pass = 0;
 
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t graph_exec = nullptr;
+  // The captured graph: its item table (and the host's copy), which no later
+  // call changes, and the workspaces that its kernels use. One of those that a
+  // later call replaces stays until the graph goes or the next replay.
+  struct {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    std::vector<ctas::Item> items;
+    ctas::Item *d_items = nullptr;
+    void *filt = nullptr;  size_t filt_cap = 0;  // bytes
+    float2 *minmax = nullptr; int *status = nullptr; int mm_cap = 0;  // slices
+  } graph;
 };

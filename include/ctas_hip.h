@@ -141,7 +141,11 @@ int ctas_fbp_repeat_dev(ctas_fbp *h, int slice, float *d_out, const float *cente
 int ctas_fbp_prepare_dev(ctas_fbp *h, const float *d_sino, int S, void *stream);
 int ctas_fbp_backproject_dev(ctas_fbp *h, float *d_out, const float *centers, int S, void *stream);
 /* Capture reconstruct_dev(d_sino, d_out, centers, S) into a hipGraph owned
- * by the handle, then replay it. No memset nodes are recorded. */
+ * by the handle, then replay it. No memset nodes are recorded. Other calls on
+ * the handle between the capture and a replay do not change what the replay
+ * does (ctas_fbp_set_angles does: the graph reads the handle's tables), and
+ * after it the filtered slices and ctas_fbp_status are the replay's. A new
+ * capture or ctas_fbp_destroy frees the graph: no replay may be running. */
 int ctas_fbp_graph_capture(ctas_fbp *h, const float *d_sino, float *d_out,
                            const float *centers, int S, void *stream);
 int ctas_fbp_graph_launch(ctas_fbp *h, void *stream);
