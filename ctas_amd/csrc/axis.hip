@@ -537,6 +537,10 @@ extern "C" int ctas_raxis_pair(const float *p0, const float *p180, int rows, int
   auto whole_errs = [&](const std::vector<int> &sh, float *e) {
     const int k = static_cast<int>(sh.size());
     if (dev_rc != CTAS_OK) return;
+    if (k < 1 || k > max_trials) {  // what the device buffers hold
+      dev_rc = fail(CTAS_E_AXIS, "Failed to calculate rotation centre.");
+      return;
+    }
     std::vector<double> acc(k);
     if (hipMemcpy(d_sh, sh.data(), sizeof(int) * k, hipMemcpyHostToDevice) != hipSuccess) {
       dev_rc = fail(CTAS_E_DEVICE, "registration: upload failed");
@@ -567,6 +571,7 @@ extern "C" int ctas_raxis_pair(const float *p0, const float *p180, int rows, int
     for (size_t i = 0; i < sh.size(); ++i) sh[i] = lo + static_cast<int>(i);
     std::vector<float> err(sh.size());
     whole_errs(sh, err.data());
+    if (dev_rc != CTAS_OK) return 0.0f;
     return improve_me(1.0f, at, e, idx, dir, [&](float x) { return err[static_cast<int>(static_cast<long>(x)) - lo]; }, rc);
   };
   std::vector<float> offsets(n_trials), errors(n_trials);
@@ -588,9 +593,10 @@ extern "C" int ctas_raxis_pair(const float *p0, const float *p180, int rows, int
   const int walk_limit = static_cast<int>((static_cast<float>(w / 2) - static_cast<float>(dir) * offsets[idx]) / kStep);
   if (walk_limit <= 0) return fail(CTAS_E_AXIS, "Failed to calculate rotation centre.");
   std::vector<float> walk_offsets(walk_limit + 2), walk_errors(walk_limit + 2);
-  walk_offsets[0] = offsets[idx - dir];
+  // a sweep of one trial (maxDev w < 8) has no neighbour: the next grid point
+  // is the bracket's other side
+  walk_offsets[0] = n_trials > 1 ? offsets[idx - dir] : offsets[idx] - static_cast<float>(dir * kStep);
   walk_offsets[1] = offsets[idx];
-  walk_errors[0] = errors[idx - dir];
   walk_errors[1] = errors[idx];
   int walk_best = 1;
   for (int i = 0; i < walk_limit; ++i) walk_offsets[i + 2] = offsets[idx] + static_cast<float>(dir * (i + 1) * kStep);

@@ -700,8 +700,9 @@ int orc_raxis_pair(const float *p0, const float *p180, int rows, int w, float ma
     if (maxSteps <= 0) { rc = -4; goto done; }
     float *v2 = (float *)malloc(sizeof(float) * (size_t)(maxSteps + 2));
     float *e2 = (float *)malloc(sizeof(float) * (size_t)(maxSteps + 2));
-    v2[0] = vax[idx - cdir]; v2[1] = vax[idx];
-    e2[0] = err[idx - cdir]; e2[1] = err[idx];
+    /* a sweep of one trial has no neighbour: the next grid point */
+    v2[0] = steps > 1 ? vax[idx - cdir] : vax[idx] - (float)(cdir * stpsz); v2[1] = vax[idx];
+    e2[0] = steps > 1 ? err[idx - cdir] : 0.0f; e2[1] = err[idx];
     int idx2 = 1;
     for (int i = 0; i < maxSteps; i++) {
       v2[i + 2] = vax[idx] + (float)(cdir * (i + 1) * stpsz);
