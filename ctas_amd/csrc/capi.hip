@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "ctas_internal.hpp"
+#include "pools.hpp"
 
 namespace ctas {
 
@@ -330,54 +331,6 @@ hipStream_t pick_stream(const ctas_fbp *h, void *stream) {
 }  // namespace
 
 namespace {
-std::mutex g_scratch_pool_mu;
-std::map<int, std::vector<void *>> g_scratch_pool;  // by device, kScratchBytes each
-}  // namespace
-
-Scratch::Scratch(size_t bytes) : bytes_(std::max<size_t>(bytes, 1)) {
-  if (hipGetDevice(&dev_) != hipSuccess) return;
-  if (bytes_ <= kScratchBytes) {
-    bytes_ = kScratchBytes;
-    std::lock_guard<std::mutex> lk(g_scratch_pool_mu);
-    auto &pool = g_scratch_pool[dev_];
-    if (!pool.empty()) {
-      p_ = pool.back();
-      pool.pop_back();
-      return;
-    }
-  }
-  if (hipMalloc(&p_, bytes_) != hipSuccess) p_ = nullptr;
-}
-
-Scratch::~Scratch() {
-  if (!p_) return;
-  if (done_ && bytes_ == kScratchBytes) {
-    std::lock_guard<std::mutex> lk(g_scratch_pool_mu);
-    auto &pool = g_scratch_pool[dev_];
-    if (pool.size() < static_cast<size_t>(kScratchKept)) {
-      pool.push_back(p_);
-      return;
-    }
-  }
-  (void)hipFree(p_);
-}
-
-namespace {
-
-// Pinned blocks, events and a stream for copies between a caller's arrays and
-// the device. The runtime's own copies of pageable memory move 4 MiB at 15
-// GB/s here (33 GB/s at 17 MB, where it pins the caller's pages). With pinned
-// blocks the host's copy to or from one runs beside the device's copy of
-// another; a kernel makes the latter, since a queued hipMemcpyAsync of a block
-// costs tens of microseconds. One slice of 1024 px x 900 angles from and to
-// host arrays: 851 us by the runtime, 534 with blocks of 512 KiB, 637 with 1
-// MiB, 670 with 256 KiB (643 by hipMemcpyAsync of 1 MiB). Allocating them
-// takes milliseconds, so a set goes back to a pool: at most kStagingSets per
-// device exist (4 MiB each), one call uses a set at a time, and a call that
-// gets none copies as before.
-constexpr size_t kStagingBlock = size_t{1} << 19;
-constexpr int kStagingBlocks = 8, kStagingSets = 4;
-constexpr size_t kStagingMost = size_t{8} << 20;  // larger copies are the runtime's
 
 // bytes / 4 words between a pinned block and device memory, both aligned to 16.
 __global__ __launch_bounds__(256) void staging_copy_kernel(uint32_t *__restrict__ dst, const uint32_t *__restrict__ src,
@@ -387,130 +340,14 @@ __global__ __launch_bounds__(256) void staging_copy_kernel(uint32_t *__restrict_
   for (int i = t; i < quads; i += stride) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
   if (t < (words & 3)) dst[4 * quads + t] = src[4 * quads + t];
 }
+
+}  // namespace
+
 hipError_t staging_copy(void *dst, const void *src, size_t bytes, hipStream_t s) {
   hipLaunchKernelGGL(staging_copy_kernel, dim3(128), dim3(256), 0, s, static_cast<uint32_t *>(dst),
                      static_cast<const uint32_t *>(src), static_cast<int>(bytes / 4));
   return hipGetLastError();
 }
-
-struct StagingSet {
-  int dev = 0;
-  unsigned char *block[kStagingBlocks] = {};
-  hipEvent_t free[kStagingBlocks] = {};  // the last copy that used the block
-  hipEvent_t mark = nullptr;
-  hipStream_t stream = nullptr;
-
-  ~StagingSet() {
-    if (stream) (void)hipStreamDestroy(stream);
-    if (mark) (void)hipEventDestroy(mark);
-    for (hipEvent_t e : free)
-      if (e) (void)hipEventDestroy(e);
-    if (block[0]) (void)hipHostFree(block[0]);
-  }
-  bool make() {
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void **>(&block[0]), kStagingBlock * kStagingBlocks) != hipSuccess)
-      return false;
-    for (int b = 0; b < kStagingBlocks; ++b) {
-      block[b] = block[0] + kStagingBlock * b;
-      if (hipEventCreateWithFlags(&free[b], hipEventDisableTiming) != hipSuccess) return false;
-    }
-    return hipEventCreateWithFlags(&mark, hipEventDisableTiming) == hipSuccess &&
-           hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) == hipSuccess;
-  }
-};
-
-std::mutex g_staging_mu;
-std::map<int, std::vector<std::unique_ptr<StagingSet>>> g_staging;  // the sets not in use
-std::map<int, int> g_staging_made;
-
-// A set of the current device for one call; given back once nothing of it is
-// in flight.
-class Staging {
- public:
-  Staging() {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return;
-    {
-      std::lock_guard<std::mutex> lk(g_staging_mu);
-      auto &idle = g_staging[dev];
-      if (!idle.empty()) {
-        set_ = std::move(idle.back());
-        idle.pop_back();
-        return;
-      }
-      if (g_staging_made[dev] >= kStagingSets) return;
-      ++g_staging_made[dev];
-    }
-    set_.reset(new StagingSet);
-    if (set_->make()) return;
-    set_.reset();
-    std::lock_guard<std::mutex> lk(g_staging_mu);
-    --g_staging_made[dev];
-  }
-  ~Staging() {
-    if (!set_) return;
-    (void)hipStreamSynchronize(set_->stream);
-    for (hipEvent_t e : set_->free) (void)hipEventSynchronize(e);
-    std::lock_guard<std::mutex> lk(g_staging_mu);
-    g_staging[set_->dev].push_back(std::move(set_));
-  }
-  Staging(const Staging &) = delete;
-  Staging &operator=(const Staging &) = delete;
-
-  explicit operator bool() const { return set_ != nullptr; }
-  hipStream_t stream() const { return set_->stream; }
-  hipEvent_t mark() const { return set_->mark; }
-
-  // Queues host -> device copies on s; src may be changed on return.
-  hipError_t upload(void *dst, const void *src, size_t bytes, hipStream_t s) {
-    if (bytes > kStagingMost) return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
-    for (size_t off = 0; off < bytes; off += kStagingBlock, next_ = (next_ + 1) % kStagingBlocks) {
-      const size_t n = std::min(kStagingBlock, bytes - off);
-      const int b = next_;
-      if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
-      std::memcpy(set_->block[b], static_cast<const unsigned char *>(src) + off, n);
-      if (hipError_t e = staging_copy(static_cast<unsigned char *>(dst) + off, set_->block[b], n, s); e != hipSuccess)
-        return e;
-      if (hipError_t e = hipEventRecord(set_->free[b], s); e != hipSuccess) return e;
-    }
-    return hipSuccess;
-  }
-  // Device -> host on the set's stream, complete on return.
-  hipError_t download(void *dst, const void *src, size_t bytes) {
-    if (bytes > kStagingMost) {
-      if (hipError_t e = hipStreamSynchronize(set_->stream); e != hipSuccess) return e;
-      return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
-    }
-    const size_t chunks = (bytes + kStagingBlock - 1) / kStagingBlock;
-    auto size = [&](size_t c) { return std::min(kStagingBlock, bytes - c * kStagingBlock); };
-    auto queue = [&](size_t c) -> hipError_t {
-      const int b = static_cast<int>(c % kStagingBlocks);
-      if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
-      if (hipError_t e = staging_copy(set_->block[b], static_cast<const unsigned char *>(src) + c * kStagingBlock,
-                                      size(c), set_->stream);
-          e != hipSuccess)
-        return e;
-      return hipEventRecord(set_->free[b], set_->stream);
-    };
-    for (size_t c = 0; c < std::min<size_t>(chunks, kStagingBlocks); ++c)
-      if (hipError_t e = queue(c); e != hipSuccess) return e;
-    for (size_t c = 0; c < chunks; ++c) {
-      const int b = static_cast<int>(c % kStagingBlocks);
-      if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
-      std::memcpy(static_cast<unsigned char *>(dst) + c * kStagingBlock, set_->block[b], size(c));
-      if (c + kStagingBlocks < chunks)
-        if (hipError_t e = queue(c + kStagingBlocks); e != hipSuccess) return e;
-    }
-    return hipSuccess;
-  }
-
- private:
-  std::unique_ptr<StagingSet> set_;
-  int next_ = 0;
-};
-
-}  // namespace
 
 int stream_wait(hipStream_t waiter, hipStream_t producer) {
   if (waiter == producer) return CTAS_OK;
@@ -1061,7 +898,7 @@ static int host_run(ctas_fbp *h, float *sino, float *out, const float *centers, 
   hipStream_t s = h->stream;
   CTAS_HIP_TRY(hipStreamSynchronize(s));
   float *d_f32 = f32_copy ? h->d_io + slice_elems * S : nullptr;
-  Staging staging;
+  Staging staging(h->device);
   // Every return below leaves no work of this call on the stream.
   struct Drain {
     hipStream_t s;
@@ -1105,7 +942,7 @@ int ctas_fbp_repeat(ctas_fbp *h, float *out, const float *centers, int n) {
   if (int rc = enqueue_repeat(h, 0, h->d_out, centers, n, h->stream)) return rc;
   CTAS_HIP_TRY(hipStreamSynchronize(h->stream));
   const size_t bytes = sizeof(float) * h->w * h->w * n;
-  Staging staging;
+  Staging staging(h->device);
   CTAS_HIP_TRY(staging ? staging.download(out, h->d_out, bytes) : hipMemcpy(out, h->d_out, bytes, hipMemcpyDeviceToHost));
   return CTAS_OK;
 }

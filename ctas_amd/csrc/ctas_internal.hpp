@@ -223,30 +223,6 @@ constexpr int kScoreChunk = 64;  // centres per scoring batch (bounds the scratc
 hipError_t launch_phantom(int N, int w, double c, int n_ell, const double *d_ell, double N0,
                           uint64_t seed, const float *d_gain, float *d_out, hipStream_t s);
 
-// Device scratch of a call that waits for its work before it returns. Small
-// buffers (up to kScratchBytes) go back to a pool of at most kScratchKept per
-// device, since allocating and freeing one costs more than most of the work
-// that needs it (about 0.3 ms for the ring filter's column means); any other
-// is freed. A buffer is in the hands of one call at a time. done(): the work
-// that used it has finished; without it the buffer is freed, which waits.
-class Scratch {
- public:
-  explicit Scratch(size_t bytes);
-  ~Scratch();
-  Scratch(const Scratch &) = delete;
-  Scratch &operator=(const Scratch &) = delete;
-  void *get() const { return p_; }  // null when the allocation failed
-  void done() { done_ = true; }
-
- private:
-  void *p_ = nullptr;
-  size_t bytes_;
-  int dev_ = 0;
-  bool done_ = false;
-};
-constexpr size_t kScratchBytes = size_t{1} << 20;
-constexpr int kScratchKept = 4;
-
 // Makes work queued next on `waiter` start after the work already queued on
 // `producer` (nullptr: the null stream, whose work is ordered with every
 // blocking stream, torch's default stream included).

@@ -1,0 +1,151 @@
+// Pools that outlive a call (pools.hpp).
+#include "pools.hpp"
+
+#include <algorithm>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <vector>
+
+namespace ctas {
+
+namespace {
+std::mutex g_scratch_pool_mu;
+std::map<int, std::vector<void *>> g_scratch_pool;  // by device, kScratchBytes each
+}  // namespace
+
+Scratch::Scratch(size_t bytes) : bytes_(std::max<size_t>(bytes, 1)) {
+  if (hipGetDevice(&dev_) != hipSuccess) return;
+  if (bytes_ <= kScratchBytes) {
+    bytes_ = kScratchBytes;
+    std::lock_guard<std::mutex> lk(g_scratch_pool_mu);
+    auto &pool = g_scratch_pool[dev_];
+    if (!pool.empty()) {
+      p_ = pool.back();
+      pool.pop_back();
+      return;
+    }
+  }
+  if (hipMalloc(&p_, bytes_) != hipSuccess) p_ = nullptr;
+}
+
+Scratch::~Scratch() {
+  if (!p_) return;
+  if (done_ && bytes_ == kScratchBytes) {
+    std::lock_guard<std::mutex> lk(g_scratch_pool_mu);
+    auto &pool = g_scratch_pool[dev_];
+    if (pool.size() < static_cast<size_t>(kScratchKept)) {
+      pool.push_back(p_);
+      return;
+    }
+  }
+  (void)hipFree(p_);
+}
+
+struct StagingSet {
+  int dev = 0;
+  unsigned char *block[kStagingBlocks] = {};
+  hipEvent_t free[kStagingBlocks] = {};  // the last copy that used the block
+  hipEvent_t mark = nullptr;
+  hipStream_t stream = nullptr;
+
+  ~StagingSet() {
+    if (stream) (void)hipStreamDestroy(stream);
+    if (mark) (void)hipEventDestroy(mark);
+    for (hipEvent_t e : free)
+      if (e) (void)hipEventDestroy(e);
+    if (block[0]) (void)hipHostFree(block[0]);
+  }
+  bool make() {
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&block[0]), kStagingBlock * kStagingBlocks) != hipSuccess)
+      return false;
+    for (int b = 0; b < kStagingBlocks; ++b) {
+      block[b] = block[0] + kStagingBlock * b;
+      if (hipEventCreateWithFlags(&free[b], hipEventDisableTiming) != hipSuccess) return false;
+    }
+    return hipEventCreateWithFlags(&mark, hipEventDisableTiming) == hipSuccess &&
+           hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) == hipSuccess;
+  }
+};
+
+namespace {
+std::mutex g_staging_mu;
+std::map<int, std::vector<std::unique_ptr<StagingSet>>> g_staging;  // the sets not in use
+std::map<int, int> g_staging_made;
+}  // namespace
+
+Staging::Staging(int dev) {
+  int current = -1;
+  if (hipGetDevice(&current) != hipSuccess || current != dev) return;
+  {
+    std::lock_guard<std::mutex> lk(g_staging_mu);
+    auto &idle = g_staging[dev];
+    if (!idle.empty()) {
+      set_ = std::move(idle.back());
+      idle.pop_back();
+      return;
+    }
+    if (g_staging_made[dev] >= kStagingSets) return;
+    ++g_staging_made[dev];
+  }
+  set_.reset(new StagingSet);
+  if (set_->make()) return;
+  set_.reset();
+  std::lock_guard<std::mutex> lk(g_staging_mu);
+  --g_staging_made[dev];
+}
+
+Staging::~Staging() {
+  if (!set_) return;
+  (void)hipStreamSynchronize(set_->stream);
+  for (hipEvent_t e : set_->free) (void)hipEventSynchronize(e);
+  std::lock_guard<std::mutex> lk(g_staging_mu);
+  g_staging[set_->dev].push_back(std::move(set_));
+}
+
+hipEvent_t Staging::mark() const { return set_->mark; }
+
+hipError_t Staging::upload(void *dst, const void *src, size_t bytes, hipStream_t s) {
+  if (bytes > kStagingMost) return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+  for (size_t off = 0; off < bytes; off += kStagingBlock, next_ = (next_ + 1) % kStagingBlocks) {
+    const size_t n = std::min(kStagingBlock, bytes - off);
+    const int b = next_;
+    if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
+    std::memcpy(set_->block[b], static_cast<const unsigned char *>(src) + off, n);
+    if (hipError_t e = staging_copy(static_cast<unsigned char *>(dst) + off, set_->block[b], n, s); e != hipSuccess)
+      return e;
+    if (hipError_t e = hipEventRecord(set_->free[b], s); e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+hipError_t Staging::download(void *dst, const void *src, size_t bytes) {
+  if (bytes > kStagingMost) {
+    if (hipError_t e = hipStreamSynchronize(set_->stream); e != hipSuccess) return e;
+    return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+  }
+  const size_t chunks = (bytes + kStagingBlock - 1) / kStagingBlock;
+  auto size = [&](size_t c) { return std::min(kStagingBlock, bytes - c * kStagingBlock); };
+  auto queue = [&](size_t c) -> hipError_t {
+    const int b = static_cast<int>(c % kStagingBlocks);
+    if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
+    if (hipError_t e = staging_copy(set_->block[b], static_cast<const unsigned char *>(src) + c * kStagingBlock,
+                                    size(c), set_->stream);
+        e != hipSuccess)
+      return e;
+    return hipEventRecord(set_->free[b], set_->stream);
+  };
+  for (size_t c = 0; c < std::min<size_t>(chunks, kStagingBlocks); ++c)
+    if (hipError_t e = queue(c); e != hipSuccess) return e;
+  for (size_t c = 0; c < chunks; ++c) {
+    const int b = static_cast<int>(c % kStagingBlocks);
+    if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
+    std::memcpy(static_cast<unsigned char *>(dst) + c * kStagingBlock, set_->block[b], size(c));
+    if (c + kStagingBlocks < chunks)
+      if (hipError_t e = queue(c + kStagingBlocks); e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+}  // namespace ctas

@@ -1,0 +1,106 @@
+// The pools of pools.cpp on a host-only stand-in for HIP; `pools_test <case>`
+// exits with 0 when the case holds.
+#include "pools.hpp"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <memory>
+#include <string>
+#include <vector>
+
+namespace {
+int g_device = 0;       // the current one
+int g_calls = 0;        // every HIP call
+bool g_refuse = false;  // allocations fail
+hipError_t g_last = hipSuccess;
+
+hipError_t call(hipError_t e = hipSuccess) {
+  ++g_calls;
+  if (e != hipSuccess) g_last = e;
+  return e;
+}
+hipError_t allocate(void **p, size_t bytes) {
+  if (g_refuse) return call(hipErrorOutOfMemory);
+  *p = std::aligned_alloc(256, (bytes + 255) / 256 * 256);
+  return call();
+}
+void check(bool ok, const char *what) {
+  if (ok) return;
+  std::printf("failed: %s\n", what);
+  std::exit(1);
+}
+}  // namespace
+
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
+hipError_t hipGetDevice(int *dev) {
+  *dev = g_device;
+  return call();
+}
+hipError_t hipMalloc(void **p, size_t bytes) { return allocate(p, bytes); }
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return allocate(p, bytes); }
+hipError_t hipFree(void *p) {
+  std::free(p);
+  return call();
+}
+hipError_t hipHostFree(void *p) { return hipFree(p); }
+hipError_t hipMemcpy(void *dst, const void *src, size_t bytes, hipMemcpyKind) {
+  std::memcpy(dst, src, bytes);
+  return call();
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return allocate(reinterpret_cast<void **>(e), 1); }
+hipError_t hipEventDestroy(hipEvent_t e) { return hipFree(e); }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return call(); }
+hipError_t hipEventSynchronize(hipEvent_t) { return call(); }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return allocate(reinterpret_cast<void **>(s), 1); }
+hipError_t hipStreamDestroy(hipStream_t s) { return hipFree(s); }
+hipError_t hipStreamSynchronize(hipStream_t) { return call(); }
+
+namespace ctas {
+hipError_t staging_copy(void *dst, const void *src, size_t bytes, hipStream_t) {
+  std::memcpy(dst, src, bytes);
+  call();
+  return hipGetLastError();  // as after a launch
+}
+}  // namespace ctas
+
+using namespace ctas;
+
+// Copies of every number of blocks arrive whole.
+void copies() {
+  for (size_t n : {size_t{1}, size_t{33}, kStagingBlock / 4, kStagingBlock / 4 + 1, kStagingBlock * 2 + 3,
+                   kStagingMost / 4, kStagingMost / 4 + 1}) {
+    std::vector<float> a(n), dev(n), b(n, -1.0f);
+    for (size_t i = 0; i < n; ++i) a[i] = static_cast<float>(i % 1000);
+    Staging st(0);
+    check(static_cast<bool>(st), "a set for the current device");
+    check(st.upload(dev.data(), a.data(), 4 * n, nullptr) == hipSuccess, "upload");
+    check(st.download(b.data(), dev.data(), 4 * n) == hipSuccess, "download");
+    check(a == b, "what comes back");
+  }
+}
+
+// A call whose device is not the current one gets no set, and one that has one
+// takes none from the others.
+void device() {
+  g_device = 1;
+  check(!Staging(0), "no set for device 0 while device 1 is current");
+  std::vector<std::unique_ptr<Staging>> held;
+  for (int k = 0; k < kStagingSets + 1; ++k) held.emplace_back(new Staging(1));
+  for (int k = 0; k < kStagingSets; ++k) check(static_cast<bool>(*held[k]), "a set for each call");
+  check(!*held[kStagingSets], "as many sets as the limit");
+  g_device = 0;
+  check(static_cast<bool>(Staging(0)), "the other device's sets are its own");
+}
+
+int main(int argc, char **argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "copies") copies();
+  else if (what == "device") device();
+  else return 2;
+  return 0;
+}
