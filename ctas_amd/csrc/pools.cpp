@@ -71,8 +71,13 @@ struct StagingSet {
 
 namespace {
 std::mutex g_staging_mu;
-std::map<int, std::vector<std::unique_ptr<StagingSet>>> g_staging;  // the sets not in use
-std::map<int, int> g_staging_made;
+struct DeviceSets {
+  StagingSet *idle[kStagingSets];  // the sets not in use
+  int n_idle = 0, made = 0;
+};
+// Raw pointers: the sets end with the process, since the runtime may be gone
+// before this file's static objects are.
+std::map<int, DeviceSets> g_staging;
 }  // namespace
 
 Staging::Staging(int dev) {
@@ -80,20 +85,19 @@ Staging::Staging(int dev) {
   if (hipGetDevice(&current) != hipSuccess || current != dev) return;
   {
     std::lock_guard<std::mutex> lk(g_staging_mu);
-    auto &idle = g_staging[dev];
-    if (!idle.empty()) {
-      set_ = std::move(idle.back());
-      idle.pop_back();
+    DeviceSets &d = g_staging[dev];
+    if (d.n_idle > 0) {
+      set_.reset(d.idle[--d.n_idle]);
       return;
     }
-    if (g_staging_made[dev] >= kStagingSets) return;
-    ++g_staging_made[dev];
+    if (d.made >= kStagingSets) return;
+    ++d.made;
   }
   set_.reset(new StagingSet);
   if (set_->make()) return;
   set_.reset();
   std::lock_guard<std::mutex> lk(g_staging_mu);
-  --g_staging_made[dev];
+  --g_staging[dev].made;
 }
 
 Staging::~Staging() {
@@ -101,7 +105,8 @@ Staging::~Staging() {
   (void)hipStreamSynchronize(set_->stream);
   for (hipEvent_t e : set_->free) (void)hipEventSynchronize(e);
   std::lock_guard<std::mutex> lk(g_staging_mu);
-  g_staging[set_->dev].push_back(std::move(set_));
+  DeviceSets &d = g_staging[set_->dev];
+  d.idle[d.n_idle++] = set_.release();  // no more than were made
 }
 
 hipEvent_t Staging::mark() const { return set_->mark; }

@@ -97,10 +97,28 @@ void device() {
   check(static_cast<bool>(Staging(0)), "the other device's sets are its own");
 }
 
+// The calls made when main ended; what runs after the static objects'
+// destructors holds the count against it.
+int g_at_end = -1;
+__attribute__((destructor)) void after_main() {
+  if (g_at_end < 0 || g_calls == g_at_end) return;
+  std::printf("failed: %d HIP calls after the end of main\n", g_calls - g_at_end);
+  std::fflush(stdout);
+  std::_Exit(1);
+}
+
+// The pools' destructors leave the runtime alone.
+void end() {
+  copies();
+  { Scratch a(100); a.done(); }
+  g_at_end = g_calls;
+}
+
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "copies") copies();
   else if (what == "device") device();
+  else if (what == "end") end();
   else return 2;
   return 0;
 }
