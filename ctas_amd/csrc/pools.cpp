@@ -10,6 +10,15 @@
 namespace ctas {
 
 namespace {
+// Whether an allocation succeeded. The error of one that failed would be
+// reported by the next launch that asks hipGetLastError, and what follows does
+// without the memory.
+bool allocated(hipError_t e) {
+  if (e == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 std::mutex g_scratch_pool_mu;
 std::map<int, std::vector<void *>> g_scratch_pool;  // by device, kScratchBytes each
 }  // namespace
@@ -26,7 +35,7 @@ Scratch::Scratch(size_t bytes) : bytes_(std::max<size_t>(bytes, 1)) {
       return;
     }
   }
-  if (hipMalloc(&p_, bytes_) != hipSuccess) p_ = nullptr;
+  if (!allocated(hipMalloc(&p_, bytes_))) p_ = nullptr;
 }
 
 Scratch::~Scratch() {
@@ -58,14 +67,14 @@ struct StagingSet {
   }
   bool make() {
     if (hipGetDevice(&dev) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void **>(&block[0]), kStagingBlock * kStagingBlocks) != hipSuccess)
+        !allocated(hipHostMalloc(reinterpret_cast<void **>(&block[0]), kStagingBlock * kStagingBlocks)))
       return false;
     for (int b = 0; b < kStagingBlocks; ++b) {
       block[b] = block[0] + kStagingBlock * b;
-      if (hipEventCreateWithFlags(&free[b], hipEventDisableTiming) != hipSuccess) return false;
+      if (!allocated(hipEventCreateWithFlags(&free[b], hipEventDisableTiming))) return false;
     }
-    return hipEventCreateWithFlags(&mark, hipEventDisableTiming) == hipSuccess &&
-           hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) == hipSuccess;
+    return allocated(hipEventCreateWithFlags(&mark, hipEventDisableTiming)) &&
+           allocated(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   }
 };
 

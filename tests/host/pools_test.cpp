@@ -97,6 +97,20 @@ void device() {
   check(static_cast<bool>(Staging(0)), "the other device's sets are its own");
 }
 
+// Without memory a call goes on without a set or scratch, and the failed
+// allocation is not what its next launch reports. Afterwards all is as before.
+void refused() {
+  float a = 1.0f, b = 0.0f;
+  g_refuse = true;
+  check(!Staging(0), "no set");
+  check(staging_copy(&b, &a, sizeof a, nullptr) == hipSuccess, "the launch after a refused set");
+  check(Scratch(100).get() == nullptr && Scratch(2 * kScratchBytes).get() == nullptr, "no scratch");
+  check(staging_copy(&b, &a, sizeof a, nullptr) == hipSuccess, "the launch after refused scratch");
+  g_refuse = false;
+  device();
+  copies();
+}
+
 // The calls made when main ended; what runs after the static objects'
 // destructors holds the count against it.
 int g_at_end = -1;
@@ -118,6 +132,7 @@ int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "copies") copies();
   else if (what == "device") device();
+  else if (what == "refused") refused();
   else if (what == "end") end();
   else return 2;
   return 0;
