@@ -36,11 +36,13 @@
 #include <cstring>
 #include <fstream>
 #include <memory>
+#include <optional>
 #include <random>
 #include <string>
 #include <vector>
 
 #include "ctas_internal.hpp"
+#include "pools.hpp"
 
 namespace ctas {
 namespace cnn {
@@ -1426,20 +1428,25 @@ static int copy_params(ctas_cnn *n, float *host, const float *dev, bool to_host)
   for (const auto &p : n->prm) count += p.n;
   // one after the other on the device first: most of the twelve are small, and
   // each copy has its own latency (gradients of 64 samples and their values on
-  // the host: 842 us with twelve copies, 702 with one)
-  // (from the network's own device; copies take any)
+  // the host: 842 us with twelve copies, 702 with one). On the network's own
+  // device (copies take any) and into scratch of this call: the network's
+  // workspace may be in use by another thread's prediction, and reading the
+  // parameters does not change the network.
   int dev_now = -1;
-  if (to_host && hipGetDevice(&dev_now) == hipSuccess && dev_now == n->device && ensure_ws(n, count) == CTAS_OK) {
+  std::optional<Scratch> packed;
+  if (to_host && hipGetDevice(&dev_now) == hipSuccess && dev_now == n->device) packed.emplace(count * 4);
+  if (packed && packed->get()) {
     ctas::cnn::Packing pk;
     for (size_t i = 0, at = 0; i < n->prm.size(); at += n->prm[i++].n) {
       pk.off[i] = static_cast<int>(n->prm[i].off);
       pk.at[i] = static_cast<int>(at);
     }
-    hipLaunchKernelGGL(pack_params, dim3((count + 255) / 256), dim3(256), 0, n->stream, dev, n->ws, pk,
-                       static_cast<int>(count));
+    hipLaunchKernelGGL(pack_params, dim3((count + 255) / 256), dim3(256), 0, n->stream, dev,
+                       static_cast<float *>(packed->get()), pk, static_cast<int>(count));
     CTAS_HIP_TRY(hipGetLastError());
     CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
-    CTAS_HIP_TRY(hipMemcpy(host, n->ws, count * 4, hipMemcpyDeviceToHost));
+    CTAS_HIP_TRY(hipMemcpy(host, packed->get(), count * 4, hipMemcpyDeviceToHost));
+    packed->done();
     return CTAS_OK;
   }
   CTAS_HIP_TRY(hipStreamSynchronize(n->stream));
