@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "ctas_internal.hpp"
+#include "score_layout.hpp"
 
 namespace ctas {
 namespace {
@@ -86,21 +87,12 @@ __device__ __forceinline__ float4 smooth4(const float *src, int st, const Taps &
 // follow there, four outputs per thread in the smoothing so that each LDS read
 // serves up to four taps. Bound by LDS reads: nine slices of 2048 px, 8
 // taps, 165 us (628 in three passes over memory).
-constexpr int kScoreTH = 32, kScoreTW = 64;      // derivatives of a tile
-constexpr int kScoreSH = kScoreTH + 4, kScoreSW = kScoreTW + 4;  // smoothed rows and columns: 34 and 66, rounded up to fours
-
-__host__ __device__ inline int score_reach(int nt) { return nt > 0 ? nt - 1 : 0; }
-inline size_t score_lds(int nt) {
-  const int e = score_reach(nt), rows = kScoreSH + e;
-  return sizeof(float) * (static_cast<size_t>(rows) * (kScoreSW + e) + static_cast<size_t>(rows) * kScoreSW);
-}
-
 __global__ __launch_bounds__(256) void score_kernel(const float *__restrict__ slices, const float *__restrict__ centres,
                                                     int w, int tiles_x, Taps taps, double *__restrict__ partial) {
-  extern __shared__ float score_buf[];
-  const int e = score_reach(taps.nt), rows = kScoreSH + e, cols = kScoreSW + e;
-  float *src = score_buf;            // [rows][cols], then the smoothed tile [kScoreSH][kScoreSW]
-  float *mid = src + rows * cols;    // [rows][kScoreSW]: smoothed along rows
+  extern __shared__ __align__(16) float score_buf[];
+  const ScoreLayout lay = score_layout(taps.nt);
+  const int e = lay.reach, rows = lay.rows, cols = lay.cols;
+  float *src = score_buf, *mid = score_buf + lay.mid;
   const int tid = threadIdx.x, k = blockIdx.y, nb = gridDim.x;
   const float c = centres[k];
   const int r = static_cast<int>(ceilf(fabsf(c)));
@@ -228,7 +220,7 @@ hipError_t launch_ag_scores(const float *d_slices, int n, int w, const float *d_
   Taps taps{};
   if (sigma > 1.0f) taps = make_taps(sigma);
   const int nb = score_tiles(w);
-  hipLaunchKernelGGL(score_kernel, dim3(nb, n), dim3(256), score_lds(taps.nt), s, d_slices, d_centres, w,
+  hipLaunchKernelGGL(score_kernel, dim3(nb, n), dim3(256), sizeof(float) * score_layout(taps.nt).floats, s, d_slices, d_centres, w,
                      (w + kScoreTW - 1) / kScoreTW, taps, d_partial);
   if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   hipLaunchKernelGGL(score_finish_kernel, dim3(n), dim3(256), 0, s, d_partial, d_scores, nb);
