@@ -332,7 +332,8 @@ hipStream_t pick_stream(const ctas_fbp *h, void *stream) {
 
 namespace {
 
-// bytes / 4 words between a pinned block and device memory, both aligned to 16.
+// bytes / 4 words between a pinned block and device memory, both aligned to 16
+// (staging_copy refuses others).
 __global__ __launch_bounds__(256) void staging_copy_kernel(uint32_t *__restrict__ dst, const uint32_t *__restrict__ src,
                                                            int words) {
   const int quads = words >> 2, stride = gridDim.x * 256;
@@ -344,6 +345,7 @@ __global__ __launch_bounds__(256) void staging_copy_kernel(uint32_t *__restrict_
 }  // namespace
 
 hipError_t staging_copy(void *dst, const void *src, size_t bytes, hipStream_t s) {
+  if (((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) != 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(staging_copy_kernel, dim3(128), dim3(256), 0, s, static_cast<uint32_t *>(dst),
                      static_cast<const uint32_t *>(src), static_cast<int>(bytes / 4));
   return hipGetLastError();
@@ -892,12 +894,14 @@ static int host_run(ctas_fbp *h, float *sino, float *out, const float *centers, 
   const size_t slice_elems = static_cast<size_t>(h->N) * h->w;
   const size_t in_bytes = sizeof(float) * slice_elems * S, out_bytes = sizeof(float) * h->w * h->w * S;
   const bool f32_copy = store_of(h->flags) != ST_F32;
-  if (int rc = grow(h->d_io, h->io_cap, in_bytes * (f32_copy ? 2 : 1))) return rc;
+  // the filtered rows' float32 copy begins on a 16-byte boundary (staging_copy)
+  const size_t f32_at = (slice_elems * S + 3) & ~size_t{3};
+  if (int rc = grow(h->d_io, h->io_cap, f32_copy ? sizeof(float) * f32_at + in_bytes : in_bytes)) return rc;
   if (do_bp)
     if (int rc = grow(h->d_out, h->out_cap, out_bytes)) return rc;
   hipStream_t s = h->stream;
   CTAS_HIP_TRY(hipStreamSynchronize(s));
-  float *d_f32 = f32_copy ? h->d_io + slice_elems * S : nullptr;
+  float *d_f32 = f32_copy ? h->d_io + f32_at : nullptr;
   Staging staging(h->device);
   // Every return below leaves no work of this call on the stream.
   struct Drain {
