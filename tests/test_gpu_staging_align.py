@@ -16,5 +16,5 @@ def test_filtered_rows_of_odd_counts(torch_cuda, S, N, w, store):
     P = np.random.default_rng(N + w).uniform(0.2, 1.0, (S, N, w)).astype(np.float32)
     filt, out = ca.CTrec(w, N, ca.ABS, "HANN", store=store).reconstruct(P, [0.25] * S)
     for s in range(S):
-        one_filt, one_out = ca.CTrec(w, N, ca.ABS, "HANN", store=store).reconstruct(P[s], 0.25)
+        one_filt, one_out = ca.CTrec(w, N, ca.ABS, "HANN", store=store).reconstruct(P[s:s + 1], [0.25])
         assert np.array_equal(filt[s], one_filt[0]) and np.array_equal(out[s], one_out[0])
