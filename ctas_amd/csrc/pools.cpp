@@ -112,7 +112,7 @@ Staging::Staging(int dev) {
 Staging::~Staging() {
   if (!set_) return;
   (void)hipStreamSynchronize(set_->stream);
-  for (hipEvent_t e : set_->free) (void)hipEventSynchronize(e);
+  for (int b = 0; b < kStagingBlocks; ++b) (void)wait(b);
   std::lock_guard<std::mutex> lk(g_staging_mu);
   DeviceSets &d = g_staging[set_->dev];
   d.idle[d.n_idle++] = set_.release();  // no more than were made
@@ -120,16 +120,30 @@ Staging::~Staging() {
 
 hipEvent_t Staging::mark() const { return set_->mark; }
 
+// A set outlives the streams of the handles that it served, and the runtime
+// looks at the stream that an event was last recorded on. So a call waits for
+// its own records only, while its stream is there; the set comes to it idle.
+hipError_t Staging::wait(int b) {
+  if (!busy_[b]) return hipSuccess;
+  busy_[b] = false;
+  return hipEventSynchronize(set_->free[b]);
+}
+
+hipError_t Staging::copy(int b, void *dst, const void *src, size_t bytes, hipStream_t s) {
+  if (hipError_t e = staging_copy(dst, src, bytes, s); e != hipSuccess) return e;
+  const hipError_t e = hipEventRecord(set_->free[b], s);
+  busy_[b] = e == hipSuccess;
+  return e;
+}
+
 hipError_t Staging::upload(void *dst, const void *src, size_t bytes, hipStream_t s) {
   if (bytes > kStagingMost) return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
   for (size_t off = 0; off < bytes; off += kStagingBlock, next_ = (next_ + 1) % kStagingBlocks) {
     const size_t n = std::min(kStagingBlock, bytes - off);
     const int b = next_;
-    if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
+    if (hipError_t e = wait(b); e != hipSuccess) return e;
     std::memcpy(set_->block[b], static_cast<const unsigned char *>(src) + off, n);
-    if (hipError_t e = staging_copy(static_cast<unsigned char *>(dst) + off, set_->block[b], n, s); e != hipSuccess)
-      return e;
-    if (hipError_t e = hipEventRecord(set_->free[b], s); e != hipSuccess) return e;
+    if (hipError_t e = copy(b, static_cast<unsigned char *>(dst) + off, set_->block[b], n, s); e != hipSuccess) return e;
   }
   return hipSuccess;
 }
@@ -143,18 +157,14 @@ hipError_t Staging::download(void *dst, const void *src, size_t bytes) {
   auto size = [&](size_t c) { return std::min(kStagingBlock, bytes - c * kStagingBlock); };
   auto queue = [&](size_t c) -> hipError_t {
     const int b = static_cast<int>(c % kStagingBlocks);
-    if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
-    if (hipError_t e = staging_copy(set_->block[b], static_cast<const unsigned char *>(src) + c * kStagingBlock,
-                                    size(c), set_->stream);
-        e != hipSuccess)
-      return e;
-    return hipEventRecord(set_->free[b], set_->stream);
+    if (hipError_t e = wait(b); e != hipSuccess) return e;
+    return copy(b, set_->block[b], static_cast<const unsigned char *>(src) + c * kStagingBlock, size(c), set_->stream);
   };
   for (size_t c = 0; c < std::min<size_t>(chunks, kStagingBlocks); ++c)
     if (hipError_t e = queue(c); e != hipSuccess) return e;
   for (size_t c = 0; c < chunks; ++c) {
     const int b = static_cast<int>(c % kStagingBlocks);
-    if (hipError_t e = hipEventSynchronize(set_->free[b]); e != hipSuccess) return e;
+    if (hipError_t e = wait(b); e != hipSuccess) return e;
     std::memcpy(static_cast<unsigned char *>(dst) + c * kStagingBlock, set_->block[b], size(c));
     if (c + kStagingBlocks < chunks)
       if (hipError_t e = queue(c + kStagingBlocks); e != hipSuccess) return e;

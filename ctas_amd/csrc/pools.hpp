@@ -72,7 +72,11 @@ class Staging {
   hipError_t download(void *dst, const void *src, size_t bytes);
 
  private:
+  hipError_t wait(int b);  // until block b's last copy of this call is done
+  hipError_t copy(int b, void *dst, const void *src, size_t bytes, hipStream_t s);  // with block b
+
   std::unique_ptr<StagingSet> set_;
+  bool busy_[kStagingBlocks] = {};  // block b's event was recorded in this call and not waited for
   int next_ = 0;
 };
 

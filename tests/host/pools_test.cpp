@@ -5,7 +5,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <memory>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -13,6 +15,8 @@ namespace {
 int g_device = 0;       // the current one
 int g_calls = 0;        // every HIP call
 bool g_refuse = false;  // allocations fail
+std::set<hipStream_t> g_streams;                  // those that exist
+std::map<hipEvent_t, hipStream_t> g_recorded;     // the stream of an event's last record
 hipError_t g_last = hipSuccess;
 
 hipError_t call(hipError_t e = hipSuccess) {
@@ -54,10 +58,25 @@ hipError_t hipMemcpy(void *dst, const void *src, size_t bytes, hipMemcpyKind) {
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return allocate(reinterpret_cast<void **>(e), 1); }
 hipError_t hipEventDestroy(hipEvent_t e) { return hipFree(e); }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return call(); }
-hipError_t hipEventSynchronize(hipEvent_t) { return call(); }
-hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return allocate(reinterpret_cast<void **>(s), 1); }
-hipError_t hipStreamDestroy(hipStream_t s) { return hipFree(s); }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  g_recorded[e] = s;
+  return call();
+}
+// An event may be waited for while the stream that it was recorded on is there.
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  const auto at = g_recorded.find(e);
+  if (at != g_recorded.end() && at->second && !g_streams.count(at->second)) return call(hipErrorInvalidValue);
+  return call();
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+  const hipError_t e = allocate(reinterpret_cast<void **>(s), 1);
+  if (e == hipSuccess) g_streams.insert(*s);
+  return e;
+}
+hipError_t hipStreamDestroy(hipStream_t s) {
+  g_streams.erase(s);
+  return hipFree(s);
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return call(); }
 
 namespace ctas {
@@ -97,6 +116,23 @@ void device() {
   check(static_cast<bool>(Staging(0)), "the other device's sets are its own");
 }
 
+// A set goes from a handle to the next after the first one's stream is gone.
+void streams() {
+  std::vector<float> a(kStagingMost / 4), dev(a.size()), b(a.size());
+  for (int handle = 0; handle < 3; ++handle) {
+    for (size_t i = 0; i < a.size(); ++i) a[i] = static_cast<float>((i + handle) % 1000);
+    hipStream_t s = nullptr;
+    check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess, "a stream");
+    {
+      Staging st(0);
+      check(st.upload(dev.data(), a.data(), 4 * a.size(), s) == hipSuccess, "upload");
+      check(st.download(b.data(), dev.data(), handle ? 4 : 4 * a.size()) == hipSuccess, "download");
+    }
+    check(hipGetLastError() == hipSuccess, "no wait for a record on a stream that is gone");
+    (void)hipStreamDestroy(s);
+  }
+}
+
 // Without memory a call goes on without a set or scratch, and the failed
 // allocation is not what its next launch reports. Afterwards all is as before.
 void refused() {
@@ -132,6 +168,7 @@ int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "copies") copies();
   else if (what == "device") device();
+  else if (what == "streams") streams();
   else if (what == "refused") refused();
   else if (what == "end") end();
   else return 2;

@@ -17,7 +17,7 @@ def pools_test(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["copies", "device", "refused", "end"])
+@pytest.mark.parametrize("case", ["copies", "device", "streams", "refused", "end"])
 def test_pools(pools_test, case):
     r = subprocess.run([str(pools_test), case], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
