@@ -32,6 +32,8 @@ sys.path.insert(0, str(ROOT))
 HBM_PEAK_GBS = 8000.0
 PEAKS_LIB = ROOT / "ctas_amd" / "libctas_peaks.so"
 COPY_BYTES = 1 << 30  # counter calibration: a plain 1 GiB copy
+# bp_group_kernel<4>, which batches of one centre take: 64x64 tiles
+GROUP_TILES = {"tile_kind": 1, "slices_per_workgroup": 4, "angles_per_pass": 16}
 
 
 def host_cpu_info() -> dict:
@@ -524,7 +526,6 @@ def main() -> int:
 
     print("[bench] fp32 CTAS", file=sys.stderr, flush=True)
     rec, ms, bp_ms, prep_ms = run_variant(ca.STORE_FP32, ca.INTERP_CTAS, args.steps, args.warmup)
-    kind, ac = rec.tiles()
     value = updates / (ms / 1e3) / 1e9
     lds_bytes = updates * 4.0  # one 4-byte sample per voxel-update (CTAS mode, FP32)
     achieved = lds_bytes / (bp_ms / 1e3) / 1e9
@@ -548,8 +549,8 @@ def main() -> int:
         "data": "synthetic (seeded ellipse phantoms, Poisson 1e5)",
         "config": {"workload": f"batched FBP {S} slices x {w} px x {N} angles, HANN, ABS, c=+{c}, "
                                "CTAS floor sampling, one hipGraph",
-                   "slices": S, "width": w, "angles": N, "filter": "HANN", "tile_kind": kind,
-                   "angles_per_pass": ac, "in_mask_fraction": round(frac_in, 4)},
+                   "slices": S, "width": w, "angles": N, "filter": "HANN", **GROUP_TILES,
+                   "in_mask_fraction": round(frac_in, 4)},
         "roofline": {"bound": "lds", "achieved": round(achieved, 1), "peak": lds_peak,
                      "unit": "GB/s", "frac": round(achieved / lds_peak, 4),
                      "traffic": (round(pmc["traffic"]) if pmc and "traffic" in pmc else None),

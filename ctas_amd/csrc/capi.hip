@@ -230,79 +230,12 @@ Item base_item(const ctas_fbp *h, int kind, bool mirror) {
   return it;
 }
 
-// One backprojection launch: `items` items from `first`, `group` slices per
-// workgroup, on tiles of `kind`.
-struct BpLaunch {
-  int first, items, group, kind;
-};
-
-// The launches that backproject S slices, and the order in which the item
-// table holds them (slices of a group lie back to back).
-//
-// Slices of one centre share their ray coordinates, so CTAS sampling of
-// float32 storage, and of 16-bit storage through mirrored angle pairs, takes
-// four or two of them per workgroup on 64x64 tiles, where that leaves enough
-// workgroups. Measured for 1 to 8 slices of 512 to 4096 px on 256 CUs, four
-// win from 448 workgroups (float32; 484 of 1400 px 445 us against 570 with
-// two and 768 alone, 288 of 768 px 274 against 258 and 353) and 484 (16-bit;
-// 544 of 2048 px 1111 us against 1387 and 1430, 288 of 1024 px 559 against
-// 513 and 454), two from 288 (float32; 183 us against 234, 256 workgroups 272
-// against 264) and 726 (16-bit; 571 us against 717, 576 workgroups 513
-// against 454). What remains is taken one by one; float32 launches of less
-// than two 64x64 tiles per CU take 32x32 tiles, and 16x32 ones up to a
-// quarter of a tile per CU (backproject.hip). Mirrored launches of few tile
-// pairs take quarters of them: LINEAR below four per CU, where whole ones do not
-// fill the chip once (144 of 1024 px 165 us against 389, 484 of 1400 px 485
-// against 532, 1008 of 1024 px 750 against 773, 1088 of 2048 px 1541 against
-// 1520), 16-bit below three (144 113 against 215, 726 of 1400 px 394 against 410). A
-// tile kind that the caller set is kept, for every slice.
 std::vector<BpLaunch> plan_backprojection(const ctas_fbp *h, const float *centers, int S, std::vector<int> *order) {
-  order->resize(S);
-  std::iota(order->begin(), order->end(), 0);
   const int kind = choose_kind(h);
-  const bool linear = mode_of(h->flags) == MODE_LINEAR, f32 = store_of(h->flags) == ST_F32 && !linear;
-  const bool mirror = use_mirror(h, kind);
-  if (h->tile_kind != TK_AUTO || (!f32 && !mirror) || static_cast<long long>(h->N) * h->w >= (1LL << 30))
-    return {{0, S, 1, kind}};
-  const long long rows = (h->w + 63) / 64, cols = mirror ? (h->w / 2 + 64) / 64 : rows;
-  const long long tiles = rows * cols, cus = h->cus;
-  const long long four = (mirror ? 15 : 14) * cus / 8, two = (mirror ? 20 : 9) * cus / 8;
-  const long long small = (linear ? 4 : 3) * cus;
-  auto single = [&](int first, int n) {
-    BpLaunch l{first, n, 1, kind};
-    if (f32 && 4 * n * tiles <= cus) l.kind = TK_16x32;
-    else if (f32 && n * tiles < 2 * cus) l.kind = TK_32x32;
-    else if (mirror && kind == TK_64x64 && n * tiles < small) l.kind = TK_32x32;
-    return l;
-  };
-  if (linear) return {single(0, S)};
-  if (f32 && S * tiles < 2 * cus) return {single(0, S)};
-  std::map<uint32_t, std::vector<int>> by_centre;
-  for (int i = 0; i < S; ++i) {
-    uint32_t bits;
-    std::memcpy(&bits, centers + i, sizeof bits);
-    by_centre[bits].push_back(i);
-  }
-  std::vector<BpLaunch> launches;
-  std::vector<int> at;
-  for (const int group : {4, 2}) {
-    long long n = 0;
-    for (const auto &c : by_centre) n += static_cast<long long>(c.second.size()) / group;
-    if (n * tiles < (group == 4 ? four : two)) continue;
-    const int first = static_cast<int>(at.size());
-    for (auto &c : by_centre) {
-      const size_t take = c.second.size() / group * group;
-      at.insert(at.end(), c.second.begin(), c.second.begin() + take);
-      c.second.erase(c.second.begin(), c.second.begin() + take);
-    }
-    launches.push_back({first, static_cast<int>(at.size()) - first, group, TK_64x64});
-  }
-  if (launches.empty()) return {single(0, S)};
-  const int first = static_cast<int>(at.size());
-  for (const auto &c : by_centre) at.insert(at.end(), c.second.begin(), c.second.end());
-  if (first < S) launches.push_back(single(first, S - first));
-  *order = at;
-  return launches;
+  const bool linear = mode_of(h->flags) == MODE_LINEAR;
+  const PlanShape shape{h->w, h->N, h->cus, kind, h->tile_kind, h->angles_per_pass,
+                        store_of(h->flags) == ST_F32 && !linear, linear, use_mirror(h, kind)};
+  return plan_launches(shape, centers, S, order);
 }
 
 // items: the host's copy of d_items
@@ -522,7 +455,7 @@ struct TuneKey {
   }
 };
 std::mutex g_tune_mu;
-std::map<TuneKey, std::pair<int, int>> g_tune;
+std::map<TuneKey, Tuned> g_tune;
 
 int width_class(int w) {
   int c = 1;
@@ -533,24 +466,21 @@ TuneKey tune_key(const ctas_fbp *h) {
   return TuneKey{width_class(h->w), width_class(h->N), mode_of(h->flags), store_of(h->flags), h->device};
 }
 
-int choose_kind(const ctas_fbp *h) {
-  if (h->tile_kind != TK_AUTO) return h->tile_kind;
-  {
+// The kind and pass length of launches of one slice per workgroup.
+std::pair<int, int> choose_tiles(const ctas_fbp *h) {
+  Tuned t;
+  if (h->tuning_ac) {
+    t.ac64 = h->tuning_ac;
+  } else {
     std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tune.find(tune_key(h));
-    if (it != g_tune.end()) return it->second.first;
+    const auto it = g_tune.find(tune_key(h));
+    if (it != g_tune.end()) t = it->second;
   }
-  return TK_64x64;  // the tuned choice at 512-4096 px on MI355X
+  return {h->tile_kind != TK_AUTO ? h->tile_kind : t.handle_kind(),
+          h->angles_per_pass ? h->angles_per_pass : t.handle_ac()};
 }
-int choose_ac(const ctas_fbp *h) {
-  if (h->angles_per_pass) return h->angles_per_pass;
-  {
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tune.find(tune_key(h));
-    if (it != g_tune.end()) return it->second.second;
-  }
-  return 32;
-}
+int choose_kind(const ctas_fbp *h) { return choose_tiles(h).first; }
+int choose_ac(const ctas_fbp *h) { return choose_tiles(h).second; }
 
 // ---- shared resources of uneven batches -------------------------------------
 struct GeomRes {
@@ -1045,7 +975,10 @@ int ctas_fbp_graph_launch(ctas_fbp *h, void *stream) {
   return CTAS_OK;
 }
 
-int ctas_fbp_autotune(ctas_fbp *h, int S) {
+// Times S slices on each tile kind and pass length, one slice per workgroup,
+// and with `plan` on the launches that the handle takes by itself, and keeps the
+// fastest for the handle's class.
+static int tune(ctas_fbp *h, int S, bool plan) {
   if (!h || S <= 0) return fail(CTAS_E_ARG, "bad arguments");
   const int keep_kind = h->tile_kind, keep_ac = h->angles_per_pass;
   const size_t slice_elems = static_cast<size_t>(h->N) * h->w;
@@ -1058,8 +991,7 @@ int ctas_fbp_autotune(ctas_fbp *h, int S) {
   // Every path below ends at the clean-up: buffers and events freed, the
   // handle's own tile settings restored.
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  float best = 1e30f;
-  int bk = TK_128x128, bac = 32;
+  Tuned best;
   auto hip = [](hipError_t e, const char *what) {
     return e == hipSuccess ? CTAS_OK : fail(CTAS_E_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
   };
@@ -1072,31 +1004,47 @@ int ctas_fbp_autotune(ctas_fbp *h, int S) {
     if (int rc = hip(hipEventCreate(&e0), "hipEventCreate")) return rc;
     if (int rc = hip(hipEventCreate(&e1), "hipEventCreate")) return rc;
     std::vector<float> centers(S, 0.0f);
+    // the fastest of five runs, after one: one slow run (a clock or cache
+    // state) must not decide between candidates a few percent apart
+    auto time = [&](float *ms) -> int {
+      if (int rc = enqueue_slices(h, d_in, d_o, nullptr, centers.data(), S, true, h->stream)) return rc;
+      *ms = 1e30f;
+      for (int r = 0; r < 5; ++r) {
+        if (int rc = hip(hipEventRecord(e0, h->stream), "hipEventRecord")) return rc;
+        if (int rc = enqueue_slices(h, d_in, d_o, nullptr, centers.data(), S, true, h->stream)) return rc;
+        if (int rc = hip(hipEventRecord(e1, h->stream), "hipEventRecord")) return rc;
+        if (int rc = hip(hipEventSynchronize(e1), "hipEventSynchronize")) return rc;
+        float one = 0.f;
+        if (int rc = hip(hipEventElapsedTime(&one, e0, e1), "hipEventElapsedTime")) return rc;
+        *ms = std::min(*ms, one);
+      }
+      return CTAS_OK;
+    };
     const int kinds[] = {TK_64x64, TK_128x64, TK_128x128};
     const int acs[] = {16, 32};
+    float least = 1e30f, least64 = 1e30f, ms = 0.f;
     for (int k : kinds) {
       for (int ac : acs) {
         h->tile_kind = k;
         h->angles_per_pass = ac;
-        if (int rc = enqueue_slices(h, d_in, d_o, nullptr, centers.data(), S, true, h->stream)) return rc;
-        // the fastest of five runs: one slow run (a clock or cache state)
-        // must not decide between candidates a few percent apart
-        float ms = 1e30f;
-        for (int r = 0; r < 5; ++r) {
-          if (int rc = hip(hipEventRecord(e0, h->stream), "hipEventRecord")) return rc;
-          if (int rc = enqueue_slices(h, d_in, d_o, nullptr, centers.data(), S, true, h->stream)) return rc;
-          if (int rc = hip(hipEventRecord(e1, h->stream), "hipEventRecord")) return rc;
-          if (int rc = hip(hipEventSynchronize(e1), "hipEventSynchronize")) return rc;
-          float one = 0.f;
-          if (int rc = hip(hipEventElapsedTime(&one, e0, e1), "hipEventElapsedTime")) return rc;
-          ms = std::min(ms, one);
+        if (int rc = time(&ms)) return rc;
+        if (ms < least) {
+          least = ms;
+          best.kind = k;
+          best.ac = ac;
         }
-        if (ms < best) {
-          best = ms;
-          bk = k;
-          bac = ac;
+        if (k == TK_64x64 && ms < least64) {
+          least64 = ms;
+          best.ac64 = ac;
         }
       }
+    }
+    if (plan) {
+      h->tile_kind = TK_AUTO;
+      h->angles_per_pass = 0;
+      h->tuning_ac = best.ac64;
+      if (int rc = time(&ms)) return rc;
+      best.beats_plan = least < ms;
     }
     return CTAS_OK;
   };
@@ -1108,11 +1056,14 @@ int ctas_fbp_autotune(ctas_fbp *h, int S) {
   (void)hipFree(d_o);
   h->tile_kind = keep_kind;
   h->angles_per_pass = keep_ac;
+  h->tuning_ac = 0;
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  g_tune[tune_key(h)] = {bk, bac};
+  g_tune[tune_key(h)] = best;
   return CTAS_OK;
 }
+
+int ctas_fbp_autotune(ctas_fbp *h, int S) { return tune(h, S, true); }
 
 int ctas_fbp_batch_uneven(const ctas_batch_item *items, int n, int contrast, int filter, float filter_param,
                           float anarc, int flags, void *stream) {
@@ -1146,12 +1097,12 @@ int ctas_fbp_batch_uneven(const ctas_batch_item *items, int n, int contrast, int
     if (!tuned) {
       ctas_fbp *t = nullptr;
       int rc = ctas_fbp_create(&t, items[i].w, items[i].n_angles, contrast, filter, filter_param, anarc, flags);
-      if (rc == CTAS_OK) rc = ctas_fbp_autotune(t, 2);
+      if (rc == CTAS_OK) rc = tune(t, 2, false);
       ctas_fbp_destroy(t);
       if (rc) return rc;
     }
     std::lock_guard<std::mutex> lk(g_tune_mu);
-    pick[cls] = g_tune[key];
+    pick[cls] = {g_tune[key].kind, g_tune[key].ac};
   }
   struct Entry {
     int src, kind, ac;

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/ctas_hip.h"
+#include "bp_plan.hpp"
 
 namespace ctas {
 
@@ -160,13 +161,6 @@ inline int store_of(int flags) {
 inline int mode_of(int flags) { return (flags & CTAS_INTERP_MASK) == CTAS_INTERP_LINEAR ? MODE_LINEAR : MODE_CTAS; }
 inline size_t store_bytes(int st) { return st == ST_F32 ? 4 : 2; }
 
-// Tile kinds: rows x cols of output per 256-thread workgroup. The two small
-// ones serve launches of CTAS sampling from float32 storage whose 64x64 tiles
-// would leave most of the chip idle; they are not among a caller's choices.
-enum TileKind { TK_AUTO = 0, TK_64x64 = 1, TK_128x64 = 2, TK_128x128 = 3, TK_32x32 = 4, TK_16x32 = 5 };
-inline int tile_rows(int kind) { return kind == TK_16x32 ? 16 : kind == TK_32x32 ? 32 : kind == TK_64x64 ? 64 : 128; }
-inline int tile_cols(int kind) { return kind >= TK_32x32 ? 32 : kind == TK_128x128 ? 128 : 64; }
-
 // ---- launchers (filter.hip, backproject.hip) ------------------------------
 // Zeros the pads around the filtered sinograms of the items (Item::pad).
 hipError_t launch_pad_zero(const Item *d_items, int n_items, hipStream_t s);
@@ -280,6 +274,7 @@ struct ctas_fbp {
 
   int tile_kind = ctas::TK_AUTO;
   int angles_per_pass = 0;
+  int tuning_ac = 0;           // while the autotuner times the handle's own launches: their pass length
 
   // The captured graph: its item table (and the host's copy), which no later
   // call changes, and the workspaces that its kernels use. One of those that a

@@ -154,12 +154,18 @@ int ctas_fbp_graph_launch(ctas_fbp *h, void *stream);
  * synchronises the handle's stream. */
 int ctas_fbp_status(ctas_fbp *h, int S, int *status);
 
-/* Tile choice for this handle's width class: rows x cols of output per
- * workgroup and angles staged per LDS pass; 0 = let the autotuner decide. */
+/* Tiles of launches of one slice per workgroup: rows x cols of output per
+ * workgroup (1: 64x64, 2: 128x64, 3: 128x128) and angles staged per LDS pass
+ * (16 or 32); 0 = the engine's choice, the autotuner's where it found a faster
+ * one. While both are 0, slices of one centre share workgroups and launches of
+ * few tiles take smaller ones, with pass lengths of their own; a kind or a pass
+ * length set here is kept for every slice, one slice per workgroup.
+ * ctas_fbp_get_tiles returns the kind and pass length of one-slice launches. */
 int ctas_fbp_set_tiles(ctas_fbp *h, int tile_kind, int angles_per_pass);
 int ctas_fbp_get_tiles(const ctas_fbp *h, int *tile_kind, int *angles_per_pass);
-/* Time the candidate tiles on the current device for this handle's shape
- * and keep the fastest (cached per width class in the process). */
+/* Time the candidate tiles on the current device for this handle's shape, and
+ * the launches that the handle takes by itself, and keep the fastest (cached per
+ * width class in the process). */
 int ctas_fbp_autotune(ctas_fbp *h, int S);
 
 /* ---- uneven batches in one launch ------------------------------------- */
