@@ -705,7 +705,8 @@ extern "C" int ctas_raxis(const float *sino, int N, int w, float anarc, float ma
   if (!best_at) {
     const int idx = scores[0] < scores[n_trials - 1] ? 0 : n_trials - 1;
     dir = idx == 0 ? -1 : 1;
-    const int walk_from = static_cast<int>(offsets[idx - dir * 2]);
+    // two grid points back; beyond the sweep where that has one or two trials
+    const int walk_from = static_cast<int>(seed_offset + static_cast<float>(kStep * (idx - dir * 2 - half)));
     const int walk_limit = static_cast<int>(static_cast<float>(w) * kShiftLimit - static_cast<float>(dir * walk_from / kStep));
     if (walk_limit <= 0) return fail(CTAS_E_AXIS, "Impossible number of n_trials.");
     std::vector<float> walk_offsets, walk_scores;

@@ -821,7 +821,8 @@ int orc_raxis(const float *sino, int N, int w, float anarc, float maxDev, int al
     if (!idxM) {
       const int idx = (err[0] < err[steps - 1]) ? 0 : steps - 1;
       cdir = (idx == 0) ? -1 : 1;
-      const int coff2 = (int)vax[idx - cdir * 2];
+      /* vax[idx - 2 cdir]; beyond the sweep where that has one or two trials */
+      const int coff2 = (int)(coffee + (float)(stpsz * (idx - cdir * 2 - hfsteps)));
       const int maxSteps = (int)((float)w * maxDevLM - (float)(cdir * coff2 / stpsz));
       if (maxSteps <= 0) { rc = -10; goto out; }
       free(vax);
