@@ -86,7 +86,7 @@ __device__ __forceinline__ float4 smooth4(const float *src, int st, const Taps &
 // into LDS once; smoothing along rows, along columns and the derivatives
 // follow there, four outputs per thread in the smoothing so that each LDS read
 // serves up to four taps. Bound by LDS reads: nine slices of 2048 px, 8
-// taps, 165 us (628 in three passes over memory).
+// taps, 148 us (628 in three passes over memory).
 __global__ __launch_bounds__(256) void score_kernel(const float *__restrict__ slices, const float *__restrict__ centres,
                                                     int w, int tiles_x, Taps taps, double *__restrict__ partial) {
   extern __shared__ __align__(16) float score_buf[];

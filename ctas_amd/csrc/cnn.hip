@@ -7,13 +7,19 @@
 // 2x180x256, then a 11264->16 fully connected layer with leaky ReLU and a
 // 16->2 output (offset in
 // downsampled detector bins, confidence logit). Activations and weights are
-// bfloat16; every product runs on the matrix cores (v_mfma_f32_16x16x32_bf16,
-// float32 accumulation) through one implicit-GEMM kernel whose operands are
-// gathered by small functors: convolution forward (W x im2col(x)), backward
-// data (W^T x col(g) with the mirrored stencil), backward weights
-// (g x im2col(x)^T, split over the pixel dimension and reduced in a fixed
-// order) and the fully connected layers. Training is Adam on float32 master
-// weights; the bfloat16 copies feed the next step.
+// bfloat16; every product of the convolutions and of the first fully connected
+// layer runs on the matrix cores (v_mfma_f32_16x16x32_bf16, float32
+// accumulation), sums that are split over workgroups reduced in a fixed order:
+// * conv_kernel: a convolution forward, with its pooling, or (the stencil
+//   mirrored, the weights transposed) the gradient of its input, from a patch
+//   of the input in LDS;
+// * wgrad_kernel, and wgrad_taps_kernel for the first layer: the weight
+//   gradients, split over the pixels;
+// * gemm_kernel, whose operands small functors gather: the first fully
+//   connected layer, forward and backward.
+// head_kernel ends the forward pass, loss_kernel begins the backward one.
+// Training is Adam on float32 master weights; the bfloat16 copies feed the next
+// step.
 //
 // Training data are made by the engine: seeded ellipse phantoms (plus small
 // dense inclusions) projected analytically on the GPU with photon noise,
@@ -233,9 +239,10 @@ __device__ __forceinline__ uint32_t pool_code(uint16_t a, uint16_t b, uint16_t c
 // other pixel gets zero, rows beyond the pooled extent too); part[b][co]
 // receives its sum before rounding. A thread takes four windows: one read of
 // their codes, one of dy, two writes. Bound by HBM, whose bytes are the
-// writes and half as many reads: 20 us a layer on average for 64 samples, 51
-// for the first (31 from activations of full size, which the forward pass then
-// has to write; 158 with the gradient in float32 and its bias sums apart).
+// writes and half as many reads. Layers two to four (the first forms its
+// gradient in wgrad_taps_kernel): 14, 9 and 6 us for 64 samples (10 a layer on
+// average; 158 with the gradient in float32 and its bias sums apart, the first
+// layer's among them).
 __global__ __launch_bounds__(256) void pool_bwd(const uint8_t *__restrict__ code, const float *__restrict__ dy,
                                                 uint16_t *__restrict__ g, float *__restrict__ part, int C, int H,
                                                 int W) {
@@ -1013,7 +1020,7 @@ __global__ void to_bf16(const float *__restrict__ p, uint16_t *__restrict__ q, i
 // a block of 1024 takes the logarithms of a row coalesced into LDS, 4096
 // columns at a time, and the 256 owners add their columns from there. One
 // thread per cell, reading its columns from memory, took 13.5 us for 1800 x
-// 2048, bound by the logarithms of three waves per CU; this takes 8.9.
+// 2048, bound by the logarithms of three waves per CU; this takes 9 to 10.
 constexpr int kFeatCols = 4096, kFeatT = 1024;
 __global__ __launch_bounds__(kFeatT) void features_kernel(const float *__restrict__ sino, int N, int w,
                                                           float *__restrict__ tmp) {
