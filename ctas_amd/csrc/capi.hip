@@ -31,6 +31,8 @@ thread_local std::string g_last_error;
 void set_error(const std::string &msg) { g_last_error = msg; }
 int fail(int code, const std::string &msg) {
   g_last_error = msg;
+  // a refused allocation's error is reported here, not by the next launch too
+  if (code == CTAS_E_NOMEM) (void)hipGetLastError();
   return code;
 }
 
@@ -72,7 +74,9 @@ int ensure_filt(ctas_fbp *h, size_t bytes) {
     h->d_filt = nullptr;
     h->filt_cap = 0;
   }
-  return grow(h->d_filt, h->filt_cap, bytes);
+  const int rc = grow(h->d_filt, h->filt_cap, bytes);
+  if (rc) h->kept_slices = 0;  // those went with the buffer
+  return rc;
 }
 
 int ensure_slices(ctas_fbp *h, int S) {

@@ -1152,7 +1152,6 @@ namespace {
 int alloc(void **p, size_t bytes) {
   if (hipMalloc(p, std::max<size_t>(bytes, 256)) != hipSuccess) {
     *p = nullptr;
-    (void)hipGetLastError();  // else the next launch reports it
     return fail(CTAS_E_NOMEM, "CNN allocation of " + std::to_string(bytes) + " bytes failed");
   }
   return CTAS_OK;
